@@ -7,14 +7,19 @@ Tensors carry the reference's strides: a [m,k] and b [n,k] are transposed views 
 fp8 storage, a_scale [m,k/128] and b_scale [ceil(n/128),k/128] are transposed views of [QK][M] /
 [QK][QN] fp32 storage, c is contiguous bf16 [m,n]. PyTorch is used for device memory and streams only.
 There is no CPU or PyTorch fallback: a missing library or a non-GPU tensor raises.
+The calls of the hot path go through a native module (csrc/torch_binding.cpp), which checks the tensors and calls the C
+ABI; everything else goes through ctypes.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libgemm.so")
+BINDING_PATH = os.path.join(_HERE, "lib", "_torch_binding.so")
 _lib = None
 
 RF_OK = 0
@@ -118,56 +123,40 @@ def last_error():
     return lib().rf_gemm_last_error().decode()
 
 
-def _check_layout(a, b, a_scale, b_scale, c):
-    if not (a.is_cuda and b.is_cuda and a_scale.is_cuda and b_scale.is_cuda and c.is_cuda):
-        raise ValueError("fp8_mm needs GPU tensors")
-    m, k = a.shape
-    n = b.shape[0]
-    qk, qn = k // 128, (n + 127) // 128
-    if a.element_size() != 1 or b.element_size() != 1:
-        raise ValueError("a and b must be 1-byte fp8 (e4m3fn) tensors")
-    if b.shape[1] != k or tuple(a_scale.shape) != (m, qk) or tuple(b_scale.shape) != (qn, qk) or tuple(c.shape) != (m, n):
-        raise ValueError("inconsistent shapes")
-    if a_scale.dtype != torch.float32 or b_scale.dtype != torch.float32 or c.dtype != torch.bfloat16:
-        raise ValueError("scales must be fp32 and c bf16")
-    # the launcher reads [K][M], [K][N], [QK][M], [QK][QN] storage: the tensors must be transposed views of that
-    def colmajor(t):
-        r, cdim = t.shape
-        return (t.stride(0) == 1 or r == 1) and (t.stride(1) == r or cdim == 1)
-    if not (colmajor(a) and colmajor(b) and colmajor(a_scale) and colmajor(b_scale) and c.is_contiguous()):
-        raise ValueError("a, b, a_scale, b_scale must be column-major (transposed views), c row-major contiguous")
-    return m, n, k
+class _Binding:
+    """The native module, loaded at the first use of one of its functions (which then replaces this stand-in)."""
+
+    def __getattr__(self, name):
+        global _native
+        if not os.path.exists(BINDING_PATH):
+            raise RuntimeError("_torch_binding.so is missing at %s: build it with `python -m radeonflow_kernels_amd.build`"
+                               % BINDING_PATH)
+        lib()
+        loader = importlib.machinery.ExtensionFileLoader("_torch_binding", BINDING_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_binding", loader))
+        loader.exec_module(module)
+        _native = module
+        return getattr(module, name)
+
+
+_native = _Binding()
 
 
 def fp8_mm(a, b, a_scale, b_scale, c, config=None):
     """c[m,n] = bf16(sum_kb a_scale*b_scale * (A_kb . B_kb^T)) on the current HIP stream; returns None."""
-    m, n, k = _check_layout(a, b, a_scale, b_scale, c)
-    stream = ctypes.c_void_p(torch.cuda.current_stream(a.device).cuda_stream)
-    L = lib()
-    cfg = ctypes.byref(config) if config is not None else None
-    with torch.cuda.device(a.device):
-        rc = L.rf_fp8_gemm_ex(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr(),
-                              m, n, k, cfg, stream)
-    if rc != RF_OK:
-        raise RuntimeError("rf_fp8_gemm failed (%d): %s" % (rc, last_error()))
+    _native.fp8_mm(a, b, a_scale, b_scale, c, 0 if config is None else ctypes.addressof(config))
 
 
 def fp8_mm_static(a, b, a_scale, b_scale, c):
     """fp8_mm through rf_fp8_gemm_static: same result, no device memory is allocated or freed by the call (temporary
     data lives in a static 32 MiB device array; shapes that need more raise)."""
-    m, n, k = _check_layout(a, b, a_scale, b_scale, c)
-    stream = ctypes.c_void_p(torch.cuda.current_stream(a.device).cuda_stream)
-    with torch.cuda.device(a.device):
-        rc = lib().rf_fp8_gemm_static(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr(),
-                                      m, n, k, stream)
-    if rc != RF_OK:
-        raise RuntimeError("rf_fp8_gemm_static failed (%d): %s" % (rc, last_error()))
+    _native.fp8_mm_static(a, b, a_scale, b_scale, c)
 
 
 def fp8_mm_time(a, b, a_scale, b_scale, c, config=None, warmup=3, iters=20):
     """Average microseconds per launch of fp8_mm over `iters` back-to-back launches timed inside the library (no
     per-launch Python overhead, which exceeds the GPU time of small shapes)."""
-    m, n, k = _check_layout(a, b, a_scale, b_scale, c)
+    m, n, k = _native.check_operands(a, b, a_scale, b_scale, c)
     stream = ctypes.c_void_p(torch.cuda.current_stream(a.device).cuda_stream)
     us = ctypes.c_float(0.0)
     cfg = ctypes.byref(config) if config is not None else None
@@ -185,25 +174,7 @@ def fp8_mm_grouped(a, b, a_scale, b_scale, c, row_offsets, variant=-1):
       a [M_total, K] fp8 stride (1, M_total); a_scale [M_total, K/128] fp32 stride (1, M_total);
       b [G, N, K] fp8 stride (K*N, 1, N); b_scale [G, ceil(N/128), K/128] fp32 stride (QK*QN, 1, QN);
       c [M_total, N] bf16 contiguous; row_offsets: sequence of G+1 ints on the host."""
-    m_total, k = a.shape
-    groups, n, _ = b.shape
-    qk, qn = k // 128, (n + 127) // 128
-    ok = (a.dtype == torch.float8_e4m3fn and b.dtype == torch.float8_e4m3fn and c.dtype == torch.bfloat16
-          and a_scale.dtype == torch.float32 and b_scale.dtype == torch.float32
-          and tuple(b.shape) == (groups, n, k) and tuple(c.shape) == (m_total, n) and c.is_contiguous()
-          and (m_total <= 1 or k == 1 or a.stride() == (1, m_total)) and tuple(a_scale.shape) == (m_total, qk)
-          and (m_total <= 1 or qk == 1 or a_scale.stride() == (1, m_total))
-          and (b.stride() == (k * n, 1, n) or (groups == 1 and b.stride()[1:] == (1, n))) and tuple(b_scale.shape) == (groups, qn, qk)
-          and (b_scale.stride() == (qk * qn, 1, qn) or qn == 1 or qk == 1 or (groups == 1 and b_scale.stride()[1:] == (1, qn))) and len(row_offsets) == groups + 1)
-    if not ok:
-        raise ValueError("fp8_mm_grouped: operands do not have the documented dtypes / shapes / strides")
-    offs = (ctypes.c_int32 * (groups + 1))(*[int(x) for x in row_offsets])
-    stream = ctypes.c_void_p(torch.cuda.current_stream(a.device).cuda_stream)
-    with torch.cuda.device(a.device):
-        rc = lib().rf_fp8_gemm_grouped(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr(),
-                                       offs, groups, n, k, variant, stream)
-    if rc != RF_OK:
-        raise RuntimeError("rf_fp8_gemm_grouped failed (%d): %s" % (rc, last_error()))
+    _native.fp8_mm_grouped(a, b, a_scale, b_scale, c, row_offsets, variant)
 
 
 def grouped_variant_for(row_offsets, n, k, num_cu=256):
@@ -234,48 +205,13 @@ def quantize_a_grouped(x, row_offsets):
     """Activations [M_total, K] (fp32 or bf16, contiguous, on the GPU) of groups that own rows row_offsets[g] ..
     row_offsets[g+1]-1 -> (a, a_scale) in the padded layout fp8_mm_grouped_padded takes: a [M_pad, K] stride (1, M_pad),
     a_scale [M_pad, K/128] stride (1, M_pad); padding rows hold zeros with scale 1."""
-    if x.dim() != 2 or not x.is_contiguous() or x.dtype not in (torch.float32, torch.bfloat16):
-        raise ValueError("source must be a contiguous 2-D fp32 or bf16 tensor [rows, K]")
-    rows, k = x.shape
-    if k < 128 or k % 128 or int(row_offsets[-1]) != rows:
-        raise ValueError("K must be a positive multiple of 128 and row_offsets must end at the number of rows")
-    groups = len(row_offsets) - 1
-    m_pad = grouped_padded_offsets(row_offsets)[-1]
-    a = torch.empty((k, m_pad), dtype=torch.float8_e4m3fn, device=x.device)
-    a_scale = torch.empty((k // 128, m_pad), dtype=torch.float32, device=x.device)
-    offs = (ctypes.c_int32 * (groups + 1))(*[int(v) for v in row_offsets])
-    name = "rf_quantize_a_grouped_%s" % ("f32" if x.dtype == torch.float32 else "bf16")
-    stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-    with torch.cuda.device(x.device):
-        rc = getattr(lib(), name)(x.data_ptr(), offs, groups, k, a.data_ptr(), a_scale.data_ptr(), stream)
-    if rc != RF_OK:
-        raise RuntimeError("%s failed (%d): %s" % (name, rc, last_error()))
-    return a.T, a_scale.T
+    return _native.quantize_a_grouped(x, row_offsets)
 
 
 def fp8_mm_grouped_padded(a, b, a_scale, b_scale, c, row_offsets, variant=-1):
     """fp8_mm_grouped on activations already in the padded layout (quantize_a_grouped): a [M_pad, K] stride (1, M_pad),
     a_scale [M_pad, K/128] stride (1, M_pad); b, b_scale, c and row_offsets as for fp8_mm_grouped."""
-    m_pad, k = a.shape
-    groups, n, _ = b.shape
-    qk, qn = k // 128, (n + 127) // 128
-    m_total = int(row_offsets[-1])
-    ok = (a.dtype == torch.float8_e4m3fn and b.dtype == torch.float8_e4m3fn and c.dtype == torch.bfloat16
-          and a_scale.dtype == torch.float32 and b_scale.dtype == torch.float32 and len(row_offsets) == groups + 1
-          and m_pad == grouped_padded_offsets(row_offsets)[-1] and a.stride() == (1, m_pad)
-          and tuple(a_scale.shape) == (m_pad, qk) and (qk == 1 or a_scale.stride() == (1, m_pad))
-          and tuple(b.shape) == (groups, n, k) and (b.stride() == (k * n, 1, n) or (groups == 1 and b.stride()[1:] == (1, n)))
-          and tuple(b_scale.shape) == (groups, qn, qk) and (b_scale.stride() == (qk * qn, 1, qn) or qn == 1 or qk == 1 or (groups == 1 and b_scale.stride()[1:] == (1, qn)))
-          and tuple(c.shape) == (m_total, n) and c.is_contiguous())
-    if not ok:
-        raise ValueError("fp8_mm_grouped_padded: operands do not have the documented dtypes / shapes / strides")
-    offs = (ctypes.c_int32 * (groups + 1))(*[int(x) for x in row_offsets])
-    stream = ctypes.c_void_p(torch.cuda.current_stream(a.device).cuda_stream)
-    with torch.cuda.device(a.device):
-        rc = lib().rf_fp8_gemm_grouped_padded(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(),
-                                              c.data_ptr(), offs, groups, n, k, variant, stream)
-    if rc != RF_OK:
-        raise RuntimeError("rf_fp8_gemm_grouped_padded failed (%d): %s" % (rc, last_error()))
+    _native.fp8_mm_grouped_padded(a, b, a_scale, b_scale, c, row_offsets, variant)
 
 
 def custom_kernel(data):
@@ -287,7 +223,7 @@ def custom_kernel(data):
 
 def run_with_metrics(a, b, a_scale, b_scale, c):
     """Calls the drop-in `run` entry with a PerfMetrics record; returns (time_ms, gflops) after a sync."""
-    m, n, k = _check_layout(a, b, a_scale, b_scale, c)
+    m, n, k = _native.check_operands(a, b, a_scale, b_scale, c)
     pm = PerfMetrics()
     stream = ctypes.c_void_p(torch.cuda.current_stream(a.device).cuda_stream)
     with torch.cuda.device(a.device):
@@ -295,24 +231,6 @@ def run_with_metrics(a, b, a_scale, b_scale, c):
                   ctypes.byref(pm), stream)
         torch.cuda.synchronize(a.device)
     return pm.entries[0].time, pm.entries[0].gflops, pm.count
-
-
-def _quantize(x, per_row):
-    if x.dim() != 2 or not x.is_contiguous() or x.dtype not in (torch.float32, torch.bfloat16):
-        raise ValueError("source must be a contiguous 2-D fp32 or bf16 tensor [rows, K]")
-    rows, k = x.shape
-    if k < 128 or k % 128:
-        raise ValueError("K must be a positive multiple of 128")
-    q = torch.empty((k, rows), dtype=torch.float8_e4m3fn, device=x.device)
-    nscale = rows if per_row else (rows + 127) // 128
-    scales = torch.empty((k // 128, nscale), dtype=torch.float32, device=x.device)
-    name = "rf_quantize_%s_%s" % ("a" if per_row else "b", "f32" if x.dtype == torch.float32 else "bf16")
-    stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-    with torch.cuda.device(x.device):
-        rc = getattr(lib(), name)(x.data_ptr(), rows, k, q.data_ptr(), scales.data_ptr(), stream)
-    if rc != RF_OK:
-        raise RuntimeError("%s failed (%d): %s" % (name, rc, last_error()))
-    return q.T, scales.T         # the transposed views fp8_mm takes: [rows, K] stride (1, rows), [rows or QN, K/128]
 
 
 def cast_to_e4m3fn(x):
@@ -331,12 +249,12 @@ def cast_to_e4m3fn(x):
 def quantize_a(x):
     """Activations [M, K] (fp32 or bf16, on the GPU) -> (a, a_scale) as fp8_mm takes them: one scale per
     (row, 128-wide K block), scale = amax/448, value = e4m3fn_rne(x / scale)."""
-    return _quantize(x, True)
+    return _native.quantize(x, True)
 
 
 def quantize_b(w):
     """Weights [N, K] -> (b, b_scale): one scale per 128x128 block."""
-    return _quantize(w, False)
+    return _native.quantize(w, False)
 
 
 def select_config(m, n, k):
