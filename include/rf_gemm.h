@@ -10,11 +10,13 @@
  *   bs  fp32,             [K/128][ceil(N/128)]
  *   c   bf16,             [M][N] row-major, fully overwritten
  * All pointers are device pointers. K must be a positive multiple of 128; M, N >= 1.
- * Shapes with M%16==0, N%16==0 and 16-byte aligned a/b/c take the tiled MFMA path as they are. Anything else is
- * staged: the operands that need it are copied with rows padded to a multiple of 16 (zeros) into an internal buffer
+ * Shapes with M%16==0, N%16==0 and 16-byte aligned a/b/c take the tiled MFMA path as they are. Anything else goes to
+ * the few-rows kernels, which take any shape and alignment, where M is small (up to a few hundred rows, whichever is
+ * estimated to be faster), and is staged otherwise: the operands that need it are copied with rows padded to a multiple of 16 (zeros) into an internal buffer
  * grown on demand, the tiled path runs on the padded shape, and c receives the result without the padding (cost: one
- * pass over a; when N is ragged or c unaligned also one over b and a staged copy of c). Problems below 2^21 multiply-adds, and explicit plans with
- * variant = -1, take a bounds-checked kernel instead (the role of the reference's legacy kernel,
+ * pass over a; when N is ragged or c unaligned also one over b and a staged copy of c). Such problems
+ * below 2^21 multiply-adds always take the few-rows kernels (their plan is reported as variant = -1); explicit plans with
+ * variant = -1 take a bounds-checked kernel (the role of the reference's legacy kernel,
  * src/gemm/gemm_kernel_legacy.cpp:237-374).
  * Temporary device memory (split-K partial sums, staging copies, stream-K counters) is kept per (device, stream), for
  * the device that is current at the call: launches on different streams of one device may overlap, launches on one
@@ -56,7 +58,9 @@ enum { RF_SCHEDULE_TILES = 0, RF_SCHEDULE_STREAM_K = 1, RF_SCHEDULE_PERSISTENT =
 /* One launch plan: which kernel variant and how K is split.
  * Replaces a DISPATCH_GEMM(...) line of the reference (src/gemm/gemm_launcher.cpp:158-162,229-259). */
 typedef struct rf_gemm_config {
-    int variant;      /* index into the variant table, see rf_gemm_variant_info(); -1 = bounds-checked kernel */
+    int variant;      /* index into the variant table, see rf_gemm_variant_info(); -1 = bounds-checked kernel. Variants 14
+                         to 20 are the few-rows kernels (16 to 64 rows x 32 to 128 columns per workgroup): any shape with
+                         M and N below 2^25, any alignment, K splits summed inside the launch */
     int split_k;      /* >= 1; K blocks are divided over this many partial sums */
     int group_m;      /* tile-order grouping along M for L2 reuse (>=1) */
     int stream_k;     /* schedule, one of RF_SCHEDULE_*:

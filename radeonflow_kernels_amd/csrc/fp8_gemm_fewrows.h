@@ -1,0 +1,294 @@
+// Few-rows form of the block-scaled fp8 GEMM: M up to a few dozen rows, any M and N, operands at any alignment.
+//
+// A decode step multiplies a handful of rows by a whole weight matrix: the launch is the streaming of B (N * K bytes), and
+// at 5 to 130 KB of it per compute unit what counts is how soon all of it has been asked for and how little follows.
+//   * a workgroup owns a strip of 32 to 128 columns and the K range of its split; its waves take K blocks in turn, so K is
+//     split between the waves as well: each wave streams its own K blocks with no barrier, and one exchange through LDS at
+//     the end adds the waves' sums in wave order;
+//   * loads go to registers (16 bytes a lane; a wave asks for up to DEPTH K blocks, 6 to 20 KB each, before it uses the
+//     first), then through a private LDS region of the wave, from which the transpose reads take MFMA fragments. Loads
+//     into registers may start at any byte, which LDS-DMA may not: a row of A is M bytes ([K][M]) and is fetched as
+//     16-byte pieces whatever M is; pieces that reach past M bring bytes of the next K row, whose results belong to rows
+//     of C that do not exist and are not stored. So nothing is staged or padded for any M or N;
+//   * pieces of the matrix's last K rows could reach past its end: every load's offset is cut to the last 16 bytes of the
+//     matrix, and in its last K block the bytes are shifted back into place;
+//   * SPLIT: the workgroups of a strip hand their sums over in memory, and the one that arrives last adds them in split
+//     order and writes C. Nobody waits. With 2 to 16 KB per workgroup this chain (write-through store, counter, read
+//     back) is a microsecond shorter than a second kernel and spares its launch (32 x 1536 x 7168: 8.7 -> 7.6 us), unlike
+//     for the 98 KB tiles of the tiled kernels.
+// Measured with operand sets that rotate out of L2, M x N x K, best tiled plan (with its staging, where M or N is ragged) ->
+// here: 1 x 7168 x 2048 11.5 -> 6.2 us, 16 x 7168 x 2048 9.2 -> 6.2, 7 x 3072 x 1536 10.1 -> 3.7, 1 x 1536 x 7168 12.4 -> 6.9,
+// 32 x 1536 x 7168 8.7 -> 7.5, 16 x 4608 x 7168 11.2 -> 10.1 (33 MB of weights: 5.1 TB/s beyond the 3.5 us of launch and
+// hand-over), 64 x 5003 x 2048 23.4 -> 8.2. What is left is launch, one or two trips to memory and the hand-over.
+// Numerics are those of the tiled kernels: per K block the products are summed inside the MFMA from zero and folded with
+// acc = fma(a_scale * b_scale, partial, acc); a wave's K blocks in order, then the waves in order, then the splits in
+// order, one bf16 rounding.
+#pragma once
+#include "fp8_gemm_kernels.h"
+
+namespace rf {
+
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1), may_alias));
+typedef uint32_t u32x4_lds __attribute__((ext_vector_type(4), may_alias));
+
+// TM 16-row tiles of A (and of C) per workgroup, TN 16-column tiles, NW waves, DEPTH K blocks asked for at a time.
+template <int TM_, int TN_, int NW_, int DEPTH_>
+struct FewRowsGeom {
+    static constexpr int TM = TM_, TN = TN_, NW = NW_, DEPTH = DEPTH_;
+    static constexpr int BM = 16 * TM, BN = 16 * TN;
+    static constexpr int REGION = BK * (BM + BN);                     // one K block of A and of B, private to a wave
+    static constexpr int EXCHANGE = NW * TM * TN * 1024;              // the waves' sums, over the regions
+    static constexpr int LDS_BYTES = NW * REGION > EXCHANGE ? NW * REGION : EXCHANGE;
+    static_assert(LDS_BYTES <= 160 * 1024, "the waves' regions fit the CU's LDS");
+    static_assert((TM & (TM - 1)) == 0 && (TN & (TN - 1)) == 0, "powers of two: the chunk swizzle stays inside a row");
+};
+
+// Byte offset of 16-byte chunk c of row k in a region whose rows are 16 * T bytes. The 32 lanes the LDS serves together
+// in a transpose read point at 8 rows of two 32-row groups; rows of one chunk are spread by moving every second
+// 32-row group by 8 rows (128 bytes), wider rows by the chunk swizzle of the tiled kernels.
+template <int T>
+__device__ __forceinline__ uint32_t fewrows_at(int k, int c) {
+    if constexpr (T == 1) return (uint32_t)((k ^ (((k >> 5) & 1) << 3)) << 4);
+    else return (uint32_t)(k * 16 * T + ((c ^ swizzle_of_row<16 * T>(k)) << 4));
+}
+
+// 16 bytes from base + off of a matrix that ends at base + end (end >= 16): past the end the bytes are undefined but
+// nothing is read there. SHIFT false: the caller knows that off + 16 <= end.
+template <bool SHIFT>
+__device__ __forceinline__ u32x4_lds load16(const uint8_t *base, uint32_t off, uint32_t end) {
+    if constexpr (!SHIFT) return *(const u32x4_any *)(base + off);
+    const uint32_t at = off < end - 16 ? off : end - 16;
+    return *(const u32x4_any *)(base + at);
+}
+// Moves the bytes of a cut load back to where they would have been.
+__device__ __forceinline__ u32x4_lds shift_back(u32x4_lds v, uint32_t off, uint32_t end) {
+    const uint32_t d = off < end - 16 ? 0 : off - (end - 16);         // 16 and more: every byte is past the end
+    const uint32_t x0 = d & 8 ? v[2] : v[0], x1 = d & 8 ? v[3] : v[1];
+    const uint32_t y0 = d & 4 ? x1 : x0, y1 = d & 4 ? (d & 8 ? 0 : v[2]) : x1, y2 = d & 4 ? v[3] : v[2], y3 = v[3];
+    u32x4_lds r;
+    r[0] = __builtin_amdgcn_alignbyte(y1, y0, d & 3);
+    r[1] = __builtin_amdgcn_alignbyte(y2, y1, d & 3);
+    r[2] = __builtin_amdgcn_alignbyte(y3, y2, d & 3);
+    r[3] = __builtin_amdgcn_alignbyte(0, y3, d & 3);
+    return r;
+}
+
+// Grid: x = column strips * row blocks (row blocks innermost: they share the strip's B), y = K splits of kb_per_split
+// blocks, every split at least one. A [K][ldm] (M of the ldm columns belong to this problem), SA [K/128][ldm], B [K][N],
+// C [M][N]. Any M, N >= 1, any alignment of A, B and C; ldm and N below 2^25 (32-bit offsets inside a K block). BYTES
+// false needs N % 16 == 0 and a 16-byte aligned B. SPLIT (gridDim.y > 1): counters holds a zero per item (gridDim.x) and
+// is zero again afterwards, slots gridDim.x * gridDim.y * TM * TN KiB, 16-byte aligned.
+template <int TM, int TN, int NW, int DEPTH, bool SPLIT, bool BYTES>
+__global__ __launch_bounds__(NW * 64) void gemm_fp8_blockscale_fewrows(
+    const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
+    const float *__restrict__ SB, uint16_t *__restrict__ C, int M, int ldm, int N, int K, int kb_per_split, int row_blocks,
+    unsigned *__restrict__ counters, float *__restrict__ slots) {
+    using G = FewRowsGeom<TM, TN, NW, DEPTH>;
+    constexpr int NLA = 2 * TM, NLB = 2 * TN;                         // 16-byte loads per lane and K block
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int L = lane & 15, g = lane >> 4;
+    // neighbouring strips on one XCD: a 32-column piece of a row of B is a quarter of a cache line
+    const int xcd = blockIdx.x % NUM_XCD, idx = blockIdx.x / NUM_XCD, per = gridDim.x / NUM_XCD, rem = gridDim.x % NUM_XCD;
+    const int item = xcd * per + (xcd < rem ? xcd : rem) + idx;
+    const int n0 = item / row_blocks * G::BN, m0 = item % row_blocks * G::BM;
+    const int QK = K / BK, QN = (N + 127) / 128;
+    const int kb_begin = blockIdx.y * kb_per_split, kb_end = kb_begin + kb_per_split < QK ? kb_begin + kb_per_split : QK;
+    const int count = (kb_end - kb_begin - wave + NW - 1) / NW;       // this wave's K blocks: kb_begin + wave + NW * i
+    uint8_t *region = lds + wave * G::REGION;
+
+    // Load i of a lane: 16-byte chunk lane % T of K row lane / T + i * 64 / T of the block
+    uint32_t off_a0, off_b0;
+    {
+        int m = m0 + 16 * (lane % TM), n = n0 + 16 * (lane % TN);
+        if (m >= M) m = m0;                                           // a whole chunk past M or N: any bytes will do
+        if (n >= N) n = n0;
+        off_a0 = (uint32_t)(lane / TM) * (uint32_t)ldm + (uint32_t)m;
+        off_b0 = (uint32_t)(lane / TN) * (uint32_t)N + (uint32_t)n;
+    }
+    auto off_a = [&](int i) { return off_a0 + (uint32_t)(i * (64 / TM)) * (uint32_t)ldm; };
+    auto off_b = [&](int i) { return off_b0 + (uint32_t)(i * (64 / TN)) * (uint32_t)N; };
+    auto dst_a = [&](int i) { return fewrows_at<TM>(lane / TM + i * (64 / TM), lane % TM); };
+    auto dst_b = [&](int i) { return BK * G::BM + fewrows_at<TN>(lane / TN + i * (64 / TN), lane % TN); };
+    const int nb = n0 >> 7;
+    static_assert(128 % G::BN == 0, "a strip lies in one b_scale block");
+    int row_s[TM];
+#pragma unroll
+    for (int j = 0; j < TM; j++) row_s[j] = m0 + 16 * j + L < M ? m0 + 16 * j + L : M - 1;
+
+    // One K block on its way: raw bytes of A and B, scales. Bytes from the K block's first row to the end of the matrix
+    // are needed to cut the loads of the last rows (below 2^32 always suffices: a K block's own offsets are).
+    struct Block {
+        u32x4_lds a[NLA], b[NLB];
+        float sa[TM], sb;
+    };
+    auto rest = [&](int kb, int ld) -> uint32_t {
+        const unsigned long long r = (unsigned long long)(K - kb * BK) * (unsigned)ld;
+        return r < 0xffffffffull ? (uint32_t)r : 0xffffffffu;
+    };
+    auto fetch = [&](Block &x, int i) {
+        const int kb = kb_begin + wave + NW * i;
+        const uint8_t *pb = B + (size_t)kb * BK * N, *pa = A + (size_t)kb * BK * ldm;
+        const uint32_t end_b = rest(kb, N), end_a = rest(kb, ldm);
+#pragma unroll
+        for (int q = 0; q < NLB; q++) x.b[q] = load16<BYTES>(pb, off_b(q), end_b);
+#pragma unroll
+        for (int q = 0; q < NLA; q++) x.a[q] = load16<true>(pa, off_a(q), end_a);
+#pragma unroll
+        for (int j = 0; j < TM; j++) x.sa[j] = SA[(size_t)kb * ldm + row_s[j]];
+        x.sb = SB[(size_t)kb * QN + nb];
+    };
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int j = 0; j < TM; j++)
+#pragma unroll
+        for (int i = 0; i < TN; i++) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int krow = 32 * g + (L >> 1);
+    auto fragment = [&](uint32_t at, int pitch) {                     // four transpose reads, 8 rows apart
+        i32x8 f;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const i32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((RF_LDS i32x2 *)(region + at + t * 8 * pitch));
+            f[2 * t] = v[0];
+            f[2 * t + 1] = v[1];
+        }
+        return f;
+    };
+    // rows 8 t further on lie at a fixed distance except in regions of one-chunk rows, whose every second 32-row group
+    // is moved by 8 rows: row ^ 8 there
+    auto fragment_1 = [&](uint32_t base) {
+        i32x8 f;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const i32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                (RF_LDS i32x2 *)(region + base + fewrows_at<1>(krow + 8 * t, 0) + 8 * (L & 1)));
+            f[2 * t] = v[0];
+            f[2 * t + 1] = v[1];
+        }
+        return f;
+    };
+    auto consume = [&](Block &x, int i) {
+        const int kb = kb_begin + wave + NW * i;
+        if (kb == QK - 1) {                                           // only the matrix's last rows have cut loads
+            const uint32_t end_b = rest(kb, N), end_a = rest(kb, ldm);
+            if constexpr (BYTES)
+#pragma unroll
+                for (int q = 0; q < NLB; q++) x.b[q] = shift_back(x.b[q], off_b(q), end_b);
+#pragma unroll
+            for (int q = 0; q < NLA; q++) x.a[q] = shift_back(x.a[q], off_a(q), end_a);
+        }
+#pragma unroll
+        for (int q = 0; q < NLB; q++) *(u32x4_lds *)(region + dst_b(q)) = x.b[q];
+#pragma unroll
+        for (int q = 0; q < NLA; q++) *(u32x4_lds *)(region + dst_a(q)) = x.a[q];
+        i32x8 bf[TN], af[TM];
+#pragma unroll
+        for (int c = 0; c < TN; c++)
+            bf[c] = TN == 1 ? fragment_1(BK * G::BM) : fragment(BK * G::BM + fewrows_at<TN>(krow, c) + 8 * (L & 1), G::BN);
+#pragma unroll
+        for (int c = 0; c < TM; c++)
+            af[c] = TM == 1 ? fragment_1(0) : fragment(fewrows_at<TM>(krow, c) + 8 * (L & 1), G::BM);
+#pragma unroll
+        for (int j = 0; j < TM; j++) {
+            const float s = x.sa[j] * x.sb;
+#pragma unroll
+            for (int c = 0; c < TN; c++) {
+                const f32x4 p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[c], af[j], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0,
+                                                                                 0, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[j][c][e] = __builtin_fmaf(s, p[e], acc[j][c][e]);
+            }
+        }
+    };
+
+    // up to DEPTH K blocks asked for, then used in order; straight-line code for every count, so that each wait is for a
+    // known number of younger loads
+    auto batch = [&](auto count_c, int i) {
+        constexpr int n = decltype(count_c)::value;
+        Block x[n];
+#pragma unroll
+        for (int d = 0; d < n; d++) fetch(x[d], i + d);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < n; d++) {
+            consume(x[d], i + d);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    static_assert(DEPTH >= 1 && DEPTH <= 4, "one to four K blocks at a time");
+    int i = 0;
+    for (; i + DEPTH <= count; i += DEPTH) batch(IntTag<DEPTH>{}, i);
+    if (DEPTH > 3 && count - i == 3) batch(IntTag<3>{}, i);
+    else if (DEPTH > 2 && count - i == 2) batch(IntTag<2>{}, i);
+    else if (DEPTH > 1 && count - i == 1) batch(IntTag<1>{}, i);
+
+    // the waves' sums through LDS, tile (j, c) of wave w at ((w * TM + j) * TN + c) * 1 KiB, lane l at + 16 l
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < TM; j++)
+#pragma unroll
+        for (int c = 0; c < TN; c++) *(f32x4 *)(lds + ((wave * TM + j) * TN + c) * 1024 + lane * 16) = acc[j][c];
+    __syncthreads();
+    auto store = [&](int t, const f32x4 &s) {                         // lane holds C[m][n .. n + 3] of tile t
+        const int m = m0 + 16 * (t / TN) + L, n = n0 + 16 * (t % TN) + 4 * g;
+        if (m >= M) return;
+        uint16_t *out = C + (size_t)m * N + n;
+        const uint32_t lo = pack_bf16x2(s[0], s[1]), hi = pack_bf16x2(s[2], s[3]);
+        if (n + 4 <= N && ((uintptr_t)out & 7) == 0) {
+            *(uint2 *)out = make_uint2(lo, hi);
+        } else {
+            if (n < N) out[0] = (uint16_t)lo;
+            if (n + 1 < N) out[1] = (uint16_t)(lo >> 16);
+            if (n + 2 < N) out[2] = (uint16_t)hi;
+            if (n + 3 < N) out[3] = (uint16_t)(hi >> 16);
+        }
+    };
+    const int splits = gridDim.y;
+    float *mine = slots + ((size_t)item * splits + blockIdx.y) * (TM * TN * 256) + lane * 4;
+    for (int t = wave; t < TM * TN; t += NW) {
+        f32x4 s = *(const f32x4 *)(lds + t * 1024 + lane * 16);
+#pragma unroll
+        for (int w = 1; w < NW; w++) {
+            const f32x4 v = *(const f32x4 *)(lds + (w * TM * TN + t) * 1024 + lane * 16);
+            s[0] += v[0]; s[1] += v[1]; s[2] += v[2]; s[3] += v[3];
+        }
+        if constexpr (SPLIT) {
+            // system scope: written through, so that the acknowledgement below means "where every XCD's loads look"
+            asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" :: "v"(mine + t * 256), "v"(s) : "memory");
+        } else {
+            store(t, s);
+        }
+    }
+    if constexpr (SPLIT) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        volatile unsigned *mailbox = (volatile unsigned *)lds;        // every wave has read the sums exchanged there
+        // wraps to zero at the last arrival: ready for the next launch
+        if (threadIdx.x == 0) *mailbox = atomicInc(counters + item, (unsigned)(splits - 1));
+        __syncthreads();
+        if (*mailbox != (unsigned)(splits - 1)) return;
+        const float *first = slots + (size_t)item * splits * (TM * TN * 256) + lane * 4;
+        for (int t = wave; t < TM * TN; t += NW) {
+            f32x4 s = {0.f, 0.f, 0.f, 0.f};
+            for (int q0 = 0; q0 < splits; q0 += 8) {
+                uint64_t v[8][2];
+#pragma unroll
+                for (int q = 0; q < 8; q++)
+                    if (q0 + q < splits) {
+                        const uint64_t *p = (const uint64_t *)(first + ((size_t)(q0 + q) * TM * TN + t) * 256);
+                        v[q][0] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        v[q][1] = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+#pragma unroll
+                for (int q = 0; q < 8; q++)
+                    if (q0 + q < splits) {
+                        const f32x2 lo = __builtin_bit_cast(f32x2, v[q][0]), hi = __builtin_bit_cast(f32x2, v[q][1]);
+                        s[0] += lo[0]; s[1] += lo[1]; s[2] += hi[0]; s[3] += hi[1];
+                    }
+            }
+            store(t, s);
+        }
+    }
+}
+
+}  // namespace rf

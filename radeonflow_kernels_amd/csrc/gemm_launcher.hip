@@ -19,6 +19,7 @@
 #include "fp8_gemm_kernels.h"
 #include "fp8_gemm_persistent.h"
 #include "fp8_gemm_skinny.h"
+#include "fp8_gemm_fewrows.h"
 #include "quantize_kernels.h"
 
 // Scratch memory of rf_fp8_gemm_static, the entry point that allocates nothing: split-K partial sums and staging
@@ -26,6 +27,10 @@
 // own address until the process ends; host code never uses this name as an address (see ensure_device_info).
 constexpr size_t kStaticScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) uint8_t scratch[kStaticScratchBytes];
+// and its arrival counters (few-rows kernels with a K split): zero when the library is loaded, and every launch that uses
+// them leaves them at zero
+constexpr int kMaxTileCounters = 16384;
+static __device__ unsigned scratch_counters[kMaxTileCounters];
 
 namespace {
 
@@ -49,6 +54,8 @@ typedef void (*streamk_kernel_t)(const uint8_t *, const uint8_t *, const float *
                                  int, int, int, int, unsigned *, float *);
 typedef void (*persistent_kernel_t)(const uint8_t *, const uint8_t *, const float *, const float *, uint16_t *, int, int,
                                     int, int, int, int, int);
+typedef void (*fewrows_kernel_t)(const uint8_t *, const uint8_t *, const float *, const float *, uint16_t *, int, int, int,
+                                 int, int, int, unsigned *, float *);
 struct Variant {
     int bm, bn, waves_m, waves_n, lds;
     tile_kernel_t direct, partial;
@@ -57,6 +64,8 @@ struct Variant {
     int lds_persistent;
     persistent_kernel_t persistent_half_tail = nullptr;   // null: no form that ends with half tiles
     int k_groups = 1;                    // > 1: wave groups of one workgroup split K between them (needs K/128 % k_groups == 0)
+    fewrows_kernel_t fewrows[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};   // [K split][any alignment of B]; null: a tiled variant
+    bool is_fewrows() const { return fewrows[0][0] != nullptr; }
     int lds_bytes() const { return lds; }
     int threads() const { return waves_m * waves_n * 64 * k_groups; }
 };
@@ -81,6 +90,14 @@ struct Variant {
     Variant { BM, BN, WM, WN, rf::TileGeom<BM, BN, WM, WN, 3>::LDS_BYTES,                  \
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, false, 3>,                      \
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true, 3>, nullptr, nullptr, 0 }
+// few-rows kernels (fp8_gemm_fewrows.h): any shape, any alignment, K splits reduced inside the launch
+#define RF_VARIANT_FEWROWS(TM, TN, NW, DEPTH)                                              \
+    Variant { 16 * TM, 16 * TN, 1, NW, rf::FewRowsGeom<TM, TN, NW, DEPTH>::LDS_BYTES,      \
+              nullptr, nullptr, nullptr, nullptr, 0, nullptr, 1,                           \
+              {{rf::gemm_fp8_blockscale_fewrows<TM, TN, NW, DEPTH, false, false>,          \
+                rf::gemm_fp8_blockscale_fewrows<TM, TN, NW, DEPTH, false, true>},          \
+               {rf::gemm_fp8_blockscale_fewrows<TM, TN, NW, DEPTH, true, false>,           \
+                rf::gemm_fp8_blockscale_fewrows<TM, TN, NW, DEPTH, true, true>}} }
 const Variant kVariants[] = {
     Variant{256, 256, 2, 4, rf::TileGeom<256, 256, 2, 4>::LDS_BYTES, rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, false>,
             rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, true>, rf::gemm_fp8_blockscale_streamk<256, 256, 2, 4>,
@@ -104,7 +121,15 @@ const Variant kVariants[] = {
     // 13: the 128 x 128 two-stage tile with K split between two wave groups (8 waves, 130 KiB LDS)
     Variant{128, 128, 2, 2, rf::InWgSplitGeom<128, 128, 2, 2, 2, 2>::LDS_BYTES,
             rf::gemm_fp8_blockscale_tile_ksplit_in_wg<128, 128, 2, 2, 2, 2>, nullptr, nullptr, nullptr, 0, nullptr, 2},
+    RF_VARIANT_FEWROWS(1, 2, 8, 3),   // 14: 16 rows x 32 columns
+    RF_VARIANT_FEWROWS(1, 4, 8, 2),   // 15: 16 x 64
+    RF_VARIANT_FEWROWS(1, 8, 8, 1),   // 16: 16 x 128
+    RF_VARIANT_FEWROWS(2, 2, 8, 2),   // 17: 32 x 32
+    RF_VARIANT_FEWROWS(2, 4, 8, 2),   // 18: 32 x 64
+    RF_VARIANT_FEWROWS(4, 2, 8, 2),   // 19: 64 x 32
+    RF_VARIANT_FEWROWS(4, 4, 8, 1),   // 20: 64 x 64
 };
+constexpr int kFewRows64x64 = 20;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
 // ---- process-wide state ---------------------------------------------------------------------
@@ -137,6 +162,7 @@ struct State {
     uint64_t tick = 0;
     bool attrs_set = false, grouped_attrs_set = false;
     int num_cu = 0;
+    unsigned *static_counters = nullptr; // this device's copy of the file-scope counters
     uint8_t *static_scratch = nullptr;   // this device's copy of the file-scope scratch array (rf_fp8_gemm_static)
     std::mutex ev_mu;                    // guards free_events only: the timing callback takes no other lock
     std::vector<std::pair<hipEvent_t, hipEvent_t>> free_events;
@@ -144,6 +170,7 @@ struct State {
 struct Shared {
     std::mutex mu;
     std::vector<TunedPlan> user_plans;   // rf_gemm_load_plans / RF_GEMM_PLANS: looked up before the built-in table
+    int plan_generation = 0;             // counts changes of user_plans
     bool env_plans_checked = false;
 };
 constexpr int kMaxDevices = 64;
@@ -198,6 +225,7 @@ int ensure_device_info(State &s) {
         if (const char *path = getenv("RF_GEMM_PLANS")) {
             int rc = parse_plans(path, shared().user_plans);
             if (rc != RF_OK) return rc;
+            shared().plan_generation++;
         }
         shared().env_plans_checked = true;
     }
@@ -209,7 +237,11 @@ int ensure_device_info(State &s) {
         return fail(RF_ERR_HIP, std::string("libgemm.so is built for gfx950 only, device is ") + prop.gcnArchName);
     s.num_cu = prop.multiProcessorCount;
     for (const Variant &v : kVariants) {
-        RF_HIP(hipFuncSetAttribute((const void *)v.direct, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
+        for (auto &pair : v.fewrows)
+            for (fewrows_kernel_t f : pair)
+                if (f) RF_HIP(hipFuncSetAttribute((const void *)f, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
+        if (v.direct)
+            RF_HIP(hipFuncSetAttribute((const void *)v.direct, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
         if (v.partial)
             RF_HIP(hipFuncSetAttribute((const void *)v.partial, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
         if (v.streamk)
@@ -233,11 +265,11 @@ int ensure_device_info(State &s) {
     void *scratch_ptr = nullptr;
     RF_HIP(hipGetSymbolAddress(&scratch_ptr, HIP_SYMBOL(scratch)));
     s.static_scratch = (uint8_t *)scratch_ptr;
+    RF_HIP(hipGetSymbolAddress(&scratch_ptr, HIP_SYMBOL(scratch_counters)));
+    s.static_counters = (unsigned *)scratch_ptr;
     s.attrs_set = true;
     return RF_OK;
 }
-
-constexpr int kMaxStreamKTiles = 16384;
 
 __global__ void zero_words(unsigned *p) { p[blockIdx.x * 256 + threadIdx.x] = 0u; }
 
@@ -311,10 +343,13 @@ struct Mem {
         return rc;
     }
     int tile_counters(unsigned **out) {
-        if (fixed) return fail(RF_ERR_BAD_CONFIG, "rf_fp8_gemm_static: the stream-K schedule is not available");
+        if (fixed) {
+            *out = s.static_counters;
+            return RF_OK;
+        }
         int rc = bind();
         if (rc != RF_OK) return rc;
-        if (!sb->tile_count) RF_HIP(device_malloc((void **)&sb->tile_count, kMaxStreamKTiles * sizeof(unsigned)));
+        if (!sb->tile_count) RF_HIP(device_malloc((void **)&sb->tile_count, kMaxTileCounters * sizeof(unsigned)));
         if (!sb->tile_count_zeroed) {
             // zeroed on the stream of the launch that follows (the kernels leave the counters at zero afterwards);
             // a kernel and not a memset, so that the call may be recorded into a HIP graph. A recorded fill has not
@@ -329,7 +364,7 @@ struct Mem {
             } else if (qe != hipSuccess) {
                 return fail(RF_ERR_HIP, std::string("hipStreamIsCapturing: ") + hipGetErrorString(qe));
             }
-            hipLaunchKernelGGL(zero_words, dim3(kMaxStreamKTiles / 256), dim3(256), 0, sb->stream, sb->tile_count);
+            hipLaunchKernelGGL(zero_words, dim3(kMaxTileCounters / 256), dim3(256), 0, sb->stream, sb->tile_count);
             RF_HIP(hipGetLastError());
             sb->tile_count_zeroed = st == hipStreamCaptureStatusNone;
         }
@@ -418,11 +453,14 @@ bool skinny_ok(int m, int n, int k) {
     return k >= rf::BK && k <= 4 * rf::BK && k % rf::BK == 0 && m >= 16 && m % 16 == 0 && n >= 64 && n % 64 == 0;
 }
 
+// Few-rows kernels keep offsets inside a K block in 32 bits.
+bool fewrows_ok(int ldm, int n) { return ldm < (1 << 25) && n < (1 << 25); }
+
 // Stream-K: at least one tile per workgroup (then a split tile has exactly two contributors, which is all the kernel
 // handles) and no more tiles than arrival counters.
 bool stream_k_ok(const Variant &v, int m, int n, int num_cu) {
     const long t = (long)ceil_div(m, v.bm) * ceil_div(n, v.bn);
-    return v.streamk && t >= num_cu && t <= kMaxStreamKTiles;
+    return v.streamk && t >= num_cu && t <= kMaxTileCounters;
 }
 
 // Plans measured on one MI355X by the tuner (python -m radeonflow_kernels_amd.tuner.gemm_tuner --all --emit).
@@ -435,16 +473,53 @@ const TunedPlan kTunedPlans[] = {
 
 constexpr int kTunedOnCUs = 256;
 
-// Heuristic plan for shapes without a measured entry. Inputs: shape and CU count.
-void select_config(int m, int n, int k, int num_cu, bool tiled_ok, const std::vector<TunedPlan> &user_plans,
-                   rf_gemm_config *out) {
+// Estimated time in microseconds of the best few-rows plan for a shape, and that plan. Fitted (relative error) to 12000
+// launches on operand sets that rotate out of the L2 caches: M = 1 ... 512, 23 pairs of N and K from 200 to 8192 and 128 to
+// 7168, every few-rows variant with 1 to 14 splits. The plan it picks is 4 % slower than the best one measured, on average.
+//   1.96                                       launch, and the way back
+//   + 1.12 + 0.106 per KiB of sums handed over when K is split
+//   + rounds * (b + 0.985 * batches of loads of a wave + c * K blocks of a wave * workgroups sharing a CU), a quarter more
+//     where rows of B start at any byte (any_bytes)
+//   + d * MB of A and B that all workgroups fetch
+double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_config *out) {
+    struct Fit { int variant, per_cu, depth; double b, c, d; };
+    const Fit fits[] = {{14, 2, 3, 0.0, 0.458, 0.0916},   {15, 1, 2, 0.0, 0.860, 0.0591},   {16, 1, 1, 0.790, 0.665, 0.0381},
+                        {17, 2, 2, 0.0, 0.572, 0.0755},   {18, 1, 2, 0.101, 1.090, 0.0546}, {19, 1, 2, 0.127, 1.063, 0.0593},
+                        {20, 1, 1, 1.651, 0.929, 0.0362}};
+    const int splits_tried[] = {1, 2, 3, 4, 5, 6, 8, 12, 14}, qk = k / rf::BK;
+    double best = 1e30;
+    for (const Fit &f : fits) {
+        const Variant &v = kVariants[f.variant];
+        const long items = (long)ceil_div(m, v.bm) * ceil_div(n, v.bn);
+        for (int sp : splits_tried) {
+            if (sp > qk || (sp > 1 && (items * sp > 4L * num_cu || items > kMaxTileCounters))) break;
+            const int kb = ceil_div(qk, sp), parts = ceil_div(qk, kb), own = ceil_div(kb, v.waves_n);
+            const long wgs = items * parts, rounds = (wgs + (long)num_cu * f.per_cu - 1) / ((long)num_cu * f.per_cu);
+            const double mb = (double)wgs * kb * (v.bm + v.bn) * rf::BK * 1e-6 * 256 / num_cu;
+            const double t = 1.96 + (parts > 1 ? 1.12 + 0.106 * parts * v.bm * v.bn / 1024.0 : 0.0) +
+                             rounds * (any_bytes ? 1.27 : 1.0) *
+                                 (f.b + 0.985 * ceil_div(own, f.depth) + f.c * own * (wgs > num_cu ? f.per_cu : 1)) +
+                             f.d * mb;
+            if (t < best) {
+                best = t;
+                *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};
+            }
+        }
+    }
+    return best;
+}
+constexpr int kFewRowsMaxM = 512;                           // beyond this the estimate is not measured (and never the best)
+
+// What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
+// (and of C on the way back).
+enum { kStageA = 1, kStageB = 2 };
+
+// Plan for a shape (m, n multiples of 16, the padded sizes when something is staged).
+void select_config_uncached(int m, int n, int k, int num_cu, int stage, const std::vector<TunedPlan> &user_plans,
+                            rf_gemm_config *out) {
     out->split_k = 1;
     out->group_m = 8;
     out->stream_k = 0;
-    if (!tiled_ok) {
-        out->variant = -1;
-        return;
-    }
     auto usable = [&](const TunedPlan &p) {
         return p.m == m && p.n == n && p.k == k && p.variant < kNumVariants && p.split_k <= k / rf::BK &&
                (kVariants[p.variant].k_groups == 1 || (p.split_k == 1 && (k / rf::BK) % kVariants[p.variant].k_groups == 0)) &&
@@ -459,16 +534,12 @@ void select_config(int m, int n, int k, int num_cu, bool tiled_ok, const std::ve
     // the compiled-in table was measured on a device with kTunedOnCUs compute units: round counts, and with them the
     // best tile and split, change with the unit count, so another device takes the cost model below (which counts
     // rounds for the device at hand) unless the caller has loaded plans measured there
+    auto take = [&](const TunedPlan &p) { *out = {p.variant, p.split_k, p.group_m, p.stream_k}; };
+    if (hit) return take(*hit);
     if (num_cu == kTunedOnCUs)
         for (const TunedPlan &p : kTunedPlans)
             if (!hit && usable(p)) hit = &p;
-    if (hit) {
-        out->variant = hit->variant;
-        out->split_k = hit->split_k;
-        out->group_m = hit->group_m;
-        out->stream_k = hit->stream_k;
-        return;
-    }
+    if (hit && (!stage || kVariants[hit->variant].is_fewrows())) return take(*hit);
     // Up to four K blocks and a large C: the launch is a streaming store, which the skinny-K schedule does best
     // (measured against the best tiled plan at N = 7168, K = 256: 1024 rows 6.5 against 6.9 us, 2048 rows 7.8 against
     // 10.3, 6144 rows 18.2 against 22.1; below about six million outputs the 64 x 128 tiles win, e.g. 2048 x 2048: 6.5
@@ -479,6 +550,7 @@ void select_config(int m, int n, int k, int num_cu, bool tiled_ok, const std::ve
     if (skinny_ok(m, n, k) &&
         (k <= 2 * rf::BK ? (double)m * n >= 6.0e6
                          : (double)m * n >= 2.0e6 && (k == 3 * rf::BK || ceil_div(n, 256) <= 16))) {
+        if (hit) return take(*hit);
         out->variant = 0;
         out->stream_k = RF_SCHEDULE_SKINNY_K;
         return;
@@ -553,6 +625,56 @@ void select_config(int m, int n, int k, int num_cu, bool tiled_ok, const std::ve
             }
         }
     }
+    if (hit) take(*hit);                                    // a measured plan, but one that would run on staged copies
+    // Few rows: the few-rows kernels, which need no staging, when they come out faster. The model above ranks tiled plans;
+    // what their launches take is 3.1 us + 0.67 of its figure, and staging adds the copies' launches and bytes
+    // (fitted to the same measurements as fewrows_plan). Over 280 shapes the choice between the two families is within 4 %
+    // of the best plan of either, on average.
+    if (m <= kFewRowsMaxM && fewrows_ok(m, n)) {
+        double tiled = 3.1 + 0.67 * best_cost;
+        if (stage & kStageA) tiled += 3.2 + 2.0 * k * m / 4e6;
+        if (stage & kStageB) tiled += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
+        rf_gemm_config few;
+        if (fewrows_plan(m, n, k, num_cu, (stage & kStageB) != 0, &few) < tiled) *out = few;
+    }
+}
+
+// The same through a small table of plans already worked out (the models take 1 to 3 us of host time, as long as a small
+// launch). Entries hold for one generation of the loaded plan files; the caller holds the lock.
+void select_config(int m, int n, int k, int num_cu, int stage, rf_gemm_config *out) {
+    struct Entry { int m, n, k, num_cu, stage, generation; rf_gemm_config cfg; };
+    constexpr unsigned kEntries = 1024;
+    static Entry table[kEntries];                           // zeroed: no entry has k == 0
+    const unsigned h = ((unsigned)m * 2654435761u) ^ ((unsigned)n * 2246822519u) ^ ((unsigned)k * 3266489917u) ^ (unsigned)(stage * 668265263);
+    Entry &e = table[(h >> 7) % kEntries];
+    if (e.m != m || e.n != n || e.k != k || e.num_cu != num_cu || e.stage != stage || e.generation != shared().plan_generation) {
+        e = {m, n, k, num_cu, stage, shared().plan_generation, {}};
+        select_config_uncached(m, n, k, num_cu, stage, shared().user_plans, &e.cfg);
+    }
+    *out = e.cfg;
+}
+
+// m rows out of ldm (the distance between two K rows of a and as); any shape and alignment. splits >= 1.
+int launch_fewrows(Mem &mem, const Variant &v, const void *a, const void *b, const float *as, const float *bs, void *c, int m,
+                   int ldm, int n, int k, int splits, hipStream_t stream) {
+    const int qk = k / rf::BK, row_blocks = ceil_div(m, v.bm), items = ceil_div(n, v.bn) * row_blocks;
+    const int kb_per_split = ceil_div(qk, splits);
+    splits = ceil_div(qk, kb_per_split);                    // every split owns at least one K block
+    unsigned *counters = nullptr;
+    float *slots = nullptr;
+    if (splits > 1) {
+        if (items > kMaxTileCounters) return fail(RF_ERR_BAD_CONFIG, "too many tiles for a K split of this variant");
+        int rc = mem.tile_counters(&counters);
+        if (rc != RF_OK) return rc;
+        rc = mem.workspace((size_t)items * splits * v.bm * v.bn * sizeof(float), &slots);
+        if (rc != RF_OK) return rc;
+    }
+    const bool any = n % 16 != 0 || (uintptr_t)b % 16 != 0;
+    hipLaunchKernelGGL(v.fewrows[splits > 1][any], dim3(items, splits), dim3(v.threads()), v.lds_bytes(), stream,
+                       (const uint8_t *)a, (const uint8_t *)b, as, bs, (uint16_t *)c, m, ldm, n, k, kb_per_split, row_blocks,
+                       counters, slots);
+    RF_HIP(hipGetLastError());
+    return RF_OK;
 }
 
 // The launch proper; the caller holds the lock and has checked shape and pointers. m_store >= 0: c has only m_store
@@ -566,9 +688,11 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
     if (user_cfg) {
         cfg = *user_cfg;
         if (cfg.variant >= kNumVariants || cfg.variant < -1 || cfg.split_k < 1 || cfg.group_m < 1 ||
-            cfg.split_k > k / rf::BK || (cfg.variant >= 0 && !tiled_ok) || (cfg.variant < 0 && cfg.split_k != 1) ||
+            cfg.split_k > k / rf::BK || (cfg.variant >= 0 && !kVariants[cfg.variant].is_fewrows() && !tiled_ok) || (cfg.variant < 0 && cfg.split_k != 1) ||
             (cfg.stream_k != 0 && (cfg.variant < 0 || cfg.split_k != 1)))
             return fail(RF_ERR_BAD_CONFIG, "configuration not usable for this shape");
+        if (cfg.variant >= 0 && kVariants[cfg.variant].is_fewrows() && !fewrows_ok(m, n))
+            return fail(RF_ERR_BAD_CONFIG, "the few-rows kernels need M and N below 2^25");
         if (cfg.variant >= 0 && kVariants[cfg.variant].k_groups > 1 &&
             (cfg.split_k != 1 || cfg.stream_k != RF_SCHEDULE_TILES || (k / rf::BK) % kVariants[cfg.variant].k_groups != 0))
             return fail(RF_ERR_BAD_CONFIG, "this variant splits K inside the workgroup: it needs split_k == 1, the tile "
@@ -593,17 +717,20 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
             return fail(RF_ERR_BAD_CONFIG, "unknown schedule");
         }
     } else {
-        select_config(m, n, k, s.num_cu, tiled_ok, shared().user_plans, &cfg);
+        if (tiled_ok) select_config(m, n, k, s.num_cu, 0, &cfg);
+        else cfg = {-1, 1, 8, RF_SCHEDULE_TILES};
     }
 
     if (mem.fixed && cfg.variant >= 0) {
         // rf_fp8_gemm_static: the plan has to live inside what is left of the static array. A stream-K plan (only a
         // plan file can name one) is replaced by the cost model's plan; a K split whose partial sums do not fit is cut
         // down to the number of parts that do, a single part needing no scratch memory at all.
-        if (cfg.stream_k == RF_SCHEDULE_STREAM_K) select_config(m, n, k, s.num_cu, true, std::vector<TunedPlan>(), &cfg);
+        if (cfg.stream_k == RF_SCHEDULE_STREAM_K) select_config_uncached(m, n, k, s.num_cu, 0, std::vector<TunedPlan>(), &cfg);
         if (cfg.stream_k == RF_SCHEDULE_STREAM_K) cfg.stream_k = RF_SCHEDULE_TILES;
         if (cfg.split_k > 1) {
-            const size_t per_part = (size_t)m * n * sizeof(float);
+            const Variant &fv = kVariants[cfg.variant];
+            const size_t per_part = !fv.is_fewrows() ? (size_t)m * n * sizeof(float)
+                : (size_t)ceil_div(m, fv.bm) * fv.bm * ceil_div(n, fv.bn) * fv.bn * sizeof(float);
             const int qk_ = k / rf::BK, kb_per = ceil_div(qk_, cfg.split_k), parts = ceil_div(qk_, kb_per);
             const size_t fit = mem.fixed_left() / per_part;
             if ((size_t)parts > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;
@@ -611,6 +738,13 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
     }
     if (m_store != m && (cfg.variant < 0 || cfg.stream_k == RF_SCHEDULE_STREAM_K))
         return fail(RF_ERR_BAD_CONFIG, "internal: this schedule cannot write fewer rows than it computes");
+    if (cfg.variant < 0 && !user_cfg && fewrows_ok(m, n)) {
+        // a small problem the tiled kernels do not take (reported as plan -1: no tile variant): the few-rows kernels do. A wave
+        // of the bounds-checked kernel gathers bytes K block after K block, 13 to 27 us where these take 3 to 4
+        // (M x N x K = 4 x 200 x 2048: 27.8 -> 3.7, 8 x 1000 x 384: 13.6 -> 3.1).
+        fewrows_plan(m, n, k, s.num_cu, n % 16 != 0, &cfg);
+        return launch_fewrows(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, stream);
+    }
     if (cfg.variant < 0) {
         dim3 grid(ceil_div(n, 16), ceil_div(m, 16));
         hipLaunchKernelGGL(rf::gemm_fp8_blockscale_checked, grid, dim3(64), 0, stream, (const uint8_t *)a,
@@ -620,6 +754,7 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
     }
 
     const Variant &v = kVariants[cfg.variant];
+    if (v.is_fewrows()) return launch_fewrows(mem, v, a, b, as, bs, c, m_store, m, n, k, cfg.split_k, stream);
     const int tiles_m = ceil_div(m, v.bm), tiles_n = ceil_div(n, v.bn);
     const int qk = k / rf::BK;
     const int kb_per_split = ceil_div(qk, cfg.split_k);
@@ -827,7 +962,7 @@ rf::GroupTable one_group(int cols, int cols_pad) {
 // rows of the problem are cut into pieces (row ranges of A, a_scale and C are independent GEMMs), each piece is staged,
 // computed and, where C is staged too, copied back before the next one re-uses the same memory; the stream orders them.
 // The staged copy of B (ragged N or an unaligned b) is shared by all pieces and has to fit beside them: when it takes
-// more than half of the array, the bounds-checked kernel computes the whole problem in place instead.
+// more than half of the array, the 64 x 64 few-rows kernel computes the whole problem in place instead.
 int launch_padded_in_pieces(State &s, Mem &mem, const void *a, const void *b, const float *as, const float *bs, void *c,
                             int m, int n, int k, hipStream_t stream) {
     auto pad16 = [](int x) { return x < 16 ? 16 : (x + 15) / 16 * 16; };
@@ -842,6 +977,8 @@ int launch_padded_in_pieces(State &s, Mem &mem, const void *a, const void *b, co
     const size_t left = mem.fixed_left() > b_bytes ? mem.fixed_left() - b_bytes : 0;
     long rows_fit = (long)((left - left / 4) / per_row) / 16 * 16 - 16;
     if (b_bytes > mem.fixed_left() / 2 || rows_fit < 16) {
+        if (fewrows_ok(m, n))
+            return launch_fewrows(mem, kVariants[kFewRows64x64], a, b, as, bs, c, m, m, n, k, 1, stream);
         hipLaunchKernelGGL(rf::gemm_fp8_blockscale_checked, dim3(ceil_div(n, 16), ceil_div(m, 16)), dim3(64), 0, stream,
                            (const uint8_t *)a, (const uint8_t *)b, as, bs, (uint16_t *)c, m, m, n, k);
         RF_HIP(hipGetLastError());
@@ -872,7 +1009,7 @@ int launch_padded_in_pieces(State &s, Mem &mem, const void *a, const void *b, co
         launch_pad_a_and_scales((const uint8_t *)a + r0, as + r0, m, rp, k, 1, pa, (float *)psa, one_group(rows, rp), stream);
         RF_HIP(hipGetLastError());
         rf_gemm_config cfg;
-        select_config(rp, np, k, s.num_cu, true, shared().user_plans, &cfg);
+        select_config(rp, np, k, s.num_cu, 0, &cfg);
         void *c_piece = copy_c ? (void *)pc : (void *)((uint16_t *)c + (size_t)r0 * n);
         rc = launch_locked(s, mem, pa, b2, (const float *)psa, bs, c_piece, rp, np, k, &cfg, stream, copy_c ? rp : rows);
         if (rc != RF_OK) return rc;
@@ -894,7 +1031,16 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     // tile, persistent) write the m true rows straight into c (their stores are masked by row); otherwise C is staged
     // and copied back.
     rf_gemm_config cfg;
-    select_config(mp, np, k, s.num_cu, true, shared().user_plans, &cfg);
+    select_config(mp, np, k, s.num_cu, (copy_a ? kStageA : 0) | (copy_b || (uintptr_t)c % 16 != 0 ? kStageB : 0), &cfg);
+    if (kVariants[cfg.variant].is_fewrows()) {
+        if (mem.fixed && cfg.split_k > 1) {                // as many K parts as the static array holds
+            const Variant &v = kVariants[cfg.variant];
+            const size_t per_part = (size_t)ceil_div(m, v.bm) * v.bm * ceil_div(n, v.bn) * v.bn * sizeof(float);
+            const size_t fit = mem.fixed_left() / per_part;
+            if ((size_t)cfg.split_k > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;
+        }
+        return launch_fewrows(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, stream);
+    }
     const bool copy_c = np != n || (uintptr_t)c % 16 != 0 || (mp != m && cfg.stream_k == RF_SCHEDULE_STREAM_K);
     size_t off = 0;
     const size_t off_a = off;  off += copy_a ? align((size_t)k * mp) : 0;
@@ -948,6 +1094,14 @@ int launch(const void *a, const void *b, const float *as, const float *bs, void 
     if (!user_cfg && !tiled_path_ok(a, b, c, m, n) && (double)m * n * k >= kPadThresholdMacs)
         return launch_padded(s, mem, a, b, as, bs, c, m, n, k, stream);
     return launch_locked(s, mem, a, b, as, bs, c, m, n, k, user_cfg, stream);
+}
+
+// The plan a launch with aligned pointers takes: a shape the tiled kernels do not take as it is is planned at its padded size.
+void plan_of_shape(int m, int n, int k, int num_cu, rf_gemm_config *out) {
+    auto pad16 = [](int x) { return x < 16 ? 16 : (x + 15) / 16 * 16; };
+    const int mp = pad16(m), np = pad16(n);
+    if ((mp != m || np != n) && (double)m * n * k < kPadThresholdMacs) *out = {-1, 1, 8, RF_SCHEDULE_TILES};
+    else select_config(mp, np, k, num_cu, (mp != m ? kStageA : 0) | (np != n ? kStageB : 0), out);
 }
 
 // ---- timing record for run() ----------------------------------------------------------------
@@ -1033,15 +1187,7 @@ int rf_gemm_select_config(int m, int n, int k, rf_gemm_config *out) {
     std::lock_guard<std::mutex> lock(shared().mu);
     int rc = ensure_device_info(s);
     if (rc != RF_OK) return rc;
-    const bool tiled = m >= 16 && n >= 16 && m % 16 == 0 && n % 16 == 0;
-    if (!tiled && (double)m * n * k >= kPadThresholdMacs) {
-        // the launch pads such a shape to multiples of 16 and plans for the padded shape (see launch_padded)
-        m = m < 16 ? 16 : (m + 15) / 16 * 16;
-        n = n < 16 ? 16 : (n + 15) / 16 * 16;
-        select_config(m, n, k, s.num_cu, true, shared().user_plans, out);
-        return RF_OK;
-    }
-    select_config(m, n, k, s.num_cu, tiled, shared().user_plans, out);
+    plan_of_shape(m, n, k, s.num_cu, out);
     return RF_OK;
 }
 
@@ -1050,14 +1196,7 @@ int rf_gemm_plan_for(int m, int n, int k, int num_cu, rf_gemm_config *out) {
     if (!out) return fail(RF_ERR_NULL_POINTER, "out is null");
     if (m < 1 || n < 1 || k < rf::BK || k % rf::BK != 0 || num_cu < 1) return fail(RF_ERR_BAD_SHAPE, "unsupported shape");
     std::lock_guard<std::mutex> lock(shared().mu);
-    const bool tiled = m >= 16 && n >= 16 && m % 16 == 0 && n % 16 == 0;
-    if (!tiled && (double)m * n * k >= kPadThresholdMacs) {
-        m = m < 16 ? 16 : (m + 15) / 16 * 16;
-        n = n < 16 ? 16 : (n + 15) / 16 * 16;
-        select_config(m, n, k, num_cu, true, shared().user_plans, out);
-        return RF_OK;
-    }
-    select_config(m, n, k, num_cu, tiled, shared().user_plans, out);
+    plan_of_shape(m, n, k, num_cu, out);
     return RF_OK;
 }
 
@@ -1068,6 +1207,7 @@ int rf_gemm_load_plans(const char *path, int *count) {
     const size_t before = shared().user_plans.size();
     int rc = parse_plans(path, shared().user_plans);
     if (rc != RF_OK) return rc;
+    shared().plan_generation++;
     if (count) *count = (int)(shared().user_plans.size() - before);
     return RF_OK;
 }
@@ -1075,6 +1215,7 @@ int rf_gemm_load_plans(const char *path, int *count) {
 void rf_gemm_clear_plans(void) {
     std::lock_guard<std::mutex> lock(shared().mu);
     shared().user_plans.clear();
+    shared().plan_generation++;
 }
 
 int rf_gemm_num_variants(void) { return kNumVariants; }
@@ -1113,6 +1254,10 @@ size_t rf_gemm_workspace_bytes(int m, int n, int k) {
         return (size_t)2 * s.num_cu * kVariants[cfg.variant].bm * kVariants[cfg.variant].bn * sizeof(float);
     }
     if (cfg.split_k <= 1) return 0;
+    if (kVariants[cfg.variant].is_fewrows()) {
+        m = ceil_div(m, kVariants[cfg.variant].bm) * kVariants[cfg.variant].bm;
+        n = ceil_div(n, kVariants[cfg.variant].bn) * kVariants[cfg.variant].bn;
+    }
     const int qk = k / rf::BK;
     const int kb_per_split = ceil_div(qk, cfg.split_k);
     return (size_t)m * n * sizeof(float) * ceil_div(qk, kb_per_split);

@@ -77,6 +77,9 @@ def tune_shape(rfk, m, n, k, log=print):
     ncu = torch.cuda.get_device_properties(0).multi_processor_count
     for v in rfk.variants():
         tiles = -(-m // v["block_m"]) * -(-n // v["block_n"])
+        few_rows = v["variant"] >= 14                    # no tile order to group; never the fastest beyond some hundred rows
+        if few_rows and m > 512:
+            continue
         # schedules: 0 = one workgroup per tile (with K splits), 1 = stream-K, 2 = persistent whole tiles,
         # 3 = persistent with a last round of half tiles, 4 = skinny K (K = 128 ... 512; listed under variant 0)
         for split, sk in [(sp, 0) for sp in SPLITS] + [(1, 1), (1, 2), (1, 3), (1, 4)]:
@@ -92,7 +95,9 @@ def tune_shape(rfk, m, n, k, log=print):
                 left = tiles % ncu
                 if v["variant"] != 0 or tiles < ncu or left == 0 or (left + 7) // 8 * 8 + left > ncu:
                     continue
-            for gm in (GROUPS if sk != 4 else GROUPS[1:2]):          # the skinny-K schedule has no tile order to group
+            if few_rows and split > 1 and tiles * split > 4 * ncu:
+                continue
+            for gm in (GROUPS if sk != 4 and not few_rows else GROUPS[1:2]):   # the skinny-K schedule has no tile order either
                 cfg = rfk.GemmConfig(v["variant"], split, gm, sk)
                 args[4].zero_()
                 us = _time(rfk, args, cfg, iters)

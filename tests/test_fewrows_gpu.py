@@ -1,0 +1,89 @@
+"""The few-rows kernels (variants 14 to 20): any shape and alignment, K split between waves and between workgroups."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import bf16_bits, exact_problem, oracle_bf16, to_gpu
+
+pytestmark = pytest.mark.gpu
+FEW_ROWS = range(14, 21)
+
+
+@pytest.fixture(scope="module")
+def rfk():
+    import radeonflow_kernels_amd as r
+    assert torch.cuda.is_available(), "these tests need the GPU"
+    r.lib()
+    return r
+
+
+# edges of the 16-row tiles and of the 32 to 128 column strips, one K block (seven idle waves), K blocks that do and do not
+# divide among eight waves and splits; M = 1 and N = 1: loads of the last rows are cut at the matrix's end
+@pytest.mark.parametrize("m,n,k", [(1, 1, 128), (1, 7168, 256), (2, 130, 1152), (15, 33, 2432), (16, 144, 1024), (17, 127, 3200),
+                                   (31, 257, 640), (33, 500, 2048), (64, 96, 7168), (65, 129, 896), (130, 47, 384)])
+def test_fewrows_bit_exact_on_any_shape(rfk, m, n, k):
+    """Exact data: every plan gives the oracle's bits whatever its summation order, nothing is stored past the end of C; two
+    launches in a row (the arrival counters of a K split are back at zero)."""
+    data = exact_problem(m, n, k, seed=5 * m + n + k)
+    exp = oracle_bf16(data)
+    g, buf = to_gpu(data, 300)
+    for v in FEW_ROWS:
+        for split in (1, 2, 5):
+            if split > k // 128:
+                continue
+            for rep in range(2):
+                g[4].fill_(-1.0)
+                rfk.fp8_mm(*g, config=rfk.GemmConfig(v, split, 1, 0))
+                torch.cuda.synchronize()
+                assert np.array_equal(bf16_bits(g[4]), exp), "variant %d split %d launch %d" % (v, split, rep)
+    assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
+
+
+@pytest.mark.parametrize("off_a,off_b,off_c", [(1, 0, 0), (0, 3, 0), (7, 15, 1), (16, 16, 2)])
+def test_fewrows_takes_operands_at_any_byte(rfk, off_a, off_b, off_c):
+    """Operands that start off_a, off_b bytes (C: off_c elements) into 16-byte aligned buffers, under the automatic plan and an
+    explicit one; the buffers end with the operands, so a load past the end would leave the allocation's data."""
+    m, n, k = 24, 176, 1280
+    data = exact_problem(m, n, k, seed=11)
+    exp = oracle_bf16(data)
+    a, b, sa, sb = to_gpu(data)[:4]
+
+    def shifted(t, off):
+        rows, cols = t.shape
+        flat = torch.empty(rows * cols + off, dtype=torch.uint8, device="cuda")
+        flat[off:].copy_(t.T.contiguous().view(torch.uint8).reshape(-1))
+        return flat[off:].view(torch.float8_e4m3fn).view(cols, rows).T
+
+    for cfg in (None, rfk.GemmConfig(18, 3, 1, 0)):
+        c = torch.zeros(m * n + off_c, dtype=torch.bfloat16, device="cuda")[off_c:].view(m, n)
+        rfk.fp8_mm(shifted(a, off_a), shifted(b, off_b), sa, sb, c, config=cfg)
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(c), exp), "plan %r" % (cfg,)
+
+
+def test_fewrows_static_entry_and_graph_replay(rfk):
+    """The allocation-free entry (its own counters and slots) and replays of a captured launch give the same bits."""
+    m, n, k = 7, 1536, 7168
+    plan = rfk.select_config(m, n, k)
+    assert plan.variant in FEW_ROWS and plan.split_k > 1
+    data = exact_problem(m, n, k, seed=3)
+    exp = oracle_bf16(data)
+    g = to_gpu(data)
+    rfk.fp8_mm(*g)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits(g[4]), exp)
+    for rep in range(2):
+        g[4].zero_()
+        rfk.fp8_mm_static(*g)
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(g[4]), exp)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rfk.fp8_mm_static(*g)
+    for rep in range(3):
+        g[4].fill_(-1.0)
+        rfk.fp8_mm(g[0], g[1], g[2], g[3], torch.empty_like(g[4]))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(g[4]), exp), "replay %d" % rep
