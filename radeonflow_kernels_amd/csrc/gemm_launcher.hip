@@ -1304,6 +1304,8 @@ const char *rf_gemm_last_error(void) { return g_last_error.c_str(); }
 }  // extern "C"
 
 namespace {
+// Up to this many elements the activations' quantiser works in 16-row pieces instead of 128-row blocks (see quantize_rows16).
+constexpr double kQuantRows16Elements = 1.0e7;
 // rows x K source (row-major, K contiguous) -> fp8 [K][rows] + scales; see quantize_kernels.h
 template <bool PER_ROW, bool IN_BF16>
 int launch_quantize(const void *x, int rows, int k, void *out, float *scales, hipStream_t stream) {
@@ -1320,11 +1322,17 @@ int launch_quantize(const void *x, int rows, int k, void *out, float *scales, hi
         int rc = ensure_device_info(s);
         if (rc != RF_OK) return rc;
     }
+    if (PER_ROW && (double)rows * k <= kQuantRows16Elements) {
+        hipLaunchKernelGGL((rf::quantize_rows16<IN_BF16>), dim3(k / rf::BK, ceil_div(rows, 16)), dim3(256), 0, stream, x, rows, k,
+                           (uint8_t *)out, scales);
+        RF_HIP(hipGetLastError());
+        return RF_OK;
+    }
     const bool vector_store = rows % 16 == 0 && (uintptr_t)out % 16 == 0;
     const int row_blocks = ceil_div(rows, 128);
     dim3 grid(k / rf::BK, row_blocks);
-    hipLaunchKernelGGL((rf::quantize_block128<PER_ROW, IN_BF16>), grid, dim3(256), 0, stream, x, rows, k, (uint8_t *)out,
-                       scales, PER_ROW ? rows : row_blocks, vector_store);
+    hipLaunchKernelGGL((rf::quantize_block128<PER_ROW, IN_BF16>), grid, dim3(rf::QuantShape<IN_BF16>::NT), 0, stream, x, rows,
+                       k, (uint8_t *)out, scales, PER_ROW ? rows : row_blocks, vector_store);
     RF_HIP(hipGetLastError());
     return RF_OK;
 }
@@ -1638,8 +1646,12 @@ int quantize_a_grouped(const void *x, const int *row_offsets, int groups, int k,
         int rc = ensure_device_info(s);
         if (rc != RF_OK) return rc;
     }
-    hipLaunchKernelGGL((rf::quantize_block128_grouped<IN_BF16>), dim3(k / rf::BK, ceil_div(at, 128)), dim3(256), 0, stream, x,
-                       at, k, (uint8_t *)a, as, tab);
+    if ((double)at * k <= kQuantRows16Elements)
+        hipLaunchKernelGGL((rf::quantize_rows16_grouped<IN_BF16>), dim3(k / rf::BK, at / 16), dim3(256), 0, stream, x, at, k,
+                           (uint8_t *)a, as, tab);
+    else
+        hipLaunchKernelGGL((rf::quantize_block128_grouped<IN_BF16>), dim3(k / rf::BK, ceil_div(at, 128)),
+                           dim3(rf::QuantShape<IN_BF16>::NT), 0, stream, x, at, k, (uint8_t *)a, as, tab);
     RF_HIP(hipGetLastError());
     return RF_OK;
 }

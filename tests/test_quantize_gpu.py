@@ -198,3 +198,33 @@ def test_quantize_a_source_beyond_4_gib(rfk):
     got_scales = s[idx].contiguous().cpu().numpy().T
     assert np.array_equal(got_scales.view(np.uint32), np.asarray(as_ref).view(np.uint32))
     assert np.array_equal(got_codes, np.asarray(a_ref))
+
+
+@pytest.mark.parametrize("rows", [1536, 1501, 2033])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_blocks_of_128_rows_equal_pieces_of_16(rfk, rows, dtype):
+    """Sources of more than ten million elements are quantised in blocks of 128 rows, smaller ones in pieces of 16: the same
+    bytes and scales, for whole blocks, ragged rows (stores at any byte) and a last block of one to 125 rows."""
+    k = 7168
+    x = torch.from_numpy(_source(rows, k, rows, "special")).cuda().to(dtype)
+    q, s = rfk.quantize_a(x)
+    for r0, r1 in ((0, 257), (257, 1000), (1000, rows)):
+        q1, s1 = rfk.quantize_a(x[r0:r1].contiguous())
+        assert torch.equal(q[r0:r1].view(torch.uint8), q1.view(torch.uint8)) and torch.equal(s[r0:r1], s1)
+
+
+@pytest.mark.parametrize("sizes", [[1, 0, 15, 16, 17, 0, 0, 3], [700, 1, 0, 333, 500, 16, 31, 97]])
+def test_grouped_quantiser_equals_the_plain_one_per_group(rfk, sizes):
+    """16-row pieces (little work) and 128-row blocks: every group's rows, and zeros with scale 1 in the padding."""
+    k = 7168
+    offs = [0] + [int(v) for v in np.cumsum(sizes)]
+    x = torch.from_numpy(_source(offs[-1], k, offs[-1], "normal")).cuda().bfloat16()
+    a, sa = rfk.quantize_a_grouped(x, offs)
+    pad = rfk.grouped_padded_offsets(offs)
+    for g, n in enumerate(sizes):
+        if n:
+            q, s = rfk.quantize_a(x[offs[g]:offs[g + 1]].contiguous())
+            assert torch.equal(a[pad[g]:pad[g] + n].view(torch.uint8), q.view(torch.uint8))
+            assert torch.equal(sa[pad[g]:pad[g] + n], s)
+        assert int(a[pad[g] + n:pad[g + 1]].contiguous().view(torch.uint8).sum(dtype=torch.int64)) == 0
+        assert bool((sa[pad[g] + n:pad[g + 1]] == 1.0).all())
