@@ -39,6 +39,7 @@ struct FewRowsGeom {
     static constexpr int REGION = BK * (BM + BN);                     // one K block of A and of B, private to a wave
     static constexpr int EXCHANGE = NW * TM * TN * 1024;              // the waves' sums, over the regions
     static constexpr int LDS_BYTES = NW * REGION > EXCHANGE ? NW * REGION : EXCHANGE;
+    static constexpr int WAVES_PER_SIMD = LDS_BYTES < 80 * 1024 ? 4 : 2;   // two workgroups of eight waves, where LDS has room
     static_assert(LDS_BYTES <= 160 * 1024, "the waves' regions fit the CU's LDS");
     static_assert((TM & (TM - 1)) == 0 && (TN & (TN - 1)) == 0, "powers of two: the chunk swizzle stays inside a row");
 };
@@ -73,78 +74,66 @@ __device__ __forceinline__ u32x4_lds shift_back(u32x4_lds v, uint32_t off, uint3
     return r;
 }
 
-// Grid: x = column strips * row blocks (row blocks innermost: they share the strip's B), y = K splits of kb_per_split
-// blocks, every split at least one. A [K][ldm] (M of the ldm columns belong to this problem), SA [K/128][ldm], B [K][N],
-// C [M][N]. Any M, N >= 1, any alignment of A, B and C; ldm and N below 2^25 (32-bit offsets inside a K block). BYTES
-// false needs N % 16 == 0 and a 16-byte aligned B. SPLIT (gridDim.y > 1): counters holds a zero per item (gridDim.x) and
-// is zero again afterwards, slots gridDim.x * gridDim.y * TM * TN KiB, 16-byte aligned.
-template <int TM, int TN, int NW, int DEPTH, bool SPLIT, bool BYTES>
-__global__ __launch_bounds__(NW * 64) void gemm_fp8_blockscale_fewrows(
-    const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
-    const float *__restrict__ SB, uint16_t *__restrict__ C, int M, int ldm, int N, int K, int kb_per_split, int row_blocks,
-    unsigned *__restrict__ counters, float *__restrict__ slots) {
-    using G = FewRowsGeom<TM, TN, NW, DEPTH>;
-    constexpr int NLA = 2 * TM, NLB = 2 * TN;                         // 16-byte loads per lane and K block
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int L = lane & 15, g = lane >> 4;
-    // neighbouring strips on one XCD: a 32-column piece of a row of B is a quarter of a cache line
-    const int xcd = blockIdx.x % NUM_XCD, idx = blockIdx.x / NUM_XCD, per = gridDim.x / NUM_XCD, rem = gridDim.x % NUM_XCD;
-    const int item = xcd * per + (xcd < rem ? xcd : rem) + idx;
-    const int n0 = item / row_blocks * G::BN, m0 = item % row_blocks * G::BM;
-    const int QK = K / BK, QN = (N + 127) / 128;
-    const int kb_begin = blockIdx.y * kb_per_split, kb_end = kb_begin + kb_per_split < QK ? kb_begin + kb_per_split : QK;
-    const int count = (kb_end - kb_begin - wave + NW - 1) / NW;       // this wave's K blocks: kb_begin + wave + NW * i
-    uint8_t *region = lds + wave * G::REGION;
-
-    // Load i of a lane: 16-byte chunk lane % T of K row lane / T + i * 64 / T of the block
+// What one wave does with one K block: loads into registers, the private LDS region, fragments, MFMAs.
+template <int TM, int TN, bool BYTES>
+struct FewRowsWave {
+    static constexpr int BM = 16 * TM, BN = 16 * TN;
+    static constexpr int NLA = 2 * TM, NLB = 2 * TN;                  // 16-byte loads per lane and K block
+    static_assert(128 % BN == 0, "a strip lies in one b_scale block");
+    // One K block on its way: raw bytes of A and B, scales.
+    struct Block {
+        u32x4_lds a[NLA], b[NLB];
+        float sa[TM], sb;
+    };
+    const uint8_t *A, *B;
+    const float *SA, *SB;
+    uint8_t *region;
+    int ldm, N, K, QN, nb, lane, first;
+    int zero = 0;                                                     // see gemm_fp8_blockscale_grouped_strips
     uint32_t off_a0, off_b0;
-    {
+    int row_s[TM];
+
+    // Tile m0, n0 of a problem of M rows that starts at column `first` of an A with ldm columns.
+    __device__ __forceinline__ FewRowsWave(const uint8_t *A_, const uint8_t *B_, const float *SA_, const float *SB_, int M,
+                                           int first_, int ldm_, int N_, int K_, int m0, int n0, uint8_t *region_, int lane_)
+        : A(A_ + first_), B(B_), SA(SA_ + first_), SB(SB_), region(region_), ldm(ldm_), N(N_), K(K_), QN((N_ + 127) / 128),
+          nb(n0 >> 7), lane(lane_), first(first_) {
+        // Load i of a lane: 16-byte chunk lane % T of K row lane / T + i * 64 / T of the block
         int m = m0 + 16 * (lane % TM), n = n0 + 16 * (lane % TN);
         if (m >= M) m = m0;                                           // a whole chunk past M or N: any bytes will do
         if (n >= N) n = n0;
         off_a0 = (uint32_t)(lane / TM) * (uint32_t)ldm + (uint32_t)m;
         off_b0 = (uint32_t)(lane / TN) * (uint32_t)N + (uint32_t)n;
-    }
-    auto off_a = [&](int i) { return off_a0 + (uint32_t)(i * (64 / TM)) * (uint32_t)ldm; };
-    auto off_b = [&](int i) { return off_b0 + (uint32_t)(i * (64 / TN)) * (uint32_t)N; };
-    auto dst_a = [&](int i) { return fewrows_at<TM>(lane / TM + i * (64 / TM), lane % TM); };
-    auto dst_b = [&](int i) { return BK * G::BM + fewrows_at<TN>(lane / TN + i * (64 / TN), lane % TN); };
-    const int nb = n0 >> 7;
-    static_assert(128 % G::BN == 0, "a strip lies in one b_scale block");
-    int row_s[TM];
 #pragma unroll
-    for (int j = 0; j < TM; j++) row_s[j] = m0 + 16 * j + L < M ? m0 + 16 * j + L : M - 1;
-
-    // One K block on its way: raw bytes of A and B, scales. Bytes from the K block's first row to the end of the matrix
-    // are needed to cut the loads of the last rows (below 2^32 always suffices: a K block's own offsets are).
-    struct Block {
-        u32x4_lds a[NLA], b[NLB];
-        float sa[TM], sb;
-    };
-    auto rest = [&](int kb, int ld) -> uint32_t {
-        const unsigned long long r = (unsigned long long)(K - kb * BK) * (unsigned)ld;
+        for (int j = 0; j < TM; j++) {
+            const int row = m0 + 16 * j + (lane & 15);
+            row_s[j] = row < M ? row : M - 1;
+        }
+    }
+    __device__ __forceinline__ uint32_t off_a(int i) const { return off_a0 + (uint32_t)(i * (64 / TM)) * (uint32_t)ldm; }
+    __device__ __forceinline__ uint32_t off_b(int i) const { return off_b0 + (uint32_t)(i * (64 / TN)) * (uint32_t)N; }
+    __device__ __forceinline__ uint32_t dst_a(int i) const { return fewrows_at<TM>(lane / TM + i * (64 / TM), lane % TM); }
+    __device__ __forceinline__ uint32_t dst_b(int i) const {
+        return BK * BM + fewrows_at<TN>(lane / TN + i * (64 / TN), lane % TN);
+    }
+    // Bytes from a K block's first row (column `skip` of it) to the end of the matrix, needed to cut the loads of the last
+    // rows (below 2^32 always suffices: a K block's own offsets are).
+    __device__ __forceinline__ uint32_t rest(int kb, int ld, int skip) const {
+        const unsigned long long r = (unsigned long long)(K - kb * BK) * (unsigned)ld - (unsigned)skip;
         return r < 0xffffffffull ? (uint32_t)r : 0xffffffffu;
-    };
-    auto fetch = [&](Block &x, int i) {
-        const int kb = kb_begin + wave + NW * i;
+    }
+    __device__ __forceinline__ void fetch(Block &x, int kb) const {
         const uint8_t *pb = B + (size_t)kb * BK * N, *pa = A + (size_t)kb * BK * ldm;
-        const uint32_t end_b = rest(kb, N), end_a = rest(kb, ldm);
+        const uint32_t end_b = rest(kb, N, 0), end_a = rest(kb, ldm, first);
 #pragma unroll
         for (int q = 0; q < NLB; q++) x.b[q] = load16<BYTES>(pb, off_b(q), end_b);
 #pragma unroll
         for (int q = 0; q < NLA; q++) x.a[q] = load16<true>(pa, off_a(q), end_a);
 #pragma unroll
         for (int j = 0; j < TM; j++) x.sa[j] = SA[(size_t)kb * ldm + row_s[j]];
-        x.sb = SB[(size_t)kb * QN + nb];
-    };
-    f32x4 acc[TM][TN];
-#pragma unroll
-    for (int j = 0; j < TM; j++)
-#pragma unroll
-        for (int i = 0; i < TN; i++) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const int krow = 32 * g + (L >> 1);
-    auto fragment = [&](uint32_t at, int pitch) {                     // four transpose reads, 8 rows apart
+        x.sb = SB[(size_t)kb * QN + nb + zero];
+    }
+    __device__ __forceinline__ i32x8 fragment(uint32_t at, int pitch) const {       // four transpose reads, 8 rows apart
         i32x8 f;
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -153,10 +142,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_fp8_blockscale_fewrows(
             f[2 * t + 1] = v[1];
         }
         return f;
-    };
+    }
     // rows 8 t further on lie at a fixed distance except in regions of one-chunk rows, whose every second 32-row group
     // is moved by 8 rows: row ^ 8 there
-    auto fragment_1 = [&](uint32_t base) {
+    __device__ __forceinline__ i32x8 fragment_1(uint32_t base, int krow, int L) const {
         i32x8 f;
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -166,11 +155,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_fp8_blockscale_fewrows(
             f[2 * t + 1] = v[1];
         }
         return f;
-    };
-    auto consume = [&](Block &x, int i) {
-        const int kb = kb_begin + wave + NW * i;
-        if (kb == QK - 1) {                                           // only the matrix's last rows have cut loads
-            const uint32_t end_b = rest(kb, N), end_a = rest(kb, ldm);
+    }
+    // The bytes of the block into the region. Its registers are free afterwards, but for the scales.
+    __device__ __forceinline__ void stage(Block &x, int kb) const {
+        if (kb == K / BK - 1) {                                       // only the matrix's last rows have cut loads
+            const uint32_t end_b = rest(kb, N, 0), end_a = rest(kb, ldm, first);
             if constexpr (BYTES)
 #pragma unroll
                 for (int q = 0; q < NLB; q++) x.b[q] = shift_back(x.b[q], off_b(q), end_b);
@@ -181,33 +170,88 @@ __global__ __launch_bounds__(NW * 64) void gemm_fp8_blockscale_fewrows(
         for (int q = 0; q < NLB; q++) *(u32x4_lds *)(region + dst_b(q)) = x.b[q];
 #pragma unroll
         for (int q = 0; q < NLA; q++) *(u32x4_lds *)(region + dst_a(q)) = x.a[q];
+    }
+    // The products of the staged block: use(j, c, p) for every 16 x 16 tile, p summed from zero.
+    template <typename Use>
+    __device__ __forceinline__ void multiply(Use use) const {
+        const int L = lane & 15, krow = 32 * (lane >> 4) + (L >> 1);
         i32x8 bf[TN], af[TM];
 #pragma unroll
         for (int c = 0; c < TN; c++)
-            bf[c] = TN == 1 ? fragment_1(BK * G::BM) : fragment(BK * G::BM + fewrows_at<TN>(krow, c) + 8 * (L & 1), G::BN);
+            bf[c] = TN == 1 ? fragment_1(BK * BM, krow, L) : fragment(BK * BM + fewrows_at<TN>(krow, c) + 8 * (L & 1), BN);
 #pragma unroll
         for (int c = 0; c < TM; c++)
-            af[c] = TM == 1 ? fragment_1(0) : fragment(fewrows_at<TM>(krow, c) + 8 * (L & 1), G::BM);
+            af[c] = TM == 1 ? fragment_1(0, krow, L) : fragment(fewrows_at<TM>(krow, c) + 8 * (L & 1), BM);
 #pragma unroll
-        for (int j = 0; j < TM; j++) {
+        for (int j = 0; j < TM; j++)
+#pragma unroll
+            for (int c = 0; c < TN; c++)
+                use(j, c, __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[c], af[j], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0,
+                                                                           0, 0));
+    }
+};
+
+// Stores a lane's C[m][n .. n + 3] of tile t of a workgroup's tile.
+template <int TN>
+__device__ __forceinline__ void fewrows_store(uint16_t *C, int M, int N, int m0, int n0, int t, int lane, const f32x4 &s) {
+    const int m = m0 + 16 * (t / TN) + (lane & 15), n = n0 + 16 * (t % TN) + 4 * (lane >> 4);
+    if (m >= M) return;
+    uint16_t *out = C + (size_t)m * N + n;
+    const uint32_t lo = pack_bf16x2(s[0], s[1]), hi = pack_bf16x2(s[2], s[3]);
+    if (n + 4 <= N && ((uintptr_t)out & 7) == 0) {
+        *(uint2 *)out = make_uint2(lo, hi);
+    } else {
+        if (n < N) out[0] = (uint16_t)lo;
+        if (n + 1 < N) out[1] = (uint16_t)(lo >> 16);
+        if (n + 2 < N) out[2] = (uint16_t)hi;
+        if (n + 3 < N) out[3] = (uint16_t)(hi >> 16);
+    }
+}
+
+// Grid: x = column strips * row blocks (row blocks innermost: they share the strip's B), y = K splits of kb_per_split
+// blocks, every split at least one. A [K][ldm] (M of the ldm columns belong to this problem), SA [K/128][ldm], B [K][N],
+// C [M][N]. Any M, N >= 1, any alignment of A, B and C; ldm and N below 2^25 (32-bit offsets inside a K block). BYTES
+// false needs N % 16 == 0 and a 16-byte aligned B. SPLIT (gridDim.y > 1): counters holds a zero per item (gridDim.x) and
+// is zero again afterwards, slots gridDim.x * gridDim.y * TM * TN KiB, 16-byte aligned.
+template <int TM, int TN, int NW, int DEPTH, bool SPLIT, bool BYTES>
+__global__ __launch_bounds__(NW * 64, (FewRowsGeom<TM, TN, NW, DEPTH>::WAVES_PER_SIMD)) void gemm_fp8_blockscale_fewrows(
+    const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
+    const float *__restrict__ SB, uint16_t *__restrict__ C, int M, int ldm, int N, int K, int kb_per_split, int row_blocks,
+    unsigned *__restrict__ counters, float *__restrict__ slots) {
+    using G = FewRowsGeom<TM, TN, NW, DEPTH>;
+    using W = FewRowsWave<TM, TN, BYTES>;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // neighbouring strips on one XCD: a 32-column piece of a row of B is a quarter of a cache line
+    const int xcd = blockIdx.x % NUM_XCD, idx = blockIdx.x / NUM_XCD, per = gridDim.x / NUM_XCD, rem = gridDim.x % NUM_XCD;
+    const int item = xcd * per + (xcd < rem ? xcd : rem) + idx;
+    const int n0 = item / row_blocks * G::BN, m0 = item % row_blocks * G::BM;
+    const int QK = K / BK;
+    const int kb_begin = blockIdx.y * kb_per_split, kb_end = kb_begin + kb_per_split < QK ? kb_begin + kb_per_split : QK;
+    const int count = (kb_end - kb_begin - wave + NW - 1) / NW;       // this wave's K blocks: kb_begin + wave + NW * i
+    const W w(A, B, SA, SB, M, 0, ldm, N, K, m0, n0, lds + wave * G::REGION, lane);
+    auto kb_of = [&](int i) { return kb_begin + wave + NW * i; };
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int j = 0; j < TM; j++)
+#pragma unroll
+        for (int i = 0; i < TN; i++) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto consume = [&](typename W::Block &x, int i) {
+        w.stage(x, kb_of(i));
+        w.multiply([&](int j, int c, const f32x4 &p) {
             const float s = x.sa[j] * x.sb;
 #pragma unroll
-            for (int c = 0; c < TN; c++) {
-                const f32x4 p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[c], af[j], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0,
-                                                                                 0, 0, 0, 0);
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[j][c][e] = __builtin_fmaf(s, p[e], acc[j][c][e]);
-            }
-        }
+            for (int e = 0; e < 4; e++) acc[j][c][e] = __builtin_fmaf(s, p[e], acc[j][c][e]);
+        });
     };
 
     // up to DEPTH K blocks asked for, then used in order; straight-line code for every count, so that each wait is for a
     // known number of younger loads
     auto batch = [&](auto count_c, int i) {
         constexpr int n = decltype(count_c)::value;
-        Block x[n];
+        typename W::Block x[n];
 #pragma unroll
-        for (int d = 0; d < n; d++) fetch(x[d], i + d);
+        for (int d = 0; d < n; d++) w.fetch(x[d], kb_of(i + d));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int d = 0; d < n; d++) {
@@ -229,27 +273,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_fp8_blockscale_fewrows(
 #pragma unroll
         for (int c = 0; c < TN; c++) *(f32x4 *)(lds + ((wave * TM + j) * TN + c) * 1024 + lane * 16) = acc[j][c];
     __syncthreads();
-    auto store = [&](int t, const f32x4 &s) {                         // lane holds C[m][n .. n + 3] of tile t
-        const int m = m0 + 16 * (t / TN) + L, n = n0 + 16 * (t % TN) + 4 * g;
-        if (m >= M) return;
-        uint16_t *out = C + (size_t)m * N + n;
-        const uint32_t lo = pack_bf16x2(s[0], s[1]), hi = pack_bf16x2(s[2], s[3]);
-        if (n + 4 <= N && ((uintptr_t)out & 7) == 0) {
-            *(uint2 *)out = make_uint2(lo, hi);
-        } else {
-            if (n < N) out[0] = (uint16_t)lo;
-            if (n + 1 < N) out[1] = (uint16_t)(lo >> 16);
-            if (n + 2 < N) out[2] = (uint16_t)hi;
-            if (n + 3 < N) out[3] = (uint16_t)(hi >> 16);
-        }
-    };
+    auto store = [&](int t, const f32x4 &s) { fewrows_store<TN>(C, M, N, m0, n0, t, lane, s); };
     const int splits = gridDim.y;
     float *mine = slots + ((size_t)item * splits + blockIdx.y) * (TM * TN * 256) + lane * 4;
     for (int t = wave; t < TM * TN; t += NW) {
         f32x4 s = *(const f32x4 *)(lds + t * 1024 + lane * 16);
 #pragma unroll
-        for (int w = 1; w < NW; w++) {
-            const f32x4 v = *(const f32x4 *)(lds + (w * TM * TN + t) * 1024 + lane * 16);
+        for (int u = 1; u < NW; u++) {
+            const f32x4 v = *(const f32x4 *)(lds + (u * TM * TN + t) * 1024 + lane * 16);
             s[0] += v[0]; s[1] += v[1]; s[2] += v[2]; s[3] += v[3];
         }
         if constexpr (SPLIT) {
@@ -289,6 +320,170 @@ __global__ __launch_bounds__(NW * 64) void gemm_fp8_blockscale_fewrows(
             store(t, s);
         }
     }
+}
+
+// Grouped forms for groups of a few rows each (an expert layer in decode): what counts is streaming every group's weights,
+// N * K bytes each. A is read where the caller has it, at any byte and with a group starting at any column, so nothing is
+// staged; the sums are those of the tiled forms to the bit, K blocks in order.
+// Grid as for gemm_fp8_blockscale_grouped, a work item being a strip of columns and a block of 16 TM rows (row blocks of a
+// strip side by side). table.row_start[g]: column of A at which group g starts (any number), out_row_start: its rows of C
+// and their number. N % 16 == 0, B 16-byte aligned.
+//
+// First form: every wave has columns of its own and walks all of K with DEPTH K blocks on their way in registers; the waves
+// share nothing, so there is no barrier. Strips of 128 columns (TN = 8): a load instruction then covers eight whole cache
+// lines, and all strips of a launch are resident at once. Narrower strips ran at half the rate: 32 groups of 48 rows in all,
+// 2048 x 7168 (382 MB of weights), columns per wave 16: 228 us, 32: 139, 64: 100, 128: 75 us with two K blocks on their
+// way (5.1 TB/s) against 96.7 us for the tiled form with its staging copy. Bound by the streaming of B; with fewer than
+// about one strip per compute unit by the chain of 56 loads (0.95 us each).
+template <int TM, int TN, int NW, int DEPTH, int WAVES_PER_SIMD>
+__global__ __launch_bounds__(NW * 64, WAVES_PER_SIMD) void gemm_fp8_blockscale_grouped_strips(
+    const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
+    const float *__restrict__ SB, uint16_t *__restrict__ C, int M_total, int N, int K, int groups, const GroupTable table) {
+    using W = FewRowsWave<TM, TN, false>;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    int grp, local;
+    if (!grouped_work_item(table, groups, grp, local)) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int out0 = table.out_row_start[grp], rows = table.out_row_start[grp + 1] - out0;
+    const int row_blocks = (rows + 16 * TM - 1) / (16 * TM);
+    const int m0 = local % row_blocks * (16 * TM), n0 = (local / row_blocks * NW + wave) * (16 * TN);
+    if (n0 >= N) return;                                              // waves share nothing
+    const int QK = K / BK, QN = (N + 127) / 128;
+    W w(A, B + (size_t)grp * K * N, SA, SB + (size_t)grp * QK * QN, rows, table.row_start[grp], M_total, N, K, m0, n0,
+        lds + wave * (BK * 16 * (TM + TN)), lane);
+    // b_scale's index in a vector register: a scalar load on its way would make every wait for LDS a wait for memory
+    asm("" : "+v"(w.zero));
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int j = 0; j < TM; j++)
+#pragma unroll
+        for (int c = 0; c < TN; c++) acc[j][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    typename W::Block x[DEPTH];
+    auto fetch = [&](typename W::Block &b, int kb) { w.fetch(b, kb < QK ? kb : QK - 1); };   // (past the end: not used)
+    auto step = [&](typename W::Block &b, int kb, auto more) {
+        w.stage(b, kb);
+        float s[TM];
+#pragma unroll
+        for (int j = 0; j < TM; j++) s[j] = b.sa[j] * b.sb;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(more)::value) fetch(b, kb + DEPTH);
+        __builtin_amdgcn_sched_barrier(0);
+        w.multiply([&](int j, int c, const f32x4 &p) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[j][c][e] = __builtin_fmaf(s[j], p[e], acc[j][c][e]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) fetch(x[d], d);
+    int kb = 0;
+    for (; kb + DEPTH < QK; kb += DEPTH)
+#pragma unroll
+        for (int d = 0; d < DEPTH; d++) step(x[d], kb + d, IntTag<1>{});
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++)
+        if (kb + d < QK) step(x[d], kb + d, IntTag<0>{});
+#pragma unroll
+    for (int j = 0; j < TM; j++)
+#pragma unroll
+        for (int c = 0; c < TN; c++) fewrows_store<TN>(C + (size_t)out0 * N, rows, N, m0, n0, j * TN + c, lane, acc[j][c]);
+}
+
+// Second form, for launches of few strips: the waves of a workgroup take K blocks in turn. After every round of NW K blocks
+// they leave the blocks' products and scales in their regions, and the wave that holds an output tile folds them in K order;
+// the next rounds' loads stay in flight across the round's two barriers. 8 groups of 2 rows, 2048 x 7168: 76 us (tiled) and
+// 54 us (first form) -> 36 us; with four strips per compute unit the barriers cost more than the parallel chain saves.
+template <int TM, int TN, int NW, int DEPTH, int WAVES_PER_SIMD>
+__global__ __launch_bounds__(NW * 64, WAVES_PER_SIMD) void gemm_fp8_blockscale_grouped_ksplit(
+    const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
+    const float *__restrict__ SB, uint16_t *__restrict__ C, int M_total, int N, int K, int groups, const GroupTable table) {
+    using W = FewRowsWave<TM, TN, false>;
+    constexpr int REGION = BK * 16 * (TM + TN), SCALES = TM * TN * 1024;
+    static_assert(SCALES + TM * 64 <= REGION, "a round's products and scales take the place of its operands");
+    constexpr int TILES = (TM * TN + NW - 1) / NW;                    // output tiles a wave folds: wave, wave + NW, ...
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    int grp, local;
+    if (!grouped_work_item(table, groups, grp, local)) return;
+    const int out0 = table.out_row_start[grp], rows = table.out_row_start[grp + 1] - out0;
+    const int row_blocks = (rows + 16 * TM - 1) / (16 * TM);
+    const int m0 = local % row_blocks * (16 * TM), n0 = local / row_blocks * (16 * TN);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int QK = K / BK, QN = (N + 127) / 128, rounds = (QK + NW - 1) / NW;
+    uint8_t *region = lds + wave * REGION;
+    W w(A, B + (size_t)grp * K * N, SA, SB + (size_t)grp * QK * QN, rows, table.row_start[grp], M_total, N, K, m0, n0, region,
+        lane);
+    asm("" : "+v"(w.zero));
+    typename W::Block x[DEPTH];
+    // a wave without a K block in the last round asks for the last one and does not use it
+    auto fetch = [&](typename W::Block &b, int r) {
+        const int kb = r * NW + wave;
+        w.fetch(b, kb < QK ? kb : QK - 1);
+    };
+    f32x4 acc[TILES];
+#pragma unroll
+    for (int i = 0; i < TILES; i++) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    constexpr int H = NW < 4 ? NW : 4;
+    auto fold = [&](f32x4 &sum, int t) {
+        const uint8_t *at = lds + t * 1024 + lane * 16, *at_s = lds + SCALES + t / TN * 64 + (lane & 15) * 4;
+#pragma unroll
+        for (int b0 = 0; b0 < NW; b0 += H) {
+            f32x4 p[H];
+            float s[H];
+#pragma unroll
+            for (int b = 0; b < H; b++) {
+                p[b] = *(const f32x4 *)(at + (b0 + b) * REGION);
+                s[b] = *(const float *)(at_s + (b0 + b) * REGION);
+            }
+#pragma unroll
+            for (int b = 0; b < H; b++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum[e] = __builtin_fmaf(s[b], p[b][e], sum[e]);
+        }
+    };
+    auto step = [&](typename W::Block &b, int r, auto more) {
+        const int kb = r * NW + wave;
+        float s[TM];
+        if (kb < QK) {
+            w.stage(b, kb);
+#pragma unroll
+            for (int j = 0; j < TM; j++) s[j] = b.sa[j] * b.sb;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(more)::value) fetch(b, r + DEPTH);
+        __builtin_amdgcn_sched_barrier(0);
+        auto leave = [&](int j, int c, const f32x4 &p) { *(f32x4 *)(region + (j * TN + c) * 1024 + lane * 16) = p; };
+        if (kb < QK) {
+            w.multiply(leave);
+        } else {                                                      // -0 * 0 = -0, and x + -0 = x for every x
+#pragma unroll
+            for (int j = 0; j < TM; j++) {
+                s[j] = -0.f;
+#pragma unroll
+                for (int c = 0; c < TN; c++) leave(j, c, (f32x4){0.f, 0.f, 0.f, 0.f});
+            }
+        }
+        if (lane < 16)
+#pragma unroll
+            for (int j = 0; j < TM; j++) *(float *)(region + SCALES + j * 64 + lane * 4) = s[j];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TILES; i++)
+            if (wave + i * NW < TM * TN) fold(acc[i], wave + i * NW);
+        __syncthreads();
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) fetch(x[d], d);
+    int r = 0;
+    for (; r + DEPTH < rounds; r += DEPTH)
+#pragma unroll
+        for (int d = 0; d < DEPTH; d++) step(x[d], r + d, IntTag<1>{});
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++)
+        if (r + d < rounds) step(x[d], r + d, IntTag<0>{});
+#pragma unroll
+    for (int i = 0; i < TILES; i++)
+        if (wave + i * NW < TM * TN)
+            fewrows_store<TN>(C + (size_t)out0 * N, rows, N, m0, n0, wave + i * NW, lane, acc[i]);
 }
 
 }  // namespace rf

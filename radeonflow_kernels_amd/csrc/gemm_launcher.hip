@@ -454,7 +454,7 @@ bool skinny_ok(int m, int n, int k) {
 }
 
 // Few-rows kernels keep offsets inside a K block in 32 bits.
-bool fewrows_ok(int ldm, int n) { return ldm < (1 << 25) && n < (1 << 25); }
+bool fewrows_ok(long ldm, int n) { return ldm < (1 << 25) && n < (1 << 25); }
 
 // Stream-K: at least one tile per workgroup (then a split tile has exactly two contributors, which is all the kernel
 // handles) and no more tiles than arrival counters.
@@ -1352,6 +1352,7 @@ struct GroupedVariant {
     bool mixed;          // 256-row tiles plus one shorter tile for what is left over (one 128-row tile for at most 128
                          // rows; the queue form: 64, 128, 192 or 256 rows)
     bool queue = false;  // resident workgroups that take tiles from per-XCD queues (gemm_fp8_blockscale_grouped_queue)
+    bool fewrows = false;  // fp8_gemm_fewrows.h: groups may start at any row of a
     // row tiles of a group of `rows` rows
     int tiles_m(int rows) const {
         if (!mixed) return ceil_div(rows, bm);
@@ -1361,13 +1362,20 @@ struct GroupedVariant {
 
 #define RF_GROUPED(BM, BN, WM, WN, NS) \
     GroupedVariant { BM, BN, WM *WN * 64, rf::TileGeom<BM, BN, WM, WN, NS>::LDS_BYTES, rf::gemm_fp8_blockscale_grouped<BM, BN, WM, WN, NS>, false }
+#define RF_GROUPED_FEWROWS(KERNEL, TM, COLUMNS, TN, NW, DEPTH, WAVES_PER_SIMD)                    \
+    GroupedVariant { 16 * TM, COLUMNS, 64 * NW, NW *rf::BK * 16 * (TM + TN),                       \
+                     rf::KERNEL<TM, TN, NW, DEPTH, WAVES_PER_SIMD>, false, false, true }
 constexpr int kMixedLds = rf::TileGeom<256, 256, 2, 4>::LDS_BYTES > rf::TileGeom<128, 256, 2, 4, 3>::LDS_BYTES
                               ? rf::TileGeom<256, 256, 2, 4>::LDS_BYTES : rf::TileGeom<128, 256, 2, 4, 3>::LDS_BYTES;
 const GroupedVariant kGroupedVariants[] = {
     RF_GROUPED(256, 256, 2, 4, 2), RF_GROUPED(128, 256, 2, 4, 3), RF_GROUPED(128, 128, 2, 2, 2), RF_GROUPED(128, 64, 2, 1, 2),
     GroupedVariant{256, 256, 512, kMixedLds, rf::gemm_fp8_blockscale_grouped_mixed, true},
-    GroupedVariant{256, 256, 512, rf::kQueueLds, nullptr, true, true}};
-constexpr int kGroupedMixed = 4, kGroupedQueue = 5;
+    GroupedVariant{256, 256, 512, rf::kQueueLds, nullptr, true, true},
+    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_strips, 1, 256, 8, 2, 2, 1),    // 6: 16 rows, two waves of 128 columns
+    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_strips, 1, 128, 8, 1, 1, 2),    // 7: 16 rows, one wave
+    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_strips, 2, 128, 8, 1, 1, 1),    // 8: 32 rows, one wave
+    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_ksplit, 1, 64, 4, 8, 1, 4)};    // 9: 16 rows, K split between eight waves
+constexpr int kGroupedMixed = 4, kGroupedQueue = 5, kGroupedFewRows = 6;
 // Estimated time of a 256-column tile of the queue form by its height in units of 64 rows, relative to a 256-row tile
 constexpr double kQueueTileCost[5] = {0.0, 0.68, 0.75, 0.97, 1.0};
 constexpr int kNumGroupedVariants = sizeof(kGroupedVariants) / sizeof(kGroupedVariants[0]);
@@ -1380,13 +1388,46 @@ long grouped_tiles(const GroupedVariant &v, const int *row_offsets, int groups, 
 }  // namespace
 
 namespace {
+// The few-rows form for these groups, or -1: groups of at most 16 rows (variants 6, 7 and 9) or 32 (variant 8); more rows
+// would stream the weights once per row block. Estimated time in us: the stream of the weights at the rate the form reaches
+// once the chip is full, or the chain of one wave's K blocks. Measured on 52 layouts (8 to 64 groups, 16 to 900 rows,
+// N x K = 2048 x 7168, 4096 x 7168, 7168 x 2048, 4096 x 2048) against the tiled forms with their staging copy: 3 to 50 %
+// faster wherever this picks one, 14 % on average; beyond 1 GB of weights, or max_rounds rounds of resident workgroups,
+// the tiled forms' steady state is as good or better (64 groups of 64 rows in all, 4096 x 7168: 306 us here, 284 tiled; of
+// 300 rows, 7168 x 2048: 210 against 191).
+int choose_grouped_fewrows(const int *row_offsets, int groups, int n, int k, int num_cu) {
+    int most = 0, busy = 0;
+    for (int g = 0; g < groups; g++) {
+        const int rows = row_offsets[g + 1] - row_offsets[g];
+        most = std::max(most, rows);
+        busy += rows > 0;
+    }
+    const double bytes = (double)busy * n * k;
+    if (most < 1 || most > 32 || n % 16 != 0 || bytes > 1.0e9 || !fewrows_ok((long)row_offsets[groups] + 16 * groups, n)) return -1;
+    struct Form { int variant, wgs_per_cu; double max_rounds, start, per_k_block, bytes_per_us; };
+    const Form forms[] = {{6, 2, 3.0, 4.0, 1.0, 5.1e6}, {7, 8, 1.0, 3.5, 0.93, 4.6e6}, {8, 4, 2.0, 3.0, 1.2, 5.0e6},
+                          {9, 2, 1.0, 3.0, 0.0, 3.3e6}};
+    int best = -1;
+    double best_t = 0;
+    for (const Form &f : forms) {
+        const GroupedVariant &v = kGroupedVariants[f.variant];
+        const double rounds = (double)busy * ceil_div(n, v.bn) / (f.wgs_per_cu * num_cu);
+        if (most > v.bm || rounds > f.max_rounds) continue;
+        const double t = std::max(f.start + f.per_k_block * (k / rf::BK), 3.0 + bytes / f.bytes_per_us * 256.0 / num_cu);
+        if (best < 0 || t < best_t) { best = f.variant; best_t = t; }
+    }
+    return best;
+}
+
 // The automatic choice of rf_fp8_gemm_grouped (variant = -1) for groups of these sizes on a device with num_cu compute units.
 int choose_grouped_variant(const int *row_offsets, int groups, int n, int k, int num_cu) {
+    const int few = choose_grouped_fewrows(row_offsets, groups, n, k, num_cu);
+    if (few >= 0) return few;
     // the largest tile that still gives every CU a workgroup; failing that, the one with the most workgroups
     int variant = -1;
     long most = -1;
     int most_v = 0;
-    for (int v = 0; v < kNumGroupedVariants && variant < 0; v++) {
+    for (int v = 0; v < kGroupedFewRows && variant < 0; v++) {
         const long t = grouped_tiles(kGroupedVariants[v], row_offsets, groups, n);
         if (t >= num_cu) variant = v;
         if (t > most) { most = t; most_v = v; }
@@ -1495,9 +1536,13 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
         }
         return RF_OK;
     }
+    if (variant < 0) variant = choose_grouped_variant(row_offsets, groups, n, k, s.num_cu);
+    const GroupedVariant &v = kGroupedVariants[variant];
+    if (v.fewrows && !fewrows_ok((long)m_total + 16 * groups, n))
+        return fail(RF_ERR_BAD_CONFIG, "the few-rows forms need fewer than 2^25 rows and columns");
     rf::GroupTable table;
     int m_rows = m_total;                      // rows of the A matrix the kernel reads
-    if (stage) {
+    if (stage && !v.fewrows) {
         // Group sizes that are not multiples of 16 (token counts per expert never are): A and a_scale are copied
         // into the staging buffer with every group starting at a multiple of 16, the kernel reads those and writes
         // each group's true rows straight into the caller's C. Costs one pass over A; the bounds-checked kernel
@@ -1534,8 +1579,6 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
         for (int g = 0; g <= rf::kMaxGroups; g++)
             table.row_start[g] = table.out_row_start[g] = row_offsets[g < groups ? g : groups];
     }
-    if (variant < 0) variant = choose_grouped_variant(row_offsets, groups, n, k, s.num_cu);
-    const GroupedVariant &v = kGroupedVariants[variant];
     const int tiles_n = ceil_div(n, v.bn);
     int tiles = 0;
     for (int g = 0; g < groups; g++) {

@@ -259,3 +259,16 @@ def test_grouped_variant_choice_on_the_host():
     for bad in (([0, 16, 8], 256, 256), ([1, 16], 256, 256), ([0, 16], 256, 100), ([0, 16], 0, 256)):
         with pytest.raises(RuntimeError):
             rfk.grouped_variant_for(*bad)
+
+
+def test_grouped_few_rows_choice_on_the_host():
+    """Groups of up to 16 rows take a few-rows form (6, 7 or 9), up to 32 rows the 32-row one (8); longer groups, ragged widths
+    and more than 1 GB of weights keep the tiled forms."""
+    import radeonflow_kernels_amd as rfk
+
+    def choice(rows, groups, n, k):
+        return rfk.grouped_variant_for([rows * g for g in range(groups + 1)], n, k)
+
+    assert choice(2, 8, 2048, 7168) == 9 and choice(2, 16, 2048, 7168) == 7 and choice(16, 32, 2048, 7168) == 6
+    assert choice(17, 32, 2048, 7168) == 8 and choice(32, 32, 2048, 7168) == 8
+    assert choice(33, 32, 2048, 7168) < 6 and choice(16, 32, 2056, 7168) < 6 and choice(16, 64, 4096, 7168) < 6

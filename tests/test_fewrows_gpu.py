@@ -87,3 +87,39 @@ def test_fewrows_static_entry_and_graph_replay(rfk):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(bf16_bits(g[4]), exp), "replay %d" % rep
+
+
+# groups at the edges of the 16 and 32 row blocks and over them, idle ones, starting at any byte; K blocks fewer than, as many as
+# and no multiple of a workgroup's waves; widths that end inside a 256, 128 and 64 column strip
+@pytest.mark.parametrize("rows,n,k", [([1], 16, 2048), ([3, 0, 16, 17, 1, 32, 33], 144, 1152), ([15, 16, 48], 272, 128),
+                                      ([0, 2, 70, 5] * 3, 320, 3328), ([int(x) for x in np.arange(64) % 5], 256, 1024)])
+@pytest.mark.parametrize("shift", [0, 5])
+def test_grouped_fewrows_bits_of_the_tiled_form(rfk, rows, n, k, shift):
+    """Rounding in every product: the few-rows forms sum K blocks in order and so give the bits of the 128 x 256 tiles, on
+    operands back to back (a at any byte, its buffer ending with it) and in the padded layout; rows of C past the groups keep
+    their fill."""
+    fp8, groups = torch.float8_e4m3fn, len(rows)
+    offs = [0] + [int(x) for x in np.cumsum(rows)]
+    m = offs[-1]
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    raw = torch.randint(0, 120, (k * m + shift,), dtype=torch.uint8, device="cuda", generator=gen)
+    a = raw[shift:].view(k, m).view(fp8).T
+    b = torch.randint(0, 120, (groups, k, n), dtype=torch.uint8, device="cuda", generator=gen).view(fp8).permute(0, 2, 1)
+    sa = (torch.rand((k // 128, m), device="cuda", generator=gen) * 1e-2).T
+    sb = (torch.rand((groups, k // 128, (n + 127) // 128), device="cuda", generator=gen) * 1e-2).permute(0, 2, 1)
+    pad = rfk.grouped_padded_offsets(offs)
+    a_pad, sa_pad = torch.zeros((k, pad[-1]), dtype=torch.uint8, device="cuda"), torch.ones((k // 128, pad[-1]), device="cuda")
+    for g in range(groups):
+        a_pad[:, pad[g]:pad[g] + rows[g]] = a.T.view(torch.uint8)[:, offs[g]:offs[g + 1]]
+        sa_pad[:, pad[g]:pad[g] + rows[g]] = sa.T[:, offs[g]:offs[g + 1]]
+
+    def launch(call, x, sx, variant):
+        buf = torch.full((m * n + 300,), -7.0, dtype=torch.bfloat16, device="cuda")
+        call(x, b, sx, sb, buf[:m * n].view(m, n), offs, variant=variant)
+        torch.cuda.synchronize()
+        return bf16_bits(buf)
+
+    expect = launch(rfk.fp8_mm_grouped, a, sa, 1)
+    for variant in (6, 7, 8, 9, -1):
+        assert np.array_equal(launch(rfk.fp8_mm_grouped, a, sa, variant), expect), variant
+        assert np.array_equal(launch(rfk.fp8_mm_grouped_padded, a_pad.view(fp8).T, sa_pad.T, variant), expect), variant
