@@ -59,7 +59,7 @@ enum { RF_SCHEDULE_TILES = 0, RF_SCHEDULE_STREAM_K = 1, RF_SCHEDULE_PERSISTENT =
  * Replaces a DISPATCH_GEMM(...) line of the reference (src/gemm/gemm_launcher.cpp:158-162,229-259). */
 typedef struct rf_gemm_config {
     int variant;      /* index into the variant table, see rf_gemm_variant_info(); -1 = bounds-checked kernel. Variants 14
-                         to 20 are the few-rows kernels (16 to 64 rows x 32 to 128 columns per workgroup): any shape with
+                         to 21 are the few-rows kernels (16 to 64 rows x 32 to 128 columns per workgroup): any shape with
                          M and N below 2^25, any alignment, K splits summed inside the launch */
     int split_k;      /* >= 1; K blocks are divided over this many partial sums */
     int group_m;      /* tile-order grouping along M for L2 reuse (>=1) */

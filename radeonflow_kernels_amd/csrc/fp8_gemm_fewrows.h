@@ -39,7 +39,8 @@ struct FewRowsGeom {
     static constexpr int REGION = BK * (BM + BN);                     // one K block of A and of B, private to a wave
     static constexpr int EXCHANGE = NW * TM * TN * 1024;              // the waves' sums, over the regions
     static constexpr int LDS_BYTES = NW * REGION > EXCHANGE ? NW * REGION : EXCHANGE;
-    static constexpr int WAVES_PER_SIMD = LDS_BYTES < 80 * 1024 ? 4 : 2;   // two workgroups of eight waves, where LDS has room
+    // waves per SIMD: two workgroups per CU, where LDS has room
+    static constexpr int WAVES_PER_SIMD = (LDS_BYTES < 80 * 1024 ? 2 : 1) * NW / 4;
     static_assert(LDS_BYTES <= 160 * 1024, "the waves' regions fit the CU's LDS");
     static_assert((TM & (TM - 1)) == 0 && (TN & (TN - 1)) == 0, "powers of two: the chunk swizzle stays inside a row");
 };

@@ -128,6 +128,8 @@ const Variant kVariants[] = {
     RF_VARIANT_FEWROWS(2, 4, 8, 2),   // 18: 32 x 64
     RF_VARIANT_FEWROWS(4, 2, 8, 2),   // 19: 64 x 32
     RF_VARIANT_FEWROWS(4, 4, 8, 1),   // 20: 64 x 64
+    RF_VARIANT_FEWROWS(4, 4, 4, 1),   // 21: 64 x 64, four waves: two workgroups per CU (200 x 5003 x 2048, 316 workgroups:
+                                      // one round of the chip instead of two, 23.2 -> 19.8 us)
 };
 constexpr int kFewRows64x64 = 20;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
@@ -485,7 +487,7 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
     struct Fit { int variant, per_cu, depth; double b, c, d; };
     const Fit fits[] = {{14, 2, 3, 0.0, 0.458, 0.0916},   {15, 1, 2, 0.0, 0.860, 0.0591},   {16, 1, 1, 0.790, 0.665, 0.0381},
                         {17, 2, 2, 0.0, 0.572, 0.0755},   {18, 1, 2, 0.101, 1.090, 0.0546}, {19, 1, 2, 0.127, 1.063, 0.0593},
-                        {20, 1, 1, 1.651, 0.929, 0.0362}};
+                        {20, 1, 1, 1.651, 0.929, 0.0362},   {21, 2, 1, 2.48, 0.424, 0.0231}};
     const int splits_tried[] = {1, 2, 3, 4, 5, 6, 8, 12, 14}, qk = k / rf::BK;
     double best = 1e30;
     for (const Fit &f : fits) {
@@ -508,7 +510,10 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
     }
     return best;
 }
-constexpr int kFewRowsMaxM = 512;                           // beyond this the estimate is not measured (and never the best)
+// Beyond these the estimate is not measured. Aligned rows of B: never the best. A staged copy of B costs a tiled plan three
+// launches and three passes over B and C, which variant 21 beats up to a few thousand rows: 700 x 5003 x 1024 36.4 -> 24.0 us,
+// 1000 x 1000 x 1024 19.4 -> 8.5, 2000 x 2003 x 1024 34.9 -> 24.0, 3000 x 1000 x 384 21.0 -> 11.0.
+constexpr int kFewRowsMaxM = 512, kFewRowsMaxMStagedB = 4096;
 
 // What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
 // (and of C on the way back).
@@ -630,7 +635,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // what their launches take is 3.1 us + 0.67 of its figure, and staging adds the copies' launches and bytes
     // (fitted to the same measurements as fewrows_plan). Over 280 shapes the choice between the two families is within 4 %
     // of the best plan of either, on average.
-    if (m <= kFewRowsMaxM && fewrows_ok(m, n)) {
+    if (m <= (stage & kStageB ? kFewRowsMaxMStagedB : kFewRowsMaxM) && fewrows_ok(m, n)) {
         double tiled = 3.1 + 0.67 * best_cost;
         if (stage & kStageA) tiled += 3.2 + 2.0 * k * m / 4e6;
         if (stage & kStageB) tiled += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;

@@ -1,4 +1,4 @@
-"""The few-rows kernels (variants 14 to 20): any shape and alignment, K split between waves and between workgroups."""
+"""The few-rows kernels (variants 14 to 21): any shape and alignment, K split between waves and between workgroups."""
 import numpy as np
 import pytest
 import torch
@@ -6,7 +6,7 @@ import torch
 from helpers import bf16_bits, exact_problem, oracle_bf16, to_gpu
 
 pytestmark = pytest.mark.gpu
-FEW_ROWS = range(14, 21)
+FEW_ROWS = range(14, 22)
 
 
 @pytest.fixture(scope="module")
