@@ -853,8 +853,8 @@ constexpr double kPadThresholdMacs = 2097152.0;            // below this the bou
 // pieces of kPadRows rows when rows are longer), and every thread finds its group by a search in LDS instead of a walk
 // over the kernel argument. A source piece starts at any byte and is one unaligned 16-byte load, cut at the end of the matrix.
 // 1001 x 7168 bytes: 7.7 -> 6.8 us (rocprofv3), 48 rows in 32 groups x 7168: 10.6 -> 5.8 us, 2.8 us of either being what
-// the shortest kernel takes.
-constexpr int kPadRows = 4;
+// the shortest kernel takes; two rounds instead of four, so twice the workgroups: 601x3072x1536 14.3 -> 13.3 us.
+constexpr int kPadRows = 2;
 template <typename T>
 __device__ __forceinline__ void pad_group_rows_body(const T *__restrict__ src, int first, int m_total, int m_pad, int rows,
                                                     int groups, T *__restrict__ dst, const rf::GroupTable &table,
@@ -942,10 +942,38 @@ __global__ __launch_bounds__(256) void pad_group_rows_a_and_scales(const uint8_t
                                    blockIdx.y);
 }
 
-// grid of pad_group_rows for `rows` rows of m_pad elements of `size` bytes
-dim3 pad_grid(int m_pad, int size, int rows) {
-    const int pieces = m_pad / (16 / size), per_block = kPadRows * (pieces < 256 ? 256 / pieces : 1);
+// The way back: the first n columns of C's padded copy [rows][ld], ld a multiple of 16, to the caller's [rows][n]. The same
+// split, a piece per thread; a piece is one aligned load and one 16-byte store at any element, the last piece of a row stored by elements.
+// (hipMemcpy2DAsync took 120 us for 6160 x 5003, a width whose rows start at odd elements: 6160 x 5003 x 2048 202 -> 104 us.)
+__global__ __launch_bounds__(256) void unpad_rows_bf16(const uint16_t *__restrict__ src, int ld, int n, int rows,
+                                                       uint16_t *__restrict__ dst) {
+    const int pieces = (n + 7) / 8;
+    const int per_block = pieces < 256 ? 256 / pieces : 1;
+    const int trow = pieces < 256 ? (int)threadIdx.x / pieces : 0;
+    const int piece = pieces < 256 ? (int)threadIdx.x - trow * pieces : (int)(blockIdx.y * 256 + threadIdx.x);
+    const int r = (int)blockIdx.x * per_block + trow, col = piece * 8;
+    if (trow >= per_block || piece >= pieces || r >= rows) return;
+    const rf::u32x4_lds w = *(const rf::u32x4_lds *)(src + (size_t)r * ld + col);
+    uint16_t *out = dst + (size_t)r * n + col;
+    if (col + 8 <= n) {
+        *(rf::u32x4_any *)out = w;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 7; e++)
+            if (col + e < n) out[e] = (uint16_t)(w[e / 2] >> (16 * (e % 2)));
+    }
+}
+
+// grid of these copies for `rows` rows of `pieces` 16-byte pieces, `rounds` rows per thread
+dim3 pad_grid_of_pieces(int pieces, int rows, int rounds) {
+    const int per_block = rounds * (pieces < 256 ? 256 / pieces : 1);
     return dim3((unsigned)ceil_div(rows, per_block), (unsigned)ceil_div(pieces, 256));     // rows on x: no 65535 limit
+}
+dim3 pad_grid(int m_pad, int size, int rows) { return pad_grid_of_pieces(m_pad / (16 / size), rows, kPadRows); }
+
+void launch_unpad_rows(const void *src, int ld, int n, int rows, void *dst, hipStream_t stream) {
+    hipLaunchKernelGGL(unpad_rows_bf16, pad_grid_of_pieces(ceil_div(n, 8), rows, 1), dim3(256), 0, stream, (const uint16_t *)src,
+                       ld, n, rows, (uint16_t *)dst);
 }
 
 // Stages A and a_scale with one launch: columns first, first + 1, ... of matrices of m_total columns.
@@ -1023,9 +1051,10 @@ int launch_padded_in_pieces(State &s, Mem &mem, const void *a, const void *b, co
         void *c_piece = copy_c ? (void *)pc : (void *)((uint16_t *)c + (size_t)r0 * n);
         rc = launch_locked(s, mem, pa, b2, (const float *)psa, bs, c_piece, rp, np, k, &cfg, stream, copy_c ? rp : rows);
         if (rc != RF_OK) return rc;
-        if (copy_c)
-            RF_HIP(hipMemcpy2DAsync((uint16_t *)c + (size_t)r0 * n, (size_t)n * 2, pc, (size_t)np * 2, (size_t)n * 2, rows,
-                                    hipMemcpyDeviceToDevice, stream));
+        if (copy_c) {
+            launch_unpad_rows(pc, np, n, rows, (uint16_t *)c + (size_t)r0 * n, stream);
+            RF_HIP(hipGetLastError());
+        }
     }
     return RF_OK;
 }
@@ -1082,8 +1111,10 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     RF_HIP(hipGetLastError());
     rc = launch_locked(s, mem, a2, b2, as2, bs, c2, mp, np, k, &cfg, stream, copy_c ? mp : m);
     if (rc != RF_OK) return rc;
-    if (copy_c)
-        RF_HIP(hipMemcpy2DAsync(c, (size_t)n * 2, c2, (size_t)np * 2, (size_t)n * 2, m, hipMemcpyDeviceToDevice, stream));
+    if (copy_c) {
+        launch_unpad_rows(c2, np, n, m, c, stream);
+        RF_HIP(hipGetLastError());
+    }
     return RF_OK;
 }
 

@@ -23,3 +23,20 @@ def test_staged_rows_bit_exact(m):
     torch.cuda.synchronize()
     assert np.array_equal(bf16_bits(c), exp)
     assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
+
+
+# more rows than the few-rows kernels take with a ragged width, so the plan is a tiled one on staged copies: widths below a
+# piece of eight, rows of a workgroup's 256 pieces and a few more; c at an odd element
+@pytest.mark.parametrize("m,n,k,off_c", [(4112, 5, 512, 0), (4100, 130, 256, 0), (4128, 2045, 128, 1), (4099, 2057, 128, 0)])
+def test_staged_output_bit_exact(m, n, k, off_c):
+    import radeonflow_kernels_amd as rfk
+    data = exact_problem(m, n, k, seed=n)
+    exp = oracle_bf16(data)
+    g, _ = to_gpu(data, 300)
+    buf = torch.full((m * n + 300,), -7.0, dtype=torch.bfloat16, device="cuda")
+    c = buf[off_c:off_c + m * n].view(m, n)
+    rfk.fp8_mm(*g[:4], c)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits(c), exp)
+    rest = torch.cat([buf[:off_c], buf[off_c + m * n:]]).float()
+    assert float(rest.min()) == -7.0 == float(rest.max())
