@@ -510,7 +510,8 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
     }
     return best;
 }
-// Beyond these the estimate is not measured. Aligned rows of B: never the best. A staged copy of B costs a tiled plan three
+// Beyond these the estimate is not measured (the second one: on devices with kTunedOnCUs units only, others keep the first,
+// and with it the plans of their padded shapes). Aligned rows of B: never the best. A staged copy of B costs a tiled plan three
 // launches and three passes over B and C, which variant 21 beats up to a few thousand rows: 700 x 5003 x 1024 36.4 -> 24.0 us,
 // 1000 x 1000 x 1024 19.4 -> 8.5, 2000 x 2003 x 1024 34.9 -> 24.0, 3000 x 1000 x 384 21.0 -> 11.0.
 constexpr int kFewRowsMaxM = 512, kFewRowsMaxMStagedB = 4096;
@@ -635,7 +636,8 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // what their launches take is 3.1 us + 0.67 of its figure, and staging adds the copies' launches and bytes
     // (fitted to the same measurements as fewrows_plan). Over 280 shapes the choice between the two families is within 4 %
     // of the best plan of either, on average.
-    if (m <= (stage & kStageB ? kFewRowsMaxMStagedB : kFewRowsMaxM) && fewrows_ok(m, n)) {
+    const int max_m = (stage & kStageB) && num_cu == kTunedOnCUs ? kFewRowsMaxMStagedB : kFewRowsMaxM;
+    if (m <= max_m && fewrows_ok(m, n)) {
         double tiled = 3.1 + 0.67 * best_cost;
         if (stage & kStageA) tiled += 3.2 + 2.0 * k * m / 4e6;
         if (stage & kStageB) tiled += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
