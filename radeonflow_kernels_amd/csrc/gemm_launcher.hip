@@ -1471,6 +1471,13 @@ int choose_grouped_variant(const int *row_offsets, int groups, int n, int k, int
         if (t > most) { most = t; most_v = v; }
     }
     if (variant < 0) variant = most_v;
+    // Too few 128 x 256 tiles for every CU: a launch is the chain of one tile's K blocks, which is as long for the 128 x 64
+    // tiles as for the 128 x 128 ones (two stages) and 10 % longer for the 128 x 256 ones (three), so smaller tiles pay
+    // only while they are alone on their CU. us on N x K = 2048 x 7168 with tiles of 64, 128 and 256 columns: 1000 rows in 8
+    // groups 92, 71, 78; 3000 rows (more 128 x 128 tiles than CUs) 176, 102, 87; 4096 x 2048: 3000 rows 91, 65, 57. (Below
+    // K = 2048 not measured.)
+    if ((variant == 2 || variant == 3) && k >= 2048)
+        return grouped_tiles(kGroupedVariants[2], row_offsets, groups, n) <= num_cu ? 2 : 1;
     if (variant == 1) variant = 0;      // 128-row tiles fill the chip: the 256-wide family, chosen below
     // Enough tiles for the 256-wide family (128-row tiles would give every CU one): 256-row tiles, 128-row tiles
     // (three stages) or the mixed form, by a
@@ -1504,8 +1511,9 @@ int choose_grouped_variant(const int *row_offsets, int groups, int n, int k, int
             if (best_t == 0 || t < best_t) { best_t = t; variant = cand; }
         }
         // The queue form (tiles of 64 to 256 rows, resident workgroups): where its shorter last tiles save at least
-        // 7 % of the rows the chosen tiles compute and it has enough items to go round (1.5 per CU; 2.5 when K is
-        // below 4096 and an item is short against the cost of drawing it). Measured on 68 layouts (8 to 128 groups of
+        // 7 % of the rows the chosen tiles compute and it has enough items to go round (a few more than CUs; 2.5 per
+        // CU when K is below 4096 and an item is short against the cost of drawing it; K = 7168 and 1.1 to 1.4 items per
+        // CU: 166 -> 155, 178 -> 164, 162 -> 150 us, with no more items than CUs 107 -> 111). Measured on 68 layouts (8 to 128 groups of
         // uniform, exponential or equal sizes; N x K = 4096 x 7168, 7168 x 2048, 2048 x 7168, 4096 x 2048) against
         // the best of the four 256-wide forms: this rule 0.8 % behind on average, 11 % at worst; never the queue form
         // 4.6 % and 16 %; the queue form on row savings alone 2.2 % and 41 % (16 groups of 16..384 rows at
@@ -1518,7 +1526,7 @@ int choose_grouped_variant(const int *row_offsets, int groups, int n, int k, int
             rows_chosen += variant == 0 ? ceil_div(rows, 256) * 256 : variant == 1 ? ceil_div(rows, 128) * 128
                            : rows / 256 * 256 + (rows % 256 == 0 ? 0 : rows % 256 <= 128 ? 128 : 256);
         }
-        const long items_needed = k >= 4096 ? 3L * num_cu / 2 : 5L * num_cu / 2;
+        const long items_needed = k >= 4096 ? 17L * num_cu / 16 : 5L * num_cu / 2;
         if (rows_queue * 100 <= rows_chosen * 93 && items_queue >= items_needed) variant = kGroupedQueue;
     }
     return variant;
