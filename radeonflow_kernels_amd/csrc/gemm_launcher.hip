@@ -56,6 +56,8 @@ typedef void (*persistent_kernel_t)(const uint8_t *, const uint8_t *, const floa
                                     int, int, int, int, int);
 typedef void (*fewrows_kernel_t)(const uint8_t *, const uint8_t *, const float *, const float *, uint16_t *, int, int, int,
                                  int, int, int, unsigned *, float *);
+typedef void (*any_c_kernel_t)(const uint8_t *, const uint8_t *, const float *, const float *, uint16_t *, int, int, int, int,
+                               int, int, int, int);
 struct Variant {
     int bm, bn, waves_m, waves_n, lds;
     tile_kernel_t direct, partial;
@@ -65,22 +67,24 @@ struct Variant {
     persistent_kernel_t persistent_half_tail = nullptr;   // null: no form that ends with half tiles
     int k_groups = 1;                    // > 1: wave groups of one workgroup split K between them (needs K/128 % k_groups == 0)
     fewrows_kernel_t fewrows[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};   // [K split][any alignment of B]; null: a tiled variant
+    any_c_kernel_t any_c = nullptr;      // the direct form for a C of any width and alignment
     bool is_fewrows() const { return fewrows[0][0] != nullptr; }
     int lds_bytes() const { return lds; }
     int threads() const { return waves_m * waves_n * 64 * k_groups; }
 };
+#define RF_ANY_C(BM, BN, WM, WN, NS) nullptr, 1, {}, rf::gemm_fp8_blockscale_tile_any_c<BM, BN, WM, WN, NS>
 #define RF_VARIANT(BM, BN, WM, WN)                                                         \
     Variant { BM, BN, WM, WN, rf::TileGeom<BM, BN, WM, WN>::LDS_BYTES,                     \
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, false>,                         \
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true>,                          \
               rf::gemm_fp8_blockscale_streamk<BM, BN, WM, WN>,                             \
               rf::gemm_fp8_blockscale_persistent<BM, BN, WM, WN>,                          \
-              rf::PersistentGeom<BM, BN, WM, WN>::LDS_BYTES }
+              rf::PersistentGeom<BM, BN, WM, WN>::LDS_BYTES, RF_ANY_C(BM, BN, WM, WN, 2) }
 // tiles with sides that are not powers of two, same inner loop: one workgroup per tile only
 #define RF_VARIANT_TILE_ONLY(BM, BN, WM, WN)                                               \
     Variant { BM, BN, WM, WN, rf::TileGeom<BM, BN, WM, WN>::LDS_BYTES,                     \
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, false>,                         \
-              rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true>, nullptr, nullptr, 0 }
+              rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true>, nullptr, nullptr, 0, RF_ANY_C(BM, BN, WM, WN, 2) }
 // the same with three LDS stages: two K blocks in flight instead of one. A K block of these tiles is 0.4 us of MFMAs,
 // less than a load takes to come back from L2 or the Infinity Cache on a busy chip, so with two stages the loop ran at
 // the latency of its loads: 1024 x 4608 x 7168 45.6 -> 39.0 us, 256 x 7168 x 2304 15.6 -> 13.1 us; the best plan of 86
@@ -89,7 +93,7 @@ struct Variant {
 #define RF_VARIANT_TILE_ONLY_NS3(BM, BN, WM, WN)                                           \
     Variant { BM, BN, WM, WN, rf::TileGeom<BM, BN, WM, WN, 3>::LDS_BYTES,                  \
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, false, 3>,                      \
-              rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true, 3>, nullptr, nullptr, 0 }
+              rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true, 3>, nullptr, nullptr, 0, RF_ANY_C(BM, BN, WM, WN, 3) }
 // few-rows kernels (fp8_gemm_fewrows.h): any shape, any alignment, K splits reduced inside the launch
 #define RF_VARIANT_FEWROWS(TM, TN, NW, DEPTH)                                              \
     Variant { 16 * TM, 16 * TN, 1, NW, rf::FewRowsGeom<TM, TN, NW, DEPTH>::LDS_BYTES,      \
@@ -102,7 +106,8 @@ const Variant kVariants[] = {
     Variant{256, 256, 2, 4, rf::TileGeom<256, 256, 2, 4>::LDS_BYTES, rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, false>,
             rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, true>, rf::gemm_fp8_blockscale_streamk<256, 256, 2, 4>,
             rf::gemm_fp8_blockscale_persistent<256, 256, 2, 4>, rf::PersistentGeom<256, 256, 2, 4>::LDS_BYTES,
-            rf::gemm_fp8_blockscale_persistent<256, 256, 2, 4, true>},   // 0: 8 waves, wave tile 128(m) x 64(n), 128 KiB LDS
+            rf::gemm_fp8_blockscale_persistent<256, 256, 2, 4, true>, 1, {},
+            rf::gemm_fp8_blockscale_tile_any_c<256, 256, 2, 4, 2>},   // 0: 8 waves, wave tile 128(m) x 64(n), 128 KiB LDS
     RF_VARIANT(128, 128, 2, 2),   // 1: 4 waves, wave tile 64 x 64, 64 KiB LDS (2 workgroups per CU)
     RF_VARIANT(256, 128, 2, 2),   // 2: 4 waves, wave tile 128 x 64, 96 KiB LDS
     RF_VARIANT(128, 256, 2, 4),   // 3: 8 waves, wave tile 64 x 64, 96 KiB LDS
@@ -244,6 +249,8 @@ int ensure_device_info(State &s) {
                 if (f) RF_HIP(hipFuncSetAttribute((const void *)f, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
         if (v.direct)
             RF_HIP(hipFuncSetAttribute((const void *)v.direct, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
+        if (v.any_c)
+            RF_HIP(hipFuncSetAttribute((const void *)v.any_c, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
         if (v.partial)
             RF_HIP(hipFuncSetAttribute((const void *)v.partial, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
         if (v.streamk)
@@ -843,8 +850,8 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
 // the bounds-checked kernel, which is 7 to 35 times slower (M = 100, N = 4096, K = 7168: 129 us against 17 us for
 // M = 112). Token counts are arbitrary in practice, so for anything but tiny problems the operands that need it are
 // copied into a staging buffer with rows padded to a multiple of 16 (zeros: padded rows and columns produce values
-// nobody reads), the tiled kernels run on the padded shape under the automatic plan, and C is copied back without the
-// padding. b_scale needs no copy: ceil(N/128) does not change. The copies cost K*M (+ K*N when N is ragged) bytes.
+// nobody reads), the tiled kernels run on the padded shape under the automatic plan and store into the caller's C where they
+// can (one K part, one workgroup per tile); otherwise C is copied back without the padding. b_scale needs no copy: ceil(N/128) does not change. The copies cost K*M (+ K*N when N is ragged) bytes.
 constexpr double kPadThresholdMacs = 2097152.0;            // below this the bounds-checked kernel is as fast
 
 // The grouped GEMM's staging copy: the caller's [rows][m_total] matrix (A with T = bytes, a_scale with T = float), in
@@ -1069,8 +1076,8 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     const bool copy_a = mp != m || (uintptr_t)a % 16 != 0, copy_b = np != n || (uintptr_t)b % 16 != 0;
     const bool copy_sa = mp != m;
     // The plan of the padded shape. With whole columns and an aligned c, the whole-tile schedules (one workgroup per
-    // tile, persistent) write the m true rows straight into c (their stores are masked by row); otherwise C is staged
-    // and copied back.
+    // tile, persistent) write the m true rows straight into c (their stores are masked by row), and the tile kernels
+    // have a form for any c; otherwise C is staged and copied back.
     rf_gemm_config cfg;
     select_config(mp, np, k, s.num_cu, (copy_a ? kStageA : 0) | (copy_b || (uintptr_t)c % 16 != 0 ? kStageB : 0), &cfg);
     if (kVariants[cfg.variant].is_fewrows()) {
@@ -1082,7 +1089,10 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
         }
         return launch_fewrows(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, stream);
     }
-    const bool copy_c = np != n || (uintptr_t)c % 16 != 0 || (mp != m && cfg.stream_k == RF_SCHEDULE_STREAM_K);
+    // whole K in one part, one workgroup per tile: the kernel stores into any c itself
+    const bool any_c = (np != n || (uintptr_t)c % 16 != 0) && cfg.split_k == 1 && cfg.stream_k == RF_SCHEDULE_TILES &&
+                       cfg.variant >= 0 && kVariants[cfg.variant].any_c;
+    const bool copy_c = !any_c && (np != n || (uintptr_t)c % 16 != 0 || (mp != m && cfg.stream_k == RF_SCHEDULE_STREAM_K));
     size_t off = 0;
     const size_t off_a = off;  off += copy_a ? align((size_t)k * mp) : 0;
     const size_t off_b = off;  off += copy_b ? align((size_t)k * np) : 0;
@@ -1090,7 +1100,7 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     const size_t off_c = off;  off += copy_c ? align((size_t)mp * np * 2) : 0;
     if (mem.fixed && off > mem.fixed_left()) return launch_padded_in_pieces(s, mem, a, b, as, bs, c, m, n, k, stream);
     uint8_t *pad = nullptr;
-    int rc = mem.pad(off, &pad);
+    int rc = off ? mem.pad(off, &pad) : RF_OK;
     if (rc != RF_OK) return rc;
     const void *a2 = a, *b2 = b;
     const float *as2 = as;
@@ -1111,6 +1121,14 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     }
     if (copy_c) c2 = pad + off_c;
     RF_HIP(hipGetLastError());
+    if (any_c) {
+        const Variant &v = kVariants[cfg.variant];
+        const int tiles_m = ceil_div(mp, v.bm), tiles_n = ceil_div(np, v.bn);
+        hipLaunchKernelGGL(v.any_c, dim3(tiles_m * tiles_n), dim3(v.threads()), v.lds_bytes(), stream, (const uint8_t *)a2,
+                           (const uint8_t *)b2, as2, bs, (uint16_t *)c, mp, np, k, tiles_m, tiles_n, cfg.group_m, m, n);
+        RF_HIP(hipGetLastError());
+        return RF_OK;
+    }
     rc = launch_locked(s, mem, a2, b2, as2, bs, c2, mp, np, k, &cfg, stream, copy_c ? mp : m);
     if (rc != RF_OK) return rc;
     if (copy_c) {

@@ -25,9 +25,11 @@ def test_staged_rows_bit_exact(m):
     assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
 
 
-# more rows than the few-rows kernels take with a ragged width, so the plan is a tiled one on staged copies: widths below a
-# piece of eight, rows of a workgroup's 256 pieces and a few more; c at an odd element
-@pytest.mark.parametrize("m,n,k,off_c", [(4112, 5, 512, 0), (4100, 130, 256, 0), (4128, 2045, 128, 1), (4099, 2057, 128, 0)])
+# more rows than the few-rows kernels take with a ragged width, so the plan is a tiled one: tiles that store into the ragged C
+# and, where K is split (17 columns of it long), a padded C written back; widths below a piece of eight, rows of a
+# workgroup's 256 pieces and a few more; c at an odd element, also with a width that needs nothing else
+@pytest.mark.parametrize("m,n,k,off_c", [(4112, 5, 512, 0), (4100, 130, 256, 0), (4128, 2045, 128, 1), (4099, 2057, 128, 0),
+                                         (4112, 17, 7168, 0), (4112, 17, 7168, 3), (4112, 1008, 256, 5)])
 def test_staged_output_bit_exact(m, n, k, off_c):
     import radeonflow_kernels_amd as rfk
     data = exact_problem(m, n, k, seed=n)
