@@ -332,9 +332,9 @@ __global__ __launch_bounds__(NW * 64, (FewRowsGeom<TM, TN, NW, DEPTH>::WAVES_PER
 //
 // First form: every wave has columns of its own and walks all of K with DEPTH K blocks on their way in registers; the waves
 // share nothing, so there is no barrier. Strips of 128 columns (TN = 8): a load instruction then covers eight whole cache
-// lines, and all strips of a launch are resident at once. Narrower strips ran at half the rate: 32 groups of 48 rows in all,
-// 2048 x 7168 (382 MB of weights), columns per wave 16: 228 us, 32: 139, 64: 100, 128: 75 us with two K blocks on their
-// way (5.1 TB/s) against 96.7 us for the tiled form with its staging copy. Bound by the streaming of B; with fewer than
+// lines, and all strips of a launch are resident at once. Narrower strips ran at half the rate: 48 rows over 32 groups,
+// 2048 x 7168 (366 MB of weights), columns per wave 16: 228 us, 32: 139, 64: 100, 128: 72 us with two K blocks on their
+// way (5.1 TB/s, the rate of a large copy) against 96.7 us for the tiled form with its staging copy. Bound by the streaming of B; with fewer than
 // about one strip per compute unit by the chain of 56 loads (0.95 us each).
 template <int TM, int TN, int NW, int DEPTH, int WAVES_PER_SIMD>
 __global__ __launch_bounds__(NW * 64, WAVES_PER_SIMD) void gemm_fp8_blockscale_grouped_strips(
