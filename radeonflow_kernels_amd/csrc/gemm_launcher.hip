@@ -1447,8 +1447,8 @@ namespace {
 // The few-rows form for these groups, or -1: groups of at most 16 rows (variants 6, 7 and 9) or 32 (variant 8); more rows
 // would stream the weights once per row block. Estimated time in us: the stream of the weights at the rate the form reaches
 // once the chip is full, or the chain of one wave's K blocks. Measured on 52 layouts (8 to 64 groups, 16 to 900 rows,
-// N x K = 2048 x 7168, 4096 x 7168, 7168 x 2048, 4096 x 2048) against the tiled forms with their staging copy: 3 to 50 %
-// faster wherever this picks one, 14 % on average; beyond 1 GB of weights, or max_rounds rounds of resident workgroups,
+// N x K = 2048 x 7168, 4096 x 7168, 7168 x 2048, 4096 x 2048) against the tiled forms with their staging copy: up to 50 %
+// faster where this picks one, 14 % on average, never slower; beyond 1 GB of weights, or max_rounds rounds of resident workgroups,
 // the tiled forms' steady state is as good or better (64 groups of 64 rows in all, 4096 x 7168: 306 us here, 284 tiled; of
 // 300 rows, 7168 x 2048: 210 against 191).
 int choose_grouped_fewrows(const int *row_offsets, int groups, int n, int k, int num_cu) {

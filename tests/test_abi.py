@@ -272,3 +272,5 @@ def test_grouped_few_rows_choice_on_the_host():
     assert choice(2, 8, 2048, 7168) == 9 and choice(2, 16, 2048, 7168) == 7 and choice(16, 32, 2048, 7168) == 6
     assert choice(17, 32, 2048, 7168) == 8 and choice(32, 32, 2048, 7168) == 8
     assert choice(33, 32, 2048, 7168) < 6 and choice(16, 32, 2056, 7168) < 6 and choice(16, 64, 4096, 7168) < 6
+    # few tiles: 128 x 128 while they are alone on their compute unit, then 128 x 256; short K keeps the most workgroups
+    assert choice(100, 8, 2048, 7168) == 2 and choice(300, 8, 2048, 7168) == 1 and choice(100, 8, 2048, 1024) == 3

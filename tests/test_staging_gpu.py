@@ -42,3 +42,25 @@ def test_staged_output_bit_exact(m, n, k, off_c):
     assert np.array_equal(bf16_bits(c), exp)
     rest = torch.cat([buf[:off_c], buf[off_c + m * n:]]).float()
     assert float(rest.min()) == -7.0 == float(rest.max())
+
+
+def test_every_tile_kernel_stores_into_any_c(tmp_path):
+    """Plan files name each tile variant for the padded shape: its form for a ragged C gives the oracle's bits and leaves what
+    lies around C alone."""
+    import radeonflow_kernels_amd as rfk
+    m, n, k = 4101, 205, 256
+    data = exact_problem(m, n, k, seed=7)
+    exp = oracle_bf16(data)
+    g, _ = to_gpu(data, 300)
+    plan = tmp_path / "p.plans"
+    for variant in range(12):
+        plan.write_text("4112 208 256 %d 1 8 0\n" % variant)
+        buf = torch.full((m * n + 301,), -7.0, dtype=torch.bfloat16, device="cuda")
+        try:
+            assert rfk.load_plans(str(plan)) == 1 and rfk.plan_for(m, n, k, 256).variant == variant
+            rfk.fp8_mm(*g[:4], buf[1:1 + m * n].view(m, n))
+            torch.cuda.synchronize()
+        finally:
+            rfk.clear_plans()
+        assert np.array_equal(bf16_bits(buf[1:1 + m * n].view(m, n)), exp), variant
+        assert float(buf[0]) == -7.0 and float(buf[1 + m * n:].float().min()) == -7.0 == float(buf[1 + m * n:].float().max())
