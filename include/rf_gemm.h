@@ -109,8 +109,8 @@ int rf_fp8_gemm(const void *a, const void *b, const float *as, const float *bs, 
  * K = 7168: two ranges); such results agree with rf_fp8_gemm's within the rounding of another K split, and bit for bit
  * on data whose sums are exact. Only when the staged copy of B (ragged N or an unaligned b) alone takes more than half
  * of the array does the much slower bounds-checked kernel compute the shape, in place. All calls on one GPU share that
- * GPU's array: two calls that overlap in time (different streams, or graph replays beside eager launches) race; calls on
- * one stream are ordered by the stream. */
+ * GPU's array: two calls that overlap in time (different streams, or graph replays beside eager launches) race, and the
+ * results of both are undefined (later calls are not affected); calls on one stream are ordered by the stream. */
 int rf_fp8_gemm_static(const void *a, const void *b, const float *as, const float *bs, void *c,
                        int m, int n, int k, hipStream_t stream);
 size_t rf_gemm_static_scratch_bytes(void);

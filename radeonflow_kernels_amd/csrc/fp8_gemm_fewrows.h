@@ -295,10 +295,12 @@ __global__ __launch_bounds__(NW * 64, (FewRowsGeom<TM, TN, NW, DEPTH>::WAVES_PER
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         volatile unsigned *mailbox = (volatile unsigned *)lds;        // every wave has read the sums exchanged there
-        // wraps to zero at the last arrival: ready for the next launch
-        if (threadIdx.x == 0) *mailbox = atomicInc(counters + item, (unsigned)(splits - 1));
+        if (threadIdx.x == 0) {
+            const unsigned w = arrival_weight(blockIdx.y, (unsigned)splits);
+            *mailbox = __hip_atomic_fetch_add(counters + item, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + w;
+        }
         __syncthreads();
-        if (*mailbox != (unsigned)(splits - 1)) return;
+        if (*mailbox != 0u) return;                                   // not the last
         const float *first = slots + (size_t)item * splits * (TM * TN * 256) + lane * 4;
         for (int t = wave; t < TM * TN; t += NW) {
             f32x4 s = {0.f, 0.f, 0.f, 0.f};

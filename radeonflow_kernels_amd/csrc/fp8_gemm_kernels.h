@@ -27,6 +27,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "arrival_counter.h"
+
 namespace rf {
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
@@ -859,9 +861,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64 * GROUPS) void gemm_fp8_block
 // work units and cut into P equal contiguous ranges, so every CU gets the same number of MFMAs whatever T is
 // (432 tiles on 256 CUs is 1.69 tiles each, not 2). A workgroup walks its range tile by tile. A tile whose K
 // range is shared by several workgroups is finished by whichever of them arrives last: each one stores its fp32
-// partial tile to its workspace slot with write-through stores and bumps the tile's counter; the one that
-// reads count == parts-1 adds the other partials and writes bf16. Nobody waits for anybody, so there is nothing to
-// deadlock, and the last arriver resets the counter: the counters are zero again when the kernel ends.
+// partial tile to its workspace slot with write-through stores and adds to the tile's arrival counter; the one that
+// arrives last (arrival_counter.h) adds the other partials and writes bf16. Nobody waits for anybody, so there is nothing
+// to deadlock, and the counters are zero again when the kernel ends.
 // Used only when every range is at least QK units long (T >= P), so a split tile has exactly 2 contributors.
 // ws: tile_count[T] (unsigned, zero on entry), then at byte offset ws_slots_off 2*P slots of BM*BN floats.
 // ---------------------------------------------------------------------------------------------
@@ -905,13 +907,13 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_str
             // the counter move
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
-            if (threadIdx.x == 0)
-                *mailbox = __hip_atomic_fetch_add(tile_count + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (threadIdx.x == 0) {
+                const unsigned w = arrival_weight((unsigned)(slot - s_first), 2u);
+                *mailbox = __hip_atomic_fetch_add(tile_count + tile, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + w;
+            }
             __syncthreads();
-            if (*mailbox == 1u) {            // the other contributor arrived first: I finish the tile
+            if (*mailbox == 0u) {            // the other contributor arrived first: I finish the tile
                 exchange_tile_f32<BM, BN, WAVES_M, WAVES_N, true>(acc, slot_ptr(other));
-                if (threadIdx.x == 0)        // ready for the next launch
-                    __hip_atomic_store(tile_count + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 write_c = true;
             }
         }
