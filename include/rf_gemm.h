@@ -18,7 +18,7 @@
  * below 2^21 multiply-adds always take the few-rows kernels (their plan is reported as variant = -1); explicit plans with
  * variant = -1 take a bounds-checked kernel (the role of the reference's legacy kernel,
  * src/gemm/gemm_kernel_legacy.cpp:237-374).
- * Temporary device memory (split-K partial sums, staging copies, stream-K counters) is kept per (device, stream), for
+ * Temporary device memory (split-K partial sums, staging copies) is kept per (device, stream), for
  * the device that is current at the call: launches on different streams of one device may overlap, launches on one
  * stream are ordered by the stream. Calls are serialised by one lock only while they enqueue. A buffer that has to grow
  * is replaced and the old one freed by rf_gemm_destroy, so no call waits for the device. A stream gets a buffer set only
@@ -26,8 +26,13 @@
  * own, and when one more asks, the least recently used set changes hands: the new stream waits on the device for the
  * old stream's work enqueued so far (an event, no host wait). A stream that is being captured into a HIP graph cannot
  * take a set over and gets RF_ERR_BAD_CONFIG (its first 32 streams capture fine; rf_fp8_gemm_static never needs a set).
- * HIP graphs captured through this library refer to these buffers: destroy them before rf_gemm_destroy, and do not
- * replay a graph captured on a stream whose set has since changed hands.
+ * HIP graphs captured through this library refer to these buffers: a replay counts as a launch on the stream the graph
+ * was captured on, whatever stream it runs on, and must not overlap that stream's other launches or the replays of
+ * another graph captured on it (results of launches that do overlap are undefined; for the grouped queue form also those
+ * of later launches on the stream, until rf_gemm_destroy). Destroy such graphs before rf_gemm_destroy, and do not replay
+ * a graph captured on a stream whose set has since changed hands. The counters of launches whose workgroups hand their
+ * work over (K split inside a few-rows launch, stream-K, queues) are static device memory, zero from the start: no call
+ * allocates or clears them.
  */
 #ifndef RF_GEMM_H
 #define RF_GEMM_H
@@ -189,7 +194,7 @@ void rf_gemm_destroy(void);
  * variant: -1 = automatic, else an index into {256x256, 128x256, 128x128, 128x64} tiles, or 4 = 256-row tiles with a
  * 128 x 256 tile for a group's last rows when at most 128 are left, or 5 = 256-row tiles with a last tile of 64, 128,
  * 192 or 256 rows, run by one resident workgroup per CU that takes tiles from a queue per XCD (the automatic choice
- * for groups of uneven size; its queues are counters in the stream's buffer set, like the stream-K schedule's), or 6 to 9 =
+ * for groups of uneven size; its queues are counters of the stream's buffer set), or 6 to 9 =
  * the few-rows forms (16 x 256, 16 x 128, 32 x 128 and 16 x 64 tiles; the automatic choice for groups of up to 16 or 32
  * rows), which read a as it is, without the copy. */
 int rf_fp8_gemm_grouped(const void *a, const void *b, const float *as, const float *bs, void *c, const int *row_offsets,

@@ -27,10 +27,18 @@
 // own address until the process ends; host code never uses this name as an address (see ensure_device_info).
 constexpr size_t kStaticScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) uint8_t scratch[kStaticScratchBytes];
-// and its arrival counters (few-rows kernels with a K split): zero when the library is loaded, and every launch that uses
-// them leaves them at zero
-constexpr int kMaxTileCounters = 16384;
-static __device__ unsigned scratch_counters[kMaxTileCounters];
+// Counters of a launch: arrivals at tiles that several workgroups finish (few-rows kernels with a K split, stream-K), and
+// the draws from the grouped GEMM's queues, in words of their own. One set per buffer set (StreamBuffers) and one for
+// rf_fp8_gemm_static. They are zero when the library is loaded, and every launch that uses them leaves them at zero: nothing
+// is allocated or cleared on the way to a launch, also not under graph capture (a counter buffer allocated and zeroed by the
+// first launch that ran eagerly put a kernel of 16384 words in front of every captured one).
+constexpr int kMaxTileCounters = 16384, kQueueCounters = 64;
+constexpr int kMaxStreamBuffers = 32;    // per device; one more stream takes over the least recently used set
+struct CounterSet {
+    unsigned tile[kMaxTileCounters], queue[kQueueCounters];
+};
+static_assert(rf::NUM_XCD <= kQueueCounters, "a counter per queue");
+static __device__ CounterSet counter_sets[kMaxStreamBuffers + 1];
 
 namespace {
 
@@ -147,7 +155,7 @@ struct TunedPlan {
 // Buffers, counters and kernel attributes belong to a device: one State per device, chosen by the device that is
 // current at the call. Plans and the lock are shared by the process.
 //
-// Temporary device memory (split-K partial sums, stream-K slots and counters, staging copies of ragged operands) is
+// Temporary device memory (split-K partial sums, stream-K slots, staging copies of ragged operands) is
 // kept per (device, stream): two launches on different streams of one device never share a buffer, so they may overlap,
 // and launches on one stream are ordered by the stream. A buffer that has to grow is replaced, and the old one is kept
 // until rf_gemm_destroy: work enqueued earlier may still use it, and waiting for that work here would block the host
@@ -158,18 +166,15 @@ struct StreamBuffers {
     size_t pad_bytes = 0;
     float *ws = nullptr;                 // split-K partial sums / stream-K slots
     size_t ws_bytes = 0;
-    unsigned *tile_count = nullptr;      // stream-K arrival counters, zero between launches
-    bool tile_count_zeroed = false;
     uint64_t last_use = 0;
 };
-constexpr int kMaxStreamBuffers = 32;    // per device; one more stream takes over the least recently used set
 struct State {
-    std::vector<StreamBuffers> buffers;
+    std::vector<StreamBuffers> buffers;  // set i has counters[i]
     std::vector<void *> retired;         // outgrown buffers, freed by rf_gemm_destroy
     uint64_t tick = 0;
     bool attrs_set = false, grouped_attrs_set = false;
     int num_cu = 0;
-    unsigned *static_counters = nullptr; // this device's copy of the file-scope counters
+    CounterSet *counters = nullptr;      // this device's copy of counter_sets, the last one for rf_fp8_gemm_static
     uint8_t *static_scratch = nullptr;   // this device's copy of the file-scope scratch array (rf_fp8_gemm_static)
     std::mutex ev_mu;                    // guards free_events only: the timing callback takes no other lock
     std::vector<std::pair<hipEvent_t, hipEvent_t>> free_events;
@@ -274,13 +279,11 @@ int ensure_device_info(State &s) {
     void *scratch_ptr = nullptr;
     RF_HIP(hipGetSymbolAddress(&scratch_ptr, HIP_SYMBOL(scratch)));
     s.static_scratch = (uint8_t *)scratch_ptr;
-    RF_HIP(hipGetSymbolAddress(&scratch_ptr, HIP_SYMBOL(scratch_counters)));
-    s.static_counters = (unsigned *)scratch_ptr;
+    RF_HIP(hipGetSymbolAddress(&scratch_ptr, HIP_SYMBOL(counter_sets)));
+    s.counters = (CounterSet *)scratch_ptr;
     s.attrs_set = true;
     return RF_OK;
 }
-
-__global__ void zero_words(unsigned *p) { p[blockIdx.x * 256 + threadIdx.x] = 0u; }
 
 // hipMalloc that also works while the calling thread records a stream into a HIP graph: an allocation is not part
 // of the recorded work, so the capture mode is relaxed around it (under the default mode the call would fail and
@@ -351,33 +354,14 @@ struct Mem {
         *out = sb->ws;
         return rc;
     }
-    int tile_counters(unsigned **out) {
+    int counters(CounterSet **out) {
         if (fixed) {
-            *out = s.static_counters;
+            *out = s.counters + kMaxStreamBuffers;
             return RF_OK;
         }
         int rc = bind();
         if (rc != RF_OK) return rc;
-        if (!sb->tile_count) RF_HIP(device_malloc((void **)&sb->tile_count, kMaxTileCounters * sizeof(unsigned)));
-        if (!sb->tile_count_zeroed) {
-            // zeroed on the stream of the launch that follows (the kernels leave the counters at zero afterwards);
-            // a kernel and not a memset, so that the call may be recorded into a HIP graph. A recorded fill has not
-            // run yet, so it does not count: launches keep filling first until one has done so for real.
-            // (on the legacy null stream the query itself is refused while another thread captures in global mode:
-            // that counts as "capturing", so the fill is issued and the flag stays false)
-            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-            const hipError_t qe = hipStreamIsCapturing(sb->stream, &st);
-            if (qe == hipErrorStreamCaptureImplicit || qe == hipErrorStreamCaptureUnsupported) {
-                (void)hipGetLastError();
-                st = hipStreamCaptureStatusActive;
-            } else if (qe != hipSuccess) {
-                return fail(RF_ERR_HIP, std::string("hipStreamIsCapturing: ") + hipGetErrorString(qe));
-            }
-            hipLaunchKernelGGL(zero_words, dim3(kMaxTileCounters / 256), dim3(256), 0, sb->stream, sb->tile_count);
-            RF_HIP(hipGetLastError());
-            sb->tile_count_zeroed = st == hipStreamCaptureStatusNone;
-        }
-        *out = sb->tile_count;
+        *out = s.counters + (sb - s.buffers.data());
         return RF_OK;
     }
 };
@@ -674,11 +658,11 @@ int launch_fewrows(Mem &mem, const Variant &v, const void *a, const void *b, con
     const int qk = k / rf::BK, row_blocks = ceil_div(m, v.bm), items = ceil_div(n, v.bn) * row_blocks;
     const int kb_per_split = ceil_div(qk, splits);
     splits = ceil_div(qk, kb_per_split);                    // every split owns at least one K block
-    unsigned *counters = nullptr;
+    CounterSet *counters = nullptr;
     float *slots = nullptr;
     if (splits > 1) {
         if (items > kMaxTileCounters) return fail(RF_ERR_BAD_CONFIG, "too many tiles for a K split of this variant");
-        int rc = mem.tile_counters(&counters);
+        int rc = mem.counters(&counters);
         if (rc != RF_OK) return rc;
         rc = mem.workspace((size_t)items * splits * v.bm * v.bn * sizeof(float), &slots);
         if (rc != RF_OK) return rc;
@@ -686,7 +670,7 @@ int launch_fewrows(Mem &mem, const Variant &v, const void *a, const void *b, con
     const bool any = n % 16 != 0 || (uintptr_t)b % 16 != 0;
     hipLaunchKernelGGL(v.fewrows[splits > 1][any], dim3(items, splits), dim3(v.threads()), v.lds_bytes(), stream,
                        (const uint8_t *)a, (const uint8_t *)b, as, bs, (uint16_t *)c, m, ldm, n, k, kb_per_split, row_blocks,
-                       counters, slots);
+                       counters ? counters->tile : nullptr, slots);
     RF_HIP(hipGetLastError());
     return RF_OK;
 }
@@ -814,14 +798,14 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
     }
     if (cfg.stream_k == RF_SCHEDULE_STREAM_K) {
         const int P = s.num_cu;
-        unsigned *tile_count = nullptr;
+        CounterSet *counters = nullptr;
         float *ws = nullptr;
-        rc = mem.tile_counters(&tile_count);
+        rc = mem.counters(&counters);
         if (rc != RF_OK) return rc;
         rc = mem.workspace((size_t)2 * P * v.bm * v.bn * sizeof(float), &ws);
         if (rc != RF_OK) return rc;
         hipLaunchKernelGGL(v.streamk, dim3(P), block, v.lds_bytes(), stream, (const uint8_t *)a, (const uint8_t *)b, as,
-                           bs, (uint16_t *)c, m, n, k, tiles_m, tiles_n, cfg.group_m, tile_count, ws);
+                           bs, (uint16_t *)c, m, n, k, tiles_m, tiles_n, cfg.group_m, counters->tile, ws);
         RF_HIP(hipGetLastError());
         return RF_OK;
     }
@@ -1347,7 +1331,11 @@ void rf_gemm_destroy(void) {
     for (StreamBuffers &b : s.buffers) {
         if (b.ws) (void)hipFree(b.ws);
         if (b.pad) (void)hipFree(b.pad);
-        if (b.tile_count) (void)hipFree(b.tile_count);
+    }
+    // a fresh start also after launches that overlapped on a queue's counters (every other use leaves zeros behind)
+    if (!s.buffers.empty()) {
+        (void)hipMemset(s.counters, 0, s.buffers.size() * sizeof(CounterSet));
+        (void)hipDeviceSynchronize();
     }
     s.buffers.clear();
     for (void *p : s.retired) (void)hipFree(p);
@@ -1712,12 +1700,12 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
         if (tiles < queues.workgroups) queues.workgroups = ceil_div(tiles, rf::NUM_XCD) * rf::NUM_XCD;
         Mem mem{s};
         mem.stream = stream;
-        unsigned *counters = nullptr;
-        rc = mem.tile_counters(&counters);
+        CounterSet *counters = nullptr;
+        rc = mem.counters(&counters);
         if (rc != RF_OK) return rc;
         hipLaunchKernelGGL(rf::gemm_fp8_blockscale_grouped_queue, dim3(queues.workgroups), dim3(v.threads), v.lds, stream,
                            (const uint8_t *)a, (const uint8_t *)b, as, bs, (uint16_t *)c, m_rows, n, k, groups, table,
-                           queues, counters);
+                           queues, counters->queue);
         RF_HIP(hipGetLastError());
         return RF_OK;
     }

@@ -197,3 +197,66 @@ def test_small_grouped_problem_takes_the_variant_with_the_most_workgroups(rfk):
         torch.cuda.synchronize()
         out[variant] = bf16_bits(c)
     assert np.any(out[3] != 0) and np.array_equal(out[-1], out[3])
+
+
+@pytest.mark.parametrize("rows,n,k", [((32,), 1536, 7168), ((1,), 200, 7168), ((40, 700, 300, 500), 4096, 4096)])
+def test_a_captured_launch_is_one_kernel_and_replays_right(rfk, rows, n, k):
+    """fp8_mm with a K split summed inside the launch (plans of an aligned and of a small ragged shape) and the grouped queue
+    form use counters: captured on a stream that has never run anything, each is one graph node, and three replays with eager
+    calls of the same stream between them give the eager result."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    grouped = len(rows) > 1
+    offs = [0] + [int(x) for x in np.cumsum(rows)]
+    m = offs[-1]
+    data = exact_problem(m, n, k, seed=m + n)
+    g = to_gpu(data)
+    exp = oracle_bf16(data)
+
+    def launch():
+        if grouped:                                      # every group with the same weights
+            rfk.fp8_mm_grouped_padded(a_pad, b3, sa_pad, sb3, g[4], offs, variant=5)
+        else:
+            rfk.fp8_mm(*g)
+
+    if grouped:
+        pad = rfk.grouped_padded_offsets(offs)
+        a_pad = torch.zeros((k, pad[-1]), dtype=torch.uint8, device="cuda")
+        sa_pad = torch.ones((k // 128, pad[-1]), device="cuda")
+        for i, r in enumerate(rows):
+            a_pad[:, pad[i]:pad[i] + r] = g[0].T.view(torch.uint8)[:, offs[i]:offs[i + 1]]
+            sa_pad[:, pad[i]:pad[i] + r] = g[2].T[:, offs[i]:offs[i + 1]]
+        a_pad, sa_pad = a_pad.view(torch.float8_e4m3fn).T, sa_pad.T
+        b3 = g[1].T.view(torch.uint8).repeat(len(rows), 1, 1).view(torch.float8_e4m3fn).transpose(1, 2)
+        sb3 = g[3].T.repeat(len(rows), 1, 1).transpose(1, 2)
+    elif n % 16 == 0:
+        assert rfk.select_config(m, n, k).split_k > 1
+    rfk.lib().rf_gemm_destroy()                          # the capture's stream is the first to use counters
+    handle, graph, graph_exec = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+    stream = torch.cuda.ExternalStream(handle.value)
+    try:
+        with torch.cuda.stream(stream):
+            assert hip.hipStreamBeginCapture(handle, 2) == 0     # hipStreamCaptureModeRelaxed
+            try:
+                launch()
+            finally:
+                assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+            count = ctypes.c_size_t()
+            assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0 and count.value == 1
+            assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, 0) == 0
+            for replay in range(3):
+                g[4].fill_(-1.0)
+                torch.cuda.synchronize()
+                assert hip.hipGraphLaunch(graph_exec, handle) == 0
+                torch.cuda.synchronize()
+                assert np.array_equal(bf16_bits(g[4]), exp), "replay %d" % replay
+                g[4].fill_(-1.0)
+                launch()
+                torch.cuda.synchronize()
+                assert np.array_equal(bf16_bits(g[4]), exp), "eager call after replay %d" % replay
+            hip.hipGraphExecDestroy(graph_exec)
+            hip.hipGraphDestroy(graph)
+    finally:
+        torch.cuda.synchronize()
+        rfk.lib().rf_gemm_destroy()
+        hip.hipStreamDestroy(handle)
