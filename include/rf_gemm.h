@@ -25,7 +25,8 @@
  * when a launch on it needs temporary memory (most plans need none); up to 32 streams per device have a set of their
  * own, and when one more asks, the least recently used set changes hands: the new stream waits on the device for the
  * old stream's work enqueued so far (an event, no host wait). A stream that is being captured into a HIP graph cannot
- * take a set over and gets RF_ERR_BAD_CONFIG (its first 32 streams capture fine; rf_fp8_gemm_static never needs a set).
+ * take a set over and gets RF_ERR_BAD_CONFIG (its first 32 streams capture fine; rf_fp8_gemm_static never needs a set; an
+ * automatic few-rows plan with a K split first gives way to one without temporary memory where the shape has one).
  * HIP graphs captured through this library refer to these buffers: a replay counts as a launch on the stream the graph
  * was captured on, whatever stream it runs on, and must not overlap that stream's other launches or the replays of
  * another graph captured on it (results of launches that do overlap are undefined; for the grouped queue form also those
@@ -166,8 +167,9 @@ int rf_gemm_variant_has_persistent(int variant);
  * the tile schedule only, and K/128 must be a multiple of the count (RF_ERR_BAD_CONFIG otherwise). */
 int rf_gemm_variant_k_groups(int variant);
 
-/* Device workspace (split-K partial sums) needed for a shape under the automatic plan, in bytes. The staging copies
- * of ragged or unaligned operands are not part of it: that buffer grows on the first such call. */
+/* Device workspace (split-K partial sums) needed for a shape under the automatic plan of aligned operands, in bytes, also
+ * for the small shapes whose plan is reported as variant -1. The staging copies of ragged or unaligned operands are not
+ * part of it: that buffer grows on the first such call. */
 size_t rf_gemm_workspace_bytes(int m, int n, int k);
 
 /* Optional explicit set-up / tear-down of the current device's workspace. run() and

@@ -508,8 +508,8 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
 constexpr int kFewRowsMaxM = 512, kFewRowsMaxMStagedB = 4096;
 
 // What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
-// (and of C on the way back).
-enum { kStageA = 1, kStageB = 2 };
+// (and of C on the way back). kTiledOnly: no few-rows plan.
+enum { kStageA = 1, kStageB = 2, kTiledOnly = 4 };
 
 // Plan for a shape (m, n multiples of 16, the padded sizes when something is staged).
 void select_config_uncached(int m, int n, int k, int num_cu, int stage, const std::vector<TunedPlan> &user_plans,
@@ -519,6 +519,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     out->stream_k = 0;
     auto usable = [&](const TunedPlan &p) {
         return p.m == m && p.n == n && p.k == k && p.variant < kNumVariants && p.split_k <= k / rf::BK &&
+               !((stage & kTiledOnly) && kVariants[p.variant].is_fewrows()) &&
                (kVariants[p.variant].k_groups == 1 || (p.split_k == 1 && (k / rf::BK) % kVariants[p.variant].k_groups == 0)) &&
                (p.stream_k != RF_SCHEDULE_PERSISTENT || persistent_ok(kVariants[p.variant], m, n, k)) &&
                (p.stream_k != RF_SCHEDULE_STREAM_K || stream_k_ok(kVariants[p.variant], m, n, num_cu)) &&
@@ -536,7 +537,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     if (num_cu == kTunedOnCUs)
         for (const TunedPlan &p : kTunedPlans)
             if (!hit && usable(p)) hit = &p;
-    if (hit && (!stage || kVariants[hit->variant].is_fewrows())) return take(*hit);
+    if (hit && (!(stage & (kStageA | kStageB)) || kVariants[hit->variant].is_fewrows())) return take(*hit);
     // Up to four K blocks and a large C: the launch is a streaming store, which the skinny-K schedule does best
     // (measured against the best tiled plan at N = 7168, K = 256: 1024 rows 6.5 against 6.9 us, 2048 rows 7.8 against
     // 10.3, 6144 rows 18.2 against 22.1; below about six million outputs the 64 x 128 tiles win, e.g. 2048 x 2048: 6.5
@@ -628,7 +629,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // (fitted to the same measurements as fewrows_plan). Over 280 shapes the choice between the two families is within 4 %
     // of the best plan of either, on average.
     const int max_m = (stage & kStageB) && num_cu == kTunedOnCUs ? kFewRowsMaxMStagedB : kFewRowsMaxM;
-    if (m <= max_m && fewrows_ok(m, n)) {
+    if (m <= max_m && fewrows_ok(m, n) && !(stage & kTiledOnly)) {
         double tiled = 3.1 + 0.67 * best_cost;
         if (stage & kStageA) tiled += 3.2 + 2.0 * k * m / 4e6;
         if (stage & kStageB) tiled += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
@@ -652,6 +653,23 @@ void select_config(int m, int n, int k, int num_cu, int stage, rf_gemm_config *o
     *out = e.cfg;
 }
 
+// Bytes in which the workgroups of a few-rows launch with K in `parts` parts hand over their sums.
+size_t fewrows_slot_bytes(const Variant &v, int m, int n, int parts) {
+    return (size_t)ceil_div(m, v.bm) * v.bm * ceil_div(n, v.bn) * v.bn * sizeof(float) * parts;
+}
+
+// Whether the memory of a few-rows plan's K split is to be had: not on a stream under capture that would have to take over
+// another stream's buffers, nor when device memory has run out. (Static mode: the caller cuts the split down beforehand.)
+bool fewrows_split_fits(Mem &mem, const Variant &v, int m, int n, int k, int splits) {
+    if (splits == 1 || mem.fixed) return true;
+    const int qk = k / rf::BK;
+    float *slots = nullptr;
+    if (mem.workspace(fewrows_slot_bytes(v, m, n, ceil_div(qk, ceil_div(qk, splits))), &slots) == RF_OK) return true;
+    (void)hipGetLastError();
+    g_last_error.clear();
+    return false;
+}
+
 // m rows out of ldm (the distance between two K rows of a and as); any shape and alignment. splits >= 1.
 int launch_fewrows(Mem &mem, const Variant &v, const void *a, const void *b, const float *as, const float *bs, void *c, int m,
                    int ldm, int n, int k, int splits, hipStream_t stream) {
@@ -664,7 +682,7 @@ int launch_fewrows(Mem &mem, const Variant &v, const void *a, const void *b, con
         if (items > kMaxTileCounters) return fail(RF_ERR_BAD_CONFIG, "too many tiles for a K split of this variant");
         int rc = mem.counters(&counters);
         if (rc != RF_OK) return rc;
-        rc = mem.workspace((size_t)items * splits * v.bm * v.bn * sizeof(float), &slots);
+        rc = mem.workspace(fewrows_slot_bytes(v, m, n, splits), &slots);
         if (rc != RF_OK) return rc;
     }
     const bool any = n % 16 != 0 || (uintptr_t)b % 16 != 0;
@@ -717,6 +735,10 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
     } else {
         if (tiled_ok) select_config(m, n, k, s.num_cu, 0, &cfg);
         else cfg = {-1, 1, 8, RF_SCHEDULE_TILES};
+        // no memory for a few-rows plan's sums: the tiled plan, which often needs none
+        if (cfg.variant >= 0 && kVariants[cfg.variant].is_fewrows() &&
+            !fewrows_split_fits(mem, kVariants[cfg.variant], m, n, k, cfg.split_k))
+            select_config(m, n, k, s.num_cu, kTiledOnly, &cfg);
     }
 
     if (mem.fixed && cfg.variant >= 0) {
@@ -727,8 +749,7 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         if (cfg.stream_k == RF_SCHEDULE_STREAM_K) cfg.stream_k = RF_SCHEDULE_TILES;
         if (cfg.split_k > 1) {
             const Variant &fv = kVariants[cfg.variant];
-            const size_t per_part = !fv.is_fewrows() ? (size_t)m * n * sizeof(float)
-                : (size_t)ceil_div(m, fv.bm) * fv.bm * ceil_div(n, fv.bn) * fv.bn * sizeof(float);
+            const size_t per_part = fv.is_fewrows() ? fewrows_slot_bytes(fv, m, n, 1) : (size_t)m * n * sizeof(float);
             const int qk_ = k / rf::BK, kb_per = ceil_div(qk_, cfg.split_k), parts = ceil_div(qk_, kb_per);
             const size_t fit = mem.fixed_left() / per_part;
             if ((size_t)parts > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;
@@ -741,6 +762,7 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         // of the bounds-checked kernel gathers bytes K block after K block, 13 to 27 us where these take 3 to 4
         // (M x N x K = 4 x 200 x 2048: 27.8 -> 3.7, 8 x 1000 x 384: 13.6 -> 3.1).
         fewrows_plan(m, n, k, s.num_cu, n % 16 != 0, &cfg);
+        if (!fewrows_split_fits(mem, kVariants[cfg.variant], m, n, k, cfg.split_k)) cfg.split_k = 1;
         return launch_fewrows(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, stream);
     }
     if (cfg.variant < 0) {
@@ -1067,8 +1089,7 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     if (kVariants[cfg.variant].is_fewrows()) {
         if (mem.fixed && cfg.split_k > 1) {                // as many K parts as the static array holds
             const Variant &v = kVariants[cfg.variant];
-            const size_t per_part = (size_t)ceil_div(m, v.bm) * v.bm * ceil_div(n, v.bn) * v.bn * sizeof(float);
-            const size_t fit = mem.fixed_left() / per_part;
+            const size_t fit = mem.fixed_left() / fewrows_slot_bytes(v, m, n, 1);
             if ((size_t)cfg.split_k > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;
         }
         return launch_fewrows(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, stream);
@@ -1290,22 +1311,18 @@ int rf_gemm_variant_has_stream_k(int variant) {
 
 size_t rf_gemm_workspace_bytes(int m, int n, int k) {
     rf_gemm_config cfg;
-    if (rf_gemm_select_config(m, n, k, &cfg) != RF_OK || cfg.variant < 0) return 0;
+    if (rf_gemm_select_config(m, n, k, &cfg) != RF_OK) return 0;
+    State &s = state();
+    if (cfg.variant < 0 && fewrows_ok(m, n)) fewrows_plan(m, n, k, s.num_cu, n % 16 != 0, &cfg);   // as launch_locked
+    if (cfg.variant < 0) return 0;
+    const Variant &v = kVariants[cfg.variant];
+    if (cfg.stream_k == RF_SCHEDULE_STREAM_K) return (size_t)2 * s.num_cu * v.bm * v.bn * sizeof(float);
+    const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, cfg.split_k));
+    if (parts <= 1) return 0;
+    if (v.is_fewrows()) return fewrows_slot_bytes(v, m, n, parts);
     // a ragged shape runs (and splits K) at its padded size; its staging copies live in a buffer of their own
-    m = m < 16 ? 16 : (m + 15) / 16 * 16;
-    n = n < 16 ? 16 : (n + 15) / 16 * 16;
-    if (cfg.stream_k == RF_SCHEDULE_STREAM_K) {
-        State &s = state();
-        return (size_t)2 * s.num_cu * kVariants[cfg.variant].bm * kVariants[cfg.variant].bn * sizeof(float);
-    }
-    if (cfg.split_k <= 1) return 0;
-    if (kVariants[cfg.variant].is_fewrows()) {
-        m = ceil_div(m, kVariants[cfg.variant].bm) * kVariants[cfg.variant].bm;
-        n = ceil_div(n, kVariants[cfg.variant].bn) * kVariants[cfg.variant].bn;
-    }
-    const int qk = k / rf::BK;
-    const int kb_per_split = ceil_div(qk, cfg.split_k);
-    return (size_t)m * n * sizeof(float) * ceil_div(qk, kb_per_split);
+    const size_t mp = m < 16 ? 16 : (m + 15) / 16 * 16, np = n < 16 ? 16 : (n + 15) / 16 * 16;
+    return mp * np * sizeof(float) * parts;
 }
 
 int rf_gemm_init(size_t workspace_bytes) {

@@ -260,3 +260,79 @@ def test_a_captured_launch_is_one_kernel_and_replays_right(rfk, rows, n, k):
         torch.cuda.synchronize()
         rfk.lib().rf_gemm_destroy()
         hip.hipStreamDestroy(handle)
+
+
+def test_small_few_rows_calls_under_capture_need_no_buffer_set(rfk):
+    """All 32 buffer sets belong to other streams, and a stream under capture cannot take one over. Automatic few-rows plans
+    with a K split give way to K in one part (small ragged shapes) or to the tiled plan (an aligned shape whose tiled plan
+    needs no memory) and are recorded all the same; an explicit plan with a K split is refused."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    L = rfk.lib()
+    L.rf_gemm_destroy()
+    handles = []
+    for _ in range(33):
+        h = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(h)) == 0
+        handles.append(h)
+
+    def launch(g, h, cfg=None):
+        a, b, sa, sb, c = g
+        return L.rf_fp8_gemm_ex(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), c.data_ptr(), a.shape[0], b.shape[0],
+                                a.shape[1], cfg, h)
+
+    try:
+        split = to_gpu(exact_problem(16, 1536, 7168, 1))
+        assert rfk.select_config(16, 1536, 7168).split_k > 1
+        for h in handles[:32]:
+            assert launch(split, h) == 0
+            torch.cuda.synchronize()
+        for (m, n, k) in ((1, 200, 7168), (3, 130, 5120), (256, 1024, 2304)):
+            assert L.rf_gemm_workspace_bytes(m, n, k) > 0
+            data = exact_problem(m, n, k, m + n)
+            g, exp = to_gpu(data), oracle_bf16(data)
+            torch.cuda.synchronize()
+            cap, graph, graph_exec = handles[32], ctypes.c_void_p(), ctypes.c_void_p()
+            assert hip.hipStreamBeginCapture(cap, 2) == 0            # hipStreamCaptureModeRelaxed
+            rc = launch(g, cap)
+            rc_explicit = launch(g, cap, ctypes.byref(rfk.GemmConfig(14, 2, 8, 0)))
+            assert hip.hipStreamEndCapture(cap, ctypes.byref(graph)) == 0
+            assert rc == 0 and rc_explicit == 4, (m, n, k)
+            assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, 0) == 0
+            for _ in range(3):
+                g[4].fill_(-1.0)
+                torch.cuda.synchronize()
+                assert hip.hipGraphLaunch(graph_exec, cap) == 0
+                torch.cuda.synchronize()
+                assert np.array_equal(bf16_bits(g[4]), exp), (m, n, k)
+                assert launch(split, handles[0]) == 0                # eager work between the replays
+                torch.cuda.synchronize()
+            hip.hipGraphExecDestroy(graph_exec)
+            hip.hipGraphDestroy(graph)
+    finally:
+        torch.cuda.synchronize()
+        L.rf_gemm_destroy()
+        for h in handles:
+            hip.hipStreamDestroy(h)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 200, 7168), (7, 1536, 7168), (100, 72, 256), (1024, 1536, 7168), (1000, 1536, 7168)])
+def test_workspace_bytes_covers_the_plan_that_runs(rfk, m, n, k):
+    """rf_gemm_init with rf_gemm_workspace_bytes: for a tabled, a padded and a small ragged shape the figure is that of a K
+    split's partial sums under the plan the call takes (reported as variant -1 for the small ones: few-rows kernels)."""
+    got = rfk.lib().rf_gemm_workspace_bytes(m, n, k)
+    plan = rfk.select_config(m, n, k)
+    qk = k // 128
+
+    def bytes_of(v, split):
+        parts = -(-qk // -(-qk // split))
+        if parts == 1:
+            return 0
+        if v["variant"] >= 14:
+            return -(-m // v["block_m"]) * v["block_m"] * -(-n // v["block_n"]) * v["block_n"] * 4 * parts
+        return -(-m // 16) * 16 * -(-n // 16) * 16 * 4 * parts
+
+    if plan.variant >= 0:
+        assert got == bytes_of(rfk.variants()[plan.variant], plan.split_k)
+    else:
+        assert got in {bytes_of(v, split) for v in rfk.variants() if v["variant"] >= 14 for split in range(1, qk + 1)}
+        assert (got > 0) == (k > 1024)                     # 56 K blocks in few tiles are split, two are not
