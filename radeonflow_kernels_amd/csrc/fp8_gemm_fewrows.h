@@ -294,7 +294,7 @@ __global__ __launch_bounds__(NW * 64, (FewRowsGeom<TM, TN, NW, DEPTH>::WAVES_PER
     if constexpr (SPLIT) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        volatile unsigned *mailbox = (volatile unsigned *)lds;        // every wave has read the sums exchanged there
+        RF_LDS unsigned *mailbox = (RF_LDS unsigned *)lds;            // every wave has read the sums exchanged there
         if (threadIdx.x == 0) {
             const unsigned w = arrival_weight(blockIdx.y, (unsigned)splits);
             *mailbox = __hip_atomic_fetch_add(counters + item, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + w;
