@@ -517,9 +517,14 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     out->split_k = 1;
     out->group_m = 8;
     out->stream_k = 0;
+    auto fewrows_usable = [&](const TunedPlan &p) {
+        const Variant &v = kVariants[p.variant];
+        return !(stage & kTiledOnly) && p.stream_k == RF_SCHEDULE_TILES && fewrows_ok(m, n) &&
+               (p.split_k == 1 || (long)ceil_div(m, v.bm) * ceil_div(n, v.bn) <= kMaxTileCounters);
+    };
     auto usable = [&](const TunedPlan &p) {
         return p.m == m && p.n == n && p.k == k && p.variant < kNumVariants && p.split_k <= k / rf::BK &&
-               !((stage & kTiledOnly) && kVariants[p.variant].is_fewrows()) &&
+               (!kVariants[p.variant].is_fewrows() || fewrows_usable(p)) &&
                (kVariants[p.variant].k_groups == 1 || (p.split_k == 1 && (k / rf::BK) % kVariants[p.variant].k_groups == 0)) &&
                (p.stream_k != RF_SCHEDULE_PERSISTENT || persistent_ok(kVariants[p.variant], m, n, k)) &&
                (p.stream_k != RF_SCHEDULE_STREAM_K || stream_k_ok(kVariants[p.variant], m, n, num_cu)) &&

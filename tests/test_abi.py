@@ -231,6 +231,27 @@ def test_planner_arithmetic_on_the_host_for_any_compute_unit_count(tmp_path):
     assert rfk.lib().rf_gemm_plan_for(16, 16, 128, 256, None) == 2
 
 
+def test_few_rows_plans_that_cannot_run_are_skipped_at_lookup(tmp_path):
+    """Plan files may name a few-rows variant for a shape it does not take: 2^25 rows, more tiles than arrival counters with a
+    K split, another schedule than one workgroup per tile. Such a plan is skipped (it failed the call); one that fits is used."""
+    import radeonflow_kernels_amd as rfk
+    plans = tmp_path / "few.plans"
+    big = 16385 * 32
+    plans.write_text("33554432 16 128 14 1 8 0\n16 33554432 128 14 1 8 0\n16 %d 256 14 2 8 0\n16 %d 384 14 1 8 0\n"
+                     "16 256 256 14 1 8 4\n16 %d 256 14 2 8 0\n" % (big, big, big - 32))
+    try:
+        assert rfk.load_plans(str(plans)) == 6
+        assert rfk.plan_for(33554432, 16, 128, 256).variant < 14
+        assert rfk.plan_for(16, 33554432, 128, 256).variant < 14
+        assert rfk.plan_for(16, big, 256, 256).split_k == 1
+        assert rfk.plan_for(16, 256, 256, 256).stream_k != 4
+        for shape, split in (((16, big, 384), 1), ((16, big - 32, 256), 2)):
+            got = rfk.plan_for(*shape, 256)
+            assert (got.variant, got.split_k) == (14, split)
+    finally:
+        rfk.clear_plans()
+
+
 def test_grouped_variant_choice_on_the_host():
     """rf_grouped_variant_for needs no device. The queue form (5) is taken where its last tiles of 64..256 rows save at
     least 7 % of the rows the other 256-wide forms compute and it has 1.5 items per compute unit (2.5 below K = 4096);
