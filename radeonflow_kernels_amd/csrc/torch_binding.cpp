@@ -56,9 +56,13 @@ void call(const char *name, const F &f) {
         raise(PyExc_RuntimeError, std::string(name) + " failed (" + std::to_string(rc) + "): " + rf_gemm_last_error());
 }
 
-// Every function: arguments by position, C++ exceptions turned into Python ones.
-template <PyObject *(*F)(PyObject *const *)>
-PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t) {
+// Every function: COUNT arguments by position, C++ exceptions turned into Python ones.
+template <PyObject *(*F)(PyObject *const *), int COUNT>
+PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t count) {
+    if (count != COUNT) {
+        PyErr_Format(PyExc_TypeError, "expected %d arguments, got %zd", COUNT, count);
+        return nullptr;
+    }
     try {
         return F(args);
     } catch (const PyError &) {
@@ -283,14 +287,14 @@ PyObject *py_quantize_a_grouped(PyObject *const *v) {
     return pair_of(a, s);
 }
 
-#define RF_ENTRY(name, f) {name, (PyCFunction)(void (*)(void))entry<f>, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {RF_ENTRY("check_operands", py_check_operands),
-                         RF_ENTRY("fp8_mm", py_fp8_mm),
-                         RF_ENTRY("fp8_mm_static", py_fp8_mm_static),
-                         RF_ENTRY("fp8_mm_grouped", py_fp8_mm_grouped),
-                         RF_ENTRY("fp8_mm_grouped_padded", py_fp8_mm_grouped_padded),
-                         RF_ENTRY("quantize", py_quantize),
-                         RF_ENTRY("quantize_a_grouped", py_quantize_a_grouped),
+#define RF_ENTRY(name, f, count) {name, (PyCFunction)(void (*)(void))entry<f, count>, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {RF_ENTRY("check_operands", py_check_operands, 5),
+                         RF_ENTRY("fp8_mm", py_fp8_mm, 6),
+                         RF_ENTRY("fp8_mm_static", py_fp8_mm_static, 5),
+                         RF_ENTRY("fp8_mm_grouped", py_fp8_mm_grouped, 7),
+                         RF_ENTRY("fp8_mm_grouped_padded", py_fp8_mm_grouped_padded, 7),
+                         RF_ENTRY("quantize", py_quantize, 2),
+                         RF_ENTRY("quantize_a_grouped", py_quantize_a_grouped, 2),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_binding", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
