@@ -130,7 +130,7 @@ PyObject *py_fp8_mm_static(PyObject *const *v) {
     Py_RETURN_NONE;
 }
 
-// A sequence of ints (or of things int() takes) as the C ABI's row offsets.
+// A sequence of ints (or of things int() takes) as the C ABI's row offsets; ValueError for one that 32 bits do not hold.
 std::vector<int> offsets_of(PyObject *o) {
     PyObject *seq = PySequence_Fast(o, "row_offsets must be a sequence");
     if (!seq) throw PyError();
@@ -140,8 +140,12 @@ std::vector<int> offsets_of(PyObject *o) {
         PyObject *x = PySequence_Fast_GET_ITEM(seq, i);
         PyObject *num = PyLong_Check(x) ? (Py_INCREF(x), x) : PyNumber_Long(x);
         if (num) {
-            out[(size_t)i] = (int)PyLong_AsUnsignedLongMask(num);
+            int overflow = 0;
+            const long long value = PyLong_AsLongLongAndOverflow(num, &overflow);
             Py_DECREF(num);
+            out[(size_t)i] = (int)value;
+            if (!PyErr_Occurred() && (overflow || value != out[(size_t)i]))
+                PyErr_SetString(PyExc_ValueError, "row_offsets must fit 32 bits");
         }
         if (PyErr_Occurred()) {
             Py_DECREF(seq);

@@ -20,3 +20,13 @@ def test_a_call_with_another_number_of_arguments_is_refused(native, name, count)
     for n in (0, count - 1, count + 1):
         with pytest.raises(TypeError, match="expected %d arguments, got %d" % (count, n)):
             getattr(native, name)(*[x] * n)
+
+
+@pytest.mark.parametrize("last", [2**32 + 16, 2**31, -2**31 - 1, 2**70])
+def test_row_offsets_that_32_bits_do_not_hold_are_refused(native, last):
+    """2^32 + 16 used to count as 16, the number of rows, and went on to the device check."""
+    x = torch.zeros((16, 128))
+    with pytest.raises(ValueError, match="32 bits"):
+        native.quantize_a_grouped(x, [0, last])
+    with pytest.raises(ValueError, match="on the GPU"):
+        native.quantize_a_grouped(x, torch.tensor([0, 16]))           # anything int() takes
