@@ -10,6 +10,8 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 
@@ -228,7 +230,12 @@ void check_source(const at::Tensor &x) {
 // A [rows, cols] tensor over [cols][rows] storage: the transposed view that fp8_mm takes.
 at::Tensor empty_column_major(const at::Tensor &like, int64_t rows, int64_t cols, at::ScalarType type) {
     const int64_t size[2] = {rows, cols}, stride[2] = {1, rows};
-    return at::detail::empty_strided_cuda(size, stride, type, like.device());
+    // Straight to the allocation where nothing listens on the way: no dispatch mode, functorch level, autocast, inference mode
+    // or profiler of this thread. Through the dispatcher a tensor costs 0.28 us more (quantize_a on 7 x 1536: 4.4 -> 4.95 us).
+    const c10::impl::LocalDispatchKeySet keys = c10::impl::tls_local_dispatch_key_set();
+    if (keys.included_ == c10::default_included_set && keys.excluded_ == c10::default_excluded_set && !at::hasCallbacks())
+        return at::detail::empty_strided_cuda(size, stride, type, like.device());
+    return at::empty_strided(size, stride, at::TensorOptions().dtype(type).device(like.device()));
 }
 
 PyObject *pair_of(const at::Tensor &x, const at::Tensor &y) {

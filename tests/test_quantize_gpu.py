@@ -228,3 +228,30 @@ def test_grouped_quantiser_equals_the_plain_one_per_group(rfk, sizes):
             assert torch.equal(sa[pad[g]:pad[g] + n], s)
         assert int(a[pad[g] + n:pad[g + 1]].contiguous().view(torch.uint8).sum(dtype=torch.int64)) == 0
         assert bool((sa[pad[g] + n:pad[g + 1]] == 1.0).all())
+
+
+def test_outputs_are_allocated_through_the_dispatcher():
+    """A dispatch mode and the profiler see the tensors that the quantisers allocate, as they see torch.empty, and inference mode
+    gives inference tensors."""
+    import radeonflow_kernels_amd as rfk
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Count(TorchDispatchMode):
+        allocated = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.allocated += "empty" in str(func)
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn((32, 256), device="cuda")
+    for call in (lambda: rfk.quantize_a(x), lambda: rfk.quantize_b(x), lambda: rfk.quantize_a_grouped(x, [0, 20, 32])):
+        with Count() as mode:
+            call()
+        assert mode.allocated == 2
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CPU]) as prof:
+        rfk.quantize_a(x)
+    assert sum(e.count for e in prof.key_averages() if "empty" in e.key) >= 2
+    with torch.inference_mode():
+        q, s = rfk.quantize_a(x)
+    assert q.is_inference() and s.is_inference()
