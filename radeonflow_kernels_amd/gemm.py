@@ -133,8 +133,13 @@ class _Binding:
                                % BINDING_PATH)
         lib()
         loader = importlib.machinery.ExtensionFileLoader("_torch_binding", BINDING_PATH)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_binding", loader))
-        loader.exec_module(module)
+        try:
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_binding", loader))
+            loader.exec_module(module)
+        except ImportError as e:
+            raise RuntimeError("_torch_binding.so at %s does not load with PyTorch %s: it belongs to the PyTorch (and Python) it "
+                               "was built with, build it again with `python -m radeonflow_kernels_amd.build` (%s)"
+                               % (BINDING_PATH, torch.__version__, e)) from e
         _native = module
         return getattr(module, name)
 

@@ -30,3 +30,16 @@ def test_row_offsets_that_32_bits_do_not_hold_are_refused(native, last):
         native.quantize_a_grouped(x, [0, last])
     with pytest.raises(ValueError, match="on the GPU"):
         native.quantize_a_grouped(x, torch.tensor([0, 16]))           # anything int() takes
+
+
+def test_a_module_built_for_another_torch_says_how_to_build_it_again(tmp_path, monkeypatch):
+    """A library with a symbol that this PyTorch does not have, as one built against another version would be."""
+    import subprocess
+    from radeonflow_kernels_amd import gemm
+    src, so = tmp_path / "m.cpp", str(tmp_path / "_torch_binding.so")
+    src.write_text('extern "C" int no_such_torch_symbol(); extern "C" void *PyInit__torch_binding() '
+                   '{ return no_such_torch_symbol() ? nullptr : nullptr; }')
+    subprocess.run(["g++", "-shared", "-fPIC", "-Wl,-z,now", "-o", so, str(src)], check=True)
+    monkeypatch.setattr(gemm, "BINDING_PATH", so)
+    with pytest.raises(RuntimeError, match="radeonflow_kernels_amd.build.*no_such_torch_symbol"):
+        gemm._Binding().fp8_mm()
