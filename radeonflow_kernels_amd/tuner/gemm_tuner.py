@@ -8,7 +8,7 @@ DISPATCH_GEMM(...) line. Here nothing is recompiled: every kernel variant is alr
   python -m radeonflow_kernels_amd.tuner.gemm_tuner --M 6144 --N 4608 --K 7168        one shape
   python -m radeonflow_kernels_amd.tuner.gemm_tuner --all [--extended] --emit          every known shape (and M = 16 ...
                                                                                        8192 for each of their (N, K)),
-                                                                                       then rewrite csrc/tuned_plans.inc
+                                                                                       then update csrc/tuned_plans.inc
   python -m radeonflow_kernels_amd.tuner.gemm_tuner --M .. --N .. --K .. --emit-file my.plans
                                                   append the winner to a plan file: rf_gemm_load_plans(path) or the
                                                   environment variable RF_GEMM_PLANS uses it without a rebuild
@@ -38,6 +38,7 @@ SHAPES = [
 EXTENDED_M = (16, 32, 48, 64, 96, 128, 192, 256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192)
 EXTENDED = [(m, n, k) for (n, k) in sorted({(n, k) for _, n, k in SHAPES if (n, k) != (64, 128)}) for m in EXTENDED_M
             if (m, n, k) not in SHAPES]
+ROTATED_ROWS = 512
 SPLITS = (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16)
 GROUPS = (4, 8, 16)
 
@@ -53,23 +54,63 @@ def _inputs(m, n, k):
     return a, b, sa, sb, c
 
 
-def _time(rfk, args, cfg, iters):
-    # timed inside the library: a Python call costs more than the GPU time of the small shapes
-    return rfk.fp8_mm_time(*args, config=cfg, warmup=3, iters=iters)
+def operand_sets(m, n, k, least_bytes=64 << 20, most=16):
+    """Operand sets of one shape, together at least least_bytes (twice the L2 caches) where `most` of them are enough."""
+    return [_inputs(m, n, k) for _ in range(max(2, min(most, -(-least_bytes // (k * (m + n))))))]
+
+
+def rotated_us(rfk, sets, cfg, launches=64, replays=3):
+    """Microseconds per launch over operand sets in rotation: the launches are captured into a graph (a Python call takes
+    longer than a small launch), the fastest of a few replays counts."""
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = float("inf")
+    with torch.cuda.stream(stream):
+        rfk.fp8_mm(*sets[0], config=cfg)                 # temporary memory is there before the capture
+        stream.synchronize()
+        graph.capture_begin()
+        try:
+            for i in range(launches):
+                rfk.fp8_mm(*sets[i % len(sets)], config=cfg)
+        finally:
+            graph.capture_end()
+        for _ in range(1 + replays):                     # the first one warms up
+            start.record()
+            graph.replay()
+            stop.record()
+            stream.synchronize()
+            best = min(best, start.elapsed_time(stop) * 1e3 / launches)
+    return best
+
+
+def settle(rfk, seconds=0.4):
+    """Clocks ramp up over tens of milliseconds of load."""
+    args = _inputs(1024, 1536, 7168)
+    rfk.fp8_mm_time(*args, warmup=3, iters=int(seconds * 1e6 / rfk.fp8_mm_time(*args, warmup=3, iters=20)))
+
+
+def _time(rfk, sets, cfg, iters):
+    # up to ROTATED_ROWS rows: a weight matrix that stays in L2 between launches flatters narrow strips. Beyond, one operand
+    # set, timed by the library's launch loop.
+    if len(sets) > 1:
+        return rotated_us(rfk, sets, cfg, launches=-(-iters // len(sets)) * len(sets))
+    return rfk.fp8_mm_time(*sets[0], config=cfg, warmup=3, iters=iters)
 
 
 def tune_shape(rfk, m, n, k, log=print):
     """Times every usable plan; returns a list of dicts sorted by time."""
-    args = _inputs(m, n, k)
+    sets = operand_sets(m, n, k) if m <= ROTATED_ROWS else [_inputs(m, n, k)]
+    args = sets[0]
     default = rfk.select_config(m, n, k)
     if default.variant < 0:
-        log("%dx%dx%d: bounds-checked kernel only (M or N not a multiple of 16)" % (m, n, k))
+        log("%dx%dx%d: a small ragged shape, which takes the few-rows kernel estimated fastest and no plan" % (m, n, k))
         return []
     flop = 2.0 * m * n * k
     # clocks ramp up over tens of milliseconds of load: warm up with the default plan before comparing
-    t_est = _time(rfk, args, None, 20)
-    _time(rfk, args, None, max(20, int(60e3 / max(t_est, 1.0))))
-    iters = max(20, min(400, int(20e3 / max(t_est, 1.0))))
+    t_est = rfk.fp8_mm_time(*args, warmup=3, iters=20)
+    rfk.fp8_mm_time(*args, warmup=3, iters=max(20, int(60e3 / max(t_est, 1.0))))
+    iters = max(20, min(400, int(20e3 / max(t_est, 1.0)))) if len(sets) == 1 else 48
     rfk.fp8_mm(*args)
     torch.cuda.synchronize()
     ref = args[4].clone()
@@ -100,7 +141,7 @@ def tune_shape(rfk, m, n, k, log=print):
             for gm in (GROUPS if sk != 4 and not few_rows else GROUPS[1:2]):   # the skinny-K schedule has no tile order either
                 cfg = rfk.GemmConfig(v["variant"], split, gm, sk)
                 args[4].zero_()
-                us = _time(rfk, args, cfg, iters)
+                us = _time(rfk, sets, cfg, iters)
                 # every plan must reproduce the default plan's output up to split-K reassociation
                 err = (args[4].float() - ref.float()).abs().max().item()
                 scale = ref.float().abs().max().item() + 1e-30
@@ -122,17 +163,41 @@ def best_for_table(cands):
     return None
 
 
+PLANS_HEADER = (
+    "// Measured on one MI355X by radeonflow_kernels_amd/tuner/gemm_tuner.py --all [--extended] --emit; the plans of up to 512 rows on",
+    "// operand sets that rotate out of the L2 caches (a weight matrix that stays in L2 between launches flatters narrow strips). A",
+    "// shape's plan is replaced only when a sweep finds one at least 2 % faster in the same sweep. A plan's time is that of the",
+    "// sweep that chose it.",
+    "// {M, N, K, variant, split_k, group_m, stream_k},   time, TFLOP/s")
+REPLACE_FROM = 0.98
+
+
+def read_plans(path):
+    """Plan lines of a tuned_plans.inc: {(M, N, K): line}, in order; {} if there is no such file."""
+    if not os.path.exists(path):
+        return {}
+    with open(path) as f:
+        lines = [l.rstrip("\n") for l in f if l.startswith("{")]
+    return {tuple(int(x) for x in l[1:].split(",")[:3]): l for l in lines}
+
+
 def emit_plans(results, path=PLANS_INC):
-    lines = ["// Generated by radeonflow_kernels_amd/tuner/gemm_tuner.py --all [--extended] --emit on one MI355X; do not edit by hand.",
-             "// {M, N, K, variant, split_k, group_m, stream_k},   best time, TFLOP/s"]
+    """Writes the plan table: the lines of the file that is there, with the plans of swept shapes that have a plan at least 2 %
+    faster than the present one (both times from this sweep) replaced, and new shapes added."""
+    plans = read_plans(path)
     for (m, n, k), cands in results.items():
         b = best_for_table(cands)
         if b is None:
             continue
-        lines.append("{%d, %d, %d, %d, %d, %d, %d},   // %.2f us, %.1f TFLOP/s" % (
-            m, n, k, b["variant"], b["split_k"], b["group_m"], b["stream_k"], b["us"], b["tflops"]))
+        if (m, n, k) in plans:
+            present = tuple(int(x) for x in plans[m, n, k].split("}")[0][1:].split(",")[3:])
+            now = [c["us"] for c in cands if (c["variant"], c["split_k"], c["group_m"], c["stream_k"]) == present]
+            if now and b["us"] > REPLACE_FROM * min(now):
+                continue
+        plans[m, n, k] = "{%d, %d, %d, %d, %d, %d, %d},   // %.2f us, %.1f TFLOP/s" % (
+            m, n, k, b["variant"], b["split_k"], b["group_m"], b["stream_k"], b["us"], b["tflops"])
     with open(path, "w") as f:
-        f.write("\n".join(lines) + "\n")
+        f.write("\n".join(PLANS_HEADER + tuple(plans.values())) + "\n")
 
 
 def main():
@@ -143,7 +208,7 @@ def main():
     ap.add_argument("--all", action="store_true")
     ap.add_argument("--extended", action="store_true", help="with --all: also M = 16 ... 8192 for every (N, K) of the list")
     ap.add_argument("--emit", nargs="?", const=PLANS_INC, default=None, metavar="PATH",
-                    help="rewrite csrc/tuned_plans.inc, or PATH if given (rebuild libgemm.so afterwards)")
+                    help="update csrc/tuned_plans.inc, or PATH if given (rebuild libgemm.so afterwards)")
     ap.add_argument("--emit-file", default=None, help="append the best plan of every tuned shape to this plan file")
     ap.add_argument("--out", default=None)
     ap.add_argument("--part", default=None, metavar="I/N", help="with --all: only every N-th shape, starting at the I-th (a sweep in N runs)")

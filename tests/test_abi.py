@@ -175,6 +175,24 @@ def test_tuner_never_writes_a_stream_k_winner_into_a_table_or_plan_file(tmp_path
     assert len(lines) == 1 and lines[0].startswith("{512, 512, 256, 0, 1, 4, 0}")
 
 
+def test_tuner_replaces_a_tabled_plan_only_when_a_sweep_finds_one_two_percent_faster(tmp_path):
+    """Both times come from the same sweep; shapes that were not swept keep their lines, a plan that can no longer run is
+    replaced. An emit of nothing over a copy of the compiled-in table writes the same bytes."""
+    from radeonflow_kernels_amd.tuner import gemm_tuner as t
+    cand = lambda variant, us: dict(variant=variant, split_k=1, group_m=8, stream_k=0, us=us, tflops=1.0)
+    inc = tmp_path / "plans.inc"
+    inc.write_text("{16, 16, 128, 3, 1, 8, 0},   // 5.00 us\n{32, 16, 128, 3, 1, 8, 0},   // 5.00 us\n"
+                   "{48, 16, 128, 3, 1, 8, 0},   // 5.00 us\n{64, 16, 128, 3, 1, 8, 0},   // 5.00 us\n")
+    t.emit_plans({(16, 16, 128): [cand(7, 9.85), cand(3, 10.0)], (32, 16, 128): [cand(7, 9.8), cand(3, 10.0)],
+                  (48, 16, 128): [cand(7, 11.0)], (80, 16, 128): [cand(7, 1.0)]}, str(inc))
+    assert {s: int(l.split(",")[3]) for s, l in t.read_plans(str(inc)).items()} == {
+        (16, 16, 128): 3, (32, 16, 128): 7, (48, 16, 128): 7, (64, 16, 128): 3, (80, 16, 128): 7}
+    before = open(t.PLANS_INC).read()
+    inc.write_text(before)
+    t.emit_plans({}, str(inc))
+    assert inc.read_text() == before
+
+
 def test_planner_arithmetic_on_the_host_for_any_compute_unit_count(tmp_path):
     """rf_gemm_plan_for needs no device. With 256 compute units a tabled shape gets its tabled plan; with any other count
     the table (measured on 256) is left aside and the cost model counts rounds for the count given: every plan names an
