@@ -466,9 +466,11 @@ const TunedPlan kTunedPlans[] = {
 
 constexpr int kTunedOnCUs = 256;
 
-// Estimated time in microseconds of the best few-rows plan for a shape, and that plan. Fitted (relative error) to 12000
-// launches on operand sets that rotate out of the L2 caches: M = 1 ... 512, 23 pairs of N and K from 200 to 8192 and 128 to
-// 7168, every few-rows variant with 1 to 14 splits. The plan it picks is 4 % slower than the best one measured, on average.
+// Estimated time in microseconds of the best few-rows plan for a shape, and that plan. Fitted (relative error) to about 12900
+// plans on operand sets that rotate out of the L2 caches: M = 1 ... 512, 23 pairs of N and K from 200 to 8192 and 128 to
+// 7168, every few-rows variant with 1 to 14 splits (tuner/fewrows_model.py: --measure takes them, --fit fits; the model
+// stands there too). The plan it picks is 4.1 % slower than the best one measured on average and 29 % at worst; constants
+// fitted anew to a second measurement pick no better ones.
 //   1.96                                       launch, and the way back
 //   + 1.12 + 0.106 per KiB of sums handed over when K is split
 //   + rounds * (b + 0.985 * batches of loads of a wave + c * K blocks of a wave * workgroups sharing a CU), a quarter more
@@ -501,10 +503,13 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
     }
     return best;
 }
-// Beyond these the estimate is not measured (the second one: on devices with kTunedOnCUs units only, others keep the first,
-// and with it the plans of their padded shapes). Aligned rows of B: never the best. A staged copy of B costs a tiled plan three
-// launches and three passes over B and C, which variant 21 beats up to a few thousand rows: 700 x 5003 x 1024 36.4 -> 24.0 us,
-// 1000 x 1000 x 1024 19.4 -> 8.5, 2000 x 2003 x 1024 34.9 -> 24.0, 3000 x 1000 x 384 21.0 -> 11.0.
+// Rows up to which the few-rows kernels are considered; the second one where B (or C) needs staging, on devices with
+// kTunedOnCUs units only (others keep the first, and with it the plans of their padded shapes). The estimate is fitted up to
+// 512 rows and comes out 9 % low beyond. A staged B costs a tiled plan up to three launches, which variant 21 beats up to a
+// few thousand rows while N is small: few rows against the best of 25 tiled plans with their staging (fewrows_model.py
+// --meet), us: 1000 x 1000 x 1024 8.5, 15.8; 1500 x 1000 x 2048 17.6, 22.8; 3000 x 1000 x 384 11.0, 13.9; 700 x 5003 x 1024
+// 24.1, 21.3; 2000 x 2003 x 1024 24.4, 18.6. Only M ragged: tiled plans above 512 rows, also where a small N would have the
+// few-rows kernels ahead (1037 x 336 x 1024 11.8, few rows 7.0; but 1001 x 576 x 7168 22.0, few rows 24.0).
 constexpr int kFewRowsMaxM = 512, kFewRowsMaxMStagedB = 4096;
 
 // What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
@@ -630,9 +635,13 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     }
     if (hit) take(*hit);                                    // a measured plan, but one that would run on staged copies
     // Few rows: the few-rows kernels, which need no staging, when they come out faster. The model above ranks tiled plans;
-    // what their launches take is 3.1 us + 0.67 of its figure, and staging adds the copies' launches and bytes
-    // (fitted to the same measurements as fewrows_plan). Over 280 shapes the choice between the two families is within 4 %
-    // of the best plan of either, on average.
+    // what their launches take is 3.1 us + 0.67 of its figure, and staging adds the copies' launches and bytes. B's term
+    // counts C's way back for every plan, although plans of one K part and one workgroup per tile store into a ragged C
+    // themselves. Measured with that in place on 82 shapes of ragged N and 100 to 4096 rows, the plan taken is 4.0 % behind
+    // the best of either family on average, 39 % at worst (4096 x 1000 x 1024: 20.1 us on 128 x 128 tiles and a copy of C,
+    // 14.7 on 128 x 192 tiles); only M ragged, up to 512 rows: 3.0 % and 17 %. Counting C's way back (1.0 us + 0.9 us per
+    // million outputs) per plan instead made 33 of 187 shapes 5 % faster on average, but ten of them 1 to 31 % slower
+    // (664 x 3001 x 7168 43 -> 56 us: the figure of a K split is too high against that of one part).
     const int max_m = (stage & kStageB) && num_cu == kTunedOnCUs ? kFewRowsMaxMStagedB : kFewRowsMaxM;
     if (m <= max_m && fewrows_ok(m, n) && !(stage & kTiledOnly)) {
         double tiled = 3.1 + 0.67 * best_cost;

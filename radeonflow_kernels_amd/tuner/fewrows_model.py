@@ -1,0 +1,198 @@
+"""The time estimate of the few-rows kernels that the automatic plans use (fewrows_plan in csrc/gemm_launcher.hip): the
+measurements behind it, its fit, and the shapes where the few-rows and the tiled kernels meet.
+
+  python -m radeonflow_kernels_amd.tuner.fewrows_model --measure FILE    every variant and K split over M = 1 ... 512 and the
+                                                                         (N, K) of PAIRS, on operand sets in rotation
+  python -m radeonflow_kernels_amd.tuner.fewrows_model --fit FILE        how far the estimate's choice is from the fastest plan
+                                                                         measured, and the constants refitted to the file
+  python -m radeonflow_kernels_amd.tuner.fewrows_model --meet FILE       ragged shapes: the automatic few-rows plan against
+                                                                         tiled plans with their staging copies
+FILE has one line per plan: M N K variant split_k us (--meet: for each shape the times of both sides). --measure and --meet
+need the GPU; the estimate and the fit do not.
+"""
+import argparse
+import os
+import tempfile
+
+import numpy as np
+
+BK = 128
+MAX_TILE_COUNTERS = 16384
+SPLITS = (1, 2, 3, 4, 5, 6, 8, 12, 14)
+# variant: tile rows, columns, waves, workgroups that share a CU, K blocks a wave asks for at a time; b, c, d (see estimate)
+VARIANTS = {14: (16, 32, 8, 2, 3), 15: (16, 64, 8, 1, 2), 16: (16, 128, 8, 1, 1), 17: (32, 32, 8, 2, 2), 18: (32, 64, 8, 1, 2),
+            19: (64, 32, 8, 1, 2), 20: (64, 64, 8, 1, 1), 21: (64, 64, 4, 2, 1)}
+FIT = {14: (0.0, 0.458, 0.0916), 15: (0.0, 0.860, 0.0591), 16: (0.790, 0.665, 0.0381), 17: (0.0, 0.572, 0.0755),
+       18: (0.101, 1.090, 0.0546), 19: (0.127, 1.063, 0.0593), 20: (1.651, 0.929, 0.0362), 21: (2.48, 0.424, 0.0231)}
+COMMON = (1.96, 1.12, 0.106, 0.985)      # launch; handing sums over, and per KiB of them; a batch of a wave's loads
+ANY_BYTES = 1.27
+
+ROWS = (1, 7, 16, 24, 32, 48, 64, 100, 128, 200, 256, 333, 512)
+PAIRS = ((1536, 7168), (4608, 7168), (7168, 2048), (7168, 256), (576, 7168), (3072, 1536), (7168, 2304), (512, 7168), (4096, 512),
+         (4096, 7168), (256, 1024), (1024, 2048), (2048, 4096), (8192, 1024), (8192, 7168), (256, 7168), (200, 2048), (1000, 384),
+         (1000, 4096), (2003, 1024), (2003, 7168), (5003, 2048), (5003, 128))
+# ragged shapes between a few hundred and a few thousand rows: N ragged, M ragged, both
+MEET = ((601, 5003, 2048), (700, 5003, 1024), (1000, 1000, 1024), (1000, 1000, 4096), (1000, 2003, 1024), (2000, 2003, 1024),
+        (3000, 1000, 384), (700, 1000, 7168), (1008, 5003, 2048), (1500, 1000, 2048), (2000, 5003, 512), (2000, 1000, 7168),
+        (4000, 200, 2048), (4096, 1000, 1024), (4001, 2003, 384), (513, 5003, 7168), (800, 200, 7168), (3000, 2003, 2048),
+        (300, 5003, 2048), (200, 2003, 7168), (100, 5003, 7168), (500, 200, 7168),
+        (601, 1536, 7168), (513, 7168, 256), (1001, 576, 7168), (300, 512, 7168), (250, 1536, 7168), (333, 7168, 2048),
+        (130, 4608, 7168), (500, 4096, 512), (200, 3072, 1536))
+
+
+def _ceil(a, b):
+    return -(-a // b)
+
+
+def _terms(variant, m, n, k, split, num_cu):
+    """(parts, KiB of sums, rounds, batches, K blocks of a wave times workgroups sharing a CU, MB fetched), or None if the
+    planner does not consider this split."""
+    bm, bn, waves, per_cu, depth = VARIANTS[variant]
+    qk, items = k // BK, _ceil(m, bm) * _ceil(n, bn)
+    if split > qk or (split > 1 and (items * split > 4 * num_cu or items > MAX_TILE_COUNTERS)):
+        return None
+    kb = _ceil(qk, split)
+    parts, own = _ceil(qk, kb), _ceil(kb, waves)
+    wgs = items * parts
+    return (parts, parts * bm * bn / 1024.0, _ceil(wgs, num_cu * per_cu), _ceil(own, depth), own * (per_cu if wgs > num_cu else 1),
+            wgs * kb * (bm + bn) * BK * 1e-6 * 256 / num_cu)
+
+
+def estimate(variant, m, n, k, split, num_cu=256, fit=None, common=COMMON):
+    """The estimate of fewrows_plan in us, or None."""
+    t = _terms(variant, m, n, k, split, num_cu)
+    if t is None:
+        return None
+    parts, kib, rounds, batches, blocks, mb = t
+    b, c, d = (fit or FIT)[variant]
+    return common[0] + (common[1] + common[2] * kib if parts > 1 else 0.0) + rounds * (ANY_BYTES if n % 16 else 1.0) * (
+        b + common[3] * batches + c * blocks) + d * mb
+
+
+def choice(m, n, k, num_cu=256, fit=None, common=COMMON):
+    """The (variant, split_k) fewrows_plan picks."""
+    best = None
+    for v in VARIANTS:
+        for s in SPLITS:
+            t = estimate(v, m, n, k, s, num_cu, fit, common)
+            if t is None:
+                break
+            if best is None or t < best[0]:
+                best = (t, v, s)
+    return best[1:]
+
+
+def refit(rows):
+    """Least squares on relative errors; the model is linear in its constants. A constant of a variant that comes out negative
+    is taken as zero. Returns (FIT, COMMON)."""
+    names = ["launch", "split", "kib", "batch"] + [(v, i) for v in VARIANTS for i in range(3)]
+    column = {x: i for i, x in enumerate(names)}
+    a = np.zeros((len(rows), len(names)))
+    for r, (m, n, k, v, s, us) in enumerate(rows):
+        parts, kib, rounds, batches, blocks, mb = _terms(v, m, n, k, s, 256)
+        f = rounds * (ANY_BYTES if n % 16 else 1.0)
+        for x, value in (("launch", 1.0), ("split", float(parts > 1)), ("kib", kib if parts > 1 else 0.0), ("batch", f * batches),
+                         ((v, 0), f), ((v, 1), f * blocks), ((v, 2), mb)):
+            a[r, column[x]] = value / us
+    used = list(range(len(names)))
+    while True:
+        x = np.linalg.lstsq(a[:, used], np.ones(len(rows)), rcond=None)[0]
+        if (x >= 0).all():
+            break
+        used = [u for u, value in zip(used, x) if value >= 0]
+    full = np.zeros(len(names))
+    full[used] = x
+    return ({v: tuple(round(float(full[column[v, i]]), 4) for i in range(3)) for v in VARIANTS},
+            tuple(round(float(full[column[x]]), 4) for x in names[:4]))
+
+
+def read(path):
+    with open(path) as f:
+        rows = [l.split() for l in f if l[:1].isdigit()]
+    rows = [tuple(int(x) for x in r[:5]) + (float(r[5]),) for r in rows]
+    return [r for r in rows if _terms(r[3], r[0], r[1], r[2], r[4], 256)]
+
+
+def report(rows, fit, common, what):
+    """How far the model is from the measured times, and its choice from the fastest measured plan of each shape."""
+    err = [estimate(v, m, n, k, s, fit=fit, common=common) / us for m, n, k, v, s, us in rows]
+    shapes = {}
+    for m, n, k, v, s, us in rows:
+        shapes.setdefault((m, n, k), {})[v, s] = us
+    behind = [t[choice(*shape, fit=fit, common=common)] / min(t.values()) for shape, t in shapes.items()]
+    print("%s: estimate over measured %.2f ... %.2f, rms of the logarithm %.3f; choice behind the fastest of %d shapes by %.1f %% "
+          "on average, %.0f %% at worst" % (what, min(err), max(err), float(np.sqrt(np.mean(np.log(err) ** 2))), len(shapes),
+                                             100 * (np.mean(behind) - 1), 100 * (max(behind) - 1)))
+
+
+def measure(path):
+    import radeonflow_kernels_amd as rfk
+    from . import gemm_tuner as t
+    t.settle(rfk)
+    with open(path, "w") as f:
+        for n, k in PAIRS:
+            for m in ROWS:
+                sets = t.operand_sets(m, n, k)
+                for v in VARIANTS:
+                    for s in SPLITS:
+                        if _terms(v, m, n, k, s, 256):
+                            f.write("%d %d %d %d %d %.2f\n" % (m, n, k, v, s, t.rotated_us(rfk, sets, rfk.GemmConfig(v, s, 8, 0), 32, 2)))
+                f.flush()
+            print(n, k, flush=True)
+
+
+# tiled plans tried on the padded shape (variant, split_k, schedule)
+TILED = [(v, s, 0) for v in (7, 9) for s in (1, 2, 3, 4)] + [(v, s, 0) for v in (6, 8, 3, 10) for s in (1, 2, 3)] + \
+        [(v, 1, 0) for v in (0, 1, 5, 11, 12, 13)] + [(0, 1, 2), (1, 1, 2), (3, 1, 2), (8, 6, 0)]
+
+
+def meet(path):
+    """Per shape: the automatic plan, the few-rows plan the estimate picks and the fastest tiled plan (named by a plan file for
+    the padded shape), all with what they need around them."""
+    import radeonflow_kernels_amd as rfk
+    from . import gemm_tuner as t
+    t.settle(rfk)
+    with tempfile.TemporaryDirectory() as d, open(path, "w") as f:
+        plans = os.path.join(d, "p.plans")
+        for m, n, k in MEET:
+            sets = t.operand_sets(m, n, k)
+            auto = t.rotated_us(rfk, sets, None, 32)
+            few = choice(m, n, k)
+            few_us = t.rotated_us(rfk, sets, rfk.GemmConfig(few[0], few[1], 8, 0), 32)
+            plan = rfk.select_config(m, n, k)
+            best = None
+            for v, s, sched in TILED:
+                with open(plans, "w") as p:
+                    p.write("%d %d %d %d %d 8 %d\n" % (_ceil(m, 16) * 16, _ceil(n, 16) * 16, k, v, s, sched))
+                rfk.load_plans(plans)
+                got = rfk.select_config(m, n, k)
+                if (got.variant, got.split_k, got.stream_k) == (v, s, sched):
+                    us = t.rotated_us(rfk, sets, None, 16, 2)
+                    best = min(best or (us, v, s, sched), (us, v, s, sched))
+                rfk.clear_plans()
+            f.write("%d %d %d  auto %d/%d/%d %.2f  few rows %d/%d %.2f (estimate %.2f)  tiled %d/%d/%d %.2f\n" % (
+                m, n, k, plan.variant, plan.split_k, plan.stream_k, auto, few[0], few[1], few_us,
+                estimate(few[0], m, n, k, few[1]), best[1], best[2], best[3], best[0]))
+            f.flush()
+            print(m, n, k, flush=True)
+
+
+def main():
+    ap = argparse.ArgumentParser()
+    for name in ("measure", "fit", "meet"):
+        ap.add_argument("--" + name, metavar="FILE")
+    a = ap.parse_args()
+    if a.measure:
+        measure(a.measure)
+    if a.fit:
+        rows = read(a.fit)
+        report(rows, FIT, COMMON, "%d measurements, constants in use" % len(rows))
+        fit, common = refit(rows)
+        report(rows, fit, common, "refitted")
+        print("COMMON =", common, "\nFIT =", fit)
+    if a.meet:
+        meet(a.meet)
+
+
+if __name__ == "__main__":
+    main()

@@ -313,3 +313,21 @@ def test_grouped_few_rows_choice_on_the_host():
     assert choice(33, 32, 2048, 7168) < 6 and choice(16, 32, 2056, 7168) < 6 and choice(16, 64, 4096, 7168) < 6
     # few tiles: 128 x 128 while they are alone on their compute unit, then 128 x 256; short K keeps the most workgroups
     assert choice(100, 8, 2048, 7168) == 2 and choice(300, 8, 2048, 7168) == 1 and choice(100, 8, 2048, 1024) == 3
+
+
+def test_few_rows_estimate_of_the_tuner_is_the_planners():
+    """The Python statement of the few-rows kernels' time estimate (tuner/fewrows_model.py, where it is measured and fitted) picks
+    the planner's variant and K split wherever the planner takes a few-rows plan by estimate: shapes outside the table, other
+    compute unit counts, ragged ones planned at their padded size."""
+    import random
+    import radeonflow_kernels_amd as rfk
+    from radeonflow_kernels_amd.tuner import fewrows_model as fm
+    rng, seen = random.Random(3), set()
+    for i in range(400):
+        m, n = rng.choice((16, 32, 48, 80, 144, 272, 400)), 16 * rng.randint(2, 500)
+        k, num_cu = 128 * rng.randint(1, 64), rng.choice((64, 255, 256, 304))
+        got = rfk.plan_for(m, n, k, num_cu)
+        if got.variant >= 14:
+            assert (got.variant, got.split_k) == fm.choice(m, n, k, num_cu), (m, n, k, num_cu)
+            seen.add(got.variant)
+    assert len(seen) >= 5, seen
