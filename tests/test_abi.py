@@ -331,3 +331,18 @@ def test_few_rows_estimate_of_the_tuner_is_the_planners():
             assert (got.variant, got.split_k) == fm.choice(m, n, k, num_cu), (m, n, k, num_cu)
             seen.add(got.variant)
     assert len(seen) >= 5, seen
+
+
+def test_benchmark_hashes_every_gemm_source():
+    """The traffic figures under profiles/ belong to a hash of the GEMM's sources: the launcher and every header it reaches,
+    but for the quantisers' and the C ABI."""
+    import bench
+    csrc = os.path.join(ROOT, "radeonflow_kernels_amd", "csrc")
+    reached, todo = set(), ["gemm_launcher.hip"]
+    while todo:
+        name = todo.pop()
+        if name not in reached:
+            reached.add(name)
+            todo += [os.path.basename(x) for x in re.findall(r'#include "([^"]+\.h)"', open(os.path.join(csrc, name)).read())
+                     if os.path.dirname(x) == ""]
+    assert sorted(bench.KERNEL_SOURCES) == sorted(reached - {"quantize_kernels.h"})
