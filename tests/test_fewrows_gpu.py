@@ -123,3 +123,112 @@ def test_grouped_fewrows_bits_of_the_tiled_form(rfk, rows, n, k, shift):
     for variant in (6, 7, 8, 9, -1):
         assert np.array_equal(launch(rfk.fp8_mm_grouped, a, sa, variant), expect), variant
         assert np.array_equal(launch(rfk.fp8_mm_grouped_padded, a_pad.view(fp8).T, sa_pad.T, variant), expect), variant
+
+
+def test_fewrows_k_splits_on_two_streams_at_once(rfk):
+    """Different numbers of K parts on two streams, launches queued deep: every stream has counters and slots of its own, so each
+    result is the one the same plan gives alone."""
+    problems = [(to_gpu(exact_problem(m, n, k, m + k)), oracle_bf16(exact_problem(m, n, k, m + k)), cfg)
+                for m, n, k, cfg in ((7, 1536, 7168, rfk.GemmConfig(14, 4, 8, 0)), (40, 1000, 4096, rfk.GemmConfig(17, 7, 8, 0)))]
+    streams = [torch.cuda.Stream() for _ in problems]
+    outs = [[torch.full_like(g[4], -1.0) for _ in range(40)] for g, _, _ in problems]
+    torch.cuda.synchronize()
+    for i in range(40):
+        for (g, _, cfg), s, out in zip(problems, streams, outs):
+            with torch.cuda.stream(s):
+                rfk.fp8_mm(*g[:4], out[i], config=cfg)
+    torch.cuda.synchronize()
+    for (_, exp, _), out in zip(problems, outs):
+        for i, c in enumerate(out):
+            assert np.array_equal(bf16_bits(c), exp), i
+
+
+def _signed_ones_and_twos(shape, gen):
+    """e4m3fn codes of +-1 and +-2."""
+    r = torch.randint(0, 4, shape, dtype=torch.uint8, device="cuda", generator=gen)
+    return 0x38 + ((r & 1) << 3) + ((r & 2) << 6)
+
+
+# 127 rows of a K block from 16,909,320 columns on are more than 2^31 bytes: a width that starts at any byte and one of aligned
+# rows, and the same many rows of A
+@pytest.mark.parametrize("m,n", [(3, 17000003), (3, 17000016), (17000003, 16)])
+def test_fewrows_offsets_beyond_31_bits(rfk, m, n):
+    k, fp8 = 256, torch.float8_e4m3fn
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    a, b = (_signed_ones_and_twos((k, x), gen).view(fp8) for x in (m, n))
+    sa = torch.randint(1, 3, (2, m), device="cuda", generator=gen).float()
+    sb = torch.randint(1, 3, (2, (n + 127) // 128), device="cuda", generator=gen).float()
+    buf = torch.full((m * n + 300,), -7.0, dtype=torch.bfloat16, device="cuda")
+    c = buf[:m * n].view(m, n)
+    plans = FEW_ROWS if m == 3 else (14, 18, 21)
+    for v in plans:
+        c.fill_(-7.0)
+        rfk.fp8_mm(a.T, b.T, sa.T, sb.T, c, config=rfk.GemmConfig(v, 1, 8, 0))
+        step = 1 << 20
+        for x0 in range(0, max(m, n), step):                   # sums of integers below 2^12: exact in any order
+            rows, cols = (slice(None), slice(x0, x0 + step)) if n > m else (slice(x0, x0 + step), slice(None))
+            exp = 0
+            for kb in range(2):
+                part = a[kb * 128:kb * 128 + 128, rows].float().T @ b[kb * 128:kb * 128 + 128, cols].float()
+                scale_n = sb[kb].repeat_interleave(128)[:n][cols]
+                exp = exp + part * sa[kb, rows][:, None] * scale_n[None, :]
+            assert torch.equal(c[rows, cols], exp.bfloat16()), (v, x0)
+        assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max()), v
+
+
+def _with_nans_and_infinities(m, n, k, seed):
+    """Exact data with NaN codes in one row of A and one column of B and infinite scales; the expected bits, K blocks folded one
+    after the other, and where they are NaN."""
+    from oracle import cref
+    a, b, sa, sb, c = exact_problem(m, n, k, seed)
+    fp8 = torch.float8_e4m3fn
+    a8, b8, sa, sb = a.view(torch.uint8).clone(), b.view(torch.uint8).clone(), sa.clone(), sb.clone()
+    a8[m // 2, 17] = 0x7F
+    b8[n - 1, k - 1] = 0xFF
+    sa[m - 1, 0] = float("inf")
+    sb[0, k // 128 - 1] = float("-inf")
+    sa[0, k // 128 - 1] = 0.0                                  # 0 * -inf
+    exp = cref.ref_gemm_blockfold(*(x.T.contiguous().view(torch.uint8).numpy() for x in (a8, b8)),
+                                  *(x.T.contiguous().numpy() for x in (sa, sb)), rows=np.arange(m))[1]
+    nan = (exp & 0x7FFF) > 0x7F80
+    assert nan[m // 2].all() and nan[:, n - 1].all() and nan[0, :min(n, 128)].all() and not nan.all()
+    assert ((exp[m - 1] & 0x7FFF) == 0x7F80).any()
+    return (a8.view(fp8), b8.view(fp8), sa, sb, c), exp, nan
+
+
+def _assert_same_values_and_nans(c, exp, nan, what):
+    got = bf16_bits(c)
+    assert np.array_equal((got & 0x7FFF) > 0x7F80, nan), what
+    assert np.array_equal(got[~nan], exp[~nan]), what
+
+
+@pytest.mark.parametrize("m,n,k", [(7, 300, 1280), (40, 160, 1024)])
+def test_fewrows_nan_codes_and_infinite_scales(rfk, m, n, k):
+    """NaN and infinity come out where the oracle has them, under every variant with and without a K split (a sum of splits
+    meets infinities of one sign only: one K block per row and column has them)."""
+    data, exp, nan = _with_nans_and_infinities(m, n, k, 4)
+    g = to_gpu(data)
+    for cfg in [None] + [rfk.GemmConfig(v, s, 8, 0) for v in FEW_ROWS for s in (1, 3)]:
+        g[4].fill_(-1.0)
+        rfk.fp8_mm(*g, config=cfg)
+        torch.cuda.synchronize()
+        _assert_same_values_and_nans(g[4], exp, nan, "plan %r" % (cfg,))
+
+
+def test_stores_into_any_c_keep_nans_and_infinities(rfk, tmp_path):
+    """The tile kernels' stores into a ragged C (plan files name the tile for the padded shape)."""
+    m, n, k = 4101, 205, 256
+    data, exp, nan = _with_nans_and_infinities(m, n, k, 9)
+    g = to_gpu(data)
+    plan = tmp_path / "p.plans"
+    for variant in range(12):
+        plan.write_text("4112 208 256 %d 1 8 0\n" % variant)
+        buf = torch.full((m * n + 1,), -7.0, dtype=torch.bfloat16, device="cuda")
+        c = buf[1:].view(m, n)
+        try:
+            assert rfk.load_plans(str(plan)) == 1 and rfk.plan_for(m, n, k, 256).variant == variant
+            rfk.fp8_mm(*g[:4], c)
+            torch.cuda.synchronize()
+        finally:
+            rfk.clear_plans()
+        _assert_same_values_and_nans(c, exp, nan, variant)

@@ -345,6 +345,15 @@ def test_bounds_checked_kernel_on_odd_shapes(rfk, m, n, k):
     assert_few_mismatches_at_reference_atol(out, oracle_bf16(data), "checked kernel")
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 130, 256), (1, 1, 128), (17, 64, 384), (5, 257, 128), (100, 72, 256), (256, 384, 512)])
+def test_bounds_checked_kernel_named_explicitly(rfk, m, n, k):
+    """Variant -1 in an explicit plan is the bounds-checked kernel, also for the shapes whose automatic plan is reported as -1 and
+    runs the few-rows kernels."""
+    data = exact_problem(m, n, k, seed=7 * m + n)
+    out = _run(rfk, data, canary=512, config=rfk.GemmConfig(-1, 1, 1, 0))
+    assert np.array_equal(bf16_bits(out), oracle_bf16(data))
+
+
 # the reference's own test shapes and seeds (scripts/problems/gemm/task.yml:53-64), its input style
 REFERENCE_TESTS = [(64, 64, 128, 6635), (64, 1536, 7168, 6635), (64, 3072, 1536, 1236), (64, 576, 7168, 542),
                    (96, 7168, 256, 1234), (96, 7168, 2048, 4153), (96, 4608, 7168, 412), (128, 7168, 2304, 624),
