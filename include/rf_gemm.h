@@ -10,14 +10,16 @@
  *   bs  fp32,             [K/128][ceil(N/128)]
  *   c   bf16,             [M][N] row-major, fully overwritten
  * All pointers are device pointers. K must be a positive multiple of 128; M, N >= 1.
- * Shapes with M%16==0, N%16==0 and 16-byte aligned a/b/c take the tiled MFMA path as they are. Anything else goes to
- * the few-rows kernels, which take any shape and alignment, where M is small (up to a few hundred rows, whichever is
- * estimated to be faster), and is staged otherwise: the operands that need it are copied with rows padded to a multiple of 16 (zeros) into an internal buffer
- * grown on demand, the tiled path runs on the padded shape, and c receives the result without the padding (cost: one
- * pass over a; when N is ragged or c unaligned also one over b and a staged copy of c). Such problems
- * below 2^21 multiply-adds always take the few-rows kernels (their plan is reported as variant = -1); explicit plans with
- * variant = -1 take a bounds-checked kernel (the role of the reference's legacy kernel,
- * src/gemm/gemm_kernel_legacy.cpp:237-374).
+ * Shapes with M%16==0, N%16==0 and 16-byte aligned a/b/c take the tiled MFMA path, or the few-rows kernels where M is small,
+ * as they are. Anything else goes to the few-rows kernels, which take any shape and alignment, where they are estimated to be
+ * faster (M up to 512; up to 4096 when N is ragged or b or c unaligned), and is staged otherwise: the operands that need it
+ * are copied with rows padded to a multiple of 16 (zeros) into an internal buffer grown on demand, the tiled path runs on the
+ * padded shape, and c receives the result without the padding (cost: one pass over a; when N is ragged or b unaligned also
+ * one over b, and when N is ragged or c unaligned and the plan splits K or is not one workgroup per tile, a padded copy of c
+ * and the way back). Such problems below 2^21 multiply-adds always take the few-rows kernel estimated fastest, whatever
+ * plans are loaded; their plan is reported as variant = -1, which says no more than that. In an explicit plan variant = -1
+ * names a bounds-checked kernel (the role of the reference's legacy kernel, src/gemm/gemm_kernel_legacy.cpp:237-374): 13 to
+ * 27 us where the few-rows kernels take 3 to 4, so a reported -1 is not to be passed on.
  * Temporary device memory (split-K partial sums, staging copies) is kept per (device, stream), for
  * the device that is current at the call: launches on different streams of one device may overlap, launches on one
  * stream are ordered by the stream. Calls are serialised by one lock only while they enqueue. A buffer that has to grow
@@ -64,7 +66,8 @@ enum { RF_SCHEDULE_TILES = 0, RF_SCHEDULE_STREAM_K = 1, RF_SCHEDULE_PERSISTENT =
 /* One launch plan: which kernel variant and how K is split.
  * Replaces a DISPATCH_GEMM(...) line of the reference (src/gemm/gemm_launcher.cpp:158-162,229-259). */
 typedef struct rf_gemm_config {
-    int variant;      /* index into the variant table, see rf_gemm_variant_info(); -1 = bounds-checked kernel. Variants 14
+    int variant;      /* index into the variant table, see rf_gemm_variant_info(); -1 = bounds-checked kernel (reported
+                         by rf_gemm_select_config: a small ragged shape, see above). Variants 14
                          to 21 are the few-rows kernels (16 to 64 rows x 32 to 128 columns per workgroup): any shape with
                          M and N below 2^25, any alignment, K splits summed inside the launch */
     int split_k;      /* >= 1; K blocks are divided over this many partial sums */
@@ -114,7 +117,7 @@ int rf_fp8_gemm(const void *a, const void *b, const float *as, const float *bs, 
  * whose staging copies do not fit as a whole is computed in row ranges that take turns in the array (M = 6001, N = 4608,
  * K = 7168: two ranges); such results agree with rf_fp8_gemm's within the rounding of another K split, and bit for bit
  * on data whose sums are exact. Only when the staged copy of B (ragged N or an unaligned b) alone takes more than half
- * of the array does the much slower bounds-checked kernel compute the shape, in place. All calls on one GPU share that
+ * of the array does a few-rows kernel (64 x 64 tiles) compute the shape, in place. All calls on one GPU share that
  * GPU's array: two calls that overlap in time (different streams, or graph replays beside eager launches) race, and the
  * results of both are undefined (later calls are not affected); calls on one stream are ordered by the stream. */
 int rf_fp8_gemm_static(const void *a, const void *b, const float *as, const float *bs, void *c,
@@ -133,8 +136,9 @@ int rf_fp8_gemm_ex(const void *a, const void *b, const float *as, const float *b
 int rf_fp8_gemm_time(const void *a, const void *b, const float *as, const float *bs, void *c, int m, int n, int k,
                      const rf_gemm_config *cfg, int warmup, int iters, float *us_per_launch, hipStream_t stream);
 
-/* The plan rf_fp8_gemm would use for (m,n,k) on the current device: the gfx950 replacement of the
- * per-shape table in src/gemm/gemm_launcher.cpp:229-259 / tuner/gemm_tuner.py. */
+/* The plan rf_fp8_gemm would use for (m,n,k) with aligned pointers on the current device: the gfx950 replacement of the
+ * per-shape table in src/gemm/gemm_launcher.cpp:229-259 / tuner/gemm_tuner.py. A ragged shape gets the plan of its padded
+ * size; variant -1 stands for the few-rows kernel that small ragged shapes take by estimate (see the top of this file). */
 int rf_gemm_select_config(int m, int n, int k, rf_gemm_config *out);
 
 /* The plan for (m,n,k) on a device with num_cu compute units, worked out on the host alone (no device is touched, the
@@ -192,7 +196,7 @@ void rf_gemm_destroy(void);
  * numbers (token counts per expert are): when one is not a multiple of 16, or a is not 16-byte aligned, the tiled forms
  * have a and as first copied into the internal staging buffer with every group starting at a multiple of 16 (one pass over a;
  * c is written in place, rows of neighbouring groups are not touched). Ragged N, unaligned b or c, and problems below
- * 2^21 multiply-adds run the bounds-checked kernel once per group.
+ * 2^21 multiply-adds that would need that copy run the bounds-checked kernel once per group.
  * variant: -1 = automatic, else an index into {256x256, 128x256, 128x128, 128x64} tiles, or 4 = 256-row tiles with a
  * 128 x 256 tile for a group's last rows when at most 128 are left, or 5 = 256-row tiles with a last tile of 64, 128,
  * 192 or 256 rows, run by one resident workgroup per CU that takes tiles from a queue per XCD (the automatic choice

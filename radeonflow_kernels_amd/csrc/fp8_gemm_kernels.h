@@ -1144,8 +1144,8 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_grouped_queue(
 }
 
 // ---------------------------------------------------------------------------------------------
-// Bounds-checked kernel for shapes or alignments the tiled kernel does not take (M or N not a
-// multiple of 16, unaligned pointers). One wave per 16x16 output tile, bytes gathered directly
+// Bounds-checked kernel, any shape and alignment: explicit plans with variant -1, and grouped calls whose
+// shape or pointers the tiled and few-rows forms do not take. One wave per 16x16 output tile, bytes gathered directly
 // from global memory; out-of-range rows/columns contribute zeros and are not stored.
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void gemm_fp8_blockscale_checked(

@@ -866,13 +866,16 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
 }
 
 // ---- shapes and pointers the tiled kernels do not take as they are ----
-// M or N not a multiple of 16 (or below 16), or operands that are not 16-byte aligned, would leave the whole GEMM to
-// the bounds-checked kernel, which is 7 to 35 times slower (M = 100, N = 4096, K = 7168: 129 us against 17 us for
-// M = 112). Token counts are arbitrary in practice, so for anything but tiny problems the operands that need it are
-// copied into a staging buffer with rows padded to a multiple of 16 (zeros: padded rows and columns produce values
+// M or N not a multiple of 16 (or below 16), or operands that are not 16-byte aligned. Token counts are arbitrary in
+// practice. Where the few-rows kernels, which take such operands as they are, are not the faster ones, the operands that need
+// it are copied into a staging buffer with rows padded to a multiple of 16 (zeros: padded rows and columns produce values
 // nobody reads), the tiled kernels run on the padded shape under the automatic plan and store into the caller's C where they
-// can (one K part, one workgroup per tile); otherwise C is copied back without the padding. b_scale needs no copy: ceil(N/128) does not change. The copies cost K*M (+ K*N when N is ragged) bytes.
-constexpr double kPadThresholdMacs = 2097152.0;            // below this the bounds-checked kernel is as fast
+// can (one K part, one workgroup per tile); otherwise C is copied back without the padding. b_scale needs no copy:
+// ceil(N/128) does not change. The copies cost K*M (+ K*N when N is ragged) bytes.
+// Below this many multiply-adds a ragged shape takes the few-rows kernel estimated fastest without a look at the plans (a
+// launch of a few microseconds, whose plan the table and the cost model do not know better); a grouped call that would have
+// to stage runs the bounds-checked kernel.
+constexpr double kPadThresholdMacs = 2097152.0;
 
 // The grouped GEMM's staging copy: the caller's [rows][m_total] matrix (A with T = bytes, a_scale with T = float), in
 // which group g owns columns out_row_start[g] .. out_row_start[g+1]-1 (counted from column `first`), is copied to
@@ -1384,7 +1387,8 @@ const char *rf_gemm_last_error(void) { return g_last_error.c_str(); }
 }  // extern "C"
 
 namespace {
-// Up to this many elements the activations' quantiser works in 16-row pieces instead of 128-row blocks (see quantize_rows16).
+// Up to this many elements the activations' quantiser works in 16-row pieces instead of 128-row blocks (both measured at
+// quantize_rows16: the line lies between 7 and 10 million, within 8 % either way).
 constexpr double kQuantRows16Elements = 1.0e7;
 // rows x K source (row-major, K contiguous) -> fp8 [K][rows] + scales; see quantize_kernels.h
 template <bool PER_ROW, bool IN_BF16>

@@ -420,10 +420,14 @@ __global__ __launch_bounds__(QuantShape<IN_BF16>::NT) void quantize_block128_gro
 }
 
 // Activations that do not fill the chip with 128 x 128 blocks: one workgroup of 256 threads per 16 rows x 128 k, eight k of
-// one row per thread. A 128-row block of a handful of rows loaded and encoded 128 rows and stored single bytes: 7 x 1536
-// from bf16 6.4 -> 2.35 us (the rate of back-to-back launches), 512 x 7168 6.3 -> 4.0, 2048 x 2048 6.4 -> 4.2. Its stores
-// are 16-byte pieces of rows of the output, which L2 merges as long as they stay there: from about ten million elements on
-// the 128-row blocks are faster (bf16: 1024 x 7168 6.4 against 5.9 here, 2048 x 7168 9.1 against 9.3).
+// one row per thread. A 128-row block of a handful of rows loads and encodes 128 rows and stores single bytes. us with
+// 128-row blocks -> here, from bf16, on sources that rotate out of the caches (one source, which stays there, in brackets):
+// 7 x 1536 4.2 -> 2.3 (the rate of back-to-back launches), 512 x 7168 5.6 -> 4.8 (4.1 -> 3.7), 2048 x 2048 6.0 -> 5.1 (4.2 ->
+// 4.0). Its stores are 16-byte pieces of rows of the output, which L2 merges as long as they stay there: beyond seven to ten
+// million elements the 128-row blocks are faster where they store whole lines (4096 x 2048 7.9 against 8.5 here, 1024 x 7168
+// 7.5 against 8.1, 2048 x 7168 12.4 against 13.4), later where rows are ragged (1400 x 7168 11.2 against 10.7) and about as
+// fast from fp32 (1024 x 7168 9.8, 9.9; 2048 x 7168 16.5, 16.7). Between one launch and the next GEMM it runs at half the copy
+// rate: 2048 x 2048 is 12.6 MB, 2.5 us at 5.1 TB/s, beside 2.3 us that the shortest launch takes.
 template <bool IN_BF16, bool GROUPED>
 __device__ __forceinline__ void quantize_rows16_body(const void *__restrict__ X, int R, int K, uint8_t *__restrict__ out,
                                                      float *__restrict__ scales, const QuantGroups &tab) {

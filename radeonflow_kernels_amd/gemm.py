@@ -154,7 +154,7 @@ def fp8_mm(a, b, a_scale, b_scale, c, config=None):
 
 def fp8_mm_static(a, b, a_scale, b_scale, c):
     """fp8_mm through rf_fp8_gemm_static: same result, no device memory is allocated or freed by the call (temporary
-    data lives in a static 32 MiB device array; shapes that need more raise)."""
+    data lives in a static 32 MiB device array; the plans of shapes that need more are fitted to it)."""
     _native.fp8_mm_static(a, b, a_scale, b_scale, c)
 
 
@@ -184,7 +184,8 @@ def fp8_mm_grouped(a, b, a_scale, b_scale, c, row_offsets, variant=-1):
 
 def grouped_variant_for(row_offsets, n, k, num_cu=256):
     """The tile form fp8_mm_grouped takes with variant=-1 for groups of these sizes on a device with num_cu compute
-    units (0..3: 256x256, 128x256, 128x128, 128x64 tiles; 4: 256-row tiles with a 128-row last tile; 5: the queue form).
+    units (0..3: 256x256, 128x256, 128x128, 128x64 tiles; 4: 256-row tiles with a 128-row last tile; 5: the queue form; 6..9:
+    the few-rows forms).
     Host arithmetic only."""
     groups = len(row_offsets) - 1
     offs = (ctypes.c_int32 * (groups + 1))(*[int(x) for x in row_offsets])
@@ -263,6 +264,8 @@ def quantize_b(w):
 
 
 def select_config(m, n, k):
+    """The plan of fp8_mm for aligned operands of this shape. variant -1: a small ragged shape, which takes the few-rows kernel
+    estimated fastest (not the bounds-checked kernel that a GemmConfig with variant -1 names)."""
     cfg = GemmConfig()
     rc = lib().rf_gemm_select_config(m, n, k, ctypes.byref(cfg))
     if rc != RF_OK:

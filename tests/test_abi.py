@@ -272,7 +272,7 @@ def test_few_rows_plans_that_cannot_run_are_skipped_at_lookup(tmp_path):
 
 def test_grouped_variant_choice_on_the_host():
     """rf_grouped_variant_for needs no device. The queue form (5) is taken where its last tiles of 64..256 rows save at
-    least 7 % of the rows the other 256-wide forms compute and it has 1.5 items per compute unit (2.5 below K = 4096);
+    least 7 % of the rows the other 256-wide forms compute and it has 17/16 items per compute unit (2.5 below K = 4096);
     groups the other forms fit as well, or too few items, keep those forms; tiny problems take the form with the most
     workgroups; bad arguments are refused."""
     import numpy as np
