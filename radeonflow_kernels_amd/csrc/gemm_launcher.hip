@@ -95,7 +95,7 @@ struct Variant {
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true>, nullptr, nullptr, 0, RF_ANY_C(BM, BN, WM, WN, 2) }
 // the same with three LDS stages: two K blocks in flight instead of one. A K block of these tiles is 0.4 us of MFMAs,
 // less than a load takes to come back from L2 or the Infinity Cache on a busy chip, so with two stages the loop ran at
-// the latency of its loads: 1024 x 4608 x 7168 45.6 -> 39.0 us, 256 x 7168 x 2304 15.6 -> 13.1 us; the best plan of 86
+// the latency of its loads: 1024 x 4608 x 7168 45.6 -> 39.0 us, 256 x 7168 x 2304 15.6 -> 13.1 us; the plan of 50
 // of the 163 tabled shapes. The two-stage forms stay: they fit more workgroups per CU (64 x 128: three instead of
 // two), which the smallest problems prefer. (128 x 128 with three stages never won and is not built.)
 #define RF_VARIANT_TILE_ONLY_NS3(BM, BN, WM, WN)                                           \
