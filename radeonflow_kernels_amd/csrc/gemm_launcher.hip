@@ -1623,7 +1623,21 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
         }
         return RF_OK;
     }
-    if (variant < 0) variant = choose_grouped_variant(row_offsets, groups, n, k, s.num_cu);
+    if (variant < 0) {
+        variant = choose_grouped_variant(row_offsets, groups, n, k, s.num_cu);
+        if (kGroupedVariants[variant].queue) {
+            // no counters to be had (a stream under capture that would have to take over another stream's set): the form
+            // without queues, whose results are the same to the bit
+            Mem mem{s};
+            mem.stream = stream;
+            CounterSet *counters = nullptr;
+            if (mem.counters(&counters) != RF_OK) {
+                (void)hipGetLastError();
+                g_last_error.clear();
+                variant = kGroupedMixed;
+            }
+        }
+    }
     const GroupedVariant &v = kGroupedVariants[variant];
     if (v.fewrows && !fewrows_ok((long)m_total + 16 * groups, n))
         return fail(RF_ERR_BAD_CONFIG, "the few-rows forms need fewer than 2^25 rows and columns");

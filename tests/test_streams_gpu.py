@@ -336,3 +336,66 @@ def test_workspace_bytes_covers_the_plan_that_runs(rfk, m, n, k):
     else:
         assert got in {bytes_of(v, split) for v in rfk.variants() if v["variant"] >= 14 for split in range(1, qk + 1)}
         assert (got > 0) == (k > 1024)                     # 56 K blocks in few tiles are split, two are not
+
+
+def test_automatic_grouped_calls_under_capture_without_a_buffer_set_take_a_form_without_queues(rfk):
+    """All 32 buffer sets belong to other streams: a grouped call whose automatic choice is the queue form is recorded on a 33rd
+    stream all the same (in the padded layout, which needs no staging), with the queue form's bits; the explicit queue form is
+    refused."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    L = rfk.lib()
+    L.rf_gemm_destroy()
+    rows = [16 * int(x) for x in np.random.default_rng(5).integers(1, 25, 16)]
+    offs = [0] + [int(x) for x in np.cumsum(rows)]
+    m, n, k = offs[-1], 4096, 4096
+    num_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    assert rfk.grouped_variant_for(offs, n, k, num_cu) == 5
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    fp8 = torch.float8_e4m3fn
+    a = torch.randint(0, 120, (k, m), dtype=torch.uint8, device="cuda", generator=gen).view(fp8).T
+    b = torch.randint(0, 120, (len(rows), k, n), dtype=torch.uint8, device="cuda", generator=gen).view(fp8).transpose(1, 2)
+    sa = (torch.rand((k // 128, m), device="cuda", generator=gen) * 1e-2).T
+    sb = (torch.rand((len(rows), k // 128, n // 128), device="cuda", generator=gen) * 1e-2).transpose(1, 2)
+    c = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+    rfk.fp8_mm_grouped_padded(a, b, sa, sb, c, offs, variant=5)
+    torch.cuda.synchronize()
+    exp = bf16_bits(c).copy()
+    L.rf_gemm_destroy()
+    split = to_gpu(exact_problem(16, 1536, 7168, 1))
+    handles = []
+    for _ in range(33):
+        h = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(h)) == 0
+        handles.append(h)
+    graph, graph_exec, cap = ctypes.c_void_p(), ctypes.c_void_p(), handles[32]
+    try:
+        for h in handles[:32]:
+            with torch.cuda.stream(torch.cuda.ExternalStream(h.value)):
+                rfk.fp8_mm(*split)
+            torch.cuda.synchronize()
+        c.fill_(-1.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(torch.cuda.ExternalStream(cap.value)):
+            assert hip.hipStreamBeginCapture(cap, 2) == 0                # hipStreamCaptureModeRelaxed
+            try:
+                rfk.fp8_mm_grouped_padded(a, b, sa, sb, c, offs)
+                with pytest.raises(RuntimeError, match="captured"):
+                    rfk.fp8_mm_grouped_padded(a, b, sa, sb, c, offs, variant=5)
+            finally:
+                assert hip.hipStreamEndCapture(cap, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, 0) == 0
+        for replay in range(3):
+            c.fill_(-1.0)
+            torch.cuda.synchronize()
+            assert hip.hipGraphLaunch(graph_exec, cap) == 0
+            torch.cuda.synchronize()
+            assert np.array_equal(bf16_bits(c), exp), replay
+            rfk.fp8_mm(*split)
+            torch.cuda.synchronize()
+        hip.hipGraphExecDestroy(graph_exec)
+        hip.hipGraphDestroy(graph)
+    finally:
+        torch.cuda.synchronize()
+        L.rf_gemm_destroy()
+        for h in handles:
+            hip.hipStreamDestroy(h)
