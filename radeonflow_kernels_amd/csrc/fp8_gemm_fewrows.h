@@ -56,8 +56,9 @@ __device__ __forceinline__ uint32_t fewrows_at(int k, int c) {
 
 // 16 bytes from base + off of a matrix that ends at base + end (end >= 16): past the end the bytes are undefined but
 // nothing is read there. SHIFT false: the caller knows that off + 16 <= end.
-template <bool SHIFT>
+template <bool SHIFT, bool STREAM = false>
 __device__ __forceinline__ u32x4_lds load16(const uint8_t *base, uint32_t off, uint32_t end) {
+    if constexpr (STREAM) return __builtin_nontemporal_load((const u32x4_any *)(base + off));
     if constexpr (!SHIFT) return *(const u32x4_any *)(base + off);
     const uint32_t at = off < end - 16 ? off : end - 16;
     return *(const u32x4_any *)(base + at);
@@ -76,7 +77,7 @@ __device__ __forceinline__ u32x4_lds shift_back(u32x4_lds v, uint32_t off, uint3
 }
 
 // What one wave does with one K block: loads into registers, the private LDS region, fragments, MFMAs.
-template <int TM, int TN, bool BYTES>
+template <int TM, int TN, bool BYTES, bool STREAM = false>
 struct FewRowsWave {
     static constexpr int BM = 16 * TM, BN = 16 * TN;
     static constexpr int NLA = 2 * TM, NLB = 2 * TN;                  // 16-byte loads per lane and K block
@@ -127,7 +128,7 @@ struct FewRowsWave {
         const uint8_t *pb = B + (size_t)kb * BK * N, *pa = A + (size_t)kb * BK * ldm;
         const uint32_t end_b = rest(kb, N, 0), end_a = rest(kb, ldm, first);
 #pragma unroll
-        for (int q = 0; q < NLB; q++) x.b[q] = load16<BYTES>(pb, off_b(q), end_b);
+        for (int q = 0; q < NLB; q++) x.b[q] = load16<BYTES, STREAM>(pb, off_b(q), end_b);
 #pragma unroll
         for (int q = 0; q < NLA; q++) x.a[q] = load16<true>(pa, off_a(q), end_a);
 #pragma unroll
@@ -334,18 +335,23 @@ __global__ __launch_bounds__(NW * 64, (FewRowsGeom<TM, TN, NW, DEPTH>::WAVES_PER
 //
 // First form: every wave has columns of its own and walks all of K with DEPTH K blocks on their way in registers; the waves
 // share nothing, so there is no barrier. Strips of 128 columns (TN = 8): a load instruction then covers eight whole cache
-// lines, and all strips of a launch are resident at once. Narrower strips ran at half the rate: 48 rows over 32 groups,
-// 2048 x 7168 (366 MB of weights), columns per wave 16: 228 us, 32: 139, 64: 100, 128: 72 us with two K blocks on their
-// way (5.1 TB/s, the rate of a large copy) against 96.7 us for the tiled form with its staging copy. Bound by the streaming of B; with fewer than
-// about one strip per compute unit by the chain of 56 loads (0.95 us each).
-template <int TM, int TN, int NW, int DEPTH, int WAVES_PER_SIMD>
+// lines (an L1 miss fetches a line whatever part of it is asked for), and all strips of a launch are resident at once. Narrower
+// strips ran at half the rate: 48 rows over 32 groups, 2048 x 7168 (366 MB of weights), columns per wave 16: 228 us, 32: 139,
+// 64: 100, 128: 72 us with two K blocks on their way against 96.7 us for the tiled form with its staging copy.
+// Bound by the streaming of B, whose rate depends on how much of a row is read at a time and on what the reads leave in the
+// Infinity Cache (a plain read of the same matrices: 128 columns by one workgroup 4.96 TB/s, 256 5.7, 512 6.4; neighbouring
+// strips dealt to different XCDs 5.4, 6.0, 6.6; with the non-temporal hint besides 5.9, 6.5). So items are dealt, the waves of
+// a workgroup hold neighbouring strips (four where there are enough of them: 36 groups of 7168 x 2048 89.5 -> 82.3 us, 30 of
+// 4096 x 2048 48 -> 45.3), and more weights than the Infinity Cache keeps are read with the hint (STREAM): the 366 MB
+// above 72.5 -> 67.0 us = 5.5 TB/s. With fewer than about one strip per compute unit bound by the chain of 56 loads (0.95 us each).
+template <int TM, int TN, int NW, int DEPTH, int WAVES_PER_SIMD, bool STREAM>
 __global__ __launch_bounds__(NW * 64, WAVES_PER_SIMD) void gemm_fp8_blockscale_grouped_strips(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
     const float *__restrict__ SB, uint16_t *__restrict__ C, int M_total, int N, int K, int groups, const GroupTable table) {
-    using W = FewRowsWave<TM, TN, false>;
+    using W = FewRowsWave<TM, TN, false, STREAM>;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     int grp, local;
-    if (!grouped_work_item(table, groups, grp, local)) return;
+    if (!grouped_work_item<true>(table, groups, grp, local)) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int out0 = table.out_row_start[grp], rows = table.out_row_start[grp + 1] - out0;
     const int row_blocks = (rows + 16 * TM - 1) / (16 * TM);

@@ -119,9 +119,10 @@ struct TileGeom {
 // Accumulates into acc the contribution of K blocks [kb_begin, kb_end) to the BM x BN tile at (m0, n0).
 // M is the number of rows of A (and of a_scale) that may be touched, ldm the distance in elements between two
 // K rows of A and of a_scale (ldm == M for a plain GEMM, ldm > M when A is a row range of a larger matrix).
+// STREAM_B: B's loads carry the non-temporal hint (see gemm_fp8_blockscale_grouped_queue).
 // All waves of the workgroup call it together. On return every LDS-DMA load has landed, but other waves may still
 // be reading LDS: a barrier is needed before LDS is written again.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int NS = 2>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NS = 2, bool STREAM_B = false>
 __device__ __forceinline__ void tile_mainloop(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
     const float *__restrict__ SB, int M, int ldm, int N, int m0, int n0, int kb_begin, int kb_end, uint8_t *lds,
@@ -256,9 +257,14 @@ __device__ __forceinline__ void tile_mainloop(
                          : "memory", "scc");
         } else if (d < D_SA) {
             const int e = d - INST_A < INST_B ? d - INST_A : 0;
-            asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         :: "v"(goff_b[cls_b(e >= 0 ? e : 0)]), "s"(src), "s"(lds_dst_b), "n"(e * 1024 + stage * STAGE_B)
-                         : "memory", "scc");
+            if constexpr (STREAM_B)
+                asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+                             :: "v"(goff_b[cls_b(e >= 0 ? e : 0)]), "s"(src), "s"(lds_dst_b), "n"(e * 1024 + stage * STAGE_B)
+                             : "memory", "scc");
+            else
+                asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                             :: "v"(goff_b[cls_b(e >= 0 ? e : 0)]), "s"(src), "s"(lds_dst_b), "n"(e * 1024 + stage * STAGE_B)
+                             : "memory", "scc");
         } else if (d == D_SA) {
             if (wave < NSC)
                 asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
@@ -992,12 +998,13 @@ struct GroupTable {
     int tile_start[kMaxGroups + 1];     // prefix of work items (one per tile); tile_start[groups] is their number
 };
 // Work item of this workgroup: its group and its index among the group's items. False: nothing to do (the grid is
-// 8 x the longest piece).
+// 8 x the longest piece). DEALT: items dealt to the XCDs one by one instead of in pieces.
+template <bool DEALT = false>
 __device__ __forceinline__ bool grouped_work_item(const GroupTable &table, int groups, int &grp, int &local) {
     const int xcd = blockIdx.x % NUM_XCD;
     const long items = table.tile_start[groups];
-    const int item = (int)(items * xcd / NUM_XCD) + (int)(blockIdx.x / NUM_XCD);
-    if (item >= (int)(items * (xcd + 1) / NUM_XCD)) return false;
+    const int item = DEALT ? (int)blockIdx.x : (int)(items * xcd / NUM_XCD) + (int)(blockIdx.x / NUM_XCD);
+    if (item >= (DEALT ? (int)items : (int)(items * (xcd + 1) / NUM_XCD))) return false;
     // the last g with tile_start[g] <= item (empty groups own no item)
     int lo = 0, hi = groups;
     while (hi - lo > 1) {
@@ -1078,6 +1085,11 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_grouped_mixed(
 // exactly once per queue, so the counter's last draw wraps it back to zero: the counters need no clearing between
 // launches (launches that share counters must not overlap).
 // In the table of this kernel tile_start[p] counts the items of the first p groups of the line.
+// stream: the launch's weights are more than the Infinity Cache keeps (the host's kStreamBytes). Those of a group with one
+// row tile are then read once and by one workgroup, and their loads say so (nt): without the hint each of them evicts
+// something from the Infinity Cache. 2000 rows in 32 groups, 4096 x 7168: 229 -> 215 us, 4000 in 64, 2048 x 7168: 240 -> 225,
+// 8192 in 32: 358 -> 355. (The hint on every item: 351 there, but 8000 rows in 32 groups at 7168 x 2048 182 -> 190, where two
+// row tiles meet in an L2.)
 // ---------------------------------------------------------------------------------------------
 struct GroupQueues {
     int piece_start[NUM_XCD + 1];        // queue x holds items piece_start[x] .. piece_start[x + 1] - 1 of the line
@@ -1090,20 +1102,20 @@ constexpr int kQueueTileLds =
 static_assert(TileGeom<192, 256, 2, 4>::LDS_BYTES <= kQueueTileLds && TileGeom<64, 256, 2, 4, 3>::LDS_BYTES <= kQueueTileLds,
               "the 256- and 128-row tiles are the largest");
 constexpr int kQueueLds = kQueueTileLds + 16;                    // + the slot through which a draw reaches all waves
-template <int BM, int NS>
+template <int BM, int NS, bool STREAM>
 __device__ __forceinline__ void grouped_queue_tile(const uint8_t *A, const uint8_t *B, const float *SA, const float *SB,
                                                    uint16_t *C, int rows, int out_rows, int M_total, int N, int n0, int QK,
                                                    uint8_t *lds) {
     f32x4 acc[TileGeom<BM, 256, 2, 4>::TM][TileGeom<BM, 256, 2, 4>::TN];
     int vz;
     asm volatile("v_mov_b32 %0, 0" : "=v"(vz));
-    tile_mainloop<BM, 256, 2, 4, NS>(A, B, SA, SB, rows, M_total, N, 0, n0, 0, QK, lds, acc, vz);
+    tile_mainloop<BM, 256, 2, 4, NS, STREAM>(A, B, SA, SB, rows, M_total, N, 0, n0, 0, QK, lds, acc, vz);
     store_tile_bf16<BM, 256, 2, 4>(acc, C, out_rows, N, 0, n0, lds);
 }
 __global__ __launch_bounds__(512) void gemm_fp8_blockscale_grouped_queue(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
     const float *__restrict__ SB, uint16_t *__restrict__ C, int M_total, int N, int K, int groups,
-    const GroupTable table, const GroupQueues queues, unsigned *__restrict__ counters) {
+    const GroupTable table, const GroupQueues queues, int stream, unsigned *__restrict__ counters) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     volatile int *drawn = (volatile int *)(lds + kQueueTileLds);
     const int QK = K / BK, QN = (N + 127) / 128;
@@ -1135,10 +1147,16 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_grouped_queue(
             const float *SAi = SA + row0 + m0, *SBg = SB + (size_t)grp * QK * QN;
             uint16_t *Ci = C + (size_t)(out0 + m0) * N;
             const int r = rows - m0, o = out_rows - m0;
-            if (height == 4) grouped_queue_tile<256, 2>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
-            else if (height == 3) grouped_queue_tile<192, 2>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
-            else if (height == 2) grouped_queue_tile<128, 3>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
-            else grouped_queue_tile<64, 3>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            // weights that only this item reads and that the Infinity Cache does not keep anyway
+            const int form = height + (stream && tiles_m == 1 ? 4 : 0);
+            if (form == 4) grouped_queue_tile<256, 2, false>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            else if (form == 3) grouped_queue_tile<192, 2, false>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            else if (form == 2) grouped_queue_tile<128, 3, false>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            else if (form == 1) grouped_queue_tile<64, 3, false>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            else if (form == 8) grouped_queue_tile<256, 2, true>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            else if (form == 7) grouped_queue_tile<192, 2, true>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            else if (form == 6) grouped_queue_tile<128, 3, true>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
+            else grouped_queue_tile<64, 3, true>(Ai, Bg, SAi, SBg, Ci, r, o, M_total, N, n0, QK, lds);
         }
     }
 }

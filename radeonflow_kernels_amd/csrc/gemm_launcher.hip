@@ -1432,6 +1432,7 @@ struct GroupedVariant {
                          // rows; the queue form: 64, 128, 192 or 256 rows)
     bool queue = false;  // resident workgroups that take tiles from per-XCD queues (gemm_fp8_blockscale_grouped_queue)
     bool fewrows = false;  // fp8_gemm_fewrows.h: groups may start at any row of a
+    grouped_kernel_t streamed = nullptr;   // few-rows strips: the kernel for more weights than kStreamBytes
     // row tiles of a group of `rows` rows
     int tiles_m(int rows) const {
         if (!mixed) return ceil_div(rows, bm);
@@ -1441,20 +1442,27 @@ struct GroupedVariant {
 
 #define RF_GROUPED(BM, BN, WM, WN, NS) \
     GroupedVariant { BM, BN, WM *WN * 64, rf::TileGeom<BM, BN, WM, WN, NS>::LDS_BYTES, rf::gemm_fp8_blockscale_grouped<BM, BN, WM, WN, NS>, false }
-#define RF_GROUPED_FEWROWS(KERNEL, TM, COLUMNS, TN, NW, DEPTH, WAVES_PER_SIMD)                    \
-    GroupedVariant { 16 * TM, COLUMNS, 64 * NW, NW *rf::BK * 16 * (TM + TN),                       \
-                     rf::KERNEL<TM, TN, NW, DEPTH, WAVES_PER_SIMD>, false, false, true }
+#define RF_GROUPED_STRIPS(TM, NW, DEPTH, WAVES_PER_SIMD)                                            \
+    GroupedVariant { 16 * TM, 128 * NW, 64 * NW, NW *rf::BK * 16 * (TM + 8),                        \
+                     rf::gemm_fp8_blockscale_grouped_strips<TM, 8, NW, DEPTH, WAVES_PER_SIMD, false>, false, false, true, \
+                     rf::gemm_fp8_blockscale_grouped_strips<TM, 8, NW, DEPTH, WAVES_PER_SIMD, true> }
 constexpr int kMixedLds = rf::TileGeom<256, 256, 2, 4>::LDS_BYTES > rf::TileGeom<128, 256, 2, 4, 3>::LDS_BYTES
                               ? rf::TileGeom<256, 256, 2, 4>::LDS_BYTES : rf::TileGeom<128, 256, 2, 4, 3>::LDS_BYTES;
 const GroupedVariant kGroupedVariants[] = {
     RF_GROUPED(256, 256, 2, 4, 2), RF_GROUPED(128, 256, 2, 4, 3), RF_GROUPED(128, 128, 2, 2, 2), RF_GROUPED(128, 64, 2, 1, 2),
     GroupedVariant{256, 256, 512, kMixedLds, rf::gemm_fp8_blockscale_grouped_mixed, true},
     GroupedVariant{256, 256, 512, rf::kQueueLds, nullptr, true, true},
-    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_strips, 1, 256, 8, 2, 2, 1),    // 6: 16 rows, two waves of 128 columns
-    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_strips, 1, 128, 8, 1, 1, 2),    // 7: 16 rows, one wave
-    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_strips, 2, 128, 8, 1, 1, 1),    // 8: 32 rows, one wave
-    RF_GROUPED_FEWROWS(gemm_fp8_blockscale_grouped_ksplit, 1, 64, 4, 8, 1, 4)};    // 9: 16 rows, K split between eight waves
+    RF_GROUPED_STRIPS(1, 2, 2, 1),    // 6: 16 rows, two waves of 128 columns
+    RF_GROUPED_STRIPS(1, 1, 1, 2),    // 7: 16 rows, one wave
+    RF_GROUPED_STRIPS(2, 1, 1, 1),    // 8: 32 rows, one wave
+    GroupedVariant{16, 64, 512, 8 * rf::BK * 16 * 5, rf::gemm_fp8_blockscale_grouped_ksplit<1, 4, 8, 1, 4>, false, false, true},   // 9: 16 rows, K split between eight waves
+    RF_GROUPED_STRIPS(1, 4, 1, 2)};   // 10: 16 rows, four waves
 constexpr int kGroupedMixed = 4, kGroupedQueue = 5, kGroupedFewRows = 6;
+// Weights (of the groups that have rows) from which on they are read with the non-temporal hint: three quarters of the
+// Infinity Cache's 256 MB, which then cannot hold them from one call to the next beside everything else, and which the
+// hint keeps for other data. us, strips: 25 groups of 2048 x 7168 (367 MB) 72.5 -> 67.2, 16 of 4096 x 7168 (470 MB) 85.4 ->
+// 76.2, 30 of 4096 x 2048 (252 MB) 48.3 -> 44.1; but 8 of 4096 x 2048 (67 MB), which stay in the cache, 15.9 -> 18.2.
+constexpr double kStreamBytes = 192.0 * (1 << 20);
 // Estimated time of a 256-column tile of the queue form by its height in units of 64 rows, relative to a 256-row tile
 constexpr double kQueueTileCost[5] = {0.0, 0.68, 0.75, 0.97, 1.0};
 constexpr int kNumGroupedVariants = sizeof(kGroupedVariants) / sizeof(kGroupedVariants[0]);
@@ -1467,7 +1475,7 @@ long grouped_tiles(const GroupedVariant &v, const int *row_offsets, int groups, 
 }  // namespace
 
 namespace {
-// The few-rows form for these groups, or -1: groups of at most 16 rows (variants 6, 7 and 9) or 32 (variant 8); more rows
+// The few-rows form for these groups, or -1: groups of at most 16 rows (variants 6, 7, 9 and 10) or 32 (variant 8); more rows
 // would stream the weights once per row block. Estimated time in us: the stream of the weights at the rate the form reaches
 // once the chip is full, or the chain of one wave's K blocks. Measured on 52 layouts (8 to 64 groups, 16 to 900 rows,
 // N x K = 2048 x 7168, 4096 x 7168, 7168 x 2048, 4096 x 2048) against the tiled forms with their staging copy: up to 50 %
@@ -1485,13 +1493,16 @@ int choose_grouped_fewrows(const int *row_offsets, int groups, int n, int k, int
     if (most < 1 || most > 32 || n % 16 != 0 || bytes > 1.0e9 || !fewrows_ok((long)row_offsets[groups] + 16 * groups, n)) return -1;
     struct Form { int variant, wgs_per_cu; double max_rounds, start, per_k_block, bytes_per_us; };
     const Form forms[] = {{6, 2, 3.0, 4.0, 1.0, 5.1e6}, {7, 8, 1.0, 3.5, 0.93, 4.6e6}, {8, 4, 2.0, 3.0, 1.2, 5.0e6},
-                          {9, 2, 1.0, 3.0, 0.0, 3.3e6}};
+                          {9, 2, 1.0, 3.0, 0.0, 3.3e6}, {10, 2, 2.0, 4.0, 1.6, 5.4e6}};
     int best = -1;
     double best_t = 0;
     for (const Form &f : forms) {
         const GroupedVariant &v = kGroupedVariants[f.variant];
         const double rounds = (double)busy * ceil_div(n, v.bn) / (f.wgs_per_cu * num_cu);
         if (most > v.bm || rounds > f.max_rounds) continue;
+        // strips of 512 columns: only where there is nearly one for every compute unit (8 % faster than 256 columns then; with
+        // 128 of them for 256 units a third slower)
+        if (f.variant == 10 && (long)busy * ceil_div(n, v.bn) * 8 < 7L * num_cu) continue;
         const double t = std::max(f.start + f.per_k_block * (k / rf::BK), 3.0 + bytes / f.bytes_per_us * 256.0 / num_cu);
         if (best < 0 || t < best_t) { best = f.variant; best_t = t; }
     }
@@ -1594,8 +1605,8 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
     if (rc != RF_OK) return rc;
     if (!s.grouped_attrs_set) {
         for (const GroupedVariant &v : kGroupedVariants)
-            if (v.kernel)
-                RF_HIP(hipFuncSetAttribute((const void *)v.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds));
+            for (grouped_kernel_t f : {v.kernel, v.streamed})
+                if (f) RF_HIP(hipFuncSetAttribute((const void *)f, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds));
         RF_HIP(hipFuncSetAttribute((const void *)rf::gemm_fp8_blockscale_grouped_queue,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, rf::kQueueLds));
         s.grouped_attrs_set = true;
@@ -1681,11 +1692,13 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
             table.row_start[g] = table.out_row_start[g] = row_offsets[g < groups ? g : groups];
     }
     const int tiles_n = ceil_div(n, v.bn);
-    int tiles = 0;
+    int tiles = 0, busy = 0;
     for (int g = 0; g < groups; g++) {
         table.tile_start[g] = tiles;
         tiles += v.tiles_m(row_offsets[g + 1] - row_offsets[g]) * tiles_n;
+        busy += row_offsets[g + 1] > row_offsets[g];
     }
+    const bool stream_b = (double)busy * n * k > kStreamBytes;
     for (int g = groups; g <= rf::kMaxGroups; g++) table.tile_start[g] = tiles;
     if (v.queue) {
         // The line of items and its eight pieces. Estimated time of a group = column tiles x (256-row tiles + what
@@ -1754,12 +1767,13 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
         if (rc != RF_OK) return rc;
         hipLaunchKernelGGL(rf::gemm_fp8_blockscale_grouped_queue, dim3(queues.workgroups), dim3(v.threads), v.lds, stream,
                            (const uint8_t *)a, (const uint8_t *)b, as, bs, (uint16_t *)c, m_rows, n, k, groups, table,
-                           queues, counters->queue);
+                           queues, stream_b, counters->queue);
         RF_HIP(hipGetLastError());
         return RF_OK;
     }
+    const grouped_kernel_t kernel = stream_b && v.streamed ? v.streamed : v.kernel;
     const int longest = ceil_div(tiles, rf::NUM_XCD);          // every XCD takes an eighth of the tiles, rounded
-    hipLaunchKernelGGL(v.kernel, dim3(longest * rf::NUM_XCD), dim3(v.threads), v.lds, stream, (const uint8_t *)a,
+    hipLaunchKernelGGL(kernel, dim3(longest * rf::NUM_XCD), dim3(v.threads), v.lds, stream, (const uint8_t *)a,
                        (const uint8_t *)b, as, bs, (uint16_t *)c, m_rows, n, k, groups, table);
     RF_HIP(hipGetLastError());
     return RF_OK;

@@ -184,7 +184,7 @@ def fp8_mm_grouped(a, b, a_scale, b_scale, c, row_offsets, variant=-1):
 
 def grouped_variant_for(row_offsets, n, k, num_cu=256):
     """The tile form fp8_mm_grouped takes with variant=-1 for groups of these sizes on a device with num_cu compute
-    units (0..3: 256x256, 128x256, 128x128, 128x64 tiles; 4: 256-row tiles with a 128-row last tile; 5: the queue form; 6..9:
+    units (0..3: 256x256, 128x256, 128x128, 128x64 tiles; 4: 256-row tiles with a 128-row last tile; 5: the queue form; 6..10:
     the few-rows forms).
     Host arithmetic only."""
     groups = len(row_offsets) - 1

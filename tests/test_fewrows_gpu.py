@@ -125,6 +125,33 @@ def test_grouped_fewrows_bits_of_the_tiled_form(rfk, rows, n, k, shift):
         assert np.array_equal(launch(rfk.fp8_mm_grouped_padded, a_pad.view(fp8).T, sa_pad.T, variant), expect), variant
 
 
+# more weights than the Infinity Cache keeps (read with the non-temporal hint): groups of at most 16 rows for the strips, of up
+# to 300 for the queue's tiles of four heights and of one and two row tiles; a partial last strip of any width, an odd number of
+# K blocks; without the last eighteen groups, the same forms without the hint
+@pytest.mark.parametrize("variants,rows", [((6, 7, 8, 10, -1), [1, 0, 16, 7, 3]), ((5,), [64, 0, 300, 65, 130, 200, 256, 1, 257, 20])])
+@pytest.mark.parametrize("groups", [30, 12])
+def test_grouped_streamed_weights_bits_of_the_tiled_form(rfk, variants, rows, groups):
+    n, k, fp8 = 2064, 3968, torch.float8_e4m3fn
+    rows = (rows * groups)[:groups]
+    offs = [0] + [int(x) for x in np.cumsum(rows)]
+    m = offs[-1]
+    gen = torch.Generator(device="cuda").manual_seed(groups + m)
+    a = torch.randint(0, 120, (k, m), dtype=torch.uint8, device="cuda", generator=gen).view(fp8).T
+    b = torch.randint(0, 120, (groups, k, n), dtype=torch.uint8, device="cuda", generator=gen).view(fp8).permute(0, 2, 1)
+    sa = (torch.rand((k // 128, m), device="cuda", generator=gen) * 1e-2).T
+    sb = (torch.rand((groups, k // 128, (n + 127) // 128), device="cuda", generator=gen) * 1e-2).permute(0, 2, 1)
+
+    def launch(variant):
+        buf = torch.full((m * n + 300,), -7.0, dtype=torch.bfloat16, device="cuda")
+        rfk.fp8_mm_grouped(a, b, sa, sb, buf[:m * n].view(m, n), offs, variant=variant)
+        torch.cuda.synchronize()
+        return bf16_bits(buf)
+
+    expect = launch(1)
+    for variant in variants:
+        assert np.array_equal(launch(variant), expect), variant
+
+
 def test_fewrows_k_splits_on_two_streams_at_once(rfk):
     """Different numbers of K parts on two streams, launches queued deep: every stream has counters and slots of its own, so each
     result is the one the same plan gives alone."""
