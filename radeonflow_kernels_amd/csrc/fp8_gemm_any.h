@@ -1,0 +1,297 @@
+// Tile kernels for operands at any alignment: rows of A of M bytes and rows of B of N bytes, whatever M and N are.
+#pragma once
+#include "fp8_gemm_fewrows.h"
+
+namespace rf {
+
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_>
+struct AnyGeom {
+    static constexpr int BM = BM_, BN = BN_, NW = WAVES_M_ * WAVES_N_, NT = NW * 64;
+    static constexpr int CPR_A = BM / 16, CPR_B = BN / 16;
+    static constexpr int IA = BK * CPR_A / NT, IB = BK * CPR_B / NT;      // 16-byte loads per thread and K block
+    static constexpr int LDS_BYTES = TileGeom<BM_, BN_, WAVES_M_, WAVES_N_, 2>::LDS_BYTES;
+    static_assert(BK * CPR_A % NT == 0 && BK * CPR_B % NT == 0, "whole loads per thread");
+};
+
+// tile_mainloop with the operands through registers.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int SETS>
+__device__ __forceinline__ void tile_mainloop_any(
+    const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
+    const float *__restrict__ SB, int M, int ldm, int N, int QK, int m0, int n0, int kb_begin, int kb_end, uint8_t *lds,
+    f32x4 (&acc)[BM / WAVES_M / 16][BN / WAVES_N / 16]) {
+    using G = TileGeom<BM, BN, WAVES_M, WAVES_N, 2>;
+    using Y = AnyGeom<BM, BN, WAVES_M, WAVES_N>;
+    constexpr int WM = G::WM, WN = G::WN, TM = G::TM, TN = G::TN, NT = G::NT, IA = Y::IA, IB = Y::IB;
+    constexpr int STAGE_A = G::STAGE_A, STAGE_B = G::STAGE_B, STAGE_S = G::STAGE_S;
+    constexpr int OFF_B = 2 * STAGE_A, OFF_S = 2 * (STAGE_A + STAGE_B), OFF_SB = BM * 4;
+    constexpr bool ONE_SB = WN <= 128 && 128 % WN == 0;
+    static_assert(ONE_SB || (TN == 3 && WN < 128), "straddling waves: three n-tiles, split before n-tile 1 or 2");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int L = lane & 15, g = lane >> 4, wm = wave % WAVES_M, wn = wave / WAVES_M;
+    const int QN = (N + 127) / 128;
+
+    // ---- loads: per-thread offsets inside one K block, destinations inside a stage ----
+    uint32_t off_a[IA], off_b[IB], dst_a[IA], dst_b[IB];
+#pragma unroll
+    for (int i = 0; i < IA; i++) {
+        const int q = i * NT + tid, row = q / Y::CPR_A, c = q % Y::CPR_A;
+        int m = m0 + 16 * c;
+        if (m >= M) m = m0;
+        off_a[i] = (uint32_t)row * (uint32_t)ldm + (uint32_t)m;
+        dst_a[i] = row * BM + ((c ^ swizzle_of_row<BM>(row)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < IB; i++) {
+        const int q = i * NT + tid, row = q / Y::CPR_B, c = q % Y::CPR_B;
+        int n = n0 + 16 * c;
+        if (n >= N) n = n0;
+        off_b[i] = (uint32_t)row * (uint32_t)N + (uint32_t)n;
+        dst_b[i] = OFF_B + row * BN + ((c ^ swizzle_of_row<BN>(row)) << 4);
+    }
+    // scales: threads 0 .. BM - 1 the rows of the tile, the next four its column blocks, the others repeat the last one
+    static_assert(NT >= BM + 4, "a thread per scale");
+    const float *src_s;
+    uint32_t dst_s, step_s;
+    if (tid < BM) {
+        const int r = tid % WM;
+        int m = m0 + (tid / WM) * WM + 16 * (r % TM) + r / TM;
+        if (m > M - 1) m = M - 1;
+        src_s = SA + m;
+        step_s = (uint32_t)ldm;
+        dst_s = OFF_S + tid * 4;
+    } else {
+        const int l = tid - BM < 3 ? tid - BM : 3;
+        int nbq = (n0 >> 7) + l;
+        if (nbq > QN - 1) nbq = QN - 1;
+        src_s = SB + nbq;
+        step_s = (uint32_t)QN;
+        dst_s = OFF_S + OFF_SB + l * 4;
+    }
+    // bytes from a K block's first row to the end of the matrix (below 2^32 always suffices)
+    auto rest = [&](int kb, int ld) {
+        const unsigned long long r = (unsigned long long)(QK - kb) * BK * (unsigned)ld;
+        return r < 0xffffffffull ? (uint32_t)r : 0xffffffffu;
+    };
+    u32x4_lds ra[SETS][IA], rb[SETS][IB];
+    float rs[SETS];
+    const int kb_last = kb_end - 1;
+    auto clamp_kb = [&](int kb) { return kb < kb_last ? kb : kb_last; };
+    auto load_item = [&](auto set_c, int d, int kb) {
+        constexpr int set = decltype(set_c)::value;
+        kb = clamp_kb(kb);
+        if (d < IA) ra[set][d] = load16<true>(A + (size_t)kb * BK * ldm, off_a[d < IA ? d : 0], rest(kb, ldm));
+        else if (d < IA + IB) rb[set][d - IA < IB ? d - IA : 0] = load16<true>(B + (size_t)kb * BK * N, off_b[d - IA < IB && d >= IA ? d - IA : 0], rest(kb, N));
+        else rs[set] = src_s[(size_t)kb * step_s];
+    };
+    auto write_item = [&](auto set_c, int d, int stage, int kb) {
+        constexpr int set = decltype(set_c)::value;
+        if (d < IA) {
+            u32x4_lds v = ra[set][d < IA ? d : 0];
+            if (kb == QK - 1) v = shift_back(v, off_a[d < IA ? d : 0], rest(kb, ldm));
+            *(u32x4_lds *)(lds + stage * STAGE_A + dst_a[d < IA ? d : 0]) = v;
+        } else if (d < IA + IB) {
+            const int e = d - IA < IB && d >= IA ? d - IA : 0;
+            u32x4_lds v = rb[set][e];
+            if (kb == QK - 1) v = shift_back(v, off_b[e], rest(kb, N));
+            *(u32x4_lds *)(lds + stage * STAGE_B + dst_b[e]) = v;
+        } else {
+            *(float *)(lds + stage * STAGE_S + dst_s) = rs[set];
+        }
+    };
+    constexpr int NL = IA + IB + 1;
+
+    // ---- LDS -> MFMA operands (see tile_mainloop) ----
+    const int krow = 32 * g + (L >> 1);
+    constexpr bool POW2_T = (TM & (TM - 1)) == 0 && (TN & (TN - 1)) == 0;
+    const uint32_t aoff_base = krow * BM + (((wm * TM) ^ swizzle_of_row<BM>(krow)) << 4) + 8 * (L & 1);
+    const uint32_t boff_base = OFF_B + krow * BN + (((wn * TN) ^ swizzle_of_row<BN>(krow)) << 4) + 8 * (L & 1);
+    uint32_t aoff_tile[POW2_T ? 1 : TM], boff_tile[POW2_T ? 1 : TN];
+    if constexpr (!POW2_T) {
+#pragma unroll
+        for (int j = 0; j < TM; j++) aoff_tile[j] = krow * BM + (((wm * TM + j) ^ swizzle_of_row<BM>(krow)) << 4) + 8 * (L & 1);
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+            boff_tile[i] = OFF_B + krow * BN + (((wn * TN + i) ^ swizzle_of_row<BN>(krow)) << 4) + 8 * (L & 1);
+    }
+    const uint32_t soff = OFF_S + (wm * WM + L * TM) * 4;
+    const int ncol0 = n0 + wn * WN;
+    const int sb_split_raw = (((ncol0 >> 7) + 1) * 128 - ncol0) >> 4;
+    const int sb_split = __builtin_amdgcn_readfirstlane(sb_split_raw < TN ? sb_split_raw : TN);
+    const uint32_t sboff = OFF_S + OFF_SB + (((ncol0 >> 7) - (n0 >> 7)) << 2);
+    const uint32_t sboff1 = sboff + (sb_split < TN ? 4 : 0);
+    constexpr int NMFMA = TM * TN, PR = (NMFMA % 4 == 0 && TN > 3) ? 4 : 3, LAG = PR - 1, BAR_SLOT = (TM - 1) * TN;
+    static_assert(NMFMA % PR == 0 && LAG < TN && LAG < PR && TM % 2 == 0, "same schedule as tile_mainloop");
+    constexpr int PER_SLOT = (NL + BAR_SLOT - 2) / (BAR_SLOT - 1);       // writes (and loads) per slot, done a slot before the barrier
+#pragma unroll
+    for (int j = 0; j < TM; j++)
+#pragma unroll
+        for (int i = 0; i < TN; i++) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    i32x8 bfrag[TN], afrag[2];
+    f32x4 pring[PR];
+    float s[TM], s1[ONE_SB ? 1 : TM], sraw[TM], sb_raw = 0.f, sb_raw1 = 0.f;
+#pragma unroll
+    for (int r = 0; r < PR; r++) pring[r] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < TM; j++) s[j] = 0.f;
+#pragma unroll
+    for (int j = 0; j < (ONE_SB ? 1 : TM); j++) s1[j] = 0.f;
+    auto rd = [&](uint32_t stage_base, uint32_t off) {
+        return __builtin_amdgcn_ds_read_tr8_b64_v2i32((RF_LDS i32x2 *)(lds + stage_base + off));
+    };
+    auto read_bfrag = [&](int i, int stage) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            i32x2 v = rd(stage * STAGE_B, (POW2_T ? boff_base ^ (i << 4) : boff_tile[POW2_T ? 0 : i]) + t * 8 * BN);
+            bfrag[i][2 * t] = v[0];
+            bfrag[i][2 * t + 1] = v[1];
+        }
+    };
+    auto read_afrag = [&](int buf, int j, int stage) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            i32x2 v = rd(stage * STAGE_A, (POW2_T ? aoff_base ^ (j << 4) : aoff_tile[POW2_T ? 0 : j]) + t * 8 * BM);
+            afrag[buf][2 * t] = v[0];
+            afrag[buf][2 * t + 1] = v[1];
+        }
+    };
+    auto read_scales = [&](int stage) {
+#pragma unroll
+        for (int q = 0; q < TM / 2; q++) {
+            f32x2 v = *(RF_LDS f32x2 *)(lds + stage * STAGE_S + soff + q * 8);
+            sraw[2 * q] = v[0];
+            sraw[2 * q + 1] = v[1];
+        }
+        sb_raw = *(RF_LDS float *)(lds + stage * STAGE_S + sboff);
+        if constexpr (!ONE_SB) sb_raw1 = *(RF_LDS float *)(lds + stage * STAGE_S + sboff1);
+    };
+    // prologue
+    auto each_set = [&](auto f) {
+        f(IntTag<0>{});
+        f(IntTag<1>{});
+        if constexpr (SETS > 2) f(IntTag<2>{});
+    };
+    each_set([&](auto set_c) {
+#pragma unroll
+        for (int d = 0; d < NL; d++) load_item(set_c, d, kb_begin + decltype(set_c)::value);
+    });
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < NL; d++) write_item(IntTag<0>{}, d, 0, kb_begin);
+#pragma unroll
+    for (int d = 0; d < NL; d++) load_item(IntTag<0>{}, d, kb_begin + SETS);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    read_bfrag(0, 0);
+    read_afrag(0, 0, 0);
+    read_scales(0);
+#pragma unroll
+    for (int i = 1; i < TN; i++) read_bfrag(i, 0);
+    // One K block: the stage it reads (cur), the register set of the next one (set). In its first slots block kb + 1 goes from
+    // its registers into the other stage, and block kb + 1 + SETS is asked for in its place.
+    auto k_block = [&](auto cur_c, auto set_c, auto split_c, int kb) {
+        constexpr int cur = decltype(cur_c)::value, nxt = 1 - cur;
+        constexpr int split = decltype(split_c)::value;
+        const float s_last = s[TM - 1], s1_last = s1[ONE_SB ? 0 : TM - 1];
+        const int kb_next = clamp_kb(kb + 1);
+#pragma unroll
+        for (int j = 0; j < TM; j++) s[j] = sraw[j] * sb_raw;
+        if constexpr (!ONE_SB)
+#pragma unroll
+            for (int j = 0; j < TM; j++) s1[j] = sraw[j] * sb_raw1;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < NMFMA; t++) {
+            const int j = t / TN, i = t % TN;
+            if (t == BAR_SLOT) {
+                __syncthreads();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            pring[t % PR] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                bfrag[i], afrag[j & 1], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+            asm volatile("" : "+v"(pring[t % PR]));
+            __builtin_amdgcn_sched_barrier(0);
+            if (j + 1 < TM) {
+                if (i == 0) read_afrag((j + 1) & 1, j + 1, cur);
+            } else {
+                read_bfrag(i, nxt);
+                if (i == 0) {
+                    read_afrag(0, 0, nxt);
+                    read_scales(nxt);
+                }
+            }
+#pragma unroll
+            for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) write_item(set_c, d, nxt, kb_next);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) load_item(set_c, d, kb + 1 + SETS);
+            if (t >= LAG) {
+                const int u = t - LAG, ju = u / TN, iu = u % TN;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    acc[ju][iu][e] = __builtin_fmaf(iu < split ? s[ju] : s1[ONE_SB ? 0 : ju], pring[u % PR][e], acc[ju][iu][e]);
+                asm volatile("" : "+v"(acc[ju][iu]));
+            } else {
+                const int u = NMFMA + t - LAG, ju = u / TN, iu = u % TN;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    acc[ju][iu][e] = __builtin_fmaf(iu < split ? s_last : s1_last, pring[u % PR][e], acc[ju][iu][e]);
+                asm volatile("" : "+v"(acc[ju][iu]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto k_loop = [&](auto split_c) {
+        constexpr int split = decltype(split_c)::value;
+        int kb = kb_begin;
+        if constexpr (SETS == 2) {
+            for (; kb + 1 < kb_end; kb += 2) {
+                k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
+                k_block(IntTag<1>{}, IntTag<0>{}, split_c, kb + 1);
+            }
+            if (kb < kb_end) k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
+        } else {
+            for (; kb + 5 < kb_end; kb += 6) {
+                k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
+                k_block(IntTag<1>{}, IntTag<2>{}, split_c, kb + 1);
+                k_block(IntTag<0>{}, IntTag<0>{}, split_c, kb + 2);
+                k_block(IntTag<1>{}, IntTag<1>{}, split_c, kb + 3);
+                k_block(IntTag<0>{}, IntTag<2>{}, split_c, kb + 4);
+                k_block(IntTag<1>{}, IntTag<0>{}, split_c, kb + 5);
+            }
+            if (kb < kb_end) k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
+            if (kb + 1 < kb_end) k_block(IntTag<1>{}, IntTag<2>{}, split_c, kb + 1);
+            if (kb + 2 < kb_end) k_block(IntTag<0>{}, IntTag<0>{}, split_c, kb + 2);
+            if (kb + 3 < kb_end) k_block(IntTag<1>{}, IntTag<1>{}, split_c, kb + 3);
+            if (kb + 4 < kb_end) k_block(IntTag<0>{}, IntTag<2>{}, split_c, kb + 4);
+        }
+#pragma unroll
+        for (int t = 0; t < LAG; t++) {
+            const int u = NMFMA + t - LAG, ju = u / TN, iu = u % TN;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                acc[ju][iu][e] = __builtin_fmaf(iu < split ? s[TM - 1] : s1[ONE_SB ? 0 : TM - 1], pring[u % PR][e], acc[ju][iu][e]);
+        }
+    };
+    if constexpr (ONE_SB) {
+        k_loop(IntTag<TN>{});
+    } else {
+        if (sb_split == 1) k_loop(IntTag<1>{});
+        else k_loop(IntTag<2>{});
+    }
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int SETS>
+__global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_tile_any(
+    const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
+    const float *__restrict__ SB, uint16_t *__restrict__ C, int M, int ldm, int N, int K, int tiles_m, int tiles_n, int group_m) {
+    using G = TileGeom<BM, BN, WAVES_M, WAVES_N, 2>;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    int tile_m, tile_n;
+    tile_of_block(blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, group_m, true, tile_m, tile_n);
+    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    f32x4 acc[G::TM][G::TN];
+    tile_mainloop_any<BM, BN, WAVES_M, WAVES_N, SETS>(A, B, SA, SB, M, ldm, N, K / BK, m0, n0, 0, K / BK, lds, acc);
+    store_tile_bf16<BM, BN, WAVES_M, WAVES_N, default_store_passes<BM, WAVES_M>(), true, true>(acc, C, M, N, m0, n0, lds);
+}
+
+}  // namespace rf

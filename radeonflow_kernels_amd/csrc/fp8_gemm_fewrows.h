@@ -231,42 +231,71 @@ __global__ __launch_bounds__(NW * 64, (FewRowsGeom<TM, TN, NW, DEPTH>::WAVES_PER
     const int QK = K / BK;
     const int kb_begin = blockIdx.y * kb_per_split, kb_end = kb_begin + kb_per_split < QK ? kb_begin + kb_per_split : QK;
     const int count = (kb_end - kb_begin - wave + NW - 1) / NW;       // this wave's K blocks: kb_begin + wave + NW * i
-    const W w(A, B, SA, SB, M, 0, ldm, N, K, m0, n0, lds + wave * G::REGION, lane);
+    W w(A, B, SA, SB, M, 0, ldm, N, K, m0, n0, lds + wave * G::REGION, lane);
+    if constexpr (DEPTH == 1) asm("" : "+v"(w.zero));             // see gemm_fp8_blockscale_grouped_strips
     auto kb_of = [&](int i) { return kb_begin + wave + NW * i; };
     f32x4 acc[TM][TN];
 #pragma unroll
     for (int j = 0; j < TM; j++)
 #pragma unroll
         for (int i = 0; i < TN; i++) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    auto consume = [&](typename W::Block &x, int i) {
-        w.stage(x, kb_of(i));
+    auto products = [&](const float (&s)[TM]) {
         w.multiply([&](int j, int c, const f32x4 &p) {
-            const float s = x.sa[j] * x.sb;
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc[j][c][e] = __builtin_fmaf(s, p[e], acc[j][c][e]);
+            for (int e = 0; e < 4; e++) acc[j][c][e] = __builtin_fmaf(s[j], p[e], acc[j][c][e]);
         });
     };
-
-    // up to DEPTH K blocks asked for, then used in order; straight-line code for every count, so that each wait is for a
-    // known number of younger loads
-    auto batch = [&](auto count_c, int i) {
-        constexpr int n = decltype(count_c)::value;
-        typename W::Block x[n];
+    auto scales_of = [&](const typename W::Block &x, float (&s)[TM]) {
 #pragma unroll
-        for (int d = 0; d < n; d++) w.fetch(x[d], kb_of(i + d));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int d = 0; d < n; d++) {
-            consume(x[d], i + d);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int j = 0; j < TM; j++) s[j] = x.sa[j] * x.sb;
     };
     static_assert(DEPTH >= 1 && DEPTH <= 4, "one to four K blocks at a time");
-    int i = 0;
-    for (; i + DEPTH <= count; i += DEPTH) batch(IntTag<DEPTH>{}, i);
-    if (DEPTH > 3 && count - i == 3) batch(IntTag<3>{}, i);
-    else if (DEPTH > 2 && count - i == 2) batch(IntTag<2>{}, i);
-    else if (DEPTH > 1 && count - i == 1) batch(IntTag<1>{}, i);
+    if constexpr (DEPTH == 1) {
+        // The next K block is asked for as soon as this one's bytes are in LDS, and travels while this one is multiplied: for
+        // waves with two and more K blocks and too many registers in a block to ask for all of them. us against one block
+        // after the other (same tiles): 128 x 7168 x 2048 10.7 -> 9.7, 200 x 3072 x 1536 8.1 -> 7.5, 400 x 2003 x 7168 28.5 -> 25.8;
+        // against the best plan before: 48 x 7168 x 2048 8.5 -> 7.4, 77 x 2048 x 2048 6.0 -> 5.1.
+        auto step = [&](typename W::Block &x, int i, auto more) {
+            w.stage(x, kb_of(i));
+            float s[TM];
+            scales_of(x, s);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (decltype(more)::value) w.fetch(x, kb_of(i + 1));
+            __builtin_amdgcn_sched_barrier(0);
+            products(s);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (count > 0) {
+            typename W::Block x;
+            w.fetch(x, kb_of(0));
+            int i = 0;
+            for (; i + 1 < count; i++) step(x, i, IntTag<1>{});
+            step(x, i, IntTag<0>{});
+        }
+    } else {
+        // up to DEPTH K blocks asked for, then used in order; straight-line code for every count, so that each wait is for a
+        // known number of younger loads
+        auto batch = [&](auto count_c, int i) {
+            constexpr int n = decltype(count_c)::value;
+            typename W::Block x[n];
+#pragma unroll
+            for (int d = 0; d < n; d++) w.fetch(x[d], kb_of(i + d));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int d = 0; d < n; d++) {
+                w.stage(x[d], kb_of(i + d));
+                float s[TM];
+                scales_of(x[d], s);
+                products(s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int i = 0;
+        for (; i + DEPTH <= count; i += DEPTH) batch(IntTag<DEPTH>{}, i);
+        if (DEPTH > 3 && count - i == 3) batch(IntTag<3>{}, i);
+        else if (DEPTH > 2 && count - i == 2) batch(IntTag<2>{}, i);
+        else if (count - i == 1) batch(IntTag<1>{}, i);
+    }
 
     // the waves' sums through LDS, tile (j, c) of wave w at ((w * TM + j) * TN + c) * 1 KiB, lane l at + 16 l
     __syncthreads();

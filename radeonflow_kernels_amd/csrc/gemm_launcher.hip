@@ -143,6 +143,13 @@ const Variant kVariants[] = {
     RF_VARIANT_FEWROWS(4, 4, 8, 1),   // 20: 64 x 64
     RF_VARIANT_FEWROWS(4, 4, 4, 1),   // 21: 64 x 64, four waves: two workgroups per CU (200 x 5003 x 2048, 316 workgroups:
                                       // one round of the chip instead of two, 23.2 -> 19.8 us)
+    // tiles of which a wave has one K block on its way while it multiplies another (16, 20 and 21 above work like that too)
+    RF_VARIANT_FEWROWS(1, 2, 8, 1),   // 22: 16 x 32
+    RF_VARIANT_FEWROWS(1, 4, 8, 1),   // 23: 16 x 64
+    RF_VARIANT_FEWROWS(2, 2, 8, 1),   // 24: 32 x 32
+    RF_VARIANT_FEWROWS(2, 4, 8, 1),   // 25: 32 x 64
+    RF_VARIANT_FEWROWS(2, 4, 4, 1),   // 26: 32 x 64, four waves
+    RF_VARIANT_FEWROWS(2, 8, 4, 1),   // 27: 32 x 128, four waves
 };
 constexpr int kFewRows64x64 = 20;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
@@ -466,21 +473,25 @@ const TunedPlan kTunedPlans[] = {
 
 constexpr int kTunedOnCUs = 256;
 
-// Estimated time in microseconds of the best few-rows plan for a shape, and that plan. Fitted (relative error) to about 12900
-// plans on operand sets that rotate out of the L2 caches: M = 1 ... 512, 23 pairs of N and K from 200 to 8192 and 128 to
-// 7168, every few-rows variant with 1 to 14 splits (tuner/fewrows_model.py: --measure takes them, --fit fits; the model
-// stands there too). The plan it picks is 4.1 % slower than the best one measured on average and 29 % at worst; constants
-// fitted anew to a second measurement pick no better ones.
-//   1.96                                       launch, and the way back
-//   + 1.12 + 0.106 per KiB of sums handed over when K is split
-//   + rounds * (b + 0.985 * batches of loads of a wave + c * K blocks of a wave * workgroups sharing a CU), a quarter more
-//     where rows of B start at any byte (any_bytes)
-//   + d * MB of A and B that all workgroups fetch
+// Estimated time in microseconds of the best few-rows plan for a shape, and that plan. Its constants are searched on 22280
+// plans measured on operand sets that rotate out of the L2 caches: M = 1 ... 512, 23 pairs of N and K from 200 to 8192 and 128
+// to 7168, every few-rows variant with 1 to 14 splits (tuner/fewrows_model.py: --measure takes them, --fit searches; the model
+// stands there too). The plan it picks is 2.3 % slower than the best one measured on average and 19 % at worst (least
+// squares on the times: 3.9 % and 28 %); its figure is 13 % off. Variants 15 and 17 to 19 are not tried: with them the best
+// measured plans are 0.2 % faster.
+//   2.56                                       launch, and the way back
+//   + 0.64 + 0.192 per KiB of sums handed over when K is split
+//   + rounds * (b + 0.253 * batches of loads of a wave + c * K blocks of a wave * workgroups sharing a CU), a quarter more
+//     where rows of B start at any byte (any_bytes); variants that load the next K block while they multiply: one batch
+//   + d * MB of A and B that all workgroups fetch + 0.0505 * MB of A and B
 double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_config *out) {
     struct Fit { int variant, per_cu, depth; double b, c, d; };
-    const Fit fits[] = {{14, 2, 3, 0.0, 0.458, 0.0916},   {15, 1, 2, 0.0, 0.860, 0.0591},   {16, 1, 1, 0.790, 0.665, 0.0381},
-                        {17, 2, 2, 0.0, 0.572, 0.0755},   {18, 1, 2, 0.101, 1.090, 0.0546}, {19, 1, 2, 0.127, 1.063, 0.0593},
-                        {20, 1, 1, 1.651, 0.929, 0.0362},   {21, 2, 1, 2.48, 0.424, 0.0231}};
+    constexpr int kAll = 1 << 20;
+    const Fit fits[] = {{14, 2, 3, 0.0238, 0.6526, 0.0811},    {16, 1, kAll, 0.017, 1.6541, 0.0325},  {20, 1, kAll, 0.2932, 1.9032, 0.0785},
+                        {21, 2, kAll, 1.3762, 1.0315, 0.0158}, {22, 2, kAll, 0.0007, 0.6572, 0.086},  {23, 1, kAll, 0.0704, 1.4481, 0.0227},
+                        {24, 2, kAll, 0.0049, 0.9508, 0.0676}, {25, 1, kAll, 0.0106, 1.7903, 0.0289}, {26, 2, kAll, 0.3722, 0.7608, 0.0427},
+                        {27, 1, kAll, 1.0902, 1.385, 0.0109}};
+    const double operands = 0.0505e-6 * k * ((double)m + n);
     const int splits_tried[] = {1, 2, 3, 4, 5, 6, 8, 12, 14}, qk = k / rf::BK;
     double best = 1e30;
     for (const Fit &f : fits) {
@@ -491,10 +502,10 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
             const int kb = ceil_div(qk, sp), parts = ceil_div(qk, kb), own = ceil_div(kb, v.waves_n);
             const long wgs = items * parts, rounds = (wgs + (long)num_cu * f.per_cu - 1) / ((long)num_cu * f.per_cu);
             const double mb = (double)wgs * kb * (v.bm + v.bn) * rf::BK * 1e-6 * 256 / num_cu;
-            const double t = 1.96 + (parts > 1 ? 1.12 + 0.106 * parts * v.bm * v.bn / 1024.0 : 0.0) +
+            const double t = 2.5568 + (parts > 1 ? 0.6363 + 0.1919 * parts * v.bm * v.bn / 1024.0 : 0.0) +
                              rounds * (any_bytes ? 1.27 : 1.0) *
-                                 (f.b + 0.985 * ceil_div(own, f.depth) + f.c * own * (wgs > num_cu ? f.per_cu : 1)) +
-                             f.d * mb;
+                                 (f.b + 0.2531 * ceil_div(own, f.depth) + f.c * own * (wgs > num_cu ? f.per_cu : 1)) +
+                             f.d * mb + operands;
             if (t < best) {
                 best = t;
                 *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};

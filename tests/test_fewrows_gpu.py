@@ -39,6 +39,24 @@ def test_fewrows_bit_exact_on_any_shape(rfk, m, n, k):
     assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
 
 
+# tiles whose waves have their next K block on its way (16, 20, 21 and 22 to 27): waves with none, one, two and several K blocks,
+# counts that differ between the waves, the matrix's cut last K block as a wave's first, second and later one
+@pytest.mark.parametrize("m,n,k", [(1, 33, 128), (17, 100, 896), (33, 300, 1024), (31, 257, 1152), (100, 130, 2176), (64, 1000, 4096)])
+def test_fewrows_pipelined_tiles_bit_exact(rfk, m, n, k):
+    data = exact_problem(m, n, k, seed=m + n + k)
+    exp = oracle_bf16(data)
+    g, buf = to_gpu(data, 300)
+    for v in (16, 20, 21) + tuple(range(22, 28)):
+        for split in (1, 2, 5):
+            if split > k // 128:
+                continue
+            g[4].fill_(-1.0)
+            rfk.fp8_mm(*g, config=rfk.GemmConfig(v, split, 1, 0))
+            torch.cuda.synchronize()
+            assert np.array_equal(bf16_bits(g[4]), exp), "variant %d split %d" % (v, split)
+    assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
+
+
 @pytest.mark.parametrize("off_a,off_b,off_c", [(1, 0, 0), (0, 3, 0), (7, 15, 1), (16, 16, 2)])
 def test_fewrows_takes_operands_at_any_byte(rfk, off_a, off_b, off_c):
     """Operands that start off_a, off_b bytes (C: off_c elements) into 16-byte aligned buffers, under the automatic plan and an
