@@ -30,24 +30,23 @@ __device__ __forceinline__ void tile_mainloop_any(
     const int L = lane & 15, g = lane >> 4, wm = wave % WAVES_M, wn = wave / WAVES_M;
     const int QN = (N + 127) / 128;
 
-    // ---- loads: per-thread offsets inside one K block, destinations inside a stage ----
-    uint32_t off_a[IA], off_b[IB], dst_a[IA], dst_b[IB];
-#pragma unroll
-    for (int i = 0; i < IA; i++) {
-        const int q = i * NT + tid, row = q / Y::CPR_A, c = q % Y::CPR_A;
-        int m = m0 + 16 * c;
-        if (m >= M) m = m0;
-        off_a[i] = (uint32_t)row * (uint32_t)ldm + (uint32_t)m;
-        dst_a[i] = row * BM + ((c ^ swizzle_of_row<BM>(row)) << 4);
-    }
-#pragma unroll
-    for (int i = 0; i < IB; i++) {
-        const int q = i * NT + tid, row = q / Y::CPR_B, c = q % Y::CPR_B;
-        int n = n0 + 16 * c;
-        if (n >= N) n = n0;
-        off_b[i] = (uint32_t)row * (uint32_t)N + (uint32_t)n;
-        dst_b[i] = OFF_B + row * BN + ((c ^ swizzle_of_row<BN>(row)) << 4);
-    }
+    // ---- loads: load i of a thread is the 16-byte chunk tid % CPR of K row i * NT / CPR + tid / CPR, at any byte ----
+    static_assert(NT % Y::CPR_A == 0 && NT % Y::CPR_B == 0, "a thread keeps its chunk");
+    const int chunk_a = tid % Y::CPR_A, row_a = tid / Y::CPR_A, chunk_b = tid % Y::CPR_B, row_b = tid / Y::CPR_B;
+    constexpr int STEP_A = NT / Y::CPR_A, STEP_B = NT / Y::CPR_B;         // K rows between two loads
+    // (a chunk past M or N: the row's first, any bytes will do)
+    const uint32_t off_a0 = (uint32_t)row_a * (uint32_t)ldm + (uint32_t)(m0 + 16 * chunk_a < M ? m0 + 16 * chunk_a : m0),
+                   off_b0 = (uint32_t)row_b * (uint32_t)N + (uint32_t)(n0 + 16 * chunk_b < N ? n0 + 16 * chunk_b : n0);
+    auto off_a = [&](int i) { return off_a0 + (uint32_t)(i * STEP_A) * (uint32_t)ldm; };
+    auto off_b = [&](int i) { return off_b0 + (uint32_t)(i * STEP_B) * (uint32_t)N; };
+    auto dst_a = [&](int i) {
+        const int row = row_a + i * STEP_A;
+        return (uint32_t)(row * BM + ((chunk_a ^ swizzle_of_row<BM>(row)) << 4));
+    };
+    auto dst_b = [&](int i) {
+        const int row = row_b + i * STEP_B;
+        return (uint32_t)(OFF_B + row * BN + ((chunk_b ^ swizzle_of_row<BN>(row)) << 4));
+    };
     // scales: threads 0 .. BM - 1 the rows of the tile, the next four its column blocks, the others repeat the last one
     static_assert(NT >= BM + 4, "a thread per scale");
     const float *src_s;
@@ -72,31 +71,31 @@ __device__ __forceinline__ void tile_mainloop_any(
         const unsigned long long r = (unsigned long long)(QK - kb) * BK * (unsigned)ld;
         return r < 0xffffffffull ? (uint32_t)r : 0xffffffffu;
     };
-    u32x4_lds ra[SETS][IA], rb[SETS][IB];
+    u32x4_lds raw[SETS][IA + IB];
     float rs[SETS];
     const int kb_last = kb_end - 1;
     auto clamp_kb = [&](int kb) { return kb < kb_last ? kb : kb_last; };
     auto load_item = [&](auto set_c, int d, int kb) {
         constexpr int set = decltype(set_c)::value;
         kb = clamp_kb(kb);
-        if (d < IA) ra[set][d] = load16<true>(A + (size_t)kb * BK * ldm, off_a[d < IA ? d : 0], rest(kb, ldm));
-        else if (d < IA + IB) rb[set][d - IA < IB ? d - IA : 0] = load16<true>(B + (size_t)kb * BK * N, off_b[d - IA < IB && d >= IA ? d - IA : 0], rest(kb, N));
+        if (d < IA) raw[set][d] = load16<true>(A + (size_t)kb * BK * ldm, off_a(d), rest(kb, ldm));
+        else if (d < IA + IB) raw[set][d] = load16<true>(B + (size_t)kb * BK * N, off_b(d - IA), rest(kb, N));
         else rs[set] = src_s[(size_t)kb * step_s];
     };
-    auto write_item = [&](auto set_c, int d, int stage, int kb) {
+    auto write_item = [&](auto set_c, int d, int stage) {
         constexpr int set = decltype(set_c)::value;
-        if (d < IA) {
-            u32x4_lds v = ra[set][d < IA ? d : 0];
-            if (kb == QK - 1) v = shift_back(v, off_a[d < IA ? d : 0], rest(kb, ldm));
-            *(u32x4_lds *)(lds + stage * STAGE_A + dst_a[d < IA ? d : 0]) = v;
-        } else if (d < IA + IB) {
-            const int e = d - IA < IB && d >= IA ? d - IA : 0;
-            u32x4_lds v = rb[set][e];
-            if (kb == QK - 1) v = shift_back(v, off_b[e], rest(kb, N));
-            *(u32x4_lds *)(lds + stage * STAGE_B + dst_b[e]) = v;
-        } else {
-            *(float *)(lds + stage * STAGE_S + dst_s) = rs[set];
-        }
+        if (d < IA) *(u32x4_lds *)(lds + stage * STAGE_A + dst_a(d)) = raw[set][d];
+        else if (d < IA + IB) *(u32x4_lds *)(lds + stage * STAGE_B + dst_b(d - IA)) = raw[set][d];
+        else *(float *)(lds + stage * STAGE_S + dst_s) = rs[set];
+    };
+    // the matrix's last K block: bytes of cut loads back to their places
+    auto uncut = [&](auto set_c, int kb) {
+        constexpr int set = decltype(set_c)::value;
+        if (kb != QK - 1) return;
+#pragma unroll
+        for (int d = 0; d < IA; d++) raw[set][d] = shift_back(raw[set][d], off_a(d), rest(kb, ldm));
+#pragma unroll
+        for (int d = 0; d < IB; d++) raw[set][IA + d] = shift_back(raw[set][IA + d], off_b(d), rest(kb, N));
     };
     constexpr int NL = IA + IB + 1;
 
@@ -175,8 +174,9 @@ __device__ __forceinline__ void tile_mainloop_any(
         for (int d = 0; d < NL; d++) load_item(set_c, d, kb_begin + decltype(set_c)::value);
     });
     __builtin_amdgcn_sched_barrier(0);
+    uncut(IntTag<0>{}, kb_begin);
 #pragma unroll
-    for (int d = 0; d < NL; d++) write_item(IntTag<0>{}, d, 0, kb_begin);
+    for (int d = 0; d < NL; d++) write_item(IntTag<0>{}, d, 0);
 #pragma unroll
     for (int d = 0; d < NL; d++) load_item(IntTag<0>{}, d, kb_begin + SETS);
     __builtin_amdgcn_sched_barrier(0);
@@ -192,7 +192,7 @@ __device__ __forceinline__ void tile_mainloop_any(
         constexpr int cur = decltype(cur_c)::value, nxt = 1 - cur;
         constexpr int split = decltype(split_c)::value;
         const float s_last = s[TM - 1], s1_last = s1[ONE_SB ? 0 : TM - 1];
-        const int kb_next = clamp_kb(kb + 1);
+        uncut(set_c, clamp_kb(kb + 1));
 #pragma unroll
         for (int j = 0; j < TM; j++) s[j] = sraw[j] * sb_raw;
         if constexpr (!ONE_SB)
@@ -220,7 +220,7 @@ __device__ __forceinline__ void tile_mainloop_any(
                 }
             }
 #pragma unroll
-            for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) write_item(set_c, d, nxt, kb_next);
+            for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) write_item(set_c, d, nxt);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) load_item(set_c, d, kb + 1 + SETS);
@@ -280,18 +280,68 @@ __device__ __forceinline__ void tile_mainloop_any(
     }
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int SETS>
+// PARTIAL: the fp32 sums of K part blockIdx.y to ws[part][M rounded up to 16][ld_ws] (see reduce_splitk_any_c).
+template <int BM, int BN, int WAVES_M, int WAVES_N, int SETS, bool PARTIAL>
 __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_tile_any(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
-    const float *__restrict__ SB, uint16_t *__restrict__ C, int M, int ldm, int N, int K, int tiles_m, int tiles_n, int group_m) {
+    const float *__restrict__ SB, void *__restrict__ out, int M, int ldm, int N, int K, int kb_per_split, int tiles_m, int tiles_n,
+    int group_m) {
     using G = TileGeom<BM, BN, WAVES_M, WAVES_N, 2>;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     int tile_m, tile_n;
     tile_of_block(blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, group_m, true, tile_m, tile_n);
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int m0 = tile_m * BM, n0 = tile_n * BN, QK = K / BK;
+    const int kb_begin = blockIdx.y * kb_per_split, kb_end = kb_begin + kb_per_split < QK ? kb_begin + kb_per_split : QK;
     f32x4 acc[G::TM][G::TN];
-    tile_mainloop_any<BM, BN, WAVES_M, WAVES_N, SETS>(A, B, SA, SB, M, ldm, N, K / BK, m0, n0, 0, K / BK, lds, acc);
-    store_tile_bf16<BM, BN, WAVES_M, WAVES_N, default_store_passes<BM, WAVES_M>(), true, true>(acc, C, M, N, m0, n0, lds);
+    tile_mainloop_any<BM, BN, WAVES_M, WAVES_N, SETS>(A, B, SA, SB, M, ldm, N, QK, m0, n0, kb_begin, kb_end, lds, acc);
+    if constexpr (PARTIAL) {
+        const int mp = (M + 15) / 16 * 16, ld_ws = (N + 15) / 16 * 16;
+        store_tile_f32_staged<BM, BN, WAVES_M, WAVES_N>(acc, (float *)out + ((size_t)blockIdx.y * mp + m0) * ld_ws + n0, ld_ws, mp - m0,
+                                                        ld_ws - n0, lds);
+    } else {
+        store_tile_bf16<BM, BN, WAVES_M, WAVES_N, default_store_passes<BM, WAVES_M>(), true, true>(acc, (uint16_t *)out, M, N, m0, n0, lds);
+    }
+}
+
+// Sum of K parts in order, one bf16 rounding, into a C of any width and alignment: ws holds [part][rows_ws][ld] sums (ld a
+// multiple of 8), C is the first `rows` x n of them. A thread sums eight columns of a row.
+__global__ __launch_bounds__(256) void reduce_splitk_any_c(const float *__restrict__ ws, int ld, size_t part_stride, int splits, int n,
+                                                           int rows, uint16_t *__restrict__ C) {
+    const int pieces = (n + 7) / 8;
+    const int per_block = pieces < 256 ? 256 / pieces : 1;
+    const int trow = pieces < 256 ? (int)threadIdx.x / pieces : 0;
+    const int piece = pieces < 256 ? (int)threadIdx.x - trow * pieces : (int)(blockIdx.y * 256 + threadIdx.x);
+    const int r = (int)blockIdx.x * per_block + trow, col = piece * 8;
+    if (trow >= per_block || piece >= pieces || r >= rows) return;
+    const float *p = ws + (size_t)r * ld + col;
+    f32x4 s0 = *(const f32x4 *)p, s1 = *(const f32x4 *)(p + 4);
+    constexpr int BATCH = 4;
+    for (int q0 = 1; q0 < splits; q0 += BATCH) {
+        f32x4 v[BATCH][2];
+#pragma unroll
+        for (int q = 0; q < BATCH; q++)
+            if (q0 + q < splits) {
+                v[q][0] = *(const f32x4 *)(p + (size_t)(q0 + q) * part_stride);
+                v[q][1] = *(const f32x4 *)(p + (size_t)(q0 + q) * part_stride + 4);
+            }
+#pragma unroll
+        for (int q = 0; q < BATCH; q++)
+            if (q0 + q < splits)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    s0[e] += v[q][0][e];
+                    s1[e] += v[q][1][e];
+                }
+    }
+    const u32x4_lds w = {pack_bf16x2(s0[0], s0[1]), pack_bf16x2(s0[2], s0[3]), pack_bf16x2(s1[0], s1[1]), pack_bf16x2(s1[2], s1[3])};
+    uint16_t *out = C + (size_t)r * n + col;
+    if (col + 8 <= n) {
+        *(u32x4_any *)out = w;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 7; e++)
+            if (col + e < n) out[e] = (uint16_t)(w[e / 2] >> (16 * (e % 2)));
+    }
 }
 
 }  // namespace rf

@@ -20,6 +20,7 @@
 #include "fp8_gemm_persistent.h"
 #include "fp8_gemm_skinny.h"
 #include "fp8_gemm_fewrows.h"
+#include "fp8_gemm_any.h"
 #include "quantize_kernels.h"
 
 // Scratch memory of rf_fp8_gemm_static, the entry point that allocates nothing: split-K partial sums and staging
@@ -66,6 +67,8 @@ typedef void (*fewrows_kernel_t)(const uint8_t *, const uint8_t *, const float *
                                  int, int, int, unsigned *, float *);
 typedef void (*any_c_kernel_t)(const uint8_t *, const uint8_t *, const float *, const float *, uint16_t *, int, int, int, int,
                                int, int, int, int);
+typedef void (*any_tile_kernel_t)(const uint8_t *, const uint8_t *, const float *, const float *, void *, int, int, int, int, int, int,
+                                  int, int);
 struct Variant {
     int bm, bn, waves_m, waves_n, lds;
     tile_kernel_t direct, partial;
@@ -76,7 +79,10 @@ struct Variant {
     int k_groups = 1;                    // > 1: wave groups of one workgroup split K between them (needs K/128 % k_groups == 0)
     fewrows_kernel_t fewrows[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};   // [K split][any alignment of B]; null: a tiled variant
     any_c_kernel_t any_c = nullptr;      // the direct form for a C of any width and alignment
+    any_tile_kernel_t any_tile[2] = {nullptr, nullptr};   // [K split]: operands at any alignment (fp8_gemm_any.h)
     bool is_fewrows() const { return fewrows[0][0] != nullptr; }
+    bool is_any_tile() const { return any_tile[0] != nullptr; }
+    bool takes_any_shape() const { return is_fewrows() || is_any_tile(); }
     int lds_bytes() const { return lds; }
     int threads() const { return waves_m * waves_n * 64 * k_groups; }
 };
@@ -110,6 +116,10 @@ struct Variant {
                 rf::gemm_fp8_blockscale_fewrows<TM, TN, NW, DEPTH, false, true>},          \
                {rf::gemm_fp8_blockscale_fewrows<TM, TN, NW, DEPTH, true, false>,           \
                 rf::gemm_fp8_blockscale_fewrows<TM, TN, NW, DEPTH, true, true>}} }
+// tiles whose operands pass through registers, at any alignment (fp8_gemm_any.h)
+#define RF_VARIANT_ANY_TILE(BM, BN, WM, WN)                                                \
+    Variant { BM, BN, WM, WN, rf::AnyGeom<BM, BN, WM, WN>::LDS_BYTES, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 1, {}, nullptr, \
+              {rf::gemm_fp8_blockscale_tile_any<BM, BN, WM, WN, 2, false>, rf::gemm_fp8_blockscale_tile_any<BM, BN, WM, WN, 2, true>} }
 const Variant kVariants[] = {
     Variant{256, 256, 2, 4, rf::TileGeom<256, 256, 2, 4>::LDS_BYTES, rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, false>,
             rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, true>, rf::gemm_fp8_blockscale_streamk<256, 256, 2, 4>,
@@ -150,8 +160,16 @@ const Variant kVariants[] = {
     RF_VARIANT_FEWROWS(2, 4, 8, 1),   // 25: 32 x 64
     RF_VARIANT_FEWROWS(2, 4, 4, 1),   // 26: 32 x 64, four waves
     RF_VARIANT_FEWROWS(2, 8, 4, 1),   // 27: 32 x 128, four waves
+    // 28: 8 waves, wave tile 32 x 64, three stages, 100 KiB LDS. At a wave per SIMD the reads of fragments, the barrier and the
+    // loads of a K block wait for each other; with two they hide. us, variant 1 (four waves, two stages), the best plan before,
+    // this: 512 x 7168 x 2048 15.1, 14.1, 11.7; 1024 x 1536 x 7168 23.9, 23.2, 22.3; 2048 x 1536 x 7168 35.3, 32.6, 29.1. The plan of 37
+    // of the 163 tabled shapes, 10 % faster there. (Four stages: the same within 2 %. Sixteen waves on 128 x 256 tiles: 49 against
+    // 44 with eight on 1024 x 4608 x 7168.)
+    RF_VARIANT_TILE_ONLY_NS3(128, 128, 4, 2),
+    RF_VARIANT_ANY_TILE(128, 128, 4, 2),   // 29: 8 waves, wave tile 32 x 64
+    RF_VARIANT_ANY_TILE(128, 256, 2, 4),   // 30: 8 waves, wave tile 64 x 64
 };
-constexpr int kFewRows64x64 = 20;
+constexpr int kFewRows64x64 = 20, kFirstFewRows = 14;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
 // ---- process-wide state ---------------------------------------------------------------------
@@ -259,6 +277,8 @@ int ensure_device_info(State &s) {
         for (auto &pair : v.fewrows)
             for (fewrows_kernel_t f : pair)
                 if (f) RF_HIP(hipFuncSetAttribute((const void *)f, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
+        for (any_tile_kernel_t f : v.any_tile)
+            if (f) RF_HIP(hipFuncSetAttribute((const void *)f, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
         if (v.direct)
             RF_HIP(hipFuncSetAttribute((const void *)v.direct, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds_bytes()));
         if (v.any_c)
@@ -525,7 +545,39 @@ constexpr int kFewRowsMaxM = 512, kFewRowsMaxMStagedB = 4096;
 
 // What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
 // (and of C on the way back). kTiledOnly: no few-rows plan.
-enum { kStageA = 1, kStageB = 2, kTiledOnly = 4 };
+// kBytesA, kBytesB: rows of that operand do not all start at a multiple of four bytes.
+enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16 };
+
+// Estimated time in microseconds of the best any-alignment tile plan for a shape whose operands would have to be staged, and
+// that plan. Fitted (relative error, 6 %) to 640 plans of 100 random shapes on operand sets that stay in the Infinity Cache:
+//   2.9 + rounds * (f + K blocks * (c + c_a where rows of A start at any byte + c_b where rows of B do))
+//   + 0.39 per million outputs (0.45 more where rows of C start at odd elements)
+//   + 2.76 + 1.19 per million sums when K is split
+double any_tile_plan(int m, int n, int k, int num_cu, int stage, rf_gemm_config *out) {
+    struct Fit { int variant; double f, c, c_a, c_b; };
+    const Fit fits[] = {{29, 1.60, 0.595, 0.091, 0.119}, {30, 2.71, 0.771, 0.130, 0.326}};
+    const int splits_tried[] = {1, 2, 3, 4, 6, 8}, qk = k / rf::BK;
+    const double mn = (double)m * n * 1e-6;
+    double best = 1e30;
+    for (const Fit &f : fits) {
+        const Variant &v = kVariants[f.variant];
+        const long tiles = (long)ceil_div(m, v.bm) * ceil_div(n, v.bn);
+        const double per_block = f.c + (stage & kBytesA ? f.c_a : 0.0) + (stage & kBytesB ? f.c_b : 0.0);
+        for (int sp : splits_tried) {
+            if (sp > qk) break;
+            const int kb = ceil_div(qk, sp), parts = ceil_div(qk, kb);
+            if (parts > 1 && mn * parts > 40.0) break;      // no more than was measured, 150 MB of sums
+            const long rounds = (tiles * parts + num_cu - 1) / num_cu;
+            const double t = 2.9 + rounds * (f.f + kb * per_block) + mn * (0.39 + (stage & kBytesB ? 0.45 : 0.0)) +
+                             (parts > 1 ? 2.76 + 1.19 * parts * mn : 0.0);
+            if (t < best) {
+                best = t;
+                *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};
+            }
+        }
+    }
+    return best;
+}
 
 // Plan for a shape (m, n multiples of 16, the padded sizes when something is staged).
 void select_config_uncached(int m, int n, int k, int num_cu, int stage, const std::vector<TunedPlan> &user_plans,
@@ -541,6 +593,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     auto usable = [&](const TunedPlan &p) {
         return p.m == m && p.n == n && p.k == k && p.variant < kNumVariants && p.split_k <= k / rf::BK &&
                (!kVariants[p.variant].is_fewrows() || fewrows_usable(p)) &&
+               (!kVariants[p.variant].is_any_tile() || (p.stream_k == RF_SCHEDULE_TILES && fewrows_ok(m, n))) &&
                (kVariants[p.variant].k_groups == 1 || (p.split_k == 1 && (k / rf::BK) % kVariants[p.variant].k_groups == 0)) &&
                (p.stream_k != RF_SCHEDULE_PERSISTENT || persistent_ok(kVariants[p.variant], m, n, k)) &&
                (p.stream_k != RF_SCHEDULE_STREAM_K || stream_k_ok(kVariants[p.variant], m, n, num_cu)) &&
@@ -558,7 +611,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     if (num_cu == kTunedOnCUs)
         for (const TunedPlan &p : kTunedPlans)
             if (!hit && usable(p)) hit = &p;
-    if (hit && (!(stage & (kStageA | kStageB)) || kVariants[hit->variant].is_fewrows())) return take(*hit);
+    if (hit && (!(stage & (kStageA | kStageB)) || kVariants[hit->variant].takes_any_shape())) return take(*hit);
     // Up to four K blocks and a large C: the launch is a streaming store, which the skinny-K schedule does best
     // (measured against the best tiled plan at N = 7168, K = 256: 1024 rows 6.5 against 6.9 us, 2048 rows 7.8 against
     // 10.3, 6144 rows 18.2 against 22.1; below about six million outputs the 64 x 128 tiles win, e.g. 2048 x 2048: 6.5
@@ -595,10 +648,11 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // (variants 12 and 13 split K between two wave groups of one workgroup: half the K blocks per group, one launch, no
     // reduction term. Variant 12, the 64 x 128 tile: the best plan of short shapes, M <= 512, with K = 512 ... 2304.
     // Variant 13, the 128 x 128 tile: the best plan where 128 x 128 tiles fill one round, e.g. 1024 x 3072 x 1536,
-    // 512 x 7168 x 2048)
+    // 512 x 7168 x 2048. Variant 28, the 128 x 128 tile with eight waves and three stages, searched for by itself on 37
+    // further shapes, the other constants as they were: choice 1.4 % behind the best of all, 4.6 % without it)
     const Candidate cands[] = {{0, 0.905, 5.96}, {3, 0.679, 3.61}, {5, 0.80, 5.8},  {6, 0.74, 4.3},  {7, 0.85, 0.3},
                                {8, 0.52, 4.2},   {9, 0.73, 0.5},   {10, 0.53, 5.9}, {11, 0.71, 7.0}, {12, 0.93, 1.4},
-                               {13, 1.06, 3.3}};
+                               {13, 1.06, 3.3}, {28, 0.44, 2.25}};
     const double f_next = 3.3, reduce_fixed = 6.03, reduce_per_elem = 1.27e-6, c_half_tile = 0.47, f_half_tile = 5.2;
     const int splits_tried[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int qk = k / rf::BK;
@@ -653,14 +707,23 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // 14.7 on 128 x 192 tiles); only M ragged, up to 512 rows: 3.0 % and 17 %. Counting C's way back (1.0 us + 0.9 us per
     // million outputs) per plan instead made 33 of 187 shapes 5 % faster on average, but ten of them 1 to 31 % slower
     // (664 x 3001 x 7168 43 -> 56 us: the figure of a K split is too high against that of one part).
+    double t = 3.1 + 0.67 * best_cost;
+    if (stage & kStageA) t += 3.2 + 2.0 * k * m / 4e6;
+    if (stage & kStageB) t += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
+    rf_gemm_config other;
     const int max_m = (stage & kStageB) && num_cu == kTunedOnCUs ? kFewRowsMaxMStagedB : kFewRowsMaxM;
     if (m <= max_m && fewrows_ok(m, n) && !(stage & kTiledOnly)) {
-        double tiled = 3.1 + 0.67 * best_cost;
-        if (stage & kStageA) tiled += 3.2 + 2.0 * k * m / 4e6;
-        if (stage & kStageB) tiled += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
-        rf_gemm_config few;
-        if (fewrows_plan(m, n, k, num_cu, (stage & kStageB) != 0, &few) < tiled) *out = few;
+        const double few = fewrows_plan(m, n, k, num_cu, (stage & kStageB) != 0, &other);
+        if (few < t) {
+            t = few;
+            *out = other;
+        }
     }
+    // Operands that would be staged: the tiles that take them as they are. On 100 shapes drawn at random (90 to 8192 rows; M or N
+    // or both ragged) the plan taken is 1.2 % behind the best of all on average and 27 % at worst, and 10 % faster than
+    // without them (37 of the plans change, one of them for the worse by 6 %); at equal estimates they are the faster ones.
+    // On the compute unit count they were measured on.
+    if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < 1.05 * t) *out = other;
 }
 
 // The same through a small table of plans already worked out (the models take 1 to 3 us of host time, as long as a small
@@ -718,6 +781,35 @@ int launch_fewrows(Mem &mem, const Variant &v, const void *a, const void *b, con
     return RF_OK;
 }
 
+// Bytes of a part's sums in a K split of an any-alignment tile plan: rows and columns rounded up to whole 16-byte pieces.
+size_t any_tile_part_bytes(int m, int n) { return (size_t)ceil_div(m, 16) * 16 * ceil_div(n, 16) * 16 * sizeof(float); }
+
+dim3 pad_grid_of_pieces(int pieces, int rows, int rounds);
+
+// Any shape and alignment. splits >= 1.
+int launch_any_tile(Mem &mem, const Variant &v, const void *a, const void *b, const float *as, const float *bs, void *c, int m, int n,
+                    int k, int splits, int group_m, hipStream_t stream) {
+    const int qk = k / rf::BK, tiles_m = ceil_div(m, v.bm), tiles_n = ceil_div(n, v.bn), kb_per_split = ceil_div(qk, splits);
+    splits = ceil_div(qk, kb_per_split);                    // every split owns at least one K block
+    void *out = c;
+    if (splits > 1) {
+        float *ws = nullptr;
+        const int rc = mem.workspace(any_tile_part_bytes(m, n) * splits, &ws);
+        if (rc != RF_OK) return rc;
+        out = ws;
+    }
+    hipLaunchKernelGGL(v.any_tile[splits > 1], dim3(tiles_m * tiles_n, splits), dim3(v.threads()), v.lds_bytes(), stream,
+                       (const uint8_t *)a, (const uint8_t *)b, as, bs, out, m, m, n, k, kb_per_split, tiles_m, tiles_n, group_m);
+    RF_HIP(hipGetLastError());
+    if (splits > 1) {
+        const int np = ceil_div(n, 16) * 16;
+        hipLaunchKernelGGL(rf::reduce_splitk_any_c, pad_grid_of_pieces(ceil_div(n, 8), m, 1), dim3(256), 0, stream, (const float *)out, np,
+                           any_tile_part_bytes(m, n) / sizeof(float), splits, n, m, (uint16_t *)c);
+        RF_HIP(hipGetLastError());
+    }
+    return RF_OK;
+}
+
 // The launch proper; the caller holds the lock and has checked shape and pointers. m_store >= 0: c has only m_store
 // (<= m) rows, the rest of the m rows of the operands are padding (one workgroup per tile schedules only).
 int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float *as, const float *bs, void *c, int m, int n,
@@ -729,11 +821,11 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
     if (user_cfg) {
         cfg = *user_cfg;
         if (cfg.variant >= kNumVariants || cfg.variant < -1 || cfg.split_k < 1 || cfg.group_m < 1 ||
-            cfg.split_k > k / rf::BK || (cfg.variant >= 0 && !kVariants[cfg.variant].is_fewrows() && !tiled_ok) || (cfg.variant < 0 && cfg.split_k != 1) ||
+            cfg.split_k > k / rf::BK || (cfg.variant >= 0 && !kVariants[cfg.variant].takes_any_shape() && !tiled_ok) || (cfg.variant < 0 && cfg.split_k != 1) ||
             (cfg.stream_k != 0 && (cfg.variant < 0 || cfg.split_k != 1)))
             return fail(RF_ERR_BAD_CONFIG, "configuration not usable for this shape");
-        if (cfg.variant >= 0 && kVariants[cfg.variant].is_fewrows() && !fewrows_ok(m, n))
-            return fail(RF_ERR_BAD_CONFIG, "the few-rows kernels need M and N below 2^25");
+        if (cfg.variant >= 0 && kVariants[cfg.variant].takes_any_shape() && !fewrows_ok(m, n))
+            return fail(RF_ERR_BAD_CONFIG, "the few-rows and any-alignment kernels need M and N below 2^25");
         if (cfg.variant >= 0 && kVariants[cfg.variant].k_groups > 1 &&
             (cfg.split_k != 1 || cfg.stream_k != RF_SCHEDULE_TILES || (k / rf::BK) % kVariants[cfg.variant].k_groups != 0))
             return fail(RF_ERR_BAD_CONFIG, "this variant splits K inside the workgroup: it needs split_k == 1, the tile "
@@ -774,7 +866,8 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         if (cfg.stream_k == RF_SCHEDULE_STREAM_K) cfg.stream_k = RF_SCHEDULE_TILES;
         if (cfg.split_k > 1) {
             const Variant &fv = kVariants[cfg.variant];
-            const size_t per_part = fv.is_fewrows() ? fewrows_slot_bytes(fv, m, n, 1) : (size_t)m * n * sizeof(float);
+            const size_t per_part = fv.is_fewrows() ? fewrows_slot_bytes(fv, m, n, 1)
+                                    : fv.is_any_tile() ? any_tile_part_bytes(m, n) : (size_t)m * n * sizeof(float);
             const int qk_ = k / rf::BK, kb_per = ceil_div(qk_, cfg.split_k), parts = ceil_div(qk_, kb_per);
             const size_t fit = mem.fixed_left() / per_part;
             if ((size_t)parts > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;
@@ -800,6 +893,10 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
 
     const Variant &v = kVariants[cfg.variant];
     if (v.is_fewrows()) return launch_fewrows(mem, v, a, b, as, bs, c, m_store, m, n, k, cfg.split_k, stream);
+    if (v.is_any_tile()) {
+        if (cfg.stream_k != RF_SCHEDULE_TILES || m_store != m) return fail(RF_ERR_BAD_CONFIG, "the any-alignment tiles have one schedule and no padded rows");
+        return launch_any_tile(mem, v, a, b, as, bs, c, m, n, k, cfg.split_k, cfg.group_m, stream);
+    }
     const int tiles_m = ceil_div(m, v.bm), tiles_n = ceil_div(n, v.bn);
     const int qk = k / rf::BK;
     const int kb_per_split = ceil_div(qk, cfg.split_k);
@@ -1113,7 +1210,24 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     // tile, persistent) write the m true rows straight into c (their stores are masked by row), and the tile kernels
     // have a form for any c; otherwise C is staged and copied back.
     rf_gemm_config cfg;
-    select_config(mp, np, k, s.num_cu, (copy_a ? kStageA : 0) | (copy_b || (uintptr_t)c % 16 != 0 ? kStageB : 0), &cfg);
+    select_config(mp, np, k, s.num_cu, (copy_a ? kStageA : 0) | (copy_b || (uintptr_t)c % 16 != 0 ? kStageB : 0) |
+                  (m % 4 != 0 || (uintptr_t)a % 4 != 0 ? kBytesA : 0) | (n % 4 != 0 || (uintptr_t)b % 4 != 0 ? kBytesB : 0), &cfg);
+    if (kVariants[cfg.variant].is_any_tile()) {
+        const size_t part = any_tile_part_bytes(m, n);
+        if (mem.fixed && cfg.split_k > 1) {                // as many K parts as the static array holds
+            const size_t fit = mem.fixed_left() / part;
+            if ((size_t)cfg.split_k > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;
+        } else if (cfg.split_k > 1) {                      // no memory for the sums: K in one part
+            float *ws = nullptr;
+            const int qk_ = k / rf::BK, parts = ceil_div(qk_, ceil_div(qk_, cfg.split_k));
+            if (mem.workspace(part * parts, &ws) != RF_OK) {
+                (void)hipGetLastError();
+                g_last_error.clear();
+                cfg.split_k = 1;
+            }
+        }
+        return launch_any_tile(mem, kVariants[cfg.variant], a, b, as, bs, c, m, n, k, cfg.split_k, cfg.group_m, stream);
+    }
     if (kVariants[cfg.variant].is_fewrows()) {
         if (mem.fixed && cfg.split_k > 1) {                // as many K parts as the static array holds
             const Variant &v = kVariants[cfg.variant];
@@ -1195,7 +1309,8 @@ void plan_of_shape(int m, int n, int k, int num_cu, rf_gemm_config *out) {
     auto pad16 = [](int x) { return x < 16 ? 16 : (x + 15) / 16 * 16; };
     const int mp = pad16(m), np = pad16(n);
     if ((mp != m || np != n) && (double)m * n * k < kPadThresholdMacs) *out = {-1, 1, 8, RF_SCHEDULE_TILES};
-    else select_config(mp, np, k, num_cu, (mp != m ? kStageA : 0) | (np != n ? kStageB : 0), out);
+    else select_config(mp, np, k, num_cu, (mp != m ? kStageA : 0) | (np != n ? kStageB : 0) | (m % 4 != 0 ? kBytesA : 0) |
+                       (n % 4 != 0 ? kBytesB : 0), out);
 }
 
 // ---- timing record for run() ----------------------------------------------------------------
@@ -1347,7 +1462,7 @@ size_t rf_gemm_workspace_bytes(int m, int n, int k) {
     if (cfg.stream_k == RF_SCHEDULE_STREAM_K) return (size_t)2 * s.num_cu * v.bm * v.bn * sizeof(float);
     const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, cfg.split_k));
     if (parts <= 1) return 0;
-    if (v.is_fewrows()) return fewrows_slot_bytes(v, m, n, parts);
+    if (cfg.variant >= kFirstFewRows) return fewrows_slot_bytes(v, m, n, parts);   // (whole tiles: a little more than variants 28 to 30 need)
     // a ragged shape runs (and splits K) at its padded size; its staging copies live in a buffer of their own
     const size_t mp = m < 16 ? 16 : (m + 15) / 16 * 16, np = n < 16 ? 16 : (n + 15) / 16 * 16;
     return mp * np * sizeof(float) * parts;

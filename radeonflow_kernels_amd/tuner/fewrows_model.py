@@ -79,8 +79,17 @@ def estimate(variant, m, n, k, split, num_cu=256, fit=None, common=COMMON):
     return None if x is None else sum(c * y for c, y in zip(tuple(common) + (fit or FIT)[variant], x))
 
 
-def choice(m, n, k, num_cu=256, fit=None, common=COMMON):
-    """The (variant, split_k) fewrows_plan picks."""
+def tile_estimate(m, n, k, split, num_cu=256):
+    """The tiled kernels' figure for variant 28 (128 x 128), which is numbered after the few-rows kernels, in the same us."""
+    qk, tiles = k // BK, _ceil(m, 128) * _ceil(n, 128)
+    kb = _ceil(qk, split)
+    parts = _ceil(qk, kb)
+    t = _ceil(tiles * parts, num_cu) * (kb * 0.44 + 2.25)
+    return 3.1 + 0.67 * (t + (6.03 + 1.27e-6 * parts * m * n if parts > 1 else 0.0))
+
+
+def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
+    """The (variant, split_k) the planner picks from variant 14 on. tiles: variant 28 among them (not for ragged operands)."""
     best = None
     for v in fit or FIT:
         for s in SPLITS:
@@ -89,6 +98,10 @@ def choice(m, n, k, num_cu=256, fit=None, common=COMMON):
                 break
             if best is None or t < best[0]:
                 best = (t, v, s)
+    if tiles:
+        for s in (1, 2, 3, 4, 6, 8, 12, 16):
+            if s <= k // BK and tile_estimate(m, n, k, s, num_cu) < best[0]:
+                best = (tile_estimate(m, n, k, s, num_cu), 28, s)
     return best[1:]
 
 
@@ -145,7 +158,7 @@ def report(rows, fit, common, what):
     shapes = {}
     for m, n, k, v, s, us in rows:
         shapes.setdefault((m, n, k), {})[v, s] = us
-    behind = [t[choice(*shape, fit=fit, common=common)] / min(t.values()) for shape, t in shapes.items()]
+    behind = [t[choice(*shape, fit=fit, common=common, tiles=False)] / min(t.values()) for shape, t in shapes.items()]
     print("%s: estimate over measured %.2f ... %.2f, rms of the logarithm %.3f; choice behind the fastest of %d shapes by %.1f %% "
           "on average, %.0f %% at worst" % (what, min(err), max(err), float(np.sqrt(np.mean(np.log(err) ** 2))), len(shapes),
                                              100 * (np.mean(behind) - 1), 100 * (max(behind) - 1)))
@@ -183,7 +196,7 @@ def meet(path):
         for m, n, k in MEET:
             sets = t.operand_sets(m, n, k)
             auto = t.rotated_us(rfk, sets, None, 32)
-            few = choice(m, n, k)
+            few = choice(m, n, k, tiles=False)
             few_us = t.rotated_us(rfk, sets, rfk.GemmConfig(few[0], few[1], 8, 0), 32)
             plan = rfk.select_config(m, n, k)
             best = None
