@@ -1575,7 +1575,7 @@ struct GroupedVariant {
 constexpr int kMixedLds = rf::TileGeom<256, 256, 2, 4>::LDS_BYTES > rf::TileGeom<128, 256, 2, 4, 3>::LDS_BYTES
                               ? rf::TileGeom<256, 256, 2, 4>::LDS_BYTES : rf::TileGeom<128, 256, 2, 4, 3>::LDS_BYTES;
 const GroupedVariant kGroupedVariants[] = {
-    RF_GROUPED(256, 256, 2, 4, 2), RF_GROUPED(128, 256, 2, 4, 3), RF_GROUPED(128, 128, 2, 2, 2), RF_GROUPED(128, 64, 2, 1, 2),
+    RF_GROUPED(256, 256, 2, 4, 2), RF_GROUPED(128, 256, 2, 4, 3), RF_GROUPED(128, 128, 4, 2, 3), RF_GROUPED(128, 64, 2, 1, 2),
     GroupedVariant{256, 256, 512, kMixedLds, rf::gemm_fp8_blockscale_grouped_mixed, true},
     GroupedVariant{256, 256, 512, rf::kQueueLds, nullptr, true, true},
     RF_GROUPED_STRIPS(1, 2, 2, 1),    // 6: 16 rows, two waves of 128 columns
@@ -1649,10 +1649,10 @@ int choose_grouped_variant(const int *row_offsets, int groups, int n, int k, int
         if (t > most) { most = t; most_v = v; }
     }
     if (variant < 0) variant = most_v;
-    // Too few 128 x 256 tiles for every CU: a launch is the chain of one tile's K blocks, which is as long for the 128 x 64
-    // tiles as for the 128 x 128 ones (two stages) and 10 % longer for the 128 x 256 ones (three), so smaller tiles pay
-    // only while they are alone on their CU. us on N x K = 2048 x 7168 with tiles of 64, 128 and 256 columns: 1000 rows in 8
-    // groups 92, 71, 78; 3000 rows (more 128 x 128 tiles than CUs) 176, 102, 87; 4096 x 2048: 3000 rows 91, 65, 57. (Below
+    // Too few 128 x 256 tiles for every CU: a launch is the chain of one tile's K blocks, shortest for the 128 x 128 tiles (eight
+    // waves, three stages), so smaller tiles pay only while they are alone on their CU. us on N x K = 2048 x 7168 with tiles of
+    // 64, 128 and 256 columns: 1000 rows in 8 groups 92, 48, 57; 3000 rows (more 128 x 128 tiles than CUs) 176, 103, 81; 4096 x
+    // 2048: 355 rows in 8 groups -, 19, 21. With four waves and two stages the 128 x 128 tiles took 62, 95 and 23. (Below
     // K = 2048 not measured.)
     if ((variant == 2 || variant == 3) && k >= 2048)
         return grouped_tiles(kGroupedVariants[2], row_offsets, groups, n) <= num_cu ? 2 : 1;
