@@ -15,6 +15,9 @@
 // With three or four K blocks an item is 64 rows (wave share 32 x 64, two m-tiles), so that four item slots and the
 // strip's fragments (up to 128 registers) still fit; B then passes through the whole ring before the first item is
 // loaded, and a wave works through an m-tile K block by K block (one A fragment and four partial tiles live at a time).
+// Which rows and columns run where is worth as much as the loop (us, before -> after; N = 7168 and 8192): with a strip's
+// workgroups on all XCDs every XCD fetched all of B and A, 27 MB for 6144 x 7168 x 256, and waited for it; dealt in bands (see
+// skinny_work) 2048 x 7168 x 256 9.4 -> 8.0, 512 x 8192 x 512 9.4 -> 6.0, 6144 x 8192 x 256 24.7 -> 20.5, 6144 x 7168 x 256 20.7 -> 19.1.
 // Numerics are those of the tiled kernels: per K block the products are summed inside the MFMA from zero and folded
 // with acc = fma(a_scale * b_scale, partial, acc), K blocks in order; one bf16 rounding.
 //
@@ -52,25 +55,65 @@ struct SkinnyGeom {
     static_assert((RING - 1) * STORES + (RING - 2) * INST_A <= 63, "the largest wait count fits the instruction's field");
 };
 
+// How the work is dealt, from the host: every division a workgroup would have to do before its first load is 0.1 us of it.
+struct SkinnyWork {
+    int strips, per_strip;       // workgroups: strips * per_strip
+    int bands_log2;              // -1: dealt as they come
+    int rounds;                  // whole rounds: in each, a strip's workgroups take one item each, side by side
+    int share, more;             // of the rows behind them, 64-row units of a workgroup; the first `more` workgroups have one more
+};
+
+// x / d for 0 <= x < 2^24 with a quotient below 2^20, or d = 1: the reciprocal's product is off by one at most.
+__device__ __forceinline__ int small_quotient(int x, int d) {
+    int q = (int)((float)x * __builtin_amdgcn_rcpf((float)d));
+    const int r = x - q * d;
+    q += r >= d ? 1 : r < 0 ? -1 : 0;
+    return __builtin_amdgcn_readfirstlane(q);
+}
+
+// Which strip and which share of its rows a workgroup takes. Workgroups go to the XCDs in turn (id % 8). With bands, an XCD's
+// workgroups are the shares of one band of rows and of neighbouring strips, so that its L2 fetches that part of A and of B
+// only; without, an XCD's workgroups have every eighth share of all strips and fetch all of B.
+__device__ __forceinline__ void skinny_work(const SkinnyWork &w, int *strip, int *part) {
+    int lin = (int)blockIdx.x, first = 0, width = w.per_strip;
+    if (w.bands_log2 >= 0) {
+        const int total = (int)gridDim.x, xcd = lin & 7, each = total >> 3, more = total & 7;
+        lin = xcd * each + (xcd < more ? xcd : more) + (lin >> 3);   // XCD after XCD: band after band, strip after strip
+        for (int g = 0; g < 1 << w.bands_log2; g++) {
+            first = (g * w.per_strip) >> w.bands_log2;
+            width = (((g + 1) * w.per_strip) >> w.bands_log2) - first;
+            if (lin < width * w.strips) break;
+            lin -= width * w.strips;
+        }
+    }
+    *strip = small_quotient(lin, width);
+    *part = first + lin - *strip * width;
+}
+
 template <int QK>
 __global__ __launch_bounds__(512) void gemm_fp8_blockscale_skinny(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
-    const float *__restrict__ SB, uint16_t *__restrict__ C, int M, int N, int per_strip, int M_store) {
+    const float *__restrict__ SB, uint16_t *__restrict__ C, int M, int N, const SkinnyWork work, int M_store) {
     using G = SkinnyGeom<QK>;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int L = lane & 15, g = lane >> 4, wm = wave & 1, wn = wave >> 1;
     const int QN = (N + 127) / 128;
-    // this workgroup: strip blockIdx.x / per_strip, and of its rows (in units of 64) the share blockIdx.x % per_strip
-    const int strip = (int)blockIdx.x / per_strip, part = (int)blockIdx.x - strip * per_strip;
-    const int units = (M + 63) / 64;
-    const int m_begin = 64 * (int)((long)part * units / per_strip);
-    int m_end = 64 * (int)((long)(part + 1) * units / per_strip);
-    if (m_end > M) m_end = M;
-    if (m_begin >= m_end) return;
-    const int n_items = (m_end - m_begin + G::IM - 1) / G::IM;
-    const int row_lim = m_end < M_store ? m_end : M_store;             // rows of C this workgroup may write end here
+    int strip, part;
+    skinny_work(work, &strip, &part);
+    const int rounds = QK <= 2 ? work.rounds : 0, per_strip = work.per_strip;       // (known to be none with 64-row items)
+    const int rest_begin = rounds * per_strip * G::IM + 64 * (part * work.share + (part < work.more ? part : work.more));
+    int rest_end = rest_begin + 64 * (work.share + (part < work.more ? 1 : 0));
+    if (rest_end > M) rest_end = M;
+    const int n_items = rounds + (rest_end > rest_begin ? (rest_end - rest_begin + G::IM - 1) / G::IM : 0);
+    if (n_items == 0) return;
+    auto row_of = [&](int item) { return item < rounds ? (item * per_strip + part) * G::IM : rest_begin + (item - rounds) * G::IM; };
+    // rows of C this workgroup may write in an item end here
+    auto row_end = [&](int item) {
+        const int e = item < rounds ? (item * per_strip + part + 1) * G::IM : rest_end;
+        return e < M_store ? e : M_store;
+    };
     const int n0 = strip * G::BN;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(RF_LDS uint8_t *)lds;
 
@@ -105,8 +148,8 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_skinny(
             dma4((uint32_t)(kb * QN + nb) * 4u, (const uint8_t *)SB, lds_base + G::OFF_SB);
         }
     };
-    auto issue_a = [&](int item) {                                   // rows m_begin + IM item .. of A into slot item % RING
-        const int slot = item & (G::RING - 1), m0 = m_begin + item * G::IM;
+    auto issue_a = [&](int item) {                                   // rows row_of(item) .. of A into slot item % RING
+        const int slot = item & (G::RING - 1), m0 = row_of(item);
 #pragma unroll
         for (int d = 0; d < G::INST_A; d++) {
             const int q = wave * G::INST_A + d;                      // K rows RPI_A q .. of the item
@@ -194,7 +237,7 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_skinny(
     // one item; full_c: no row of it is masked
     auto compute_item = [&](int t, auto full_c) {
         constexpr bool full = decltype(full_c)::value != 0;
-        const int slot = t & (G::RING - 1), m0 = m_begin + t * G::IM;
+        const int slot = t & (G::RING - 1), m0 = row_of(t), row_lim = row_end(t);
         float sv[QK][G::TM];                                         // a_scale of row L of each m-tile, per K block
 #pragma unroll
         for (int kb = 0; kb < QK; kb++) {
@@ -324,7 +367,7 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_skinny(
             mark3 = issued;
         }
         if (active) {
-            if (m_begin + (t + 1) * G::IM <= row_lim) {
+            if (row_of(t) + G::IM <= row_end(t)) {
                 compute_item(t, IntTag<1>{});
                 issued += G::STORES;
             } else {

@@ -473,6 +473,25 @@ bool skinny_ok(int m, int n, int k) {
     return k >= rf::BK && k <= 4 * rf::BK && k % rf::BK == 0 && m >= 16 && m % 16 == 0 && n >= 64 && n % 64 == 0;
 }
 
+// Bands of rows the skinny-K schedule deals to the XCDs (see skinny_work), as a power of two; -1: none, workgroups as they
+// come. With g bands an XCD fetches 1/g of A and g/8 of B; B counts four times, since everybody waits for it at the start
+// while A streams ahead of its use. us, none -> one band / two: 512 x 7168 x 384 7.2 -> 4.9 / 5.1; 1024 x 7168 x 256 6.9 -> 5.5 / 5.5;
+// 4096 x 7168 x 256 14.9 -> 13.5 / 13.5; 6144 x 7168 x 256 21.2 -> 19.9 / 23.2; 6144 x 3072 x 512 17.4 -> 16.6 / 15.3; 8192 x 3072 x 384
+// 17.0 -> 16.8 / 15.9. None where that is the faster way:
+//   rows of C whose length is a power of two up to 8 KB put the few columns an XCD would have onto few channels of its L2
+//     (8192 x 2048 x 256 8.1 -> 9.6 with one band); rows of 16 KB need two bands (6144 x 8192 x 256 24.7 -> 23.1 / 20.9)
+//   K = 128: A and B are small next to C (3072 x 1536 x 128 4.4 -> 4.7, 4096 x 8192 x 128 12.1 -> 13.9; but 4096 x 7168 x 128 12.0 -> 11.5)
+//   few strips whose shares come in eighths: each XCD has an eighth of the rows anyway (4096 x 576 x 384 4.8 -> 5.0; with shares
+//     that do not, 6144 x 576 x 384 8.2 -> 7.2)
+int skinny_bands_log2(int m, int n, int qk, int strips, int per_strip) {
+    const bool power = (n & (n - 1)) == 0;
+    if ((power && n <= 4096) || (qk == 1 && (power || n <= 4096)) || (strips <= 8 && per_strip % 8 == 0)) return -1;
+    int best = power ? 1 : 0;
+    for (int l = best + 1; l <= 3; l++)
+        if ((double)m / (1 << l) + 0.5 * n * (1 << l) < (double)m / (1 << best) + 0.5 * n * (1 << best)) best = l;
+    return best;
+}
+
 // Few-rows kernels keep offsets inside a K block in 32 bits.
 bool fewrows_ok(long ldm, int n) { return ldm < (1 << 25) && n < (1 << 25); }
 
@@ -922,10 +941,17 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         const int strips = ceil_div(n, 256), units = ceil_div(m, 64);
         int per_strip = s.num_cu / strips;
         per_strip = per_strip < 1 ? 1 : per_strip > units ? units : per_strip;
+        // A C that the Infinity Cache does not hold is written band by band, all workgroups side by side, which memory takes
+        // faster than 256 streams far apart: K = 256, 8192 x 7168 30.7 -> 27.1 us, 6144 x 7168 19.9 -> 19.1; smaller ones are
+        // even or up to 3 % slower (1024 x 7168 5.5 -> 5.7), and so are the 64-row items of K = 384 and 512 (6144 x 7168 x 384
+        // 24.5 -> 25.0), which spend more on each item.
+        const int rounds = qk <= 2 && (double)m * n >= 4.0e7 ? m / (per_strip * rf::SkinnyGeom<2>::IM) : 0;
+        const int rest = ceil_div(m - rounds * per_strip * rf::SkinnyGeom<2>::IM, 64);
+        const rf::SkinnyWork work = {strips, per_strip, skinny_bands_log2(m, n, qk, strips, per_strip), rounds, rest / per_strip, rest % per_strip};
 #define RF_LAUNCH_SKINNY(QK)                                                                                            \
     hipLaunchKernelGGL(rf::gemm_fp8_blockscale_skinny<QK>, dim3(strips * per_strip), dim3(512),                         \
                        rf::SkinnyGeom<QK>::LDS_BYTES, stream, (const uint8_t *)a, (const uint8_t *)b, as, bs,           \
-                       (uint16_t *)c, m, n, per_strip, m_store)
+                       (uint16_t *)c, m, n, work, m_store)
         if (qk == 1) RF_LAUNCH_SKINNY(1);
         else if (qk == 2) RF_LAUNCH_SKINNY(2);
         else if (qk == 3) RF_LAUNCH_SKINNY(3);

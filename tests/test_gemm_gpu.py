@@ -282,6 +282,19 @@ def test_skinny_k_schedule_bit_exact(rfk, m, n, k):
     assert_close_to_oracle(out, oracle_bf16(noisy), RTOL, ATOL, "skinny K")
 
 
+@pytest.mark.parametrize("m,n,k", [(1040, 576, 384), (2128, 320, 256), (8000, 192, 512), (80, 8192, 256), (16, 8192, 384),
+                                   (48, 66048, 128), (8016, 5120, 128), (6001, 7168, 256), (7985, 5056, 256)])
+def test_skinny_k_bands_and_rounds_bit_exact(rfk, m, n, k):
+    """How the skinny-K schedule deals its work: bands of rows per XCD (1, 2, 4 and 8 of them, fewer shares of a strip than
+    bands, more strips than compute units), and from 40 million outputs on whole rounds of items with a rest, with rows of the
+    last item that C does not have. Exact data, bit for bit."""
+    data = exact_problem(m, n, k, seed=m + n + k)
+    cfg = rfk.GemmConfig(0, 1, 8, 4) if m % 16 == 0 else None
+    if cfg is None:
+        assert rfk.select_config(m, n, k).stream_k == 4
+    assert np.array_equal(bf16_bits(_run(rfk, data, config=cfg, canary=1024)), oracle_bf16(data))
+
+
 @pytest.mark.parametrize("m,n,k", [(64, 128, 256), (1024, 1536, 7168), (208, 576, 1024), (64, 1536, 7168), (1024, 512, 512),
                                    (208, 576, 768), (512, 3072, 1536), (128, 128, 384)])
 def test_k_split_inside_the_workgroup_equals_the_two_launch_form(rfk, m, n, k):
