@@ -753,8 +753,8 @@ __device__ __forceinline__ void exchange_tile_f32(f32x4 (&acc)[BM / WAVES_M / 16
 
 // ---------------------------------------------------------------------------------------------
 // One workgroup per (tile, K split). PARTIAL=false: writes bf16 C. PARTIAL=true: writes the fp32 partial sums of
-// the K range of split blockIdx.y to ws[split][M][N] (summed by reduce_splitk_bf16). M_store <= M is the number of
-// rows of bf16 C that exist (a caller whose M is not a multiple of 16 passes A padded to M rows and its own C).
+// the K range of split blockIdx.y to ws[split][M_store][N] (summed by reduce_splitk_bf16). M_store <= M is the number of
+// rows of C that exist (a caller whose M is not a multiple of 16 passes A padded to M rows and its own C).
 // Requirements checked by the host: M%16==0, N%16==0, M>=16, N>=16, a/b 16-byte aligned,
 // c 16-byte aligned, K%128==0.
 // ---------------------------------------------------------------------------------------------
@@ -774,8 +774,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_til
     f32x4 acc[G::TM][G::TN];
     tile_mainloop<BM, BN, WAVES_M, WAVES_N, NS>(A, B, SA, SB, M, M, N, m0, n0, kb_begin, kb_end, lds, acc);
     if constexpr (PARTIAL)
-        store_tile_f32_staged<BM, BN, WAVES_M, WAVES_N>(acc, (float *)Cout + ((size_t)blockIdx.y * M + m0) * N + n0, N,
-                                                        M - m0, N - n0, lds);
+        store_tile_f32_staged<BM, BN, WAVES_M, WAVES_N>(acc, (float *)Cout + ((size_t)blockIdx.y * M_store + m0) * N + n0, N,
+                                                        M_store - m0, N - n0, lds);
     else
         store_tile_bf16<BM, BN, WAVES_M, WAVES_N>(acc, (uint16_t *)Cout, M_store, N, m0, n0, lds);
 }
@@ -930,9 +930,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_str
 
 // Sum of split-K partials in split order 0..S-1, then one bf16 rounding
 // (the reference's reduce_kernel, src/gemm/gemm_kernel.cpp:288-303). 4 outputs per thread.
-// mn: elements of C; split_stride: elements between two splits in ws (>= mn: the partials may have more rows than C).
+// mn: elements of C, and of a split's partial sums in ws.
 __global__ __launch_bounds__(256) void reduce_splitk_bf16(const float *__restrict__ ws, uint16_t *__restrict__ C,
-                                                          size_t mn, int splits, size_t split_stride) {
+                                                          size_t mn, int splits) {
     size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= mn) return;
     const float *p = ws + i;
@@ -944,7 +944,7 @@ __global__ __launch_bounds__(256) void reduce_splitk_bf16(const float *__restric
     for (; q0 + BATCH <= splits; q0 += BATCH) {
         f32x4 v[BATCH];
 #pragma unroll
-        for (int q = 0; q < BATCH; q++) v[q] = *(const f32x4 *)(p + (size_t)(q0 + q) * split_stride);
+        for (int q = 0; q < BATCH; q++) v[q] = *(const f32x4 *)(p + (size_t)(q0 + q) * mn);
 #pragma unroll
         for (int q = 0; q < BATCH; q++) {
             s[0] += v[q][0]; s[1] += v[q][1]; s[2] += v[q][2]; s[3] += v[q][3];
@@ -954,7 +954,7 @@ __global__ __launch_bounds__(256) void reduce_splitk_bf16(const float *__restric
         f32x4 v[BATCH - 1];
 #pragma unroll
         for (int q = 0; q < BATCH - 1; q++)
-            if (q0 + q < splits) v[q] = *(const f32x4 *)(p + (size_t)(q0 + q) * split_stride);
+            if (q0 + q < splits) v[q] = *(const f32x4 *)(p + (size_t)(q0 + q) * mn);
 #pragma unroll
         for (int q = 0; q < BATCH - 1; q++)
             if (q0 + q < splits) {

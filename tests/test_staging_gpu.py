@@ -64,3 +64,29 @@ def test_every_tile_kernel_stores_into_any_c(tmp_path):
             rfk.clear_plans()
         assert np.array_equal(bf16_bits(buf[1:1 + m * n].view(m, n)), exp), variant
         assert float(buf[0]) == -7.0 and float(buf[1 + m * n:].float().min()) == -7.0 == float(buf[1 + m * n:].float().max())
+
+
+# 530 rows are planned as 544 and staged as 640 (whole lines) where that adds no tile: every schedule, K in one and in several
+# parts (whose sums are of the true rows only), tiles of 192 rows that 640 would need one more of; 520 rows need no more lines
+# with 64-row units than with 16; N = 500 (B staged, planned as 512 or 496)
+@pytest.mark.parametrize("m,n,k,plan", [(530, 512, 512, "3 1 8 0"), (530, 512, 512, "8 3 8 0"), (530, 512, 512, "5 1 8 0"),
+                                        (530, 512, 512, "28 4 8 0"), (530, 512, 512, "0 1 8 2"), (530, 512, 512, "0 1 8 4"),
+                                        (520, 512, 256, "0 1 8 4"), (530, 512, 512, "0 1 8 1"), (577, 500, 384, "10 1 8 0"),
+                                        (577, 490, 384, "8 1 8 0"), (577, 490, 384, "3 3 8 0"), (641, 130, 256, "28 1 8 0")])
+def test_staged_rows_of_whole_lines(tmp_path, m, n, k, plan):
+    import radeonflow_kernels_amd as rfk
+    data = exact_problem(m, n, k, seed=m + n)
+    exp = oracle_bf16(data)
+    g, buf = to_gpu(data, 300)
+    path = tmp_path / "p.plans"
+    path.write_text("%d %d %d %s\n" % ((m + 15) // 16 * 16, (n + 15) // 16 * 16, k, plan))
+    try:
+        assert rfk.load_plans(str(path)) == 1
+        for fill in (-1.0, 3.0):
+            g[4].fill_(fill)
+            rfk.fp8_mm(*g)
+            torch.cuda.synchronize()
+            assert np.array_equal(bf16_bits(g[4]), exp)
+    finally:
+        rfk.clear_plans()
+    assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
