@@ -993,7 +993,8 @@ __global__ __launch_bounds__(256) void reduce_splitk_bf16(const float *__restric
 // ---------------------------------------------------------------------------------------------
 constexpr int kMaxGroups = 256;
 struct GroupTable {
-    int row_start[kMaxGroups + 1];      // first row of each group in A and a_scale (multiples of 16)
+    int row_start[kMaxGroups + 1];      // first row of each group in A and a_scale (multiples of 16, each group's rows rounded
+                                        // up to one further on at least)
     int out_row_start[kMaxGroups + 1];  // first row of each group in C; the differences are the true row counts
     int tile_start[kMaxGroups + 1];     // prefix of work items (one per tile); tile_start[groups] is their number
 };
@@ -1024,8 +1025,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_gro
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     int grp, local;
     if (!grouped_work_item(table, groups, grp, local)) return;
-    const int row0 = table.row_start[grp], rows = table.row_start[grp + 1] - row0;
     const int out0 = table.out_row_start[grp], out_rows = table.out_row_start[grp + 1] - out0;
+    const int row0 = table.row_start[grp], rows = (out_rows + 15) / 16 * 16;      // A has all of them, see GroupTable
     const int tiles_m = (rows + BM - 1) / BM;
     const int m0 = (local % tiles_m) * BM, n0 = (local / tiles_m) * BN;
     const int QK = K / BK, QN = (N + 127) / 128;
@@ -1047,8 +1048,8 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_grouped_mixed(
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     int grp, local;
     if (!grouped_work_item(table, groups, grp, local)) return;
-    const int row0 = table.row_start[grp], rows = table.row_start[grp + 1] - row0;
     const int out0 = table.out_row_start[grp], out_rows = table.out_row_start[grp + 1] - out0;
+    const int row0 = table.row_start[grp], rows = (out_rows + 15) / 16 * 16;      // A has all of them, see GroupTable
     const int big_m = rows / 256 + (rows % 256 > 128 ? 1 : 0);       // 256-row tiles of this group
     const int tiles_m = rows / 256 + (rows % 256 > 0 ? 1 : 0);       // row tiles of either height
     const int tile_m = local % tiles_m, n0 = (local / tiles_m) * 256;
@@ -1137,8 +1138,8 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_grouped_queue(
                 if (table.tile_start[mid] <= item) lo = mid; else hi = mid;
             }
             const int grp = queues.order[lo], local = item - table.tile_start[lo];
-            const int row0 = table.row_start[grp], rows = table.row_start[grp + 1] - row0;
             const int out0 = table.out_row_start[grp], out_rows = table.out_row_start[grp + 1] - out0;
+            const int row0 = table.row_start[grp], rows = (out_rows + 15) / 16 * 16;
             const int full = rows / 256, rest = rows - full * 256;
             const int tiles_m = full + (rest > 0 ? 1 : 0);
             const int tile_m = local % tiles_m, n0 = (local / tiles_m) * 256, m0 = tile_m * 256;

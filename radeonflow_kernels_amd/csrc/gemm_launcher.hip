@@ -1821,11 +1821,19 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
         // into the staging buffer with every group starting at a multiple of 16, the kernel reads those and writes
         // each group's true rows straight into the caller's C. Costs one pass over A; the bounds-checked kernel
         // per group would be 10 to 30 times slower than the tiled one.
+        // Starts at a multiple of 128, whole cache lines (a tile's 128-byte pieces of A are then one line each, not two), where
+        // that makes the copy at most an eighth longer. us: 3623 rows in 8 groups, 7168 x 2048, 94.2 -> 88.4; 3077 in 16,
+        // 4096 x 7168, 167.0 -> 159.5; 1076 in 8, the same, 85.3 -> 81.9; a copy a fifth longer lost up to 2 %.
+        long by16 = 0, by128 = 0;
+        for (int g = 0; g < groups; g++) {
+            by16 += (row_offsets[g + 1] - row_offsets[g] + 15) / 16 * 16;
+            by128 += (long)ceil_div(row_offsets[g + 1] - row_offsets[g], 128) * 128;
+        }
+        const int unit = by128 * 8 <= by16 * 9 && by128 < (1L << 30) ? 128 : 16;
         int at = 0;
         for (int g = 0; g < groups; g++) {
             table.row_start[g] = at;
-            const int pr = (row_offsets[g + 1] - row_offsets[g] + 15) / 16 * 16;
-            at += pr;
+            at += ceil_div(row_offsets[g + 1] - row_offsets[g], unit) * unit;
         }
         for (int g = groups; g <= rf::kMaxGroups; g++) table.row_start[g] = at;
         for (int g = 0; g <= rf::kMaxGroups; g++) table.out_row_start[g] = row_offsets[g < groups ? g : groups];

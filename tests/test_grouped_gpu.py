@@ -107,6 +107,18 @@ def test_grouped_any_group_sizes_bit_exact(rfk, rows, n, k):
         _check_canary(g[5], g[4].numel())
 
 
+# staged with starts at multiples of 128 (2560 rows where multiples of 16 are 2336) and, the copy too much longer, of 16
+@pytest.mark.parametrize("rows", [[500, 370, 264, 250, 0, 897], [129, 0, 640, 385, 513], [500, 380, 280, 260, 900, 1, 1, 1, 1, 1]])
+def test_grouped_staged_on_whole_lines_bit_exact(rfk, rows):
+    g, offs, exp = _grouped_problem(rows, 272, 384, seed=77, exact=True)
+    for variant in (-1, 0, 1, 2, 3, 4, 5):
+        g[4].fill_(-3.0)
+        rfk.fp8_mm_grouped(*g[:5], offs, variant=variant)
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(g[4]), exp), "variant %d" % variant
+        _check_canary(g[5], g[4].numel())
+
+
 def test_grouped_any_group_sizes_quantised_data(rfk):
     rows, n, k = [77, 130, 1, 260, 45], 1024, 1024
     g, offs, exp = _grouped_problem(rows, n, k, seed=8, exact=False)
