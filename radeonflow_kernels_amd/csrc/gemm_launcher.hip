@@ -1569,8 +1569,13 @@ int launch_quantize(const void *x, int rows, int k, void *out, float *scales, hi
         if (rc != RF_OK) return rc;
     }
     if (PER_ROW && (double)rows * k <= kQuantRows16Elements) {
-        hipLaunchKernelGGL((rf::quantize_rows16<IN_BF16>), dim3(k / rf::BK, ceil_div(rows, 16)), dim3(256), 0, stream, x, rows, k,
-                           (uint8_t *)out, scales);
+        const int blocks = k / rf::BK;
+        if (blocks % rf::NUM_XCD != 0 && rows >= 128)
+            hipLaunchKernelGGL((rf::quantize_rows16<IN_BF16, true>), dim3(ceil_div(ceil_div(rows, 128) * blocks, rf::NUM_XCD) * 8 * rf::NUM_XCD),
+                               dim3(256), 0, stream, x, rows, k, (uint8_t *)out, scales);
+        else
+            hipLaunchKernelGGL((rf::quantize_rows16<IN_BF16, false>), dim3(blocks, ceil_div(rows, 16)), dim3(256), 0, stream, x, rows, k,
+                               (uint8_t *)out, scales);
         RF_HIP(hipGetLastError());
         return RF_OK;
     }

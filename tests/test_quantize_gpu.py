@@ -255,3 +255,15 @@ def test_outputs_are_allocated_through_the_dispatcher():
     with torch.inference_mode():
         q, s = rfk.quantize_a(x)
     assert q.is_inference() and s.is_inference()
+
+
+# numbers of K blocks that the eight XCDs do not divide: pieces dealt to them eight at a time; rows of one such unit, one piece
+# and one row more, fewer units than XCDs
+@pytest.mark.parametrize("rows,k", [(128, 128), (129, 384), (145, 1152), (1000, 2304), (2047, 640), (127, 384)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_pieces_dealt_to_the_xcds_match_the_oracle(rfk, rows, k, dtype):
+    x = torch.from_numpy(_source(rows, k, rows + k, "normal")).to(dtype)
+    a_ref, as_ref = cref.quantize_a(x.float().numpy())
+    a, a_scale = rfk.quantize_a(x.cuda())
+    assert np.array_equal(a.cpu().view(torch.uint8).numpy(), np.asarray(a_ref).view(np.uint8).reshape(k, rows).T)
+    assert np.array_equal(a_scale.cpu().numpy(), np.asarray(as_ref).reshape(k // 128, rows).T)
