@@ -565,7 +565,8 @@ constexpr int kFewRowsMaxM = 512, kFewRowsMaxMStagedB = 4096;
 // What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
 // (and of C on the way back). kTiledOnly: no few-rows plan.
 // kBytesA, kBytesB: rows of that operand do not all start at a multiple of four bytes.
-enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16 };
+// kFewRowsOnly: the few-rows plan (m and n as they are).
+enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16, kFewRowsOnly = 32 };
 
 // Estimated time in microseconds of the best any-alignment tile plan for a shape whose operands would have to be staged, and
 // that plan. Fitted (relative error, 6 %) to 640 plans of 100 random shapes on operand sets that stay in the Infinity Cache:
@@ -755,7 +756,8 @@ void select_config(int m, int n, int k, int num_cu, int stage, rf_gemm_config *o
     Entry &e = table[(h >> 7) % kEntries];
     if (e.m != m || e.n != n || e.k != k || e.num_cu != num_cu || e.stage != stage || e.generation != shared().plan_generation) {
         e = {m, n, k, num_cu, stage, shared().plan_generation, {}};
-        select_config_uncached(m, n, k, num_cu, stage, shared().user_plans, &e.cfg);
+        if (stage & kFewRowsOnly) fewrows_plan(m, n, k, num_cu, (stage & kStageB) != 0, &e.cfg);
+        else select_config_uncached(m, n, k, num_cu, stage, shared().user_plans, &e.cfg);
     }
     *out = e.cfg;
 }
@@ -898,7 +900,7 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         // a small problem the tiled kernels do not take (reported as plan -1: no tile variant): the few-rows kernels do. A wave
         // of the bounds-checked kernel gathers bytes K block after K block, 13 to 27 us where these take 3 to 4
         // (M x N x K = 4 x 200 x 2048: 27.8 -> 3.7, 8 x 1000 x 384: 13.6 -> 3.1).
-        fewrows_plan(m, n, k, s.num_cu, n % 16 != 0, &cfg);
+        select_config(m, n, k, s.num_cu, kFewRowsOnly | (n % 16 != 0 ? kStageB : 0), &cfg);
         if (!fewrows_split_fits(mem, kVariants[cfg.variant], m, n, k, cfg.split_k)) cfg.split_k = 1;
         return launch_fewrows(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, stream);
     }
