@@ -553,14 +553,17 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
     }
     return best;
 }
-// Rows up to which the few-rows kernels are considered; the second one where B (or C) needs staging, on devices with
-// kTunedOnCUs units only (others keep the first, and with it the plans of their padded shapes). The estimate is fitted up to
-// 512 rows and comes out 9 % low beyond. A staged B costs a tiled plan up to three launches, which variant 21 beats up to a
-// few thousand rows while N is small: few rows against the best of 25 tiled plans with their staging (fewrows_model.py
-// --meet), us: 1000 x 1000 x 1024 8.5, 15.8; 1500 x 1000 x 2048 17.6, 22.8; 3000 x 1000 x 384 11.0, 13.9; 700 x 5003 x 1024
-// 24.1, 21.3; 2000 x 2003 x 1024 24.4, 18.6. Only M ragged: tiled plans above 512 rows, also where a small N would have the
-// few-rows kernels ahead (1037 x 336 x 1024 11.8, few rows 7.0; but 1001 x 576 x 7168 22.0, few rows 24.0).
-constexpr int kFewRowsMaxM = 512, kFewRowsMaxMStagedB = 4096;
+// Rows up to which the few-rows kernels are considered; the second one where B (or C) needs staging or N is small, on devices
+// with kTunedOnCUs units only (others keep the first, and with it the plans of their padded shapes). The estimate is fitted up to
+// 512 rows and comes out 9 % low beyond, which is added where nothing but M can be ragged. A staged B costs a tiled plan up to
+// three launches, which variant 21 beats up to a few thousand rows while N is small: few rows against the best of 25 tiled plans
+// with their staging (fewrows_model.py --meet), us: 1000 x 1000 x 1024 8.5, 15.8; 1500 x 1000 x 2048 17.6, 22.8; 3000 x 1000 x 384
+// 11.0, 13.9; 700 x 5003 x 1024 24.1, 21.3; 2000 x 2003 x 1024 24.4, 18.6. A small N leaves most compute units without one of
+// the large tiles, so that those split K and sum in a second launch. Before -> with the few-rows kernels in the choice, us:
+// 528 x 256 x 2048 10.1 -> 7.7, 1833 x 256 x 2048 13.2 -> 9.1, 1919 x 512 x 2048 17.0 -> 11.6, 848 x 576 x 1024 7.9 -> 6.1,
+// 779 x 1024 x 1024 10.1 -> 7.7, 665 x 1536 x 384 6.4 -> 5.4; of 130 shapes with N = 200 ... 1536 and 513 to 4096 rows 27 are
+// faster by 2 to 47 %, none slower by more than the 2 % that runs differ by.
+constexpr int kFewRowsMaxM = 512, kFewRowsMaxMWide = 4096, kFewRowsSmallN = 1536;
 
 // What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
 // (and of C on the way back). kTiledOnly: no few-rows plan.
@@ -639,13 +642,19 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // rows 5.9 against 6.8 us, 4096 rows 12.3 against 13.8, 8192 rows 22.5 against 24.0; N = 7168, K = 384: 512 rows
     // 4.9 against 6.0, 6144 rows 25.7 against 31.8. With K = 512 and more than sixteen strips the tiled plans are as
     // fast or faster (N = 7168: 2048 rows 15.1 against 13.1 us, 6144 rows 30.6 against 30.4).
-    if (skinny_ok(m, n, k) &&
-        (k <= 2 * rf::BK ? (double)m * n >= 6.0e6
-                         : (double)m * n >= 2.0e6 && (k == 3 * rf::BK || ceil_div(n, 256) <= 16))) {
-        if (hit) return take(*hit);
-        out->variant = 0;
-        out->stream_k = RF_SCHEDULE_SKINNY_K;
-        return;
+    // Staged operands: it has to beat the tiles that take them as they are, see below.
+    const bool skinny = skinny_ok(m, n, k) &&
+                        (k <= 2 * rf::BK ? (double)m * n >= 6.0e6
+                                         : (double)m * n >= 2.0e6 && (k == 3 * rf::BK || ceil_div(n, 256) <= 16));
+    const bool staged = stage & (kStageA | kStageB);
+    if (skinny) {
+        if (hit) {
+            take(*hit);
+        } else {
+            out->variant = 0;
+            out->stream_k = RF_SCHEDULE_SKINNY_K;
+        }
+        if (!staged || num_cu != kTunedOnCUs) return;
     }
     // No measured entry: a cost model whose constants were searched on the tuner's measurements of the tabled shapes so
     // that its plan comes close to the best measured one. Searched on 213 shapes (the 163 of the table and 50 others,
@@ -677,7 +686,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     const int splits_tried[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int qk = k / rf::BK;
     double best_cost = 1e30;
-    for (const Candidate &cd : cands) {
+    if (!skinny) for (const Candidate &cd : cands) {
         const Variant &v = kVariants[cd.variant];
         const long tiles = (long)ceil_div(m, v.bm) * ceil_div(n, v.bn);
         for (int sp : splits_tried) {
@@ -730,10 +739,14 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     double t = 3.1 + 0.67 * best_cost;
     if (stage & kStageA) t += 3.2 + 2.0 * k * m / 4e6;
     if (stage & kStageB) t += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
+    // The skinny-K schedule behind a staging copy of A, fitted to 63 shapes of 321 to 8005 rows and N = 1024 ... 8192. With the
+    // estimate below the plan taken is the faster one on all of them, where 34 were up to 80 % slower: 570 x 4096 x 384 11.2 -> 6.2,
+    // 3003 x 1024 x 512 12.2 -> 7.8, 8005 x 1024 x 128 9.4 -> 7.2; 1318 x 8192 x 384 stays (13.8, the tiles 16.0).
+    if (skinny && !(stage & kStageB)) t = 7.2 + 0.9 * qk + (0.19 + 0.078 * qk) * 1e-6 * m * n;
     rf_gemm_config other;
-    const int max_m = (stage & kStageB) && num_cu == kTunedOnCUs ? kFewRowsMaxMStagedB : kFewRowsMaxM;
+    const int max_m = ((stage & kStageB) || n <= kFewRowsSmallN) && num_cu == kTunedOnCUs ? kFewRowsMaxMWide : kFewRowsMaxM;
     if (m <= max_m && fewrows_ok(m, n) && !(stage & kTiledOnly)) {
-        const double few = fewrows_plan(m, n, k, num_cu, (stage & kStageB) != 0, &other);
+        const double few = fewrows_plan(m, n, k, num_cu, (stage & kStageB) != 0, &other) * (m > kFewRowsMaxM && !(stage & kStageB) ? 1.09 : 1.0);
         if (few < t) {
             t = few;
             *out = other;
@@ -1261,6 +1274,8 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
             const Variant &v = kVariants[cfg.variant];
             const size_t fit = mem.fixed_left() / fewrows_slot_bytes(v, m, n, 1);
             if ((size_t)cfg.split_k > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;
+        } else if (!fewrows_split_fits(mem, kVariants[cfg.variant], m, n, k, cfg.split_k)) {
+            cfg.split_k = 1;                               // no memory for the sums: K in one part
         }
         return launch_fewrows(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, stream);
     }

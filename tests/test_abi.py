@@ -346,3 +346,17 @@ def test_benchmark_hashes_every_gemm_source():
             todo += [os.path.basename(x) for x in re.findall(r'#include "([^"]+\.h)"', open(os.path.join(csrc, name)).read())
                      if os.path.dirname(x) == ""]
     assert sorted(bench.KERNEL_SOURCES) == sorted(reached - {"quantize_kernels.h"})
+
+
+def test_few_rows_plans_for_a_small_n_and_any_tiles_instead_of_a_staged_skinny_k():
+    """Up to 4096 rows the few-rows kernels (variants 14 to 27) are in the choice while N is small; the skinny-K schedule behind a
+    staging copy gives way to the tiles that take ragged operands (29, 30) where those fill about one round. Both on 256 units."""
+    import radeonflow_kernels_amd as rfk
+    few = lambda *a: 14 <= rfk.plan_for(*a).variant <= 27
+    assert few(528, 256, 2048, 256) and few(1833, 256, 2048, 256) and few(848, 576, 1024, 256) and few(665, 1536, 384, 256)
+    assert not few(1833, 256, 2048, 304) and not few(4112, 256, 2048, 256) and not few(1040, 2048, 2048, 256)
+    skinny = lambda *a: rfk.plan_for(*a).stream_k == 4
+    for m, n, k in ((570, 4096, 384), (3003, 1024, 512), (8005, 1024, 128), (843, 7168, 256)):
+        assert rfk.plan_for(m, n, k, 256).variant in (29, 30) and skinny(m, n, k, 304)
+        assert not rfk.plan_for((m + 15) // 16 * 16, n, k, 256).variant in (29, 30)
+    assert skinny(1318, 8192, 384, 256) and skinny(5005, 7168, 256, 256)

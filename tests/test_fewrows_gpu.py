@@ -277,3 +277,18 @@ def test_stores_into_any_c_keep_nans_and_infinities(rfk, tmp_path):
         finally:
             rfk.clear_plans()
         _assert_same_values_and_nans(c, exp, nan, variant)
+
+
+@pytest.mark.parametrize("m,n,k", [(513, 256, 2048), (1833, 256, 2048), (848, 576, 1024), (665, 1536, 384), (2500, 256, 2048)])
+def test_fewrows_as_the_plan_of_many_rows(rfk, m, n, k):
+    """More than 512 rows and a small N: the automatic plan is a few-rows kernel, with the oracle's bits from both entries."""
+    assert 14 <= rfk.select_config(m, n, k).variant <= 27
+    data = exact_problem(m, n, k, seed=m)
+    exp = oracle_bf16(data)
+    g, buf = to_gpu(data, 300)
+    for call in (rfk.fp8_mm, rfk.fp8_mm_static):
+        g[4].fill_(-1.0)
+        call(*g)
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(g[4]), exp)
+    assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
