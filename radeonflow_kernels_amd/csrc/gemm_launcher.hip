@@ -635,18 +635,23 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
         for (const TunedPlan &p : kTunedPlans)
             if (!hit && usable(p)) hit = &p;
     if (hit && (!(stage & (kStageA | kStageB)) || kVariants[hit->variant].takes_any_shape())) return take(*hit);
-    // Up to four K blocks and a large C: the launch is a streaming store, which the skinny-K schedule does best
-    // (measured against the best tiled plan at N = 7168, K = 256: 1024 rows 6.5 against 6.9 us, 2048 rows 7.8 against
-    // 10.3, 6144 rows 18.2 against 22.1; below about six million outputs the 64 x 128 tiles win, e.g. 2048 x 2048: 6.5
-    // against 5.6 us). Three and four K blocks (items of 64 rows): from two million outputs on; N = 4096, K = 512: 1024
-    // rows 5.9 against 6.8 us, 4096 rows 12.3 against 13.8, 8192 rows 22.5 against 24.0; N = 7168, K = 384: 512 rows
-    // 4.9 against 6.0, 6144 rows 25.7 against 31.8. With K = 512 and more than sixteen strips the tiled plans are as
-    // fast or faster (N = 7168: 2048 rows 15.1 against 13.1 us, 6144 rows 30.6 against 30.4).
-    // Staged operands: it has to beat the tiles that take them as they are, see below.
-    const bool skinny = skinny_ok(m, n, k) &&
-                        (k <= 2 * rf::BK ? (double)m * n >= 6.0e6
-                                         : (double)m * n >= 2.0e6 && (k == 3 * rf::BK || ceil_div(n, 256) <= 16));
+    // Up to four K blocks and a large C: the launch is a streaming store, which the skinny-K schedule does best. Against the best
+    // tiled plan, us: K = 128, 592 x 7168 5.1, 5.4 and 1328 x 4096 5.8, 6.5, but 592 x 4096 (2.4 million outputs) 4.4, 3.9; K = 256,
+    // 848 x 7168 6.2, 6.8 and 2016 x 3072 5.9, 7.0, but 592 x 7168 6.3, 6.3 and 2048 x 2048 6.5, 5.6; K = 384, 1328 x 3072 6.3, 6.9
+    // and 848 x 7168 7.3, 7.7. With K = 512 and more than sixteen strips the tiles are as fast or faster up to 20 million outputs
+    // (2016 x 7168 13.5, 13.3) and again beyond 60 (8048 x 8192 57.5, 54.2; between them 3008 x 7168 18.7, 20.8). Three or four K blocks whose C is one
+    // round of 128 x 128 tiles: those (variant 28), 592 x 4096 x 512 7.7 -> 6.3, 1328 x 2048 x 512 7.2 -> 6.7, 848 x 4096 x 384 6.9 -> 6.2,
+    // 3008 x 576 x 512 6.7 -> 6.1; 336 x 7168 x 384 5.7, 5.8.
+    // Staged operands: the schedule has to beat the tiles that take them as they are, see below.
+    const double mn = (double)m * n;
+    const int qk = k / rf::BK;
     const bool staged = stage & (kStageA | kStageB);
+    const int tiles_128 = ceil_div(m, 128) * ceil_div(n, 128);
+    const bool one_round = !staged && num_cu == kTunedOnCUs && (qk == 3 || qk == 4) && tiles_128 <= num_cu && tiles_128 >= 96 &&
+                           (qk == 4 || mn >= 2.0e6);
+    const bool skinny = !one_round && skinny_ok(m, n, k) &&
+                        (qk == 1 ? mn >= 4.1e6 : qk == 2 ? mn >= 6.0e6 : mn >= 2.0e6 && (qk == 3 || ceil_div(n, 256) <= 16));
+    if (one_round) out->variant = 28;
     if (skinny) {
         if (hit) {
             take(*hit);
@@ -684,9 +689,8 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
                                {13, 1.06, 3.3}, {28, 0.44, 2.25}};
     const double f_next = 3.3, reduce_fixed = 6.03, reduce_per_elem = 1.27e-6, c_half_tile = 0.47, f_half_tile = 5.2;
     const int splits_tried[] = {1, 2, 3, 4, 6, 8, 12, 16};
-    const int qk = k / rf::BK;
     double best_cost = 1e30;
-    if (!skinny) for (const Candidate &cd : cands) {
+    if (!skinny && !one_round) for (const Candidate &cd : cands) {
         const Variant &v = kVariants[cd.variant];
         const long tiles = (long)ceil_div(m, v.bm) * ceil_div(n, v.bn);
         for (int sp : splits_tried) {
@@ -742,7 +746,8 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // The skinny-K schedule behind a staging copy of A, fitted to 63 shapes of 321 to 8005 rows and N = 1024 ... 8192. With the
     // estimate below the plan taken is the faster one on all of them, where 34 were up to 80 % slower: 570 x 4096 x 384 11.2 -> 6.2,
     // 3003 x 1024 x 512 12.2 -> 7.8, 8005 x 1024 x 128 9.4 -> 7.2; 1318 x 8192 x 384 stays (13.8, the tiles 16.0).
-    if (skinny && !(stage & kStageB)) t = 7.2 + 0.9 * qk + (0.19 + 0.078 * qk) * 1e-6 * m * n;
+    if (skinny && !(stage & kStageB)) t = 7.2 + 0.9 * qk + (0.19 + 0.078 * qk) * 1e-6 * mn;
+    if (one_round) t = 3.0 + 0.6 * qk + 0.36e-6 * mn;       // fitted to 32 shapes, 3 %
     rf_gemm_config other;
     const int max_m = ((stage & kStageB) || n <= kFewRowsSmallN) && num_cu == kTunedOnCUs ? kFewRowsMaxMWide : kFewRowsMaxM;
     if (m <= max_m && fewrows_ok(m, n) && !(stage & kTiledOnly)) {

@@ -360,3 +360,13 @@ def test_few_rows_plans_for_a_small_n_and_any_tiles_instead_of_a_staged_skinny_k
         assert rfk.plan_for(m, n, k, 256).variant in (29, 30) and skinny(m, n, k, 304)
         assert not rfk.plan_for((m + 15) // 16 * 16, n, k, 256).variant in (29, 30)
     assert skinny(1318, 8192, 384, 256) and skinny(5005, 7168, 256, 256)
+
+
+def test_short_k_plans_by_the_shape_of_the_output():
+    """K of three and four blocks: 128 x 128 tiles with eight waves where they are one round of 256 units, the skinny-K schedule
+    beyond; one K block: the skinny-K schedule from 4.1 million outputs on."""
+    import radeonflow_kernels_amd as rfk
+    plan = lambda m, n, k, cu=256: (lambda c: "skinny" if c.stream_k == 4 else c.variant)(rfk.plan_for(m, n, k, cu))
+    assert plan(592, 4096, 512) == plan(848, 4096, 384) == plan(592, 3072, 512) == 28
+    assert plan(1168, 4096, 512) == "skinny" and plan(592, 4096, 512, 304) == "skinny"      # 320 tiles; another device
+    assert plan(592, 7168, 128) == "skinny" and plan(560, 7168, 128) != "skinny" and plan(592, 7168, 256) != "skinny"
