@@ -103,7 +103,7 @@ struct Variant {
 // less than a load takes to come back from L2 or the Infinity Cache on a busy chip, so with two stages the loop ran at
 // the latency of its loads: 1024 x 4608 x 7168 45.6 -> 39.0 us, 256 x 7168 x 2304 15.6 -> 13.1 us; the plan of 50
 // of the 163 tabled shapes. The two-stage forms stay: they fit more workgroups per CU (64 x 128: three instead of
-// two), which the smallest problems prefer. (128 x 128 with three stages never won and is not built.)
+// two), which the smallest problems prefer. (128 x 128 with four waves and three stages never won; with eight it is variant 28.)
 #define RF_VARIANT_TILE_ONLY_NS3(BM, BN, WM, WN)                                           \
     Variant { BM, BN, WM, WN, rf::TileGeom<BM, BN, WM, WN, 3>::LDS_BYTES,                  \
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, false, 3>,                      \
@@ -1038,9 +1038,11 @@ constexpr double kPadThresholdMacs = 2097152.0;
 // pieces of kPadRows rows when rows are longer), and every thread finds its group by a search in LDS instead of a walk
 // over the kernel argument. A source piece starts at any byte and is one unaligned 16-byte load, cut at the end of the matrix.
 // 1001 x 7168 bytes: 7.7 -> 6.8 us (rocprofv3), 48 rows in 32 groups x 7168: 10.6 -> 5.8 us, 2.8 us of either being what
-// the shortest kernel takes; two rounds instead of four, so twice the workgroups: 601x3072x1536 14.3 -> 13.3 us.
-constexpr int kPadRows = 2;
-template <typename T>
+// the shortest kernel takes. One round up to kPadOneRound bytes, whose workgroups hardly fill the chip, two beyond: the GEMM with
+// its copy in two rounds -> one, us: 701 x 7168 x 2048 26.4 -> 25.7, 3001 x 7168 x 256 16.7 -> 16.0, 1990 x 2048 x 2048 21.8 -> 21.4;
+// even at 1001 x 4608 x 7168 (7.3 MB), but 5001 x 7168 x 2048 (10.5 MB) 86.3 -> 87.2. (Four rounds: up to 5 % slower.)
+constexpr double kPadOneRound = 8.0e6;
+template <typename T, int kPadRows>
 __device__ __forceinline__ void pad_group_rows_body(const T *__restrict__ src, int first, int m_total, int m_pad, int rows,
                                                     int groups, T *__restrict__ dst, const rf::GroupTable &table,
                                                     int block_row, int block_chunk) {
@@ -1108,22 +1110,23 @@ __device__ __forceinline__ void pad_group_rows_body(const T *__restrict__ src, i
     }
 }
 
-template <typename T>
+template <typename T, int kPadRows>
 __global__ __launch_bounds__(256) void pad_group_rows(const T *__restrict__ src, int m_total, int m_pad, int rows,
                                                       int groups, T *__restrict__ dst, const rf::GroupTable table) {
-    pad_group_rows_body<T>(src, 0, m_total, m_pad, rows, groups, dst, table, blockIdx.x, blockIdx.y);
+    pad_group_rows_body<T, kPadRows>(src, 0, m_total, m_pad, rows, groups, dst, table, blockIdx.x, blockIdx.y);
 }
 
 // A and a_scale in one launch (they are staged together whenever M or the group sizes are ragged): the first
 // blocks_a workgroups along x copy the bytes of A, the others the floats of a_scale.
+template <int kPadRows>
 __global__ __launch_bounds__(256) void pad_group_rows_a_and_scales(const uint8_t *__restrict__ a, const float *__restrict__ as,
                                                                    int first, int m_total, int m_pad, int k, int groups,
                                                                    uint8_t *__restrict__ a_dst, float *__restrict__ as_dst,
                                                                    int blocks_a, const rf::GroupTable table) {
     if ((int)blockIdx.x < blocks_a)
-        pad_group_rows_body<uint8_t>(a, first, m_total, m_pad, k, groups, a_dst, table, blockIdx.x, blockIdx.y);
+        pad_group_rows_body<uint8_t, kPadRows>(a, first, m_total, m_pad, k, groups, a_dst, table, blockIdx.x, blockIdx.y);
     else
-        pad_group_rows_body<float>(as, first, m_total, m_pad, k / rf::BK, groups, as_dst, table, blockIdx.x - blocks_a,
+        pad_group_rows_body<float, kPadRows>(as, first, m_total, m_pad, k / rf::BK, groups, as_dst, table, blockIdx.x - blocks_a,
                                    blockIdx.y);
 }
 
@@ -1154,7 +1157,7 @@ dim3 pad_grid_of_pieces(int pieces, int rows, int rounds) {
     const int per_block = rounds * (pieces < 256 ? 256 / pieces : 1);
     return dim3((unsigned)ceil_div(rows, per_block), (unsigned)ceil_div(pieces, 256));     // rows on x: no 65535 limit
 }
-dim3 pad_grid(int m_pad, int size, int rows) { return pad_grid_of_pieces(m_pad / (16 / size), rows, kPadRows); }
+dim3 pad_grid(int m_pad, int size, int rows, int rounds) { return pad_grid_of_pieces(m_pad / (16 / size), rows, rounds); }
 
 void launch_unpad_rows(const void *src, int ld, int n, int rows, void *dst, hipStream_t stream) {
     hipLaunchKernelGGL(unpad_rows_bf16, pad_grid_of_pieces(ceil_div(n, 8), rows, 1), dim3(256), 0, stream, (const uint16_t *)src,
@@ -1164,8 +1167,10 @@ void launch_unpad_rows(const void *src, int ld, int n, int rows, void *dst, hipS
 // Stages A and a_scale with one launch: columns first, first + 1, ... of matrices of m_total columns.
 void launch_pad_a_and_scales(const void *a, const float *as, int first, int m_total, int m_pad, int k, int groups,
                              uint8_t *a_dst, float *as_dst, const rf::GroupTable &table, hipStream_t stream) {
-    const dim3 ga = pad_grid(m_pad, 1, k), gs = pad_grid(m_pad, 4, k / rf::BK);
-    hipLaunchKernelGGL(pad_group_rows_a_and_scales, dim3(ga.x + gs.x, ga.y > gs.y ? ga.y : gs.y), dim3(256), 0, stream,
+    const bool one = (double)m_pad * k <= kPadOneRound;
+    const dim3 ga = pad_grid(m_pad, 1, k, one ? 1 : 2), gs = pad_grid(m_pad, 4, k / rf::BK, one ? 1 : 2);
+    const auto kernel = one ? &pad_group_rows_a_and_scales<1> : &pad_group_rows_a_and_scales<2>;
+    hipLaunchKernelGGL(kernel, dim3(ga.x + gs.x, ga.y > gs.y ? ga.y : gs.y), dim3(256), 0, stream,
                        (const uint8_t *)a, as, first, m_total, m_pad, k, groups, a_dst, as_dst, (int)ga.x, table);
 }
 
@@ -1179,6 +1184,14 @@ rf::GroupTable one_group(int cols, int cols_pad) {
         t.tile_start[g] = 0;
     }
     return t;
+}
+
+// Stages one matrix of K rows of `cols` bytes.
+void launch_pad_bytes(const void *src, int cols, int cols_pad, int k, uint8_t *dst, hipStream_t stream) {
+    const bool one = (double)cols_pad * k <= kPadOneRound;
+    const auto kernel = one ? &pad_group_rows<uint8_t, 1> : &pad_group_rows<uint8_t, 2>;
+    hipLaunchKernelGGL(kernel, pad_grid(cols_pad, 1, k, one ? 1 : 2), dim3(256), 0, stream, (const uint8_t *)src, cols, cols_pad, k, 1,
+                       dst, one_group(cols, cols_pad));
 }
 
 // rf_fp8_gemm_static on a ragged or unaligned shape whose staging copies do not fit the static array as a whole: the
@@ -1213,8 +1226,7 @@ int launch_padded_in_pieces(State &s, Mem &mem, const void *a, const void *b, co
         uint8_t *pb = nullptr;
         rc = mem.pad(b_bytes, &pb);
         if (rc != RF_OK) return rc;
-        hipLaunchKernelGGL(pad_group_rows<uint8_t>, pad_grid(np, 1, k), dim3(256), 0, stream, (const uint8_t *)b, n, np, k, 1,
-                           pb, one_group(n, np));
+        launch_pad_bytes(b, n, np, k, pb, stream);
         RF_HIP(hipGetLastError());
         b2 = pb;
     }
@@ -1315,13 +1327,11 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
         a2 = pad + off_a;
         as2 = (const float *)(pad + off_sa);
     } else if (copy_a) {                                   // M is fine, only the pointer is not aligned
-        hipLaunchKernelGGL(pad_group_rows<uint8_t>, pad_grid(mp, 1, k), dim3(256), 0, stream, (const uint8_t *)a, m, mp, k, 1,
-                           pad + off_a, one_group(m, mp));
+        launch_pad_bytes(a, m, mp, k, pad + off_a, stream);
         a2 = pad + off_a;
     }
     if (copy_b) {
-        hipLaunchKernelGGL(pad_group_rows<uint8_t>, pad_grid(np, 1, k), dim3(256), 0, stream, (const uint8_t *)b, n, np, k, 1,
-                           pad + off_b, one_group(n, np));
+        launch_pad_bytes(b, n, np, k, pad + off_b, stream);
         b2 = pad + off_b;
     }
     if (copy_c) c2 = pad + off_c;
