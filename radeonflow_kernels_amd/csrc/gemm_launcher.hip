@@ -21,6 +21,7 @@
 #include "fp8_gemm_skinny.h"
 #include "fp8_gemm_fewrows.h"
 #include "fp8_gemm_any.h"
+#include "plan_limits.h"
 #include "quantize_kernels.h"
 
 // Scratch memory of rf_fp8_gemm_static, the entry point that allocates nothing: split-K partial sums and staging
@@ -453,10 +454,8 @@ bool tiled_path_ok(const void *a, const void *b, const void *c, int m, int n) {
            ((uintptr_t)c % 16) == 0;
 }
 
-// (K * M and K * N below 2^32: the persistent kernel keeps a load cursor's K position in 32-bit per-lane offsets)
 bool persistent_ok(const Variant &v, int m, int n, int k) {
-    return v.persistent && m >= v.bm && m % 16 == 0 && n % v.bn == 0 && (k / rf::BK) % 2 == 0 &&
-           (unsigned long long)k * m < (1ull << 32) && (unsigned long long)k * n < (1ull << 32);
+    return v.persistent && m >= v.bm && m % 16 == 0 && n % v.bn == 0 && (k / rf::BK) % 2 == 0 && rf::persistent_offsets_fit(m, n, k);
 }
 
 // Persistent schedule that finishes the last, partial round with half tiles: one workgroup per CU, at least one whole
@@ -876,7 +875,7 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
                 return fail(RF_ERR_BAD_CONFIG, "stream_k needs at least as many tiles as compute units");
         } else if (cfg.stream_k == RF_SCHEDULE_PERSISTENT) {
             if (!persistent_ok(kVariants[cfg.variant], m, n, k))
-                return fail(RF_ERR_BAD_CONFIG, "the persistent schedule needs M >= the tile height, M % 16 == 0, N a multiple of the tile width and K/128 even");
+                return fail(RF_ERR_BAD_CONFIG, "the persistent schedule needs M >= the tile height, M % 16 == 0, N a multiple of the tile width, K/128 even, and K * M and K * N below 2^32");
         } else if (cfg.stream_k == RF_SCHEDULE_PERSISTENT_HALF_TAIL) {
             if (!half_tail_ok(kVariants[cfg.variant], m, n, k, s.num_cu))
                 return fail(RF_ERR_BAD_CONFIG, "the half-tile schedule needs the 256x256 tile, the persistent schedule's "
@@ -1301,14 +1300,14 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
                        cfg.variant >= 0 && kVariants[cfg.variant].any_c;
     const bool copy_c = !any_c && (np != n || (uintptr_t)c % 16 != 0 || (mp != m && cfg.stream_k == RF_SCHEDULE_STREAM_K));
     if (!mem.fixed && !copy_c && cfg.variant >= 0) {
-        // The staged rows become whole cache lines where that adds no tile: a row of a tile is then one or two lines, and not
-        // one more. Rows of A of 1024 bytes instead of 1008 (N x K = 4608 x 7168), of B of 4608 instead of 4592, us: 128 x 192
-        // tiles 41.4 -> 39.6, 128 x 256 46.5 -> 43.4 and 45.2 -> 43.4, 128 x 128 61.7 -> 57.7 and 63.4 -> 57.7; 256 x 256,
-        // 2032 rows, 74.5 -> 72.2 and 78.7 -> 72.2.
-        auto lines = [](int x, int tile) { return ceil_div(ceil_div(x, 128) * 128, tile) == ceil_div(x, tile) ? ceil_div(x, 128) * 128 : x; };
+        // The staged rows become whole cache lines where that adds no tile and the schedule still holds (staged_length): a row of
+        // a tile is then one or two lines, and not one more. Rows of A of 1024 bytes instead of 1008 (N x K = 4608 x 7168), of B of
+        // 4608 instead of 4592, us: 128 x 192 tiles 41.4 -> 39.6, 128 x 256 46.5 -> 43.4 and 45.2 -> 43.4, 128 x 128 61.7 -> 57.7 and
+        // 63.4 -> 57.7; 256 x 256, 2032 rows, 74.5 -> 72.2 and 78.7 -> 72.2.
         const Variant &v = kVariants[cfg.variant];
-        if (copy_a && copy_sa) mp = lines(mp, cfg.stream_k == RF_SCHEDULE_SKINNY_K ? 64 : v.bm);
-        if (copy_b && any_c) np = lines(np, v.bn);
+        const bool persistent = cfg.stream_k == RF_SCHEDULE_PERSISTENT || cfg.stream_k == RF_SCHEDULE_PERSISTENT_HALF_TAIL;
+        if (copy_a && copy_sa) mp = rf::staged_length(mp, cfg.stream_k == RF_SCHEDULE_SKINNY_K ? 64 : v.bm, np, k, persistent);
+        if (copy_b && any_c) np = rf::staged_length(np, v.bn, mp, k, false);      // (any_c: one workgroup per tile)
     }
     size_t off = 0;
     const size_t off_a = off;  off += copy_a ? align((size_t)k * mp) : 0;
