@@ -1086,7 +1086,7 @@ __global__ __launch_bounds__(512) void gemm_fp8_blockscale_grouped_mixed(
 // exactly once per queue, so the counter's last draw wraps it back to zero: the counters need no clearing between
 // launches (launches that share counters must not overlap).
 // In the table of this kernel tile_start[p] counts the items of the first p groups of the line.
-// stream: the launch's weights are more than the Infinity Cache keeps (the host's kStreamBytes). Those of a group with one
+// stream: the launch's weights leave the Infinity Cache little room (grouped_weights_streamed). Those of a group with one
 // row tile are then read once and by one workgroup, and their loads say so (nt): without the hint each of them evicts
 // something from the Infinity Cache. 2000 rows in 32 groups, 4096 x 7168: 229 -> 215 us, 4000 in 64, 2048 x 7168: 240 -> 225,
 // 8192 in 32: 358 -> 355. (The hint on every item: 351 there, but 8000 rows in 32 groups at 7168 x 2048 182 -> 190, where two

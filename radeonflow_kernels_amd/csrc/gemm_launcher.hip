@@ -1630,7 +1630,7 @@ struct GroupedVariant {
                          // rows; the queue form: 64, 128, 192 or 256 rows)
     bool queue = false;  // resident workgroups that take tiles from per-XCD queues (gemm_fp8_blockscale_grouped_queue)
     bool fewrows = false;  // fp8_gemm_fewrows.h: groups may start at any row of a
-    grouped_kernel_t streamed = nullptr;   // few-rows strips: the kernel for more weights than kStreamBytes
+    grouped_kernel_t streamed = nullptr;   // few-rows strips: the kernel whose weights carry the non-temporal hint
     // row tiles of a group of `rows` rows
     int tiles_m(int rows) const {
         if (!mixed) return ceil_div(rows, bm);
@@ -1656,11 +1656,6 @@ const GroupedVariant kGroupedVariants[] = {
     GroupedVariant{16, 64, 512, 8 * rf::BK * 16 * 5, rf::gemm_fp8_blockscale_grouped_ksplit<1, 4, 8, 1, 4>, false, false, true},   // 9: 16 rows, K split between eight waves
     RF_GROUPED_STRIPS(1, 4, 1, 2)};   // 10: 16 rows, four waves
 constexpr int kGroupedMixed = 4, kGroupedQueue = 5, kGroupedFewRows = 6;
-// Weights (of the groups that have rows) from which on they are read with the non-temporal hint: three quarters of the
-// Infinity Cache's 256 MB, which then cannot hold them from one call to the next beside everything else, and which the
-// hint keeps for other data. us, strips: 25 groups of 2048 x 7168 (367 MB) 72.5 -> 67.2, 16 of 4096 x 7168 (470 MB) 85.4 ->
-// 76.2, 30 of 4096 x 2048 (252 MB) 48.3 -> 44.1; but 8 of 4096 x 2048 (67 MB), which stay in the cache, 15.9 -> 18.2.
-constexpr double kStreamBytes = 192.0 * (1 << 20);
 // Estimated time of a 256-column tile of the queue form by its height in units of 64 rows, relative to a 256-row tile
 constexpr double kQueueTileCost[5] = {0.0, 0.68, 0.75, 0.97, 1.0};
 constexpr int kNumGroupedVariants = sizeof(kGroupedVariants) / sizeof(kGroupedVariants[0]);
@@ -1904,7 +1899,7 @@ int grouped_gemm(const void *a, const void *b, const float *as, const float *bs,
         tiles += v.tiles_m(row_offsets[g + 1] - row_offsets[g]) * tiles_n;
         busy += row_offsets[g + 1] > row_offsets[g];
     }
-    const bool stream_b = (double)busy * n * k > kStreamBytes;
+    const bool stream_b = rf::grouped_weights_streamed((double)busy * n * k, v.queue, v.bn);
     for (int g = groups; g <= rf::kMaxGroups; g++) table.tile_start[g] = tiles;
     if (v.queue) {
         // The line of items and its eight pieces. Estimated time of a group = column tiles x (256-row tiles + what

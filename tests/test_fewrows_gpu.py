@@ -143,11 +143,11 @@ def test_grouped_fewrows_bits_of_the_tiled_form(rfk, rows, n, k, shift):
         assert np.array_equal(launch(rfk.fp8_mm_grouped_padded, a_pad.view(fp8).T, sa_pad.T, variant), expect), variant
 
 
-# more weights than the Infinity Cache keeps (read with the non-temporal hint): groups of at most 16 rows for the strips, of up
-# to 300 for the queue's tiles of four heights and of one and two row tiles; a partial last strip of any width, an odd number of
-# K blocks; without the last eighteen groups, the same forms without the hint
+# groups of at most 16 rows for the strips, of up to 300 for the queue's tiles of four heights and of one and two row tiles; a
+# partial last strip of any width, an odd number of K blocks. Weights of the groups that have rows: 328 MB for the strips and 369
+# for the queue (both read with the non-temporal hint), 197 (without) and 221 (with it), 82 and 90 (both without)
 @pytest.mark.parametrize("variants,rows", [((6, 7, 8, 10, -1), [1, 0, 16, 7, 3]), ((5,), [64, 0, 300, 65, 130, 200, 256, 1, 257, 20])])
-@pytest.mark.parametrize("groups", [30, 12])
+@pytest.mark.parametrize("groups", [50, 30, 12])
 def test_grouped_streamed_weights_bits_of_the_tiled_form(rfk, variants, rows, groups):
     n, k, fp8 = 2064, 3968, torch.float8_e4m3fn
     rows = (rows * groups)[:groups]
