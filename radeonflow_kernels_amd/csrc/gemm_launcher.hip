@@ -769,8 +769,7 @@ void select_config(int m, int n, int k, int num_cu, int stage, rf_gemm_config *o
     struct Entry { int m, n, k, num_cu, stage, generation; rf_gemm_config cfg; };
     constexpr unsigned kEntries = 1024;
     static Entry table[kEntries];                           // zeroed: no entry has k == 0
-    const unsigned h = ((unsigned)m * 2654435761u) ^ ((unsigned)n * 2246822519u) ^ ((unsigned)k * 3266489917u) ^ (unsigned)(stage * 668265263);
-    Entry &e = table[(h >> 7) % kEntries];
+    Entry &e = table[rf::plan_slot(m, n, k, stage, kEntries)];
     if (e.m != m || e.n != n || e.k != k || e.num_cu != num_cu || e.stage != stage || e.generation != shared().plan_generation) {
         e = {m, n, k, num_cu, stage, shared().plan_generation, {}};
         if (stage & kFewRowsOnly) fewrows_plan(m, n, k, num_cu, (stage & kStageB) != 0, &e.cfg);

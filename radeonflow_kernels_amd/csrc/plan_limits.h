@@ -1,5 +1,5 @@
 // Rules of the launcher that look at sizes only: what a schedule holds for, how long the rows of a staged operand may become
-// under it, and which weights are read with the non-temporal hint. Host code.
+// under it, which weights are read with the non-temporal hint, and where a plan is remembered. Host code.
 #pragma once
 
 namespace rf {
@@ -33,6 +33,12 @@ constexpr int staged_length(int x, int tile, int other, int k, bool persistent) 
 //     smaller ones not measured.
 constexpr bool grouped_weights_streamed(double bytes, bool queue, int columns) {
     return bytes > (queue ? 192.0 * (1 << 20) : columns > 256 ? 256.0 * (1 << 20) : 290.0e6);
+}
+
+// Slot of a shape in the table of plans already worked out (a power of two of them, up to 2^25). All products unsigned: `stage` has
+// six bits, and as an int its product overflowed from 4 on.
+constexpr unsigned plan_slot(int m, int n, int k, int stage, unsigned entries) {
+    return ((((unsigned)m * 2654435761u) ^ ((unsigned)n * 2246822519u) ^ ((unsigned)k * 3266489917u) ^ ((unsigned)stage * 668265263u)) >> 7) % entries;
 }
 
 }  // namespace rf

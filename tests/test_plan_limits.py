@@ -58,3 +58,13 @@ def test_weights_the_infinity_cache_can_hold_are_read_without_the_hint(limits):
             assert limits.streamed(groups * n * k, 0, columns) == want, (groups, n, k)
     assert limits.streamed(33 * 4096 * 2048, 0, 512) == 1 and limits.streamed(32 * 4096 * 2048, 0, 512) == 0
     assert limits.streamed(26 * 4096 * 2048, 1, 256) == 1 and limits.streamed(23 * 4096 * 2048, 1, 256) == 0
+
+
+def test_plan_table_slot_is_defined_for_every_set_of_staging_flags(tmp_path):
+    """Evaluated by the compiler, which refuses a constant expression that overflows a signed product (flags of 4 and more did):
+    all 64 sets of flags, the largest sizes."""
+    src = tmp_path / "slot.cpp"
+    src.write_text('#include "%s"\ntemplate <int S> constexpr bool below() {\n    constexpr unsigned a = rf::plan_slot(2147483647, 2147483647, 2147483520, S, 1024), '
+                   'b = rf::plan_slot(1, 1, 128, S, 1024);\n    static_assert(a < 1024 && b < 1024, "");\n    if constexpr (S > 0) return below<S - 1>();\n'
+                   '    return true;\n}\nstatic_assert(below<63>(), "");\n' % os.path.join(ROOT, "radeonflow_kernels_amd", "csrc", "plan_limits.h"))
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", str(src)], check=True)
