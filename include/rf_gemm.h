@@ -162,6 +162,11 @@ void rf_gemm_clear_plans(void);
 /* Variant table introspection (for the tuner and tests). Returns RF_ERR_BAD_CONFIG past the end. */
 int rf_gemm_num_variants(void);
 int rf_gemm_variant_info(int variant, int *block_m, int *block_n, int *waves_m, int *waves_n, int *lds_bytes);
+/* What a variant is, -1 if the index is out of range: tiles whose operands go straight to LDS (M, N multiples of 16, aligned
+ * pointers), the kernels for few rows, or tiles whose operands pass through registers (both of any shape and alignment, M and N
+ * below 2^25; one workgroup per tile only). The indices of a kind need not be neighbours. */
+enum { RF_VARIANT_KIND_TILE = 0, RF_VARIANT_KIND_FEW_ROWS = 1, RF_VARIANT_KIND_ANY_ALIGNMENT = 2 };
+int rf_gemm_variant_kind(int variant);
 /* 1 if the variant can run with rf_gemm_config.stream_k = RF_SCHEDULE_STREAM_K / RF_SCHEDULE_PERSISTENT, 0 if not
  * (or if the index is out of range). */
 int rf_gemm_variant_has_stream_k(int variant);

@@ -1510,6 +1510,11 @@ int rf_gemm_variant_k_groups(int variant) {
     return variant >= 0 && variant < kNumVariants ? kVariants[variant].k_groups : 0;
 }
 
+int rf_gemm_variant_kind(int variant) {
+    if (variant < 0 || variant >= kNumVariants) return -1;
+    return kVariants[variant].is_fewrows() ? RF_VARIANT_KIND_FEW_ROWS : kVariants[variant].is_any_tile() ? RF_VARIANT_KIND_ANY_ALIGNMENT : RF_VARIANT_KIND_TILE;
+}
+
 int rf_gemm_variant_has_persistent(int variant) {
     return variant >= 0 && variant < kNumVariants && kVariants[variant].persistent != nullptr;
 }

@@ -49,7 +49,7 @@ EXPORTS = ("run", "rf_fp8_gemm", "rf_fp8_gemm_ex", "rf_gemm_select_config", "rf_
            "rf_gemm_last_error", "rf_fp8_gemm_grouped", "rf_quantize_a_f32", "rf_quantize_a_bf16", "rf_quantize_b_f32", "rf_quantize_b_bf16",
            "rf_cast_f32_to_e4m3fn", "rf_gemm_load_plans", "rf_gemm_clear_plans", "rf_fp8_gemm_time", "rf_fp8_gemm_static",
            "rf_gemm_static_scratch_bytes", "rf_grouped_padded_offsets", "rf_quantize_a_grouped_f32",
-           "rf_quantize_a_grouped_bf16", "rf_fp8_gemm_grouped_padded", "rf_gemm_plan_for", "rf_gemm_variant_k_groups",
+           "rf_quantize_a_grouped_bf16", "rf_fp8_gemm_grouped_padded", "rf_gemm_plan_for", "rf_gemm_variant_k_groups", "rf_gemm_variant_kind",
            "rf_grouped_variant_for")
 
 
@@ -87,6 +87,8 @@ def lib():
         L.rf_gemm_variant_info.restype = i32
         L.rf_gemm_variant_has_stream_k.argtypes = [i32]
         L.rf_gemm_variant_has_stream_k.restype = i32
+        L.rf_gemm_variant_kind.argtypes = [i32]
+        L.rf_gemm_variant_kind.restype = i32
         L.rf_gemm_variant_k_groups.argtypes = [i32]
         L.rf_gemm_variant_k_groups.restype = i32
         L.rf_gemm_variant_has_persistent.argtypes = [i32]
@@ -304,6 +306,9 @@ def plan_can_run(v, split, k):
     return v["k_groups"] == 1 or (split == 1 and (k // 128) % v["k_groups"] == 0)
 
 
+VARIANT_KINDS = ("tile", "few rows", "any alignment")
+
+
 def variants():
     L = lib()
     out = []
@@ -314,5 +319,5 @@ def variants():
                         waves_n=vals[3].value, lds_bytes=vals[4].value,
                         stream_k=bool(L.rf_gemm_variant_has_stream_k(v)),
                         persistent=bool(L.rf_gemm_variant_has_persistent(v)),
-                        k_groups=L.rf_gemm_variant_k_groups(v)))
+                        k_groups=L.rf_gemm_variant_k_groups(v), kind=VARIANT_KINDS[L.rf_gemm_variant_kind(v)]))
     return out

@@ -98,28 +98,14 @@ def _time(rfk, sets, cfg, iters):
     return rfk.fp8_mm_time(*sets[0], config=cfg, warmup=3, iters=iters)
 
 
-def tune_shape(rfk, m, n, k, log=print):
-    """Times every usable plan; returns a list of dicts sorted by time."""
-    sets = operand_sets(m, n, k) if m <= ROTATED_ROWS else [_inputs(m, n, k)]
-    args = sets[0]
-    default = rfk.select_config(m, n, k)
-    if default.variant < 0:
-        log("%dx%dx%d: a small ragged shape, which takes the few-rows kernel estimated fastest and no plan" % (m, n, k))
-        return []
-    flop = 2.0 * m * n * k
-    # clocks ramp up over tens of milliseconds of load: warm up with the default plan before comparing
-    t_est = rfk.fp8_mm_time(*args, warmup=3, iters=20)
-    rfk.fp8_mm_time(*args, warmup=3, iters=max(20, int(60e3 / max(t_est, 1.0))))
-    iters = max(20, min(400, int(20e3 / max(t_est, 1.0)))) if len(sets) == 1 else 48
-    rfk.fp8_mm(*args)
-    torch.cuda.synchronize()
-    ref = args[4].clone()
-    out = []
-    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+def plans_to_time(rfk, m, n, k, ncu):
+    """The plans of a sweep as (variant, split_k, group_m, stream_k). Left out: the any-alignment tiles (made for operands that
+    the other tiles do not take), few-rows kernels beyond the rows up to which automatic plans consider them, and plans that
+    cannot run."""
     for v in rfk.variants():
         tiles = -(-m // v["block_m"]) * -(-n // v["block_n"])
-        few_rows = v["variant"] >= 14                    # no tile order to group; never the fastest beyond some hundred rows
-        if few_rows and m > 512:
+        few_rows = v["kind"] == "few rows"               # no tile order to group
+        if v["kind"] == "any alignment" or (few_rows and m > (4096 if n <= 1536 else 512)):
             continue
         # schedules: 0 = one workgroup per tile (with K splits), 1 = stream-K, 2 = persistent whole tiles,
         # 3 = persistent with a last round of half tiles, 4 = skinny K (K = 128 ... 512; listed under variant 0)
@@ -139,15 +125,41 @@ def tune_shape(rfk, m, n, k, log=print):
             if few_rows and split > 1 and tiles * split > 4 * ncu:
                 continue
             for gm in (GROUPS if sk != 4 and not few_rows else GROUPS[1:2]):   # the skinny-K schedule has no tile order either
-                cfg = rfk.GemmConfig(v["variant"], split, gm, sk)
-                args[4].zero_()
-                us = _time(rfk, sets, cfg, iters)
-                # every plan must reproduce the default plan's output up to split-K reassociation
-                err = (args[4].float() - ref.float()).abs().max().item()
-                scale = ref.float().abs().max().item() + 1e-30
-                out.append(dict(variant=v["variant"], block_m=v["block_m"], block_n=v["block_n"], split_k=split,
-                                group_m=gm, stream_k=sk, us=round(us, 2), tflops=round(flop / us / 1e6, 1),
-                                max_abs_dev_vs_default=err, ok=bool(err <= 2e-2 * scale)))
+                yield v["variant"], split, gm, sk
+
+
+def tune_shape(rfk, m, n, k, log=print):
+    """Times every usable plan; returns a list of dicts sorted by time."""
+    sets = operand_sets(m, n, k) if m <= ROTATED_ROWS else [_inputs(m, n, k)]
+    args = sets[0]
+    default = rfk.select_config(m, n, k)
+    if default.variant < 0:
+        log("%dx%dx%d: a small ragged shape, which takes the few-rows kernel estimated fastest and no plan" % (m, n, k))
+        return []
+    flop = 2.0 * m * n * k
+    # clocks ramp up over tens of milliseconds of load: warm up with the default plan before comparing
+    t_est = rfk.fp8_mm_time(*args, warmup=3, iters=20)
+    rfk.fp8_mm_time(*args, warmup=3, iters=max(20, int(60e3 / max(t_est, 1.0))))
+    iters = max(20, min(400, int(20e3 / max(t_est, 1.0)))) if len(sets) == 1 else 48
+    rfk.fp8_mm(*args)
+    torch.cuda.synchronize()
+    ref = args[4].clone()
+    out = []
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = {v["variant"]: (v["block_m"], v["block_n"]) for v in rfk.variants()}
+    plans = list(plans_to_time(rfk, m, n, k, ncu))
+    present = (default.variant, default.split_k, default.group_m, default.stream_k)
+    if present not in plans:                             # what a winner has to beat is always among the times
+        plans.append(present)
+    for plan in plans:
+        args[4].zero_()
+        us = _time(rfk, sets, rfk.GemmConfig(*plan), iters)
+        # every plan must reproduce the default plan's output up to split-K reassociation
+        err = (args[4].float() - ref.float()).abs().max().item()
+        scale = ref.float().abs().max().item() + 1e-30
+        out.append(dict(variant=plan[0], block_m=blocks[plan[0]][0], block_n=blocks[plan[0]][1], split_k=plan[1],
+                        group_m=plan[2], stream_k=plan[3], us=round(us, 2), tflops=round(flop / us / 1e6, 1),
+                        max_abs_dev_vs_default=err, ok=bool(err <= 2e-2 * scale)))
     out = [o for o in out if o["ok"]]
     out.sort(key=lambda o: o["us"])
     return out

@@ -193,6 +193,25 @@ def test_tuner_replaces_a_tabled_plan_only_when_a_sweep_finds_one_two_percent_fa
     assert inc.read_text() == before
 
 
+def test_tuner_times_every_plan_of_the_compiled_in_table():
+    """A sweep that leaves a tabled plan out would replace it unseen: the table's lines, 128 x 128 tiles of variant 28 beyond 512
+    rows and with every tile order among them, are all timed (they were skipped when kernels for few rows were told by their
+    number); the any-alignment tiles are not."""
+    import radeonflow_kernels_amd as rfk
+    from radeonflow_kernels_amd.tuner import gemm_tuner as t
+    inc = os.path.join(ROOT, "radeonflow_kernels_amd", "csrc", "tuned_plans.inc")
+    plans = [tuple(int(x) for x in re.findall(r"-?\d+", l.split("}")[0])) for l in open(inc) if l.startswith("{")]
+    for p in plans:
+        assert p[3:] in set(t.plans_to_time(rfk, *p[:3], 256)), p
+    timed = set(t.plans_to_time(rfk, 1024, 3072, 1536, 256))
+    assert {(28, s, g, 0) for s in (1, 2, 4, 12) for g in t.GROUPS} <= timed
+    kinds = {v["variant"]: v["kind"] for v in rfk.variants()}
+    assert "any alignment" in kinds.values() and {kinds[p[0]] for p in timed} == {"tile"}
+    for shape in ((64, 3072, 1536), (848, 576, 1024)):
+        assert {kinds[p[0]] for p in t.plans_to_time(rfk, *shape, 256)} == {"tile", "few rows"}
+    assert rfk.lib().rf_gemm_variant_kind(-1) == -1 == rfk.lib().rf_gemm_variant_kind(len(kinds))
+
+
 def test_planner_arithmetic_on_the_host_for_any_compute_unit_count(tmp_path):
     """rf_gemm_plan_for needs no device. With 256 compute units a tabled shape gets its tabled plan; with any other count
     the table (measured on 256) is left aside and the cost model counts rounds for the count given: every plan names an
