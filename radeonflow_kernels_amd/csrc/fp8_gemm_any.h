@@ -14,7 +14,7 @@ struct AnyGeom {
 };
 
 // tile_mainloop with the operands through registers.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int SETS>
+template <int BM, int BN, int WAVES_M, int WAVES_N>
 __device__ __forceinline__ void tile_mainloop_any(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
     const float *__restrict__ SB, int M, int ldm, int N, int QK, int m0, int n0, int kb_begin, int kb_end, uint8_t *lds,
@@ -24,8 +24,8 @@ __device__ __forceinline__ void tile_mainloop_any(
     constexpr int WM = G::WM, WN = G::WN, TM = G::TM, TN = G::TN, NT = G::NT, IA = Y::IA, IB = Y::IB;
     constexpr int STAGE_A = G::STAGE_A, STAGE_B = G::STAGE_B, STAGE_S = G::STAGE_S;
     constexpr int OFF_B = 2 * STAGE_A, OFF_S = 2 * (STAGE_A + STAGE_B), OFF_SB = BM * 4;
-    constexpr bool ONE_SB = WN <= 128 && 128 % WN == 0;
-    static_assert(ONE_SB || (TN == 3 && WN < 128), "straddling waves: three n-tiles, split before n-tile 1 or 2");
+    static_assert(WN <= 128 && 128 % WN == 0, "a wave's columns have one b_scale");
+    static_assert((TM & (TM - 1)) == 0 && (TN & (TN - 1)) == 0, "a fragment's address is the wave's first one with the tile's index XORed in");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int L = lane & 15, g = lane >> 4, wm = wave % WAVES_M, wn = wave / WAVES_M;
     const int QN = (N + 127) / 128;
@@ -71,8 +71,8 @@ __device__ __forceinline__ void tile_mainloop_any(
         const unsigned long long r = (unsigned long long)(QK - kb) * BK * (unsigned)ld;
         return r < 0xffffffffull ? (uint32_t)r : 0xffffffffu;
     };
-    u32x4_lds raw[SETS][IA + IB];
-    float rs[SETS];
+    u32x4_lds raw[2][IA + IB];                                           // two K blocks on their way
+    float rs[2];
     const int kb_last = kb_end - 1;
     auto clamp_kb = [&](int kb) { return kb < kb_last ? kb : kb_last; };
     auto load_item = [&](auto set_c, int d, int kb) {
@@ -101,23 +101,11 @@ __device__ __forceinline__ void tile_mainloop_any(
 
     // ---- LDS -> MFMA operands (see tile_mainloop) ----
     const int krow = 32 * g + (L >> 1);
-    constexpr bool POW2_T = (TM & (TM - 1)) == 0 && (TN & (TN - 1)) == 0;
     const uint32_t aoff_base = krow * BM + (((wm * TM) ^ swizzle_of_row<BM>(krow)) << 4) + 8 * (L & 1);
     const uint32_t boff_base = OFF_B + krow * BN + (((wn * TN) ^ swizzle_of_row<BN>(krow)) << 4) + 8 * (L & 1);
-    uint32_t aoff_tile[POW2_T ? 1 : TM], boff_tile[POW2_T ? 1 : TN];
-    if constexpr (!POW2_T) {
-#pragma unroll
-        for (int j = 0; j < TM; j++) aoff_tile[j] = krow * BM + (((wm * TM + j) ^ swizzle_of_row<BM>(krow)) << 4) + 8 * (L & 1);
-#pragma unroll
-        for (int i = 0; i < TN; i++)
-            boff_tile[i] = OFF_B + krow * BN + (((wn * TN + i) ^ swizzle_of_row<BN>(krow)) << 4) + 8 * (L & 1);
-    }
     const uint32_t soff = OFF_S + (wm * WM + L * TM) * 4;
     const int ncol0 = n0 + wn * WN;
-    const int sb_split_raw = (((ncol0 >> 7) + 1) * 128 - ncol0) >> 4;
-    const int sb_split = __builtin_amdgcn_readfirstlane(sb_split_raw < TN ? sb_split_raw : TN);
     const uint32_t sboff = OFF_S + OFF_SB + (((ncol0 >> 7) - (n0 >> 7)) << 2);
-    const uint32_t sboff1 = sboff + (sb_split < TN ? 4 : 0);
     constexpr int NMFMA = TM * TN, PR = (NMFMA % 4 == 0 && TN > 3) ? 4 : 3, LAG = PR - 1, BAR_SLOT = (TM - 1) * TN;
     static_assert(NMFMA % PR == 0 && LAG < TN && LAG < PR && TM % 2 == 0, "same schedule as tile_mainloop");
     constexpr int PER_SLOT = (NL + BAR_SLOT - 2) / (BAR_SLOT - 1);       // writes (and loads) per slot, done a slot before the barrier
@@ -127,20 +115,18 @@ __device__ __forceinline__ void tile_mainloop_any(
         for (int i = 0; i < TN; i++) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
     i32x8 bfrag[TN], afrag[2];
     f32x4 pring[PR];
-    float s[TM], s1[ONE_SB ? 1 : TM], sraw[TM], sb_raw = 0.f, sb_raw1 = 0.f;
+    float s[TM], sraw[TM], sb_raw = 0.f;
 #pragma unroll
     for (int r = 0; r < PR; r++) pring[r] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < TM; j++) s[j] = 0.f;
-#pragma unroll
-    for (int j = 0; j < (ONE_SB ? 1 : TM); j++) s1[j] = 0.f;
     auto rd = [&](uint32_t stage_base, uint32_t off) {
         return __builtin_amdgcn_ds_read_tr8_b64_v2i32((RF_LDS i32x2 *)(lds + stage_base + off));
     };
     auto read_bfrag = [&](int i, int stage) {
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            i32x2 v = rd(stage * STAGE_B, (POW2_T ? boff_base ^ (i << 4) : boff_tile[POW2_T ? 0 : i]) + t * 8 * BN);
+            i32x2 v = rd(stage * STAGE_B, (boff_base ^ (i << 4)) + t * 8 * BN);
             bfrag[i][2 * t] = v[0];
             bfrag[i][2 * t + 1] = v[1];
         }
@@ -148,7 +134,7 @@ __device__ __forceinline__ void tile_mainloop_any(
     auto read_afrag = [&](int buf, int j, int stage) {
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            i32x2 v = rd(stage * STAGE_A, (POW2_T ? aoff_base ^ (j << 4) : aoff_tile[POW2_T ? 0 : j]) + t * 8 * BM);
+            i32x2 v = rd(stage * STAGE_A, (aoff_base ^ (j << 4)) + t * 8 * BM);
             afrag[buf][2 * t] = v[0];
             afrag[buf][2 * t + 1] = v[1];
         }
@@ -161,24 +147,18 @@ __device__ __forceinline__ void tile_mainloop_any(
             sraw[2 * q + 1] = v[1];
         }
         sb_raw = *(RF_LDS float *)(lds + stage * STAGE_S + sboff);
-        if constexpr (!ONE_SB) sb_raw1 = *(RF_LDS float *)(lds + stage * STAGE_S + sboff1);
     };
     // prologue
-    auto each_set = [&](auto f) {
-        f(IntTag<0>{});
-        f(IntTag<1>{});
-        if constexpr (SETS > 2) f(IntTag<2>{});
-    };
-    each_set([&](auto set_c) {
 #pragma unroll
-        for (int d = 0; d < NL; d++) load_item(set_c, d, kb_begin + decltype(set_c)::value);
-    });
+    for (int d = 0; d < NL; d++) load_item(IntTag<0>{}, d, kb_begin);
+#pragma unroll
+    for (int d = 0; d < NL; d++) load_item(IntTag<1>{}, d, kb_begin + 1);
     __builtin_amdgcn_sched_barrier(0);
     uncut(IntTag<0>{}, kb_begin);
 #pragma unroll
     for (int d = 0; d < NL; d++) write_item(IntTag<0>{}, d, 0);
 #pragma unroll
-    for (int d = 0; d < NL; d++) load_item(IntTag<0>{}, d, kb_begin + SETS);
+    for (int d = 0; d < NL; d++) load_item(IntTag<0>{}, d, kb_begin + 2);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     read_bfrag(0, 0);
@@ -187,17 +167,13 @@ __device__ __forceinline__ void tile_mainloop_any(
 #pragma unroll
     for (int i = 1; i < TN; i++) read_bfrag(i, 0);
     // One K block: the stage it reads (cur), the register set of the next one (set). In its first slots block kb + 1 goes from
-    // its registers into the other stage, and block kb + 1 + SETS is asked for in its place.
-    auto k_block = [&](auto cur_c, auto set_c, auto split_c, int kb) {
+    // its registers into the other stage, and block kb + 3 is asked for in its place.
+    auto k_block = [&](auto cur_c, auto set_c, int kb) {
         constexpr int cur = decltype(cur_c)::value, nxt = 1 - cur;
-        constexpr int split = decltype(split_c)::value;
-        const float s_last = s[TM - 1], s1_last = s1[ONE_SB ? 0 : TM - 1];
+        const float s_last = s[TM - 1];
         uncut(set_c, clamp_kb(kb + 1));
 #pragma unroll
         for (int j = 0; j < TM; j++) s[j] = sraw[j] * sb_raw;
-        if constexpr (!ONE_SB)
-#pragma unroll
-            for (int j = 0; j < TM; j++) s1[j] = sraw[j] * sb_raw1;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < NMFMA; t++) {
@@ -223,65 +199,39 @@ __device__ __forceinline__ void tile_mainloop_any(
             for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) write_item(set_c, d, nxt);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) load_item(set_c, d, kb + 1 + SETS);
+            for (int d = t * PER_SLOT; d < (t + 1) * PER_SLOT && d < NL; d++) load_item(set_c, d, kb + 3);
             if (t >= LAG) {
                 const int u = t - LAG, ju = u / TN, iu = u % TN;
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    acc[ju][iu][e] = __builtin_fmaf(iu < split ? s[ju] : s1[ONE_SB ? 0 : ju], pring[u % PR][e], acc[ju][iu][e]);
+                    acc[ju][iu][e] = __builtin_fmaf(s[ju], pring[u % PR][e], acc[ju][iu][e]);
                 asm volatile("" : "+v"(acc[ju][iu]));
             } else {
                 const int u = NMFMA + t - LAG, ju = u / TN, iu = u % TN;
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    acc[ju][iu][e] = __builtin_fmaf(iu < split ? s_last : s1_last, pring[u % PR][e], acc[ju][iu][e]);
+                    acc[ju][iu][e] = __builtin_fmaf(s_last, pring[u % PR][e], acc[ju][iu][e]);
                 asm volatile("" : "+v"(acc[ju][iu]));
             }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    auto k_loop = [&](auto split_c) {
-        constexpr int split = decltype(split_c)::value;
-        int kb = kb_begin;
-        if constexpr (SETS == 2) {
-            for (; kb + 1 < kb_end; kb += 2) {
-                k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
-                k_block(IntTag<1>{}, IntTag<0>{}, split_c, kb + 1);
-            }
-            if (kb < kb_end) k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
-        } else {
-            for (; kb + 5 < kb_end; kb += 6) {
-                k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
-                k_block(IntTag<1>{}, IntTag<2>{}, split_c, kb + 1);
-                k_block(IntTag<0>{}, IntTag<0>{}, split_c, kb + 2);
-                k_block(IntTag<1>{}, IntTag<1>{}, split_c, kb + 3);
-                k_block(IntTag<0>{}, IntTag<2>{}, split_c, kb + 4);
-                k_block(IntTag<1>{}, IntTag<0>{}, split_c, kb + 5);
-            }
-            if (kb < kb_end) k_block(IntTag<0>{}, IntTag<1>{}, split_c, kb);
-            if (kb + 1 < kb_end) k_block(IntTag<1>{}, IntTag<2>{}, split_c, kb + 1);
-            if (kb + 2 < kb_end) k_block(IntTag<0>{}, IntTag<0>{}, split_c, kb + 2);
-            if (kb + 3 < kb_end) k_block(IntTag<1>{}, IntTag<1>{}, split_c, kb + 3);
-            if (kb + 4 < kb_end) k_block(IntTag<0>{}, IntTag<2>{}, split_c, kb + 4);
-        }
+    int kb = kb_begin;
+    for (; kb + 1 < kb_end; kb += 2) {
+        k_block(IntTag<0>{}, IntTag<1>{}, kb);
+        k_block(IntTag<1>{}, IntTag<0>{}, kb + 1);
+    }
+    if (kb < kb_end) k_block(IntTag<0>{}, IntTag<1>{}, kb);
 #pragma unroll
-        for (int t = 0; t < LAG; t++) {
-            const int u = NMFMA + t - LAG, ju = u / TN, iu = u % TN;
+    for (int t = 0; t < LAG; t++) {
+        const int u = NMFMA + t - LAG, ju = u / TN, iu = u % TN;
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                acc[ju][iu][e] = __builtin_fmaf(iu < split ? s[TM - 1] : s1[ONE_SB ? 0 : TM - 1], pring[u % PR][e], acc[ju][iu][e]);
-        }
-    };
-    if constexpr (ONE_SB) {
-        k_loop(IntTag<TN>{});
-    } else {
-        if (sb_split == 1) k_loop(IntTag<1>{});
-        else k_loop(IntTag<2>{});
+        for (int e = 0; e < 4; e++) acc[ju][iu][e] = __builtin_fmaf(s[TM - 1], pring[u % PR][e], acc[ju][iu][e]);
     }
 }
 
 // PARTIAL: the fp32 sums of K part blockIdx.y to ws[part][M rounded up to 16][ld_ws] (see reduce_splitk_any_c).
-template <int BM, int BN, int WAVES_M, int WAVES_N, int SETS, bool PARTIAL>
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool PARTIAL>
 __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_tile_any(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,
     const float *__restrict__ SB, void *__restrict__ out, int M, int ldm, int N, int K, int kb_per_split, int tiles_m, int tiles_n,
@@ -293,7 +243,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64) void gemm_fp8_blockscale_til
     const int m0 = tile_m * BM, n0 = tile_n * BN, QK = K / BK;
     const int kb_begin = blockIdx.y * kb_per_split, kb_end = kb_begin + kb_per_split < QK ? kb_begin + kb_per_split : QK;
     f32x4 acc[G::TM][G::TN];
-    tile_mainloop_any<BM, BN, WAVES_M, WAVES_N, SETS>(A, B, SA, SB, M, ldm, N, QK, m0, n0, kb_begin, kb_end, lds, acc);
+    tile_mainloop_any<BM, BN, WAVES_M, WAVES_N>(A, B, SA, SB, M, ldm, N, QK, m0, n0, kb_begin, kb_end, lds, acc);
     if constexpr (PARTIAL) {
         const int mp = (M + 15) / 16 * 16, ld_ws = (N + 15) / 16 * 16;
         store_tile_f32_staged<BM, BN, WAVES_M, WAVES_N>(acc, (float *)out + ((size_t)blockIdx.y * mp + m0) * ld_ws + n0, ld_ws, mp - m0,

@@ -120,7 +120,7 @@ struct Variant {
 // tiles whose operands pass through registers, at any alignment (fp8_gemm_any.h)
 #define RF_VARIANT_ANY_TILE(BM, BN, WM, WN)                                                \
     Variant { BM, BN, WM, WN, rf::AnyGeom<BM, BN, WM, WN>::LDS_BYTES, nullptr, nullptr, nullptr, nullptr, 0, nullptr, 1, {}, nullptr, \
-              {rf::gemm_fp8_blockscale_tile_any<BM, BN, WM, WN, 2, false>, rf::gemm_fp8_blockscale_tile_any<BM, BN, WM, WN, 2, true>} }
+              {rf::gemm_fp8_blockscale_tile_any<BM, BN, WM, WN, false>, rf::gemm_fp8_blockscale_tile_any<BM, BN, WM, WN, true>} }
 const Variant kVariants[] = {
     Variant{256, 256, 2, 4, rf::TileGeom<256, 256, 2, 4>::LDS_BYTES, rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, false>,
             rf::gemm_fp8_blockscale_tile<256, 256, 2, 4, true>, rf::gemm_fp8_blockscale_streamk<256, 256, 2, 4>,
@@ -678,14 +678,13 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // no padded columns, e.g. N = 576, 1536 or 3072; the 64x128 tile where M is short or the whole problem is a few
     // microseconds); the others never won by more than a few percent.
     struct Candidate { int variant; double c, f; };
-    // (variants 12 and 13 split K between two wave groups of one workgroup: half the K blocks per group, one launch, no
-    // reduction term. Variant 12, the 64 x 128 tile: the best plan of short shapes, M <= 512, with K = 512 ... 2304.
-    // Variant 13, the 128 x 128 tile: the best plan where 128 x 128 tiles fill one round, e.g. 1024 x 3072 x 1536,
-    // 512 x 7168 x 2048. Variant 28, the 128 x 128 tile with eight waves and three stages, searched for by itself on 37
-    // further shapes, the other constants as they were: choice 1.4 % behind the best of all, 4.6 % without it)
-    const Candidate cands[] = {{0, 0.905, 5.96}, {3, 0.679, 3.61}, {5, 0.80, 5.8},  {6, 0.74, 4.3},  {7, 0.85, 0.3},
-                               {8, 0.52, 4.2},   {9, 0.73, 0.5},   {10, 0.53, 5.9}, {11, 0.71, 7.0}, {12, 0.93, 1.4},
-                               {13, 1.06, 3.3}, {28, 0.44, 2.25}};
+    // (variant 12 splits K between two wave groups of one workgroup: half the K blocks per group, one launch, no
+    // reduction term. The 64 x 128 tile: the best plan of short shapes, M <= 512, with K = 512 ... 2304. Variant 28, the
+    // 128 x 128 tile with eight waves and three stages, searched for by itself on 37 further shapes, the other constants as
+    // they were: choice 1.4 % behind the best of all, 4.6 % without it. Not among them: variants 6 (c = 0.74, f = 4.3) and 13
+    // (half of 1.06, 3.3), whose tiles 8 and 28 have at less of both)
+    const Candidate cands[] = {{0, 0.905, 5.96}, {3, 0.679, 3.61}, {5, 0.80, 5.8},  {7, 0.85, 0.3},  {8, 0.52, 4.2},
+                               {9, 0.73, 0.5},   {10, 0.53, 5.9},  {11, 0.71, 7.0}, {12, 0.93, 1.4}, {28, 0.44, 2.25}};
     const double f_next = 3.3, reduce_fixed = 6.03, reduce_per_elem = 1.27e-6, c_half_tile = 0.47, f_half_tile = 5.2;
     const int splits_tried[] = {1, 2, 3, 4, 6, 8, 12, 16};
     double best_cost = 1e30;
