@@ -567,17 +567,29 @@ constexpr int kFewRowsMaxM = 512, kFewRowsMaxMWide = 4096, kFewRowsSmallN = 1536
 // What a shape or its pointers need before the tiled kernels can run on it (see launch_padded): copies of A and a_scale, or of B
 // (and of C on the way back). kTiledOnly: no few-rows plan.
 // kBytesA, kBytesB: rows of that operand do not all start at a multiple of four bytes.
-// kFewRowsOnly: the few-rows plan (m and n as they are).
-enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16, kFewRowsOnly = 32 };
+// kFewRowsOnly: the few-rows plan (m and n as they are). kCutC: rows of C are not whole cache lines.
+// kCopyB: B is copied (kStageB without it: only C is unaligned).
+enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16, kFewRowsOnly = 32, kCutC = 64, kCopyB = 128 };
 
-// Estimated time in microseconds of the best any-alignment tile plan for a shape whose operands would have to be staged, and
-// that plan. Fitted (relative error, 6 %) to 640 plans of 100 random shapes on operand sets that stay in the Infinity Cache:
-//   2.9 + rounds * (f + K blocks * (c + c_a where rows of A start at any byte + c_b where rows of B do))
-//   + 0.39 per million outputs (0.45 more where rows of C start at odd elements)
-//   + 2.76 + 1.19 per million sums when K is split
+// The flags of a shape and its pointers (0: aligned).
+int stage_flags(int m, int n, uintptr_t a, uintptr_t b, uintptr_t c) {
+    const bool copy_b = n % 16 != 0 || b % 16 != 0;
+    return (m % 16 != 0 || a % 16 != 0 ? kStageA : 0) | (copy_b || c % 16 != 0 ? kStageB : 0) | (copy_b ? kCopyB : 0) |
+           (m % 4 != 0 || a % 4 != 0 ? kBytesA : 0) | (n % 4 != 0 || b % 4 != 0 ? kBytesB : 0) | (n % 64 != 0 || c % 128 != 0 ? kCutC : 0);
+}
+
+// The three estimates below decide what a call takes whose operands would have to be staged. Their constants are fitted (relative
+// error) to plans of 430 random shapes measured on operand sets and C in rotation, as those of fewrows_plan are
+// (tuner/staged_model.py: --measure takes them, --fit fits).
+
+// Estimated time in microseconds of the best any-alignment tile plan for a shape, and that plan. 1809 plans, 8 % off:
+//   1.84 + rounds * (f + K blocks * (c + c_a where rows of A start at any byte + c_b where rows of B do))
+//   + 0.21 per million outputs, 0.56 more where rows of C are not whole lines (two tiles then write each line at their border) and
+//     0.17 where those of B, and with a ragged N those of C, start at any byte
+//   + 3.02 + 1.03 per million sums when K is split
 double any_tile_plan(int m, int n, int k, int num_cu, int stage, rf_gemm_config *out) {
     struct Fit { int variant; double f, c, c_a, c_b; };
-    const Fit fits[] = {{29, 1.60, 0.595, 0.091, 0.119}, {30, 2.71, 0.771, 0.130, 0.326}};
+    const Fit fits[] = {{29, 2.54, 0.580, 0.093, 0.105}, {30, 3.835, 0.792, 0.093, 0.285}};
     const int splits_tried[] = {1, 2, 3, 4, 6, 8}, qk = k / rf::BK;
     const double mn = (double)m * n * 1e-6;
     double best = 1e30;
@@ -590,8 +602,8 @@ double any_tile_plan(int m, int n, int k, int num_cu, int stage, rf_gemm_config 
             const int kb = ceil_div(qk, sp), parts = ceil_div(qk, kb);
             if (parts > 1 && mn * parts > 40.0) break;      // no more than was measured, 150 MB of sums
             const long rounds = (tiles * parts + num_cu - 1) / num_cu;
-            const double t = 2.9 + rounds * (f.f + kb * per_block) + mn * (0.39 + (stage & kBytesB ? 0.45 : 0.0)) +
-                             (parts > 1 ? 2.76 + 1.19 * parts * mn : 0.0);
+            const double t = 1.837 + rounds * (f.f + kb * per_block) + (parts > 1 ? 3.021 + 1.029 * parts * mn : 0.0) +
+                             mn * (0.21 + (stage & kCutC ? 0.562 : 0.0) + (stage & kBytesB ? 0.168 : 0.0));
             if (t < best) {
                 best = t;
                 *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};
@@ -600,6 +612,23 @@ double any_tile_plan(int m, int n, int k, int num_cu, int stage, rf_gemm_config 
     }
     return best;
 }
+
+// Estimated time in microseconds of the skinny-K schedule on staged copies: `mn` million outputs in qk K blocks, the copy of A and
+// the one of B, and C's way back, which costs less beyond the 15 million outputs (30 MB) that the L2 caches hold. 154 shapes, 7 % off.
+// With it the plan taken of this schedule and any_tile_plan's is 0.9 % slower than the faster one on average and 22 % at worst.
+// Shapes with ragged N, or only B or C unaligned, had none, and all of them took any_tile_plan's: 4256 x 8000 x 256 with B at an odd byte
+// 46.8 -> 22.9 us, 6144 x 7168 x 256 with C 8 bytes off 74.2 -> 49.5, 8192 x 7160 x 256 97.5 -> 65.9, 6000 x 4090 x 128 46.9 -> 33.5; but
+// 1264 x 5632 x 256 with C 8 bytes off stays (11.3, the schedule 15.6).
+double skinny_staged_us(int qk, double mn, int stage) {
+    double t = 2.137 + 1.033 * qk + (0.265 + 0.098 * qk) * mn;
+    if (stage & kStageA) t += 2.591;
+    if (stage & kCopyB) t += 2.948;
+    if ((stage & kStageB) && (stage & kCutC)) t += 1.522 + 0.921 * std::min(mn, 15.0) + 0.369 * std::max(mn - 15.0, 0.0);
+    return t;
+}
+
+// The same of one round of 128 x 128 tiles over three or four K blocks, nothing staged. 30 shapes, 2 % off.
+double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn; }
 
 // Plan for a shape (m, n multiples of 16, the padded sizes when something is staged).
 void select_config_uncached(int m, int n, int k, int num_cu, int stage, const std::vector<TunedPlan> &user_plans,
@@ -741,11 +770,8 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     double t = 3.1 + 0.67 * best_cost;
     if (stage & kStageA) t += 3.2 + 2.0 * k * m / 4e6;
     if (stage & kStageB) t += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
-    // The skinny-K schedule behind a staging copy of A, fitted to 63 shapes of 321 to 8005 rows and N = 1024 ... 8192. With the
-    // estimate below the plan taken is the faster one on all of them, where 34 were up to 80 % slower: 570 x 4096 x 384 11.2 -> 6.2,
-    // 3003 x 1024 x 512 12.2 -> 7.8, 8005 x 1024 x 128 9.4 -> 7.2; 1318 x 8192 x 384 stays (13.8, the tiles 16.0).
-    if (skinny && !(stage & kStageB)) t = 7.2 + 0.9 * qk + (0.19 + 0.078 * qk) * 1e-6 * mn;
-    if (one_round) t = 3.0 + 0.6 * qk + 0.36e-6 * mn;       // fitted to 32 shapes, 3 %
+    if (skinny) t = skinny_staged_us(qk, 1e-6 * mn, stage);
+    if (one_round) t = one_round_us(qk, 1e-6 * mn);
     rf_gemm_config other;
     const int max_m = ((stage & kStageB) || n <= kFewRowsSmallN) && num_cu == kTunedOnCUs ? kFewRowsMaxMWide : kFewRowsMaxM;
     if (m <= max_m && fewrows_ok(m, n) && !(stage & kTiledOnly)) {
@@ -755,11 +781,10 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
             *out = other;
         }
     }
-    // Operands that would be staged: the tiles that take them as they are. On 100 shapes drawn at random (90 to 8192 rows; M or N
-    // or both ragged) the plan taken is 1.2 % behind the best of all on average and 27 % at worst, and 10 % faster than
-    // without them (37 of the plans change, one of them for the worse by 6 %); at equal estimates they are the faster ones.
-    // On the compute unit count they were measured on.
-    if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < 1.05 * t) *out = other;
+    // Operands that would be staged: the tiles that take them as they are, on the compute unit count they were measured on.
+    // On 166 shapes that the fit has not seen (100 to 8192 rows, M or N or both ragged) the plan taken is 1.2 % behind the best of few
+    // rows, these tiles with every K split and the plans of the padded shape on average, 24 % at worst.
+    if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < t) *out = other;
 }
 
 // The same through a small table of plans already worked out (the models take 1 to 3 us of host time, as long as a small
@@ -1265,8 +1290,7 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     // tile, persistent) write the m true rows straight into c (their stores are masked by row), and the tile kernels
     // have a form for any c; otherwise C is staged and copied back.
     rf_gemm_config cfg;
-    select_config(mp, np, k, s.num_cu, (copy_a ? kStageA : 0) | (copy_b || (uintptr_t)c % 16 != 0 ? kStageB : 0) |
-                  (m % 4 != 0 || (uintptr_t)a % 4 != 0 ? kBytesA : 0) | (n % 4 != 0 || (uintptr_t)b % 4 != 0 ? kBytesB : 0), &cfg);
+    select_config(mp, np, k, s.num_cu, stage_flags(m, n, (uintptr_t)a, (uintptr_t)b, (uintptr_t)c), &cfg);
     if (kVariants[cfg.variant].is_any_tile()) {
         const size_t part = any_tile_part_bytes(m, n);
         if (mem.fixed && cfg.split_k > 1) {                // as many K parts as the static array holds
@@ -1374,8 +1398,7 @@ void plan_of_shape(int m, int n, int k, int num_cu, rf_gemm_config *out) {
     auto pad16 = [](int x) { return x < 16 ? 16 : (x + 15) / 16 * 16; };
     const int mp = pad16(m), np = pad16(n);
     if ((mp != m || np != n) && (double)m * n * k < kPadThresholdMacs) *out = {-1, 1, 8, RF_SCHEDULE_TILES};
-    else select_config(mp, np, k, num_cu, (mp != m ? kStageA : 0) | (np != n ? kStageB : 0) | (m % 4 != 0 ? kBytesA : 0) |
-                       (n % 4 != 0 ? kBytesB : 0), out);
+    else select_config(mp, np, k, num_cu, stage_flags(m, n, 0, 0, 0), out);
 }
 
 // ---- timing record for run() ----------------------------------------------------------------

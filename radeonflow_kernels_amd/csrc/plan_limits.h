@@ -36,7 +36,7 @@ constexpr bool grouped_weights_streamed(double bytes, bool queue, int columns) {
 }
 
 // Slot of a shape in the table of plans already worked out (a power of two of them, up to 2^25). All products unsigned: `stage` has
-// six bits, and as an int its product overflowed from 4 on.
+// eight bits, and as an int its product overflowed from 4 on.
 constexpr unsigned plan_slot(int m, int n, int k, int stage, unsigned entries) {
     return ((((unsigned)m * 2654435761u) ^ ((unsigned)n * 2246822519u) ^ ((unsigned)k * 3266489917u) ^ ((unsigned)stage * 668265263u)) >> 7) % entries;
 }

@@ -212,6 +212,17 @@ def test_tuner_times_every_plan_of_the_compiled_in_table():
     assert rfk.lib().rf_gemm_variant_kind(-1) == -1 == rfk.lib().rf_gemm_variant_kind(len(kinds))
 
 
+@pytest.mark.parametrize("m,n,k,schedule", [(8192, 7160, 256, 4), (6000, 4090, 128, 4), (5727, 7676, 256, 4), (7137, 4404, 384, 4), (1504, 3889, 384, 0),
+                                            (700, 3001, 512, 0), (570, 4096, 384, 0), (1318, 8192, 384, 4)])
+def test_short_k_on_staged_copies_is_weighed_against_the_any_alignment_tiles(m, n, k, schedule):
+    """Short K, a large C and a ragged N: the skinny-K schedule on staged copies had no estimate and so was never taken (the first four
+    shapes: 98, 47, 76 and 61 us on the tiles, 66, 33, 54 and 48 on the schedule); a smaller C stays on the tiles, and with only M ragged
+    both sides keep what they had."""
+    import radeonflow_kernels_amd as rfk
+    plan = rfk.plan_for(m, n, k, 256)
+    assert plan.stream_k == schedule and (schedule == 4 or plan.variant in (29, 30))
+
+
 def test_planner_arithmetic_on_the_host_for_any_compute_unit_count(tmp_path):
     """rf_gemm_plan_for needs no device. With 256 compute units a tabled shape gets its tabled plan; with any other count
     the table (measured on 256) is left aside and the cost model counts rounds for the count given: every plan names an
