@@ -519,16 +519,20 @@ constexpr int kTunedOnCUs = 256;
 // measured plans are 0.2 % faster.
 //   2.56                                       launch, and the way back
 //   + 0.64 + 0.192 per KiB of sums handed over when K is split
-//   + rounds * (b + 0.253 * batches of loads of a wave + c * K blocks of a wave * workgroups sharing a CU), a quarter more
+//   + rounds * (b + 0.253 * batches of loads of a wave + c * K blocks of a wave * workgroups sharing a CU), times `any`
 //     where rows of B start at any byte (any_bytes); variants that load the next K block while they multiply: one batch
 //   + d * MB of A and B that all workgroups fetch + 0.0505 * MB of A and B
+// `any` is 1.27 but for three variants: a row of 16 and 27's 128 columns is one cache line where it is aligned and two where it is not, and of 21 two
+// workgroups share a CU and its L1. Searched on 12 pairs of ragged N from 1000 to 5003 and K from 384 to 7168, M = 1 ... 500
+// (tuner/fewrows_model.py --ragged): the plan taken, any_tile_plan's among the choice, is 1.4 % behind the fastest on average and 12 % at
+// worst, with 1.27 for all 2.5 % and 17 % (40 x 2003 x 7168 12.2 us on variant 16, 10.9 on 25).
 double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_config *out) {
-    struct Fit { int variant, per_cu, depth; double b, c, d; };
+    struct Fit { int variant, per_cu, depth; double b, c, d, any = 1.27; };
     constexpr int kAll = 1 << 20;
-    const Fit fits[] = {{14, 2, 3, 0.0238, 0.6526, 0.0811},    {16, 1, kAll, 0.017, 1.6541, 0.0325},  {20, 1, kAll, 0.2932, 1.9032, 0.0785},
-                        {21, 2, kAll, 1.3762, 1.0315, 0.0158}, {22, 2, kAll, 0.0007, 0.6572, 0.086},  {23, 1, kAll, 0.0704, 1.4481, 0.0227},
+    const Fit fits[] = {{14, 2, 3, 0.0238, 0.6526, 0.0811},    {16, 1, kAll, 0.017, 1.6541, 0.0325, 1.5},  {20, 1, kAll, 0.2932, 1.9032, 0.0785},
+                        {21, 2, kAll, 1.3762, 1.0315, 0.0158, 1.5}, {22, 2, kAll, 0.0007, 0.6572, 0.086},  {23, 1, kAll, 0.0704, 1.4481, 0.0227},
                         {24, 2, kAll, 0.0049, 0.9508, 0.0676}, {25, 1, kAll, 0.0106, 1.7903, 0.0289}, {26, 2, kAll, 0.3722, 0.7608, 0.0427},
-                        {27, 1, kAll, 1.0902, 1.385, 0.0109}};
+                        {27, 1, kAll, 1.0902, 1.385, 0.0109, 1.5}};
     const double operands = 0.0505e-6 * k * ((double)m + n);
     const int splits_tried[] = {1, 2, 3, 4, 5, 6, 8, 12, 14}, qk = k / rf::BK;
     double best = 1e30;
@@ -541,7 +545,7 @@ double fewrows_plan(int m, int n, int k, int num_cu, bool any_bytes, rf_gemm_con
             const long wgs = items * parts, rounds = (wgs + (long)num_cu * f.per_cu - 1) / ((long)num_cu * f.per_cu);
             const double mb = (double)wgs * kb * (v.bm + v.bn) * rf::BK * 1e-6 * 256 / num_cu;
             const double t = 2.5568 + (parts > 1 ? 0.6363 + 0.1919 * parts * v.bm * v.bn / 1024.0 : 0.0) +
-                             rounds * (any_bytes ? 1.27 : 1.0) *
+                             rounds * (any_bytes ? f.any : 1.0) *
                                  (f.b + 0.2531 * ceil_div(own, f.depth) + f.c * own * (wgs > num_cu ? f.per_cu : 1)) +
                              f.d * mb + operands;
             if (t < best) {

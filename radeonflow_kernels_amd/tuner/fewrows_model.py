@@ -3,12 +3,13 @@ measurements behind it, its fit, and the shapes where the few-rows and the tiled
 
   python -m radeonflow_kernels_amd.tuner.fewrows_model --measure FILE    every variant and K split over M = 1 ... 512 and the
                                                                          (N, K) of PAIRS, on operand sets in rotation
+  python -m radeonflow_kernels_amd.tuner.fewrows_model --ragged FILE     the same over ragged N: RAGGED_ROWS and RAGGED_PAIRS
   python -m radeonflow_kernels_amd.tuner.fewrows_model --fit FILE        how far the estimate's choice is from the fastest plan
                                                                          measured, and the constants refitted to the file
   python -m radeonflow_kernels_amd.tuner.fewrows_model --meet FILE       ragged shapes: the automatic few-rows plan against
                                                                          tiled plans with their staging copies
 FILE has one line per plan: M N K variant split_k us (--meet: for each shape the times of both sides). --measure and --meet
-need the GPU; the estimate and the fit do not.
+need the GPU, and so does --ragged; the estimate and the fit do not.
 """
 import argparse
 import os
@@ -30,12 +31,16 @@ FIT = {14: (0.0238, 0.6526, 0.0811), 16: (0.017, 1.6541, 0.0325), 20: (0.2932, 1
        22: (0.0007, 0.6572, 0.086), 23: (0.0704, 1.4481, 0.0227), 24: (0.0049, 0.9508, 0.0676), 25: (0.0106, 1.7903, 0.0289),
        26: (0.3722, 0.7608, 0.0427), 27: (1.0902, 1.385, 0.0109)}
 COMMON = (2.5568, 0.6363, 0.1919, 0.2531, 0.0505)   # launch; handing sums over, and per KiB of them; a batch of a wave's loads; a MB of operands
-ANY_BYTES = 1.27
+ANY_BYTES = {16: 1.5, 21: 1.5, 27: 1.5}              # where rows of B start at any byte; the other variants 1.27
 
 ROWS = (1, 7, 16, 24, 32, 48, 64, 100, 128, 200, 256, 333, 512)
 PAIRS = ((1536, 7168), (4608, 7168), (7168, 2048), (7168, 256), (576, 7168), (3072, 1536), (7168, 2304), (512, 7168), (4096, 512),
          (4096, 7168), (256, 1024), (1024, 2048), (2048, 4096), (8192, 1024), (8192, 7168), (256, 7168), (200, 2048), (1000, 384),
          (1000, 4096), (2003, 1024), (2003, 7168), (5003, 2048), (5003, 128))
+# the ragged N that ANY_BYTES is searched on
+RAGGED_ROWS = (1, 7, 16, 24, 40, 48, 64, 100, 150, 200, 333, 500)
+RAGGED_PAIRS = ((1000, 2048), (1000, 7168), (1001, 4096), (2003, 2048), (2003, 4096), (2003, 7168), (3001, 3072), (5003, 2048), (5003, 7168),
+                (1003, 1024), (2003, 384), (5003, 1024))
 # ragged shapes between a few hundred and a few thousand rows: N ragged, M ragged, both
 MEET = ((601, 5003, 2048), (700, 5003, 1024), (1000, 1000, 1024), (1000, 1000, 4096), (1000, 2003, 1024), (2000, 2003, 1024),
         (3000, 1000, 384), (700, 1000, 7168), (1008, 5003, 2048), (1500, 1000, 2048), (2000, 5003, 512), (2000, 1000, 7168),
@@ -69,7 +74,7 @@ def _features(variant, m, n, k, split, num_cu=256):
     if t is None:
         return None
     parts, kib, rounds, batches, blocks, mb = t
-    f = rounds * (ANY_BYTES if n % 16 else 1.0)
+    f = rounds * (ANY_BYTES.get(variant, 1.27) if n % 16 else 1.0)
     return (1.0, float(parts > 1), kib if parts > 1 else 0.0, f * batches, k * (m + n) * 1e-6, f, f * blocks, mb)
 
 
@@ -164,13 +169,13 @@ def report(rows, fit, common, what):
                                              100 * (np.mean(behind) - 1), 100 * (max(behind) - 1)))
 
 
-def measure(path):
+def measure(path, pairs=PAIRS, row_counts=ROWS):
     import radeonflow_kernels_amd as rfk
     from . import gemm_tuner as t
     t.settle(rfk)
     with open(path, "w") as f:
-        for n, k in PAIRS:
-            for m in ROWS:
+        for n, k in pairs:
+            for m in row_counts:
                 sets = t.operand_sets(m, n, k)
                 for v in VARIANTS:
                     for s in SPLITS:
@@ -218,11 +223,13 @@ def meet(path):
 
 def main():
     ap = argparse.ArgumentParser()
-    for name in ("measure", "fit", "meet"):
+    for name in ("measure", "ragged", "fit", "meet"):
         ap.add_argument("--" + name, metavar="FILE")
     a = ap.parse_args()
     if a.measure:
         measure(a.measure)
+    if a.ragged:
+        measure(a.ragged, RAGGED_PAIRS, RAGGED_ROWS)
     if a.fit:
         rows = read(a.fit)
         report(rows, FIT, COMMON, "%d measurements, constants in use" % len(rows))
