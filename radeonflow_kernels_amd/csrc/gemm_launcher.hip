@@ -851,9 +851,9 @@ size_t any_tile_part_bytes(int m, int n) { return (size_t)ceil_div(m, 16) * 16 *
 
 dim3 pad_grid_of_pieces(int pieces, int rows, int rounds);
 
-// Any shape and alignment. splits >= 1.
-int launch_any_tile(Mem &mem, const Variant &v, const void *a, const void *b, const float *as, const float *bs, void *c, int m, int n,
-                    int k, int splits, int group_m, hipStream_t stream) {
+// Any shape and alignment; rows of A and a_scale are ldm (>= m) long. splits >= 1.
+int launch_any_tile(Mem &mem, const Variant &v, const void *a, const void *b, const float *as, const float *bs, void *c, int m, int ldm,
+                    int n, int k, int splits, int group_m, hipStream_t stream) {
     const int qk = k / rf::BK, tiles_m = ceil_div(m, v.bm), tiles_n = ceil_div(n, v.bn), kb_per_split = ceil_div(qk, splits);
     splits = ceil_div(qk, kb_per_split);                    // every split owns at least one K block
     void *out = c;
@@ -864,7 +864,7 @@ int launch_any_tile(Mem &mem, const Variant &v, const void *a, const void *b, co
         out = ws;
     }
     hipLaunchKernelGGL(v.any_tile[splits > 1], dim3(tiles_m * tiles_n, splits), dim3(v.threads()), v.lds_bytes(), stream,
-                       (const uint8_t *)a, (const uint8_t *)b, as, bs, out, m, m, n, k, kb_per_split, tiles_m, tiles_n, group_m);
+                       (const uint8_t *)a, (const uint8_t *)b, as, bs, out, m, ldm, n, k, kb_per_split, tiles_m, tiles_n, group_m);
     RF_HIP(hipGetLastError());
     if (splits > 1) {
         const int np = ceil_div(n, 16) * 16;
@@ -959,8 +959,8 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
     const Variant &v = kVariants[cfg.variant];
     if (v.is_fewrows()) return launch_fewrows(mem, v, a, b, as, bs, c, m_store, m, n, k, cfg.split_k, stream);
     if (v.is_any_tile()) {
-        if (cfg.stream_k != RF_SCHEDULE_TILES || m_store != m) return fail(RF_ERR_BAD_CONFIG, "the any-alignment tiles have one schedule and no padded rows");
-        return launch_any_tile(mem, v, a, b, as, bs, c, m, n, k, cfg.split_k, cfg.group_m, stream);
+        if (cfg.stream_k != RF_SCHEDULE_TILES) return fail(RF_ERR_BAD_CONFIG, "the any-alignment tiles have one schedule");
+        return launch_any_tile(mem, v, a, b, as, bs, c, m_store, m, n, k, cfg.split_k, cfg.group_m, stream);
     }
     const int tiles_m = ceil_div(m, v.bm), tiles_n = ceil_div(n, v.bn);
     const int qk = k / rf::BK;
@@ -1309,7 +1309,7 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
                 cfg.split_k = 1;
             }
         }
-        return launch_any_tile(mem, kVariants[cfg.variant], a, b, as, bs, c, m, n, k, cfg.split_k, cfg.group_m, stream);
+        return launch_any_tile(mem, kVariants[cfg.variant], a, b, as, bs, c, m, m, n, k, cfg.split_k, cfg.group_m, stream);
     }
     if (kVariants[cfg.variant].is_fewrows()) {
         if (mem.fixed && cfg.split_k > 1) {                // as many K parts as the static array holds

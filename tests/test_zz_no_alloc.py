@@ -92,3 +92,26 @@ def test_static_entry_fits_the_plan_to_its_scratch_array(rfk, tmp_path):
     data = rk.generate_input_blockquant(256, 1536, 7168, 25)
     got, want = _both(rfk, data)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n", [512, 500])
+@pytest.mark.parametrize("piece", ["0 1 8 0", "28 2 8 0", "21 1 8 0", "29 1 8 0", "30 2 8 0"])
+def test_static_entry_in_row_ranges_takes_every_kind_of_plan(rfk, tmp_path, n, piece):
+    """A 36 MB staging copy of A, which a plan file's tile for the whole shape asks for: row ranges of 2512 and 2489 (padded to 2496)
+    rows, each with the plan that the file has for it: tiles with and without K parts, few-rows kernels, any-alignment tiles (these
+    were refused for a range with padded rows)."""
+    from helpers import exact_problem
+    m, k = 5001, 7168
+    plans = tmp_path / "ranges.plans"
+    plans.write_text("5008 512 7168 0 1 8 0\n2512 512 7168 %s\n2496 512 7168 %s\n" % (piece, piece))
+    data = exact_problem(m, n, k, seed=n)
+    g, buf = to_gpu(data, canary_elems=4096)
+    g[4].fill_(-3.0)
+    try:
+        assert rfk.load_plans(str(plans)) == 3
+        rfk.fp8_mm_static(*g)
+        torch.cuda.synchronize()
+    finally:
+        rfk.clear_plans()
+    assert np.array_equal(bf16_bits(g[4]), oracle_bf16(data))
+    assert bool((buf[g[4].numel():].float() == -7.0).all()), "store past the end of C"
