@@ -409,3 +409,24 @@ def test_short_k_plans_by_the_shape_of_the_output():
     assert plan(592, 4096, 512) == plan(848, 4096, 384) == plan(592, 3072, 512) == 28
     assert plan(1168, 4096, 512) == "skinny" and plan(592, 4096, 512, 304) == "skinny"      # 320 tiles; another device
     assert plan(592, 7168, 128) == "skinny" and plan(560, 7168, 128) != "skinny" and plan(592, 7168, 256) != "skinny"
+
+
+def test_staged_model_states_the_estimates_of_the_launcher():
+    """tuner/staged_model.py, where they are measured and fitted, picks what the launcher picks between the skinny-K schedule on staged
+    copies and the any-alignment tiles (beyond 4096 rows, where no few-rows kernel is considered), K split included."""
+    import numpy as np
+    import radeonflow_kernels_amd as rfk
+    from radeonflow_kernels_amd.tuner import staged_model as sm
+    seen = []
+    for i, (m, n, k, _, _) in enumerate(sm.shapes(11)):
+        m, n, k = m + 4097, -(-n // 64) * 64 - i % 16, min(k, 256)          # N padded to 16 is a multiple of 64: the schedule can run
+        if n % 16 == 0 or m * n < 6e6:
+            continue
+        tiles = min((float(np.dot(sm.any_terms(m, n, k, 0, 0, v, s), sm.ANY)), (v, s, 0)) for v in sm.ANY_TILES for s in (1, 2)
+                    if s <= k // 128 and (s == 1 or m * n * s < 3.9e7))
+        skinny = float(np.dot(sm.skinny_terms(m, n, k, 0, 0), sm.SKINNY_STAGED))
+        if abs(tiles[0] / skinny - 1) > 0.01:
+            got = rfk.plan_for(m, n, k, 256)
+            assert (got.variant, got.split_k, got.stream_k) == (tiles[1] if tiles[0] < skinny else sm.SKINNY), (m, n, k)
+            seen.append(got.stream_k)
+    assert min(seen.count(0), seen.count(4)) > 20

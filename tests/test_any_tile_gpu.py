@@ -127,3 +127,32 @@ def test_any_tile_nan_and_infinity(rfk):
         keep[:, n - 1] = False
         assert np.array_equal(bf16_bits(g[4]).reshape(m, n)[keep], clean[keep])
         assert not torch.isfinite(got[m - 1]).any()
+
+
+# rows of A or B of 17 million bytes: 127 of them, and C and the K parts' sums, are beyond 2^31
+@pytest.mark.parametrize("m,n,plans", [(130, 17000003, ((29, 1), (30, 1))), (17000003, 16, ((29, 1), (30, 1), (29, 2)))])
+def test_any_tile_offsets_beyond_31_bits(rfk, m, n, plans):
+    k, fp8 = 256, torch.float8_e4m3fn
+    gen = torch.Generator(device="cuda").manual_seed(n)
+
+    def signed_ones_and_twos(shape):                           # codes of 1, 2, -1 and -2
+        x = torch.randint(0, 4, shape, dtype=torch.uint8, device="cuda", generator=gen)
+        return 0x38 + ((x & 1) << 3) + ((x & 2) << 6)
+
+    a, b = (signed_ones_and_twos((k, x)).view(fp8) for x in (m, n))
+    sa = torch.randint(1, 3, (2, m), device="cuda", generator=gen).float()
+    sb = torch.randint(1, 3, (2, (n + 127) // 128), device="cuda", generator=gen).float()
+    buf = torch.full((m * n + 300,), -7.0, dtype=torch.bfloat16, device="cuda")
+    c = buf[:m * n].view(m, n)
+    step = 1 << 20
+    for v, split in plans:
+        c.fill_(-7.0)
+        rfk.fp8_mm(a.T, b.T, sa.T, sb.T, c, config=rfk.GemmConfig(v, split, 8, 0))
+        for x0 in range(0, max(m, n), step):                   # sums of integers below 2^12: exact in any order
+            rows, cols = (slice(None), slice(x0, x0 + step)) if n > m else (slice(x0, x0 + step), slice(None))
+            exp = 0
+            for kb in range(2):
+                part = a[kb * 128:kb * 128 + 128, rows].float().T @ b[kb * 128:kb * 128 + 128, cols].float()
+                exp = exp + part * sa[kb, rows][:, None] * sb[kb].repeat_interleave(128)[:n][cols][None, :]
+            assert torch.equal(c[rows, cols], exp.bfloat16()), (v, split, x0)
+        assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max()), (v, split)

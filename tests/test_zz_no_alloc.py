@@ -50,8 +50,8 @@ def test_static_entry_matches_the_allocating_entry_on_two_calls_in_a_row(rfk):
 
 def test_static_entry_fits_the_plan_to_its_scratch_array(rfk, tmp_path):
     """Shapes whose plan under rf_fp8_gemm needs more than the 32 MiB array still run, and allocate nothing:
-    * M = 5001 with K = 7168 (a 36 MB staging copy of A): computed in row ranges that take turns in the array;
-    * the same with a ragged N as well (B and C are staged too);
+    * M = 5001 with K = 7168 (36 MB of A): not staged, on tiles that take it as it is, with the K parts that fit;
+    * the same with a ragged N as well;
     * a plan file that asks for four K parts of 16.8 MB each: cut down to one part;
     * a stream-K plan from a plan file: replaced by the automatic plan.
     Exact data, so every fitted plan must give the oracle's bits (and rf_fp8_gemm's); then data with rounding in it
