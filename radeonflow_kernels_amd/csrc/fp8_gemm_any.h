@@ -13,7 +13,10 @@ struct AnyGeom {
     static_assert(BK * CPR_A % NT == 0 && BK * CPR_B % NT == 0, "whole loads per thread");
 };
 
-// tile_mainloop with the operands through registers.
+// tile_mainloop with the operands through registers: 16-byte loads at any byte into one of two register sets, from there into the stage
+// that the next K block reads. Bound by the latency of the loads and by LDS, which every byte is written to and read from by all waves:
+// a K block of a 128 x 128 tile takes 0.58 us, of a 128 x 256 tile 0.79, rows that start at any byte up to 0.4 us more. No copy of A or B
+// and none of C: 200 x 5003 x 2048 19.5 -> 14.3 us (few-rows kernels), 4096 x 1000 x 1024 19.8 -> 11.1 (128 x 128 tiles on a copy of B).
 template <int BM, int BN, int WAVES_M, int WAVES_N>
 __device__ __forceinline__ void tile_mainloop_any(
     const uint8_t *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ SA,

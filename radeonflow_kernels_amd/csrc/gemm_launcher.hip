@@ -102,8 +102,8 @@ struct Variant {
               rf::gemm_fp8_blockscale_tile<BM, BN, WM, WN, true>, nullptr, nullptr, 0, RF_ANY_C(BM, BN, WM, WN, 2) }
 // the same with three LDS stages: two K blocks in flight instead of one. A K block of these tiles is 0.4 us of MFMAs,
 // less than a load takes to come back from L2 or the Infinity Cache on a busy chip, so with two stages the loop ran at
-// the latency of its loads: 1024 x 4608 x 7168 45.6 -> 39.0 us, 256 x 7168 x 2304 15.6 -> 13.1 us; the plan of 50
-// of the 163 tabled shapes. The two-stage forms stay: they fit more workgroups per CU (64 x 128: three instead of
+// the latency of its loads: 1024 x 4608 x 7168 45.6 -> 39.0 us, 256 x 7168 x 2304 15.6 -> 13.1 us; the plan of 21
+// of the 163 tabled shapes, and variant 28 of 37. The two-stage forms stay: they fit more workgroups per CU (64 x 128: three instead of
 // two), which the smallest problems prefer. (128 x 128 with four waves and three stages never won; with eight it is variant 28.)
 #define RF_VARIANT_TILE_ONLY_NS3(BM, BN, WM, WN)                                           \
     Variant { BM, BN, WM, WN, rf::TileGeom<BM, BN, WM, WN, 3>::LDS_BYTES,                  \
@@ -766,11 +766,8 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // Few rows: the few-rows kernels, which need no staging, when they come out faster. The model above ranks tiled plans;
     // what their launches take is 3.1 us + 0.67 of its figure, and staging adds the copies' launches and bytes. B's term
     // counts C's way back for every plan, although plans of one K part and one workgroup per tile store into a ragged C
-    // themselves. Measured with that in place on 82 shapes of ragged N and 100 to 4096 rows, the plan taken is 4.0 % behind
-    // the best of either family on average, 39 % at worst (4096 x 1000 x 1024: 20.1 us on 128 x 128 tiles and a copy of C,
-    // 14.7 on 128 x 192 tiles); only M ragged, up to 512 rows: 3.0 % and 17 %. Counting C's way back (1.0 us + 0.9 us per
-    // million outputs) per plan instead made 33 of 187 shapes 5 % faster on average, but ten of them 1 to 31 % slower
-    // (664 x 3001 x 7168 43 -> 56 us: the figure of a K split is too high against that of one part).
+    // themselves. Counting it (1.0 us + 0.9 us per million outputs) per plan instead made 33 of 187 shapes 5 % faster on average,
+    // but ten of them 1 to 31 % slower (664 x 3001 x 7168 43 -> 56 us: the figure of a K split is too high against that of one part).
     double t = 3.1 + 0.67 * best_cost;
     if (stage & kStageA) t += 3.2 + 2.0 * k * m / 4e6;
     if (stage & kStageB) t += 7.0 + 2.0 * k * n / 5e6 + 4.0 * m * n / 5e6;
@@ -987,10 +984,11 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         const int strips = ceil_div(n, 256), units = ceil_div(m, 64);
         int per_strip = s.num_cu / strips;
         per_strip = per_strip < 1 ? 1 : per_strip > units ? units : per_strip;
-        // A C that the Infinity Cache does not hold is written band by band, all workgroups side by side, which memory takes
-        // faster than 256 streams far apart: K = 256, 8192 x 7168 30.7 -> 27.1 us, 6144 x 7168 19.9 -> 19.1; smaller ones are
-        // even or up to 3 % slower (1024 x 7168 5.5 -> 5.7), and so are the 64-row items of K = 384 and 512 (6144 x 7168 x 384
-        // 24.5 -> 25.0), which spend more on each item.
+        // From 40 million outputs on C is written band by band, all workgroups of a strip side by side, and not a stretch of rows each.
+        // Time with rounds over without, 96 shapes of 7 to 60 million outputs, N = 2048 ... 8192, operands and C in rotation: beyond 42
+        // million 0.98 on average (0.88 ... 1.02; 6272 x 7168 x 256 25.3 -> 22.3 us), 40 to 42 million 0.99, 32 to 39.5 million 1.00 at K = 128
+        // and 1.03 at K = 256, below 1.00 and 1.01 (0.94 ... 1.07, as the rows divide among the workgroups). All of these C are smaller than
+        // the Infinity Cache. The 64-row items of K = 384 and 512 spend more on each item (6144 x 7168 x 384 24.5 -> 25.0).
         const int rounds = qk <= 2 && (double)m * n >= 4.0e7 ? m / (per_strip * rf::SkinnyGeom<2>::IM) : 0;
         const int rest = ceil_div(m - rounds * per_strip * rf::SkinnyGeom<2>::IM, 64);
         const rf::SkinnyWork work = {strips, per_strip, skinny_bands_log2(m, n, qk, strips, per_strip), rounds, rest / per_strip, rest % per_strip};
