@@ -28,8 +28,8 @@
  * own, and when one more asks, the least recently used set changes hands: the new stream waits on the device for the
  * old stream's work enqueued so far (an event, no host wait). A stream that is being captured into a HIP graph cannot
  * take a set over and gets RF_ERR_BAD_CONFIG (its first 32 streams capture fine; rf_fp8_gemm_static never needs a set; an
- * automatic few-rows plan with a K split first gives way to one without temporary memory where the shape has one, and the
- * automatic grouped queue form to the mixed tiles).
+ * automatic few-rows plan with a K split first gives way to one without temporary memory where the shape has one, a plan on
+ * staged copies to tiles that take the operands as they are, and the automatic grouped queue form to the mixed tiles).
  * HIP graphs captured through this library refer to these buffers: a replay counts as a launch on the stream the graph
  * was captured on, whatever stream it runs on, and must not overlap that stream's other launches or the replays of
  * another graph captured on it (results of launches that do overlap are undefined; for the grouped queue form also those

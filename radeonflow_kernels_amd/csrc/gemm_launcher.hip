@@ -170,7 +170,7 @@ const Variant kVariants[] = {
     RF_VARIANT_ANY_TILE(128, 128, 4, 2),   // 29: 8 waves, wave tile 32 x 64
     RF_VARIANT_ANY_TILE(128, 256, 2, 4),   // 30: 8 waves, wave tile 64 x 64
 };
-constexpr int kFewRows64x64 = 20, kFirstFewRows = 14;
+constexpr int kFewRows64x64 = 20, kFirstFewRows = 14, kAnyTile128 = 29;
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
 // ---- process-wide state ---------------------------------------------------------------------
@@ -1341,6 +1341,11 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     if (mem.fixed && off > mem.fixed_left()) return launch_padded_in_pieces(s, mem, a, b, as, bs, c, m, n, k, stream);
     uint8_t *pad = nullptr;
     int rc = off ? mem.pad(off, &pad) : RF_OK;
+    if (rc != RF_OK && !mem.fixed && fewrows_ok(m, n)) {   // no memory for the copies: the tiles that need none, K in one part
+        (void)hipGetLastError();
+        g_last_error.clear();
+        return launch_any_tile(mem, kVariants[kAnyTile128], a, b, as, bs, c, m, m, n, k, 1, 8, stream);
+    }
     if (rc != RF_OK) return rc;
     const void *a2 = a, *b2 = b;
     const float *as2 = as;

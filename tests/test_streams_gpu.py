@@ -315,6 +315,56 @@ def test_small_few_rows_calls_under_capture_need_no_buffer_set(rfk):
             hip.hipStreamDestroy(h)
 
 
+def test_staged_calls_under_capture_without_a_buffer_set_take_tiles_that_need_none(rfk):
+    """All 32 buffer sets belong to other streams, and a stream under capture cannot take one over. Ragged shapes whose plan runs on
+    staged copies (the skinny-K schedule, 256 x 256 tiles) are recorded all the same, on tiles that take operands as they are."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    L = rfk.lib()
+    L.rf_gemm_destroy()
+    handles = []
+    for _ in range(33):
+        h = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(h)) == 0
+        handles.append(h)
+
+    def launch(g, h):
+        a, b, sa, sb, c = g
+        return L.rf_fp8_gemm(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), c.data_ptr(), a.shape[0], b.shape[0], a.shape[1], h)
+
+    try:
+        split = to_gpu(exact_problem(16, 1536, 7168, 1))
+        for h in handles[:32]:
+            assert launch(split, h) == 0
+            torch.cuda.synchronize()
+        for (m, n, k), schedule in (((2608, 4090, 128), 4), ((3056, 5003, 256), 0)):
+            plan = rfk.select_config(m, n, k)
+            assert (plan.variant, plan.stream_k) == (0, schedule)
+            data = exact_problem(m, n, k, m + n)
+            g, exp = to_gpu(data), oracle_bf16(data)
+            torch.cuda.synchronize()
+            cap, graph, graph_exec = handles[32], ctypes.c_void_p(), ctypes.c_void_p()
+            assert hip.hipStreamBeginCapture(cap, 2) == 0            # hipStreamCaptureModeRelaxed
+            rc = launch(g, cap)
+            assert hip.hipStreamEndCapture(cap, ctypes.byref(graph)) == 0
+            assert rc == 0, (m, n, k, L.rf_gemm_last_error())
+            assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, 0) == 0
+            for _ in range(3):
+                g[4].fill_(-1.0)
+                torch.cuda.synchronize()
+                assert hip.hipGraphLaunch(graph_exec, cap) == 0
+                torch.cuda.synchronize()
+                assert np.array_equal(bf16_bits(g[4]), exp), (m, n, k)
+                assert launch(split, handles[0]) == 0                # eager work between the replays
+                torch.cuda.synchronize()
+            hip.hipGraphExecDestroy(graph_exec)
+            hip.hipGraphDestroy(graph)
+    finally:
+        torch.cuda.synchronize()
+        L.rf_gemm_destroy()
+        for h in handles:
+            hip.hipStreamDestroy(h)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 200, 7168), (7, 1536, 7168), (100, 72, 256), (1024, 1536, 7168), (1000, 1536, 7168)])
 def test_workspace_bytes_covers_the_plan_that_runs(rfk, m, n, k):
     """rf_gemm_init with rf_gemm_workspace_bytes: for a tabled, a padded and a small ragged shape the figure is that of a K
