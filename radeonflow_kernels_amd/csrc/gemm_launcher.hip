@@ -1292,7 +1292,13 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     // tile, persistent) write the m true rows straight into c (their stores are masked by row), and the tile kernels
     // have a form for any c; otherwise C is staged and copied back.
     rf_gemm_config cfg;
-    select_config(mp, np, k, s.num_cu, stage_flags(m, n, (uintptr_t)a, (uintptr_t)b, (uintptr_t)c), &cfg);
+    const int stage = stage_flags(m, n, (uintptr_t)a, (uintptr_t)b, (uintptr_t)c);
+    select_config(mp, np, k, s.num_cu, stage, &cfg);
+    // The skinny-K schedule in the static array: a C that is staged and does not fit would be computed and copied back range by
+    // range, with launches for each, behind the tiles that write it in place: 8192 x 7160 x 256 138 us, 98; 2144 x 7860 x 256 47, 36.
+    if (mem.fixed && cfg.stream_k == RF_SCHEDULE_SKINNY_K && (np != n || (uintptr_t)c % 16 != 0) && fewrows_ok(m, n) &&
+        (size_t)mp * np * 2 + (size_t)k * ((size_t)mp + np) > mem.fixed_left())
+        any_tile_plan(mp, np, k, s.num_cu, stage, &cfg);
     if (kVariants[cfg.variant].is_any_tile()) {
         const size_t part = any_tile_part_bytes(m, n);
         if (mem.fixed && cfg.split_k > 1) {                // as many K parts as the static array holds

@@ -94,6 +94,32 @@ def test_static_entry_fits_the_plan_to_its_scratch_array(rfk, tmp_path):
     assert np.array_equal(got, want)
 
 
+def test_static_entry_writes_a_large_ragged_c_in_place(rfk):
+    """Short K, a ragged N and 33.6 MB of C: the plan stages B and C, which do not fit the array; one launch, and not one per range of
+    rows with its copies."""
+    from helpers import exact_problem
+    m, n, k = 4112, 4090, 256
+    assert rfk.select_config(m, n, k).stream_k == 4
+    data = exact_problem(m, n, k, seed=1)
+    g, buf = to_gpu(data, canary_elems=4096)
+    hip, graph, count = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p(), ctypes.c_size_t()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        handle = ctypes.c_void_p(stream.cuda_stream)
+        assert hip.hipStreamBeginCapture(handle, 2) == 0                 # hipStreamCaptureModeRelaxed
+        try:
+            rfk.fp8_mm_static(*g)
+        finally:
+            assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0 and count.value == 1
+        hip.hipGraphDestroy(graph)
+    g[4].fill_(-3.0)
+    rfk.fp8_mm_static(*g)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits(g[4]), oracle_bf16(data))
+    assert bool((buf[g[4].numel():].float() == -7.0).all()), "store past the end of C"
+
+
 @pytest.mark.parametrize("n", [512, 500])
 @pytest.mark.parametrize("piece", ["0 1 8 0", "28 2 8 0", "21 1 8 0", "29 1 8 0", "30 2 8 0"])
 def test_static_entry_in_row_ranges_takes_every_kind_of_plan(rfk, tmp_path, n, piece):
