@@ -583,8 +583,8 @@ constexpr int kFewRowsMaxM = 512, kFewRowsMaxMWide = 4096, kFewRowsSmallN = 1536
 // (and of C on the way back). kTiledOnly: no few-rows plan.
 // kBytesA, kBytesB: rows of that operand do not all start at a multiple of four bytes.
 // kFewRowsOnly: the few-rows plan (m and n as they are). kCutC: rows of C are not whole cache lines.
-// kCopyB: B is copied (kStageB without it: only C is unaligned).
-enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16, kFewRowsOnly = 32, kCutC = 64, kCopyB = 128 };
+// kCopyB: B is copied (kStageB without it: only C is unaligned). kNoSplitTiles: without split_tile_plan, whose plans want memory.
+enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16, kFewRowsOnly = 32, kCutC = 64, kCopyB = 128, kNoSplitTiles = 256 };
 
 // The flags of a shape and its pointers (0: aligned).
 int stage_flags(int m, int n, uintptr_t a, uintptr_t b, uintptr_t c) {
@@ -644,6 +644,53 @@ double skinny_staged_us(int qk, double mn, int stage) {
 
 // The same of one round of 128 x 128 tiles over three or four K blocks, nothing staged. 30 shapes, 2 % off.
 double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn; }
+
+// A plan of one workgroup per tile and K part in estimated microseconds, where K is long and the chip is not full of the largest tile:
+//   3.28 + rounds * (f + K blocks of a part * (c + g * share of the units at work)) + 0.693 per million outputs
+//   + 0.057 per million bytes of A and B + 2.47 + 1.18 per million sums when K is split
+// (the more units are at work the longer each waits for L2 and the longer a K block). Fitted to 330 shapes (48 to 2600 rows, N = 256 to
+// 8192, K = 1024 to 8192, half of them the benchmark's pairs), every variant below with 1 to 8 parts on operand sets in rotation: 6.6 % off
+// there, 6.7 % on 160 other shapes. `*out` is replaced where another plan comes out 6 % lower: 6 % of 6000 shapes drawn from these ranges
+// change plan, and 110 of those, timed in turn, are 14 % faster (geometric mean, up to 36 %), three 2 to 5 % slower. us: 1360 x 1536 x 7168
+// 41.4 (28, one part) -> 32.4 (10, three), 543 x 4096 x 7168 with its staging 46.0 -> 37.3, 255 x 8128 x 6144 38.3 -> 34.9. (Without the
+// margin 45 of 472 shapes come out more than 3 % slower.) The model in select_config_uncached, which ranks them first, counts a K split's
+// sums at twice what they cost against a K block, and a K block the same on half the chip as on all of it. Left out: the 64 x 128 tile in
+// one part, which takes plans from variant 12 that are up to 9 % faster. In 64 bits' terms the results are as exact as before (relative
+// error 1.660e-3 to 1.664e-3 on either side, the bf16 of C).
+struct SplitTileFit { int variant; double f, c, g; };
+constexpr SplitTileFit kSplitTileFits[] = {{9, 0.232, 0.462, 0.027}, {12, 0.0, 0.767, 0.401}, {28, 0.229, 0.434, 0.246}, {8, 0.716, 0.623, 0.255},
+                                           {10, 1.02, 0.77, 0.097}, {11, 0.981, 0.892, 0.085}, {0, 0.885, 1.313, 0.0}};
+double split_tile_us(const SplitTileFit &f, int m, int n, int k, int splits, int num_cu) {
+    const Variant &v = kVariants[f.variant];
+    const int qk = k / rf::BK;
+    const double wgs = (double)ceil_div(m, v.bm) * ceil_div(n, v.bn) * splits, mn = (double)m * n * 1e-6;
+    const double rounds = std::ceil(wgs / num_cu), blocks = v.k_groups > 1 ? qk / v.k_groups : ceil_div(qk, splits);
+    return 3.281 + rounds * (f.f + blocks * (f.c + f.g * wgs / num_cu / rounds)) + 0.693 * mn + 0.057e-6 * k * ((double)m + n) +
+           (splits > 1 ? 2.471 + 1.182 * mn * splits : 0.0);
+}
+void split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out) {
+    const int qk = k / rf::BK;
+    // (up to 512 rows variant 28 keeps the figure that the few-rows estimate was weighed against)
+    double best = 1e30;
+    for (const SplitTileFit &f : kSplitTileFits)
+        if (f.variant == out->variant) best = 0.94 * split_tile_us(f, m, n, k, ceil_div(qk, ceil_div(qk, out->split_k)), num_cu);
+    if (best == 1e30) return;                               // a plan that is not estimated here stays
+    for (const SplitTileFit &f : kSplitTileFits) {
+        const Variant &v = kVariants[f.variant];
+        if (f.variant == 28 && m <= kFewRowsMaxM) continue;
+        const double tiles = (double)ceil_div(m, v.bm) * ceil_div(n, v.bn);
+        for (int sp : {1, 2, 3, 4, 5, 6, 8}) {
+            if (sp > qk || ceil_div(qk, ceil_div(qk, sp)) != sp || (v.k_groups > 1 && (sp > 1 || qk % v.k_groups != 0))) continue;
+            if (sp == 1 && f.variant == 9) continue;
+            if (sp > 1 && (tiles * sp > 600 || (double)m * n * sp > 45.0e6)) continue;      // no more than was measured
+            const double t = split_tile_us(f, m, n, k, sp, num_cu);
+            if (t < best) {
+                best = t;
+                *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};
+            }
+        }
+    }
+}
 
 // Plan for a shape (m, n multiples of 16, the padded sizes when something is staged).
 void select_config_uncached(int m, int n, int k, int num_cu, int stage, const std::vector<TunedPlan> &user_plans,
@@ -797,6 +844,10 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // On 166 shapes that the fit has not seen (100 to 8192 rows, M or N or both ragged) the plan taken is 1.2 % behind the best of few
     // rows, these tiles with every K split and the plans of the padded shape on average, 24 % at worst.
     if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < t) *out = other;
+    if (!hit && num_cu == kTunedOnCUs && !(stage & (kStageB | kNoSplitTiles)) && out->stream_k == RF_SCHEDULE_TILES &&
+        !kVariants[out->variant].takes_any_shape() && qk >= 8 && m > 32 && m <= 2600 && n <= 8192 && (double)n * k <= 6.0e7 &&
+        ceil_div(m, 256) * ceil_div(n, 256) <= num_cu)
+        split_tile_plan(m, n, k, num_cu, out);
 }
 
 // The same through a small table of plans already worked out (the models take 1 to 3 us of host time, as long as a small
@@ -826,6 +877,19 @@ bool fewrows_split_fits(Mem &mem, const Variant &v, int m, int n, int k, int spl
     const int qk = k / rf::BK;
     float *slots = nullptr;
     if (mem.workspace(fewrows_slot_bytes(v, m, n, ceil_div(qk, ceil_div(qk, splits))), &slots) == RF_OK) return true;
+    (void)hipGetLastError();
+    g_last_error.clear();
+    return false;
+}
+
+// The same of a tiled plan's K split, beside `staged` bytes of copies; m rows of c.
+bool tile_split_fits(Mem &mem, const rf_gemm_config &cfg, int m, int n, int k, size_t staged) {
+    if (cfg.variant < 0 || cfg.split_k == 1 || cfg.stream_k != RF_SCHEDULE_TILES || kVariants[cfg.variant].takes_any_shape()) return true;
+    const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, cfg.split_k));
+    const size_t bytes = (size_t)m * n * sizeof(float) * parts;
+    if (mem.fixed) return bytes + staged <= mem.fixed_left();
+    float *ws = nullptr;
+    if (mem.workspace(bytes, &ws) == RF_OK) return true;
     (void)hipGetLastError();
     g_last_error.clear();
     return false;
@@ -929,13 +993,15 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         if (cfg.variant >= 0 && kVariants[cfg.variant].is_fewrows() &&
             !fewrows_split_fits(mem, kVariants[cfg.variant], m, n, k, cfg.split_k))
             select_config(m, n, k, s.num_cu, kTiledOnly, &cfg);
+        // no memory for a tiled plan's sums: the plan of the cost model alone
+        if (!tile_split_fits(mem, cfg, m_store, n, k, 0)) select_config(m, n, k, s.num_cu, kTiledOnly | kNoSplitTiles, &cfg);
     }
 
     if (mem.fixed && cfg.variant >= 0) {
         // rf_fp8_gemm_static: the plan has to live inside what is left of the static array. A stream-K plan (only a
         // plan file can name one) is replaced by the cost model's plan; a K split whose partial sums do not fit is cut
         // down to the number of parts that do, a single part needing no scratch memory at all.
-        if (cfg.stream_k == RF_SCHEDULE_STREAM_K) select_config_uncached(m, n, k, s.num_cu, 0, std::vector<TunedPlan>(), &cfg);
+        if (cfg.stream_k == RF_SCHEDULE_STREAM_K) select_config_uncached(m, n, k, s.num_cu, kNoSplitTiles, std::vector<TunedPlan>(), &cfg);
         if (cfg.stream_k == RF_SCHEDULE_STREAM_K) cfg.stream_k = RF_SCHEDULE_TILES;
         if (cfg.split_k > 1) {
             const Variant &fv = kVariants[cfg.variant];
@@ -1279,7 +1345,7 @@ int launch_padded_in_pieces(State &s, Mem &mem, const void *a, const void *b, co
         launch_pad_a_and_scales(a, as, r0, m, rp, k, 1, pa, (float *)psa, one_group(rows, rp), stream);
         RF_HIP(hipGetLastError());
         rf_gemm_config cfg;
-        select_config(rp, np, k, s.num_cu, 0, &cfg);
+        select_config(rp, np, k, s.num_cu, kNoSplitTiles, &cfg);
         void *c_piece = copy_c ? (void *)pc : (void *)((uint16_t *)c + (size_t)r0 * n);
         rc = launch_locked(s, mem, pa, b2, (const float *)psa, bs, c_piece, rp, np, k, &cfg, stream, copy_c ? rp : rows);
         if (rc != RF_OK) return rc;
@@ -1305,6 +1371,8 @@ int launch_padded(State &s, Mem &mem, const void *a, const void *b, const float 
     rf_gemm_config cfg;
     const int stage = stage_flags(m, n, (uintptr_t)a, (uintptr_t)b, (uintptr_t)c);
     select_config(mp, np, k, s.num_cu, stage, &cfg);
+    if (!(stage & kStageB) && !tile_split_fits(mem, cfg, m, n, k, (size_t)k * mp + align((size_t)qk * mp * sizeof(float)) + 1024))
+        select_config(mp, np, k, s.num_cu, stage | kNoSplitTiles, &cfg);
     // The skinny-K schedule in the static array: a C that is staged and does not fit would be computed and copied back range by
     // range, with launches for each, behind the tiles that write it in place: 8192 x 7160 x 256 138 us, 98; 2144 x 7860 x 256 47, 36.
     if (mem.fixed && cfg.stream_k == RF_SCHEDULE_SKINNY_K && (np != n || (uintptr_t)c % 16 != 0) && fewrows_ok(m, n) &&

@@ -430,3 +430,14 @@ def test_staged_model_states_the_estimates_of_the_launcher():
             assert (got.variant, got.split_k, got.stream_k) == (tiles[1] if tiles[0] < skinny else sm.SKINNY), (m, n, k)
             seen.append(got.stream_k)
     assert min(seen.count(0), seen.count(4)) > 20
+
+
+def test_long_k_on_a_part_of_the_chip_is_split():
+    """split_tile_plan: wide tiles in K parts where the model that ranks whole tiles kept one part; not for tabled shapes, staged B or C,
+    other compute unit counts, short K, or a chip full of the largest tile. Odd rows take the plan of the padded shape."""
+    import radeonflow_kernels_amd as rfk
+    plan = lambda *a: (lambda c: (c.variant, c.split_k, c.stream_k))(rfk.plan_for(*a))
+    assert plan(1360, 1536, 7168, 256) == plan(1355, 1536, 7168, 256) == (10, 3, 0)
+    assert plan(544, 4096, 7168, 256) == plan(543, 4096, 7168, 256) == (10, 3, 0) and plan(304, 1632, 2176, 256) == (9, 3, 0)
+    assert plan(1024, 1536, 7168, 256) == (28, 2, 0) and plan(1360, 1536, 7168, 304) == (28, 2, 0)
+    assert plan(1360, 1530, 7168, 256) != (10, 3, 0) and plan(1360, 1536, 896, 256)[1] == 1 and plan(8192, 8192, 7168, 256)[1] == 1

@@ -778,3 +778,26 @@ def test_k_split_inside_the_workgroup_on_random_shapes_equals_the_two_launch_for
         for v, twin in pairs:
             ref = _bits_under(rfk, ops, m, n, rfk.GemmConfig(twin, 2, 8, 0))
             assert np.array_equal(_bits_under(rfk, ops, m, n, rfk.GemmConfig(v, 1, 8, 0)), ref), (v, m, n, k)
+
+
+# K parts that divide the K blocks unevenly (17 in three), a single m-tile, odd rows (A staged); sums of 35.7 MB beyond the 32 MB static
+# array; sums that fit it alone but not beside a staged A (1195 rows); the large ones against one K part, in any order exact
+@pytest.mark.parametrize("m,n,k,oracle", [(304, 1632, 2176, True), (45, 5504, 7296, True), (48, 7856, 2304, True), (272, 8192, 7168, False),
+                                          (2256, 576, 7168, False), (1195, 1136, 7808, False)])
+def test_split_tile_plans_in_both_entries(rfk, m, n, k, oracle):
+    """Shapes that split_tile_plan moves to a K split: the bits of the oracle from the entry that allocates and from the one that cannot."""
+    assert rfk.select_config(m, n, k).split_k > 1
+    data = exact_problem(m, n, k, seed=m + n)
+    g, buf = to_gpu(data, 300)
+    if oracle:
+        exp = oracle_bf16(data)
+    else:
+        rfk.fp8_mm(*g, config=rfk.GemmConfig(29, 1, 8, 0))
+        torch.cuda.synchronize()
+        exp = bf16_bits(g[4])
+    for call in (rfk.fp8_mm, rfk.fp8_mm_static):
+        g[4].fill_(-1.0)
+        call(*g)
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(g[4]), exp), call.__name__
+    assert float(buf[m * n:].float().min()) == -7.0 == float(buf[m * n:].float().max())
