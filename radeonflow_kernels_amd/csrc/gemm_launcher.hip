@@ -660,6 +660,7 @@ double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn;
 struct SplitTileFit { int variant; double f, c, g; };
 constexpr SplitTileFit kSplitTileFits[] = {{9, 0.232, 0.462, 0.027}, {12, 0.0, 0.767, 0.401}, {28, 0.229, 0.434, 0.246}, {8, 0.716, 0.623, 0.255},
                                            {10, 1.02, 0.77, 0.097}, {11, 0.981, 0.892, 0.085}, {0, 0.885, 1.313, 0.0}};
+static_assert(kSplitTileFits[2].variant == 28, "named below");
 double split_tile_us(const SplitTileFit &f, int m, int n, int k, int splits, int num_cu) {
     const Variant &v = kVariants[f.variant];
     const int qk = k / rf::BK;
@@ -668,13 +669,14 @@ double split_tile_us(const SplitTileFit &f, int m, int n, int k, int splits, int
     return 3.281 + rounds * (f.f + blocks * (f.c + f.g * wgs / num_cu / rounds)) + 0.693 * mn + 0.057e-6 * k * ((double)m + n) +
            (splits > 1 ? 2.471 + 1.182 * mn * splits : 0.0);
 }
-void split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out) {
+// Returns the figure of the plan that it leaves in *out, 0 for one that is not estimated here.
+double split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out) {
     const int qk = k / rf::BK;
     // (up to 512 rows variant 28 keeps the figure that the few-rows estimate was weighed against)
-    double best = 1e30;
+    double kept = 0.0;
     for (const SplitTileFit &f : kSplitTileFits)
-        if (f.variant == out->variant) best = 0.94 * split_tile_us(f, m, n, k, ceil_div(qk, ceil_div(qk, out->split_k)), num_cu);
-    if (best == 1e30) return;                               // a plan that is not estimated here stays
+        if (f.variant == out->variant) kept = split_tile_us(f, m, n, k, ceil_div(qk, ceil_div(qk, out->split_k)), num_cu);
+    double best = 0.94 * kept;                              // (0: a plan that is not estimated here stays)
     for (const SplitTileFit &f : kSplitTileFits) {
         const Variant &v = kVariants[f.variant];
         if (f.variant == 28 && m <= kFewRowsMaxM) continue;
@@ -685,11 +687,12 @@ void split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out) {
             if (sp > 1 && (tiles * sp > 600 || (double)m * n * sp > 45.0e6)) continue;      // no more than was measured
             const double t = split_tile_us(f, m, n, k, sp, num_cu);
             if (t < best) {
-                best = t;
+                best = kept = t;
                 *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};
             }
         }
     }
+    return kept;
 }
 
 // Plan for a shape (m, n multiples of 16, the padded sizes when something is staged).
@@ -778,7 +781,8 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
                                {9, 0.73, 0.5},   {10, 0.53, 5.9},  {11, 0.71, 7.0}, {12, 0.93, 1.4}, {28, 0.44, 2.25}};
     const double f_next = 3.3, reduce_fixed = 6.03, reduce_per_elem = 1.27e-6, c_half_tile = 0.47, f_half_tile = 5.2;
     const int splits_tried[] = {1, 2, 3, 4, 6, 8, 12, 16};
-    double best_cost = 1e30;
+    double best_cost = 1e30, cost_28 = 1e30;
+    int split_28 = 1;
     if (!skinny && !one_round) for (const Candidate &cd : cands) {
         const Variant &v = kVariants[cd.variant];
         const long tiles = (long)ceil_div(m, v.bm) * ceil_div(n, v.bn);
@@ -802,6 +806,10 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
                 double t = sched == RF_SCHEDULE_PERSISTENT ? rounds * kb_per * cd.c + cd.f + (rounds - 1) * f_next
                                                            : rounds * (kb_per * cd.c + cd.f);
                 if (splits > 1) t += reduce_fixed + reduce_per_elem * splits * (double)m * n;
+                if (cd.variant == 28 && t < cost_28) {
+                    cost_28 = t;
+                    split_28 = sp;
+                }
                 if (t < best_cost) {
                     best_cost = t;
                     out->variant = cd.variant;
@@ -846,8 +854,18 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < t) *out = other;
     if (!hit && num_cu == kTunedOnCUs && !(stage & (kStageB | kNoSplitTiles)) && out->stream_k == RF_SCHEDULE_TILES &&
         !kVariants[out->variant].takes_any_shape() && qk >= 8 && m > 32 && m <= 2600 && n <= 8192 && (double)n * k <= 6.0e7 &&
-        ceil_div(m, 256) * ceil_div(n, 256) <= num_cu)
-        split_tile_plan(m, n, k, num_cu, out);
+        ceil_div(m, 256) * ceil_div(n, 256) <= num_cu) {
+        // The few-rows kernels again, 8 % below that figure of a plan of one K part (a tiled plan of long K has too low a `t` above), us:
+        // 256 x 3824 x 2560 17.3 -> 13.3, 384 x 2048 x 2048 10.3 -> 9.5, 64 x 8000 x 2304 14.0 -> 9.6. Of 6000 shapes 1.8 % change; 100 of them timed
+        // in turn are 9.4 % faster (geometric mean), two 5 and 7 % slower. Not against plans with a K split: 128 x 7344 x 4608 18.1 (28, four parts), 22.0.
+        // (Variant 28's best plan, which tuner/fewrows_model.py knows, has to be behind as well.)
+        const double tiled = split_tile_plan(m, n, k, num_cu, out);
+        if (m <= kFewRowsMaxM && out->split_k == 1 && !(stage & kTiledOnly) && fewrows_ok(m, n)) {
+            const double few = fewrows_plan(m, n, k, num_cu, false, &other);
+            const bool below_28 = split_28 == 1 ? few < 0.92 * split_tile_us(kSplitTileFits[2], m, n, k, 1, num_cu) : few < 3.1 + 0.67 * cost_28;
+            if (few < 0.92 * tiled && below_28) *out = other;
+        }
+    }
 }
 
 // The same through a small table of plans already worked out (the models take 1 to 3 us of host time, as long as a small

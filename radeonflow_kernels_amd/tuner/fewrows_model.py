@@ -93,6 +93,19 @@ def tile_estimate(m, n, k, split, num_cu=256):
     return 3.1 + 0.67 * (t + (6.03 + 1.27e-6 * parts * m * n if parts > 1 else 0.0))
 
 
+def long_k_tile_us(m, n, k, split, num_cu=256):
+    """split_tile_us of csrc/gemm_launcher.hip for variant 28, or None where the planner does not weigh it."""
+    qk = k // BK
+    if not (num_cu == 256 and qk >= 8 and 32 < m <= 512 and n <= 8192 and n * k <= 6.0e7 and _ceil(m, 256) * _ceil(n, 256) <= num_cu):
+        return None
+    kb = _ceil(qk, split)
+    parts = _ceil(qk, kb)
+    wgs, mn = _ceil(m, 128) * _ceil(n, 128) * parts, m * n * 1e-6
+    rounds = _ceil(wgs, num_cu)
+    return (3.281 + rounds * (0.229 + kb * (0.434 + 0.246 * wgs / num_cu / rounds)) + 0.693 * mn + 0.057e-6 * k * (m + n)
+            + (2.471 + 1.182 * mn * parts if parts > 1 else 0.0))
+
+
 def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
     """The (variant, split_k) the planner picks from variant 14 on. tiles: variant 28 among them (not for ragged operands)."""
     best = None
@@ -104,9 +117,14 @@ def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
             if best is None or t < best[0]:
                 best = (t, v, s)
     if tiles:
+        few = best
         for s in (1, 2, 3, 4, 6, 8, 12, 16):
             if s <= k // BK and tile_estimate(m, n, k, s, num_cu) < best[0]:
                 best = (tile_estimate(m, n, k, s, num_cu), 28, s)
+        if best[1:] == (28, 1):
+            us = long_k_tile_us(m, n, k, best[2], num_cu)
+            if us is not None and few[0] < 0.92 * us:
+                best = few
     return best[1:]
 
 

@@ -441,3 +441,5 @@ def test_long_k_on_a_part_of_the_chip_is_split():
     assert plan(544, 4096, 7168, 256) == plan(543, 4096, 7168, 256) == (10, 3, 0) and plan(304, 1632, 2176, 256) == (9, 3, 0)
     assert plan(1024, 1536, 7168, 256) == (28, 2, 0) and plan(1360, 1536, 7168, 304) == (28, 2, 0)
     assert plan(1360, 1530, 7168, 256) != (10, 3, 0) and plan(1360, 1536, 896, 256)[1] == 1 and plan(8192, 8192, 7168, 256)[1] == 1
+    # the few-rows kernels where they are well below the tiled plan of one part, not against a K split
+    assert plan(256, 3824, 2560, 256) == plan(384, 2048, 2048, 256) == (21, 1, 0) and plan(128, 7344, 4608, 256) == (28, 4, 0)
