@@ -21,6 +21,7 @@
 #include "fp8_gemm_skinny.h"
 #include "fp8_gemm_fewrows.h"
 #include "fp8_gemm_any.h"
+#include "grown_buffer.h"
 #include "plan_limits.h"
 #include "quantize_kernels.h"
 
@@ -352,14 +353,8 @@ struct Mem {
 
     template <typename T>
     int grow(T *&buf, size_t &have, size_t need) {
-        if (need <= have) return RF_OK;
-        // the old buffer may still be read by launches enqueued earlier: keep it until rf_gemm_destroy
-        if (buf) s.retired.push_back(buf);
-        const size_t want = need > have + have / 2 ? need : have + have / 2;
-        buf = nullptr;
-        have = 0;
-        RF_HIP(device_malloc((void **)&buf, want));
-        have = want;
+        // the old buffer may still be read by launches enqueued earlier: it is kept until rf_gemm_destroy
+        RF_HIP(rf::grow_buffer(buf, have, need, s.retired, device_malloc));
         return RF_OK;
     }
     int take_fixed(size_t bytes, void **out, const char *what) {
