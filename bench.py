@@ -49,7 +49,7 @@ EXTRA_CONFIGS = {
 RTOL, ATOL, ATOL_REFERENCE = 2e-2, 1e-2, 1e-3
 SETTLE_SECONDS = 0.4
 KERNEL_SOURCES = ("arrival_counter.h", "fp8_gemm_kernels.h", "fp8_gemm_persistent.h", "fp8_gemm_skinny.h", "fp8_gemm_fewrows.h", "fp8_gemm_any.h",
-                  "plan_limits.h", "gemm_launcher.hip")
+                  "grown_buffer.h", "plan_limits.h", "gemm_launcher.hip")
 
 
 def kernel_source_sha():
