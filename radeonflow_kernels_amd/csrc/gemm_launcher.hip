@@ -643,15 +643,16 @@ double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn;
 // A plan of one workgroup per tile and K part in estimated microseconds, where K is long and the chip is not full of the largest tile:
 //   3.28 + rounds * (f + K blocks of a part * (c + g * share of the units at work)) + 0.693 per million outputs
 //   + 0.057 per million bytes of A and B + 2.47 + 1.18 per million sums when K is split
-// (the more units are at work the longer each waits for L2 and the longer a K block). Fitted to 330 shapes (48 to 2600 rows, N = 256 to
-// 8192, K = 1024 to 8192, half of them the benchmark's pairs), every variant below with 1 to 8 parts on operand sets in rotation: 6.6 % off
-// there, 6.7 % on 160 other shapes. `*out` is replaced where another plan comes out 6 % lower: 6 % of 6000 shapes drawn from these ranges
-// change plan, and 110 of those, timed in turn, are 14 % faster (geometric mean, up to 36 %), three 2 to 5 % slower. us: 1360 x 1536 x 7168
-// 41.4 (28, one part) -> 32.4 (10, three), 543 x 4096 x 7168 with its staging 46.0 -> 37.3, 255 x 8128 x 6144 38.3 -> 34.9. (Without the
-// margin 45 of 472 shapes come out more than 3 % slower.) The model in select_config_uncached, which ranks them first, counts a K split's
-// sums at twice what they cost against a K block, and a K block the same on half the chip as on all of it. Left out: the 64 x 128 tile in
-// one part, which takes plans from variant 12 that are up to 9 % faster. In 64 bits' terms the results are as exact as before (relative
-// error 1.660e-3 to 1.664e-3 on either side, the bf16 of C).
+// (the more units are at work the longer each waits for L2 and the longer a K block). Fitted to the plans within 1.5 times the fastest of
+// 310 shapes (48 to 2464 rows, N = 256 to 8192, K = 1024 to 8192, 40 % of them the benchmark's pairs of N and K), every variant below with 1
+// to 8 parts on operand sets in rotation. 7.8 % off (root mean square, 43 % at worst) over all 6797 plans of these shapes, 6.6 % over those
+// fitted; 7.8 % and 42 % over 3583 plans of 158 other shapes. The model in select_config_uncached, which ranks plans first, counts a K
+// split's sums at twice what they cost against a K block, and a K block the same on half the chip as on all of it. `*out` is replaced where
+// another plan comes out 6 % lower, but for the exceptions in split_tile_plan: 8 % of the shapes in the range. Of 846 such shapes, drawn
+// for the purpose and timed in turn, the new plans are 16 % faster (geometric mean, up to 42 %), three 2 to 6 % slower (448 x 1600 x 3328 14.6 ->
+// 15.4). us: 1360 x 1536 x 7168 41.4 (28, one part) -> 32.4 (10, three), 543 x 4096 x 7168 with its staging 46.0 -> 37.3. Left out: the 64 x 128
+// tile in one part, which takes plans from variant 12 that are up to 9 % faster. In 64 bits' terms the results are as exact as before
+// (relative error 1.660e-3 to 1.664e-3 on either side, the bf16 of C).
 struct SplitTileFit { int variant; double f, c, g; };
 constexpr SplitTileFit kSplitTileFits[] = {{9, 0.232, 0.462, 0.027}, {12, 0.0, 0.767, 0.401}, {28, 0.229, 0.434, 0.246}, {8, 0.716, 0.623, 0.255},
                                            {10, 1.02, 0.77, 0.097}, {11, 0.981, 0.892, 0.085}, {0, 0.885, 1.313, 0.0}};
@@ -667,21 +668,29 @@ double split_tile_us(const SplitTileFit &f, int m, int n, int k, int splits, int
 // Returns the figure of the plan that it leaves in *out, 0 for one that is not estimated here.
 double split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out) {
     const int qk = k / rf::BK;
-    // (up to 512 rows variant 28 keeps the figure that the few-rows estimate was weighed against)
-    double kept = 0.0;
+    const rf_gemm_config first = *out;
+    const bool many = m > kFewRowsMaxM;
+    double before = 0.0;                                    // stays 0 for a plan that is not estimated here, which stays too
     for (const SplitTileFit &f : kSplitTileFits)
-        if (f.variant == out->variant) kept = split_tile_us(f, m, n, k, ceil_div(qk, ceil_div(qk, out->split_k)), num_cu);
-    double best = 0.94 * kept;                              // (0: a plan that is not estimated here stays)
+        if (f.variant == first.variant) before = split_tile_us(f, m, n, k, ceil_div(qk, ceil_div(qk, first.split_k)), num_cu);
+    // Where 6 % are not enough, or nothing is, of 1739 shapes whose plan it changed (timed in turn; ratio to the plan before, geometric
+    // mean and worst): a K split already and 129 to 192 rows, 95 shapes 0.98 and 1.25 (160 x 7968 x 6656 28.6 us in two parts of variant
+    // 28, 35.9 in four of 10); variant 12 replaced beyond 512 rows by 9 at all, 35 shapes 0.93 and 1.16 (640 x 1536 x 3584 14.6, 16.9), or
+    // for 6 to 10 %, 25 shapes 0.86 and 1.13 (1024 x 704 x 3072 12.9, 14.7); 28 replaced beyond 512 rows by 9 for 6 to 10 %, 21 shapes 0.93
+    // and 1.06. Mostly N is a multiple of 128 there: the plan before then reads whole lines of B and is up to 15 % below its estimate.
+    if (first.split_k > 1 && m > 128 && m <= 192) return before;
+    double kept = before, best = (many && first.variant == 12 ? 0.90 : 0.94) * before;
     for (const SplitTileFit &f : kSplitTileFits) {
         const Variant &v = kVariants[f.variant];
-        if (f.variant == 28 && m <= kFewRowsMaxM) continue;
+        // (up to 512 rows variant 28 in more parts is not tried: the few-rows kernels were weighed against its plan of the first model)
+        if ((f.variant == 28 && !many) || (f.variant == 9 && many && first.variant == 12)) continue;
         const double tiles = (double)ceil_div(m, v.bm) * ceil_div(n, v.bn);
         for (int sp : {1, 2, 3, 4, 5, 6, 8}) {
             if (sp > qk || ceil_div(qk, ceil_div(qk, sp)) != sp || (v.k_groups > 1 && (sp > 1 || qk % v.k_groups != 0))) continue;
             if (sp == 1 && f.variant == 9) continue;
             if (sp > 1 && (tiles * sp > 600 || (double)m * n * sp > 45.0e6)) continue;      // no more than was measured
             const double t = split_tile_us(f, m, n, k, sp, num_cu);
-            if (t < best) {
+            if (t < best && (f.variant != 9 || !many || t < 0.90 * before)) {
                 best = kept = t;
                 *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};
             }

@@ -443,3 +443,15 @@ def test_long_k_on_a_part_of_the_chip_is_split():
     assert plan(1360, 1530, 7168, 256) != (10, 3, 0) and plan(1360, 1536, 896, 256)[1] == 1 and plan(8192, 8192, 7168, 256)[1] == 1
     # the few-rows kernels where they are well below the tiled plan of one part, not against a K split
     assert plan(256, 3824, 2560, 256) == plan(384, 2048, 2048, 256) == (21, 1, 0) and plan(128, 7344, 4608, 256) == (28, 4, 0)
+
+
+@pytest.mark.parametrize("shape,plan", [
+    ((160, 7968, 6656), (28, 2)), ((176, 7808, 7296), (28, 2)), ((144, 8000, 6784), (28, 2)), ((176, 6016, 6912), (28, 2)),
+    ((144, 8192, 7168), (28, 2)), ((176, 7424, 8064), (28, 2)), ((144, 5808, 8192), (8, 4)), ((144, 3584, 3840), (28, 4)),
+    ((640, 1536, 3584), (12, 1)), ((592, 1536, 3328), (12, 1)), ((1024, 704, 3072), (12, 1)),
+    ((560, 1792, 3200), (28, 1))])
+def test_long_k_keeps_plans_that_a_k_split_made_slower(shape, plan):
+    """Shapes that split_tile_plan moved to a K split 3 to 25 % slower than the plan that they have without it."""
+    import radeonflow_kernels_amd as rfk
+    got = rfk.plan_for(*shape, 256)
+    assert (got.variant, got.split_k, got.stream_k) == (*plan, 0)
