@@ -860,14 +860,19 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
         !kVariants[out->variant].takes_any_shape() && qk >= 8 && m > 32 && m <= 2600 && n <= 8192 && (double)n * k <= 6.0e7 &&
         ceil_div(m, 256) * ceil_div(n, 256) <= num_cu) {
         // The few-rows kernels again, 8 % below that figure of a plan of one K part (a tiled plan of long K has too low a `t` above), us:
-        // 256 x 3824 x 2560 17.3 -> 13.3, 384 x 2048 x 2048 10.3 -> 9.5, 64 x 8000 x 2304 14.0 -> 9.6. Of 6000 shapes 1.8 % change; 100 of them timed
-        // in turn are 9.4 % faster (geometric mean), two 5 and 7 % slower. Not against plans with a K split: 128 x 7344 x 4608 18.1 (28, four parts), 22.0.
+        // 256 x 3824 x 2560 17.3 -> 13.3, 384 x 2048 x 2048 10.3 -> 9.5, 64 x 8000 x 2304 14.0 -> 9.6. Not against plans with a K split: 128 x
+        // 7344 x 4608 18.1 (28, four parts), 22.0. Where 8 % are not enough, of 654 shapes that changed plan (timed in turn; ratio to the plan
+        // before, geometric mean and worst): more than 128 rows and K below 1792, where the estimate of the tiles is up to 20 % high, 169
+        // shapes 0.97 and 1.13 (144 x 6208 x 1408 9.1 -> 9.8), none; more than 128 rows and whole lines of B, 10 to 18 % lower, 29 shapes 0.95
+        // and 1.05; up to 128 rows and K below 1792, 8 to 10 % lower, 22 shapes 0.93 and 1.04. Of 182 other shapes that still change, drawn
+        // for the purpose, all are 12 % faster (geometric mean), none more than 2 % slower.
         // (Variant 28's best plan, which tuner/fewrows_model.py knows, has to be behind as well.)
         const double tiled = split_tile_plan(m, n, k, num_cu, out);
+        const double share = m > 128 ? (qk < 14 ? 0.0 : n % 128 == 0 ? 0.82 : 0.92) : qk < 14 ? 0.90 : 0.92;
         if (m <= kFewRowsMaxM && out->split_k == 1 && !(stage & kTiledOnly) && fewrows_ok(m, n)) {
             const double few = fewrows_plan(m, n, k, num_cu, false, &other);
-            const bool below_28 = split_28 == 1 ? few < 0.92 * split_tile_us(kSplitTileFits[2], m, n, k, 1, num_cu) : few < 3.1 + 0.67 * cost_28;
-            if (few < 0.92 * tiled && below_28) *out = other;
+            const bool below_28 = split_28 == 1 ? few < share * split_tile_us(kSplitTileFits[2], m, n, k, 1, num_cu) : few < 3.1 + 0.67 * cost_28;
+            if (few < share * tiled && below_28) *out = other;
         }
     }
 }

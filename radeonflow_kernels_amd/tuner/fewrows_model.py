@@ -106,6 +106,13 @@ def long_k_tile_us(m, n, k, split, num_cu=256):
             + (2.471 + 1.182 * mn * parts if parts > 1 else 0.0))
 
 
+def long_k_share(m, n, k):
+    """What part of that figure the few-rows estimate has to stay below (0: it is not weighed)."""
+    if m > 128:
+        return 0.0 if k < 14 * BK else 0.82 if n % 128 == 0 else 0.92
+    return 0.90 if k < 14 * BK else 0.92
+
+
 def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
     """The (variant, split_k) the planner picks from variant 14 on. tiles: variant 28 among them (not for ragged operands)."""
     best = None
@@ -123,7 +130,7 @@ def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
                 best = (tile_estimate(m, n, k, s, num_cu), 28, s)
         if best[1:] == (28, 1):
             us = long_k_tile_us(m, n, k, best[2], num_cu)
-            if us is not None and few[0] < 0.92 * us:
+            if us is not None and few[0] < long_k_share(m, n, k) * us:
                 best = few
     return best[1:]
 

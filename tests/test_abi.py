@@ -455,3 +455,14 @@ def test_long_k_keeps_plans_that_a_k_split_made_slower(shape, plan):
     import radeonflow_kernels_amd as rfk
     got = rfk.plan_for(*shape, 256)
     assert (got.variant, got.split_k, got.stream_k) == (*plan, 0)
+
+
+@pytest.mark.parametrize("shape,plan", [
+    ((256, 4064, 1664), (28, 1)), ((144, 6208, 1408), (28, 1)), ((208, 4064, 1152), (28, 1)), ((160, 5440, 1152), (28, 1)),
+    ((192, 5376, 1280), (12, 1)), ((160, 5824, 1024), (12, 1)), ((240, 2944, 2048), (12, 1)), ((208, 3456, 2304), (12, 1)),
+    ((128, 7296, 1152), (28, 1))])
+def test_long_k_keeps_tiled_plans_that_few_rows_kernels_made_slower(shape, plan):
+    """Shapes that the second comparison moved to few-rows kernels 3 to 13 % slower than the tiles they have without it."""
+    import radeonflow_kernels_amd as rfk
+    got = rfk.plan_for(*shape, 256)
+    assert (got.variant, got.split_k, got.stream_k) == (*plan, 0)
