@@ -665,6 +665,10 @@ double split_tile_us(const SplitTileFit &f, int m, int n, int k, int splits, int
     return 3.281 + rounds * (f.f + blocks * (f.c + f.g * wgs / num_cu / rounds)) + 0.693 * mn + 0.057e-6 * k * ((double)m + n) +
            (splits > 1 ? 2.471 + 1.182 * mn * splits : 0.0);
 }
+// The sizes it was fitted to and checked on; plans beyond them stay as the first model has them.
+bool long_k_range(int m, int n, int k) {
+    return m >= 48 && m <= 2608 && n >= 256 && n <= 8192 && k >= 1024 && k <= 8192 && (double)n * k <= 6.0e7;
+}
 // Returns the figure of the plan that it leaves in *out, 0 for one that is not estimated here.
 double split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out) {
     const int qk = k / rf::BK;
@@ -857,8 +861,7 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     // rows, these tiles with every K split and the plans of the padded shape on average, 24 % at worst.
     if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < t) *out = other;
     if (!hit && num_cu == kTunedOnCUs && !(stage & (kStageB | kNoSplitTiles)) && out->stream_k == RF_SCHEDULE_TILES &&
-        !kVariants[out->variant].takes_any_shape() && qk >= 8 && m > 32 && m <= 2600 && n <= 8192 && (double)n * k <= 6.0e7 &&
-        ceil_div(m, 256) * ceil_div(n, 256) <= num_cu) {
+        !kVariants[out->variant].takes_any_shape() && long_k_range(m, n, k) && ceil_div(m, 256) * ceil_div(n, 256) <= num_cu) {
         // The few-rows kernels again, 8 % below that figure of a plan of one K part (a tiled plan of long K has too low a `t` above), us:
         // 256 x 3824 x 2560 17.3 -> 13.3, 384 x 2048 x 2048 10.3 -> 9.5, 64 x 8000 x 2304 14.0 -> 9.6. Not against plans with a K split: 128 x
         // 7344 x 4608 18.1 (28, four parts), 22.0. Where 8 % are not enough, of 654 shapes that changed plan (timed in turn; ratio to the plan

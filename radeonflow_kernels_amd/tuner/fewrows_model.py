@@ -96,7 +96,8 @@ def tile_estimate(m, n, k, split, num_cu=256):
 def long_k_tile_us(m, n, k, split, num_cu=256):
     """split_tile_us of csrc/gemm_launcher.hip for variant 28, or None where the planner does not weigh it."""
     qk = k // BK
-    if not (num_cu == 256 and qk >= 8 and 32 < m <= 512 and n <= 8192 and n * k <= 6.0e7 and _ceil(m, 256) * _ceil(n, 256) <= num_cu):
+    if not (num_cu == 256 and 48 <= m <= 512 and 256 <= n <= 8192 and 1024 <= k <= 8192 and n * k <= 6.0e7 and
+            _ceil(m, 256) * _ceil(n, 256) <= num_cu):
         return None
     kb = _ceil(qk, split)
     parts = _ceil(qk, kb)

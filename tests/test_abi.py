@@ -466,3 +466,12 @@ def test_long_k_keeps_tiled_plans_that_few_rows_kernels_made_slower(shape, plan)
     import radeonflow_kernels_amd as rfk
     got = rfk.plan_for(*shape, 256)
     assert (got.variant, got.split_k, got.stream_k) == (*plan, 0)
+
+
+@pytest.mark.parametrize("shape,plan", [((2349, 2064, 26496), (8, 1)), ((1796, 1264, 34304), (10, 3)), ((1904, 512, 24576), (28, 4)),
+                                        ((336, 4096, 8320), (28, 2)), ((1360, 1536, 8320), (28, 1)), ((2240, 224, 3328), (12, 1))])
+def test_long_k_estimate_is_not_used_beyond_the_sizes_it_was_measured_on(shape, plan):
+    """K above 8192 and N below 256: the plans of the model that ranks whole tiles."""
+    import radeonflow_kernels_amd as rfk
+    got = rfk.plan_for(*shape, 256)
+    assert (got.variant, got.split_k, got.stream_k) == (*plan, 0)
