@@ -1035,8 +1035,9 @@ int launch_locked(State &s, Mem &mem, const void *a, const void *b, const float 
         if (cfg.stream_k == RF_SCHEDULE_STREAM_K) cfg.stream_k = RF_SCHEDULE_TILES;
         if (cfg.split_k > 1) {
             const Variant &fv = kVariants[cfg.variant];
-            const size_t per_part = fv.is_fewrows() ? fewrows_slot_bytes(fv, m, n, 1)
-                                    : fv.is_any_tile() ? any_tile_part_bytes(m, n) : (size_t)m * n * sizeof(float);
+            // (of the rows of c, as the launches below have it)
+            const size_t per_part = fv.is_fewrows() ? fewrows_slot_bytes(fv, m_store, n, 1)
+                                    : fv.is_any_tile() ? any_tile_part_bytes(m_store, n) : (size_t)m_store * n * sizeof(float);
             const int qk_ = k / rf::BK, kb_per = ceil_div(qk_, cfg.split_k), parts = ceil_div(qk_, kb_per);
             const size_t fit = mem.fixed_left() / per_part;
             if ((size_t)parts > fit) cfg.split_k = fit < 2 ? 1 : (int)fit;

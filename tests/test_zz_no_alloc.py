@@ -141,3 +141,40 @@ def test_static_entry_in_row_ranges_takes_every_kind_of_plan(rfk, tmp_path, n, p
         rfk.clear_plans()
     assert np.array_equal(bf16_bits(g[4]), oracle_bf16(data))
     assert bool((buf[g[4].numel():].float() == -7.0).all()), "store past the end of C"
+
+
+def _plan_bits(rfk, ops, m, n, cfg):
+    """Bits of the first m rows of an aligned problem under an explicit plan."""
+    a, b, sa, sb = ops
+    c = torch.zeros((a.shape[0], n), dtype=torch.bfloat16, device="cuda")
+    rfk.fp8_mm(a, b, sa, sb, c, config=rfk.GemmConfig(*cfg, 8, 0))
+    torch.cuda.synchronize()
+    return bf16_bits(c[:m])
+
+
+def _static_bits_and_plans(rfk, m, n, k, plans):
+    """rf_fp8_gemm_static on data whose sums round, so that the bits tell the number of K parts, and each plan's bits on the same
+    problem with its rows padded to a multiple of 16."""
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    mp, qk, fp8 = -(-m // 16) * 16, k // 128, torch.float8_e4m3fn
+    a, sa = torch.randint(0, 120, (k, mp), dtype=torch.uint8, device="cuda", generator=gen), torch.rand((qk, mp), device="cuda", generator=gen)
+    a ^= torch.randint(0, 2, (k, mp), dtype=torch.uint8, device="cuda", generator=gen) << 7
+    b, sb = torch.randint(0, 120, (k, n), dtype=torch.uint8, device="cuda", generator=gen).view(fp8).T, torch.rand((qk, -(-n // 128)), device="cuda", generator=gen).T
+    c = torch.full((m, n), -3.0, dtype=torch.bfloat16, device="cuda")
+    rfk.fp8_mm_static(a[:, :m].contiguous().view(fp8).T, b, sa[:, :m].contiguous().T, sb, c)
+    torch.cuda.synchronize()
+    ops = (a.view(fp8).T, b, sa.T, sb)
+    return bf16_bits(c), [_plan_bits(rfk, ops, m, n, p) for p in plans]
+
+
+def test_static_entry_counts_the_rows_of_c_for_a_staged_k_split(rfk):
+    """Sums that fit beside the staged A as the 625 rows that are written, but not as the 640 that are computed: the plan's three
+    parts, which were cut to two."""
+    m, n, k = 625, 3792, 7040
+    cfg = rfk.select_config(m, n, k)
+    assert cfg.split_k == 3 and cfg.stream_k == 0
+    staged = k * 640 + k // 128 * 640 * 4
+    assert staged + 3 * 4 * m * n <= rfk.lib().rf_gemm_static_scratch_bytes() < staged + 3 * 4 * 640 * n
+    got, (three, two) = _static_bits_and_plans(rfk, m, n, k, [(cfg.variant, 3), (cfg.variant, 2)])
+    assert not np.array_equal(three, two)
+    assert np.array_equal(got, three)
