@@ -114,9 +114,10 @@ int rf_fp8_gemm(const void *a, const void *b, const float *as, const float *bs, 
  * rf_gemm_static_scratch_bytes() bytes (32 MiB; every GPU the library has run on holds one until the process ends),
  * and the call allocates and frees nothing. The plan is rf_fp8_gemm's, and so are the result bits, whenever that plan
  * fits the array. Otherwise the plan is fitted to it: a K split is cut down to as many parts as fit (one part needs no
- * scratch memory), a stream-K plan from a plan file is replaced by the automatic plan, and a ragged or unaligned shape
- * whose staging copies do not fit as a whole is computed in row ranges that take turns in the array (M = 6001, N = 4608,
- * K = 7168: two ranges); such results agree with rf_fp8_gemm's within the rounding of another K split, and bit for bit
+ * scratch memory) or, where it was chosen for a long K by estimate (K = 1024 to 8192, up to 2608 rows), gives way to the plan
+ * estimated fastest among those that fit, a stream-K plan from a plan file is replaced by the automatic plan, and a ragged
+ * or unaligned shape whose staging copies do not fit as a whole is computed in row ranges that take turns in the array
+ * (M = 6001, N = 4608, K = 7168: two ranges); such results agree with rf_fp8_gemm's within the rounding of another K split, and bit for bit
  * on data whose sums are exact. Only when the staged copy of B (ragged N or an unaligned b) alone takes more than half
  * of the array does a few-rows kernel (64 x 64 tiles) compute the shape, in place. All calls on one GPU share that
  * GPU's array: two calls that overlap in time (different streams, or graph replays beside eager launches) race, and the

@@ -781,7 +781,8 @@ def test_k_split_inside_the_workgroup_on_random_shapes_equals_the_two_launch_for
 
 
 # K parts that divide the K blocks unevenly (17 in three), a single m-tile, odd rows (A staged); sums of 35.7 MB beyond the 32 MB static
-# array; sums that fit it alone but not beside a staged A (1195 rows); the large ones against one K part, in any order exact
+# array; sums that fit it alone but not beside a staged A (1195 rows); the large ones against one K part. The sums are exact in any order: this
+# is a test of the bits, not of the plan that runs (test_static_entry_fits_a_long_k_plan_to_its_scratch_array tells which one does)
 @pytest.mark.parametrize("m,n,k,oracle", [(304, 1632, 2176, True), (45, 5504, 7296, True), (48, 7856, 2304, True), (272, 8192, 7168, False),
                                           (2256, 576, 7168, False), (1195, 1136, 7808, False)])
 def test_split_tile_plans_in_both_entries(rfk, m, n, k, oracle):

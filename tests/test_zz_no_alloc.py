@@ -178,3 +178,19 @@ def test_static_entry_counts_the_rows_of_c_for_a_staged_k_split(rfk):
     got, (three, two) = _static_bits_and_plans(rfk, m, n, k, [(cfg.variant, 3), (cfg.variant, 2)])
     assert not np.array_equal(three, two)
     assert np.array_equal(got, three)
+
+
+# aligned and beyond the array by itself, A staged beside the sums; the plan before the rule for long K in one part and in two
+@pytest.mark.parametrize("m,n,k,runs", [(272, 8192, 7168, (28, 1)), (400, 5664, 7936, (10, 2)), (1361, 1536, 7168, (28, 1)),
+                                        (1195, 1136, 7808, (28, 2)), (1228, 1616, 7552, (10, 3)), (716, 1952, 8192, (10, 4))])
+def test_static_entry_fits_a_long_k_plan_to_its_scratch_array(rfk, m, n, k, runs):
+    """Plans of split_tile_plan whose sums do not fit: the one that runs is neither theirs nor theirs with fewer parts unless that
+    is estimated fastest among those that fit. Data that round tell the K parts by their bits."""
+    cfg, qk = rfk.select_config(m, n, k), k // 128
+    staged = (k + 4 * qk) * -(-m // 16) * 16 if m % 16 else 0
+    fit = (rfk.lib().rf_gemm_static_scratch_bytes() - staged) // (4 * m * n)
+    assert cfg.split_k > fit and cfg.stream_k == 0 and runs[1] <= fit
+    others = [(cfg.variant, p) for p in range(1, cfg.split_k + 1) if p != runs[1] and -(-qk // -(-qk // p)) == p]
+    got, bits = _static_bits_and_plans(rfk, m, n, k, [runs] + others)
+    assert np.array_equal(got, bits[0])
+    assert not any(np.array_equal(got, x) for x in bits[1:])
