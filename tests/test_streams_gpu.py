@@ -449,3 +449,65 @@ def test_automatic_grouped_calls_under_capture_without_a_buffer_set_take_a_form_
         L.rf_gemm_destroy()
         for h in handles:
             hip.hipStreamDestroy(h)
+
+
+@pytest.mark.parametrize("m,runs", [(1360, (28, 1)), (1355, (29, 1))])
+def test_long_k_plans_under_capture_without_a_buffer_set_take_one_k_part(rfk, m, runs):
+    """All 32 buffer sets belong to other streams, and a stream under capture cannot take one over: a shape that split_tile_plan moves
+    to three K parts is recorded as one kernel of one K part, on the plan without that rule or, with A to be staged, on the tiles that
+    take operands as they are. Data that round tell which plan ran."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    L = rfk.lib()
+    L.rf_gemm_destroy()
+    n, k = 1536, 7168
+    assert rfk.select_config(m, n, k).split_k > 1
+    gen, fp8 = torch.Generator(device="cuda").manual_seed(m), torch.float8_e4m3fn
+    a, b = (torch.randint(0, 120, (k, x), dtype=torch.uint8, device="cuda", generator=gen).view(fp8).T for x in (m, n))
+    sa, sb = (torch.rand((k // 128, x), device="cuda", generator=gen).T for x in (m, n // 128))
+    c = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+
+    def bits(config=None):
+        c.fill_(-1.0)
+        rfk.fp8_mm(a, b, sa, sb, c, config=config)
+        torch.cuda.synchronize()
+        return bf16_bits(c).copy()
+
+    exp = bits(rfk.GemmConfig(*runs, 8, 0))
+    split = to_gpu(exact_problem(16, 1536, 7168, 1))
+    handles = []
+    for _ in range(33):
+        h = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(h)) == 0
+        handles.append(h)
+    graph, graph_exec, count, cap = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t(), handles[32]
+    try:
+        L.rf_gemm_destroy()
+        for h in handles[:32]:
+            with torch.cuda.stream(torch.cuda.ExternalStream(h.value)):
+                rfk.fp8_mm(*split)
+            torch.cuda.synchronize()
+        with torch.cuda.stream(torch.cuda.ExternalStream(cap.value)):
+            assert hip.hipStreamBeginCapture(cap, 2) == 0                # hipStreamCaptureModeRelaxed
+            try:
+                rfk.fp8_mm(a, b, sa, sb, c)
+            finally:
+                assert hip.hipStreamEndCapture(cap, ctypes.byref(graph)) == 0
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0 and count.value == 1
+        assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, 0) == 0
+        for replay in range(3):
+            c.fill_(-1.0)
+            torch.cuda.synchronize()
+            assert hip.hipGraphLaunch(graph_exec, cap) == 0
+            torch.cuda.synchronize()
+            assert np.array_equal(bf16_bits(c), exp), replay
+            with torch.cuda.stream(torch.cuda.ExternalStream(handles[0].value)):
+                rfk.fp8_mm(*split)                                       # eager work between the replays
+            torch.cuda.synchronize()
+        hip.hipGraphExecDestroy(graph_exec)
+        hip.hipGraphDestroy(graph)
+        assert not np.array_equal(bits(), exp), "with a buffer set the plan has three K parts"
+    finally:
+        torch.cuda.synchronize()
+        L.rf_gemm_destroy()
+        for h in handles:
+            hip.hipStreamDestroy(h)
