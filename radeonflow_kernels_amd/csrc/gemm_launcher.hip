@@ -580,6 +580,7 @@ constexpr int kFewRowsMaxM = 512, kFewRowsMaxMWide = 4096, kFewRowsSmallN = 1536
 // kFewRowsOnly: the few-rows plan (m and n as they are). kCutC: rows of C are not whole cache lines.
 // kCopyB: B is copied (kStageB without it: only C is unaligned). kNoSplitTiles: without split_tile_plan, whose plans want memory.
 enum { kStageA = 1, kStageB = 2, kTiledOnly = 4, kBytesA = 8, kBytesB = 16, kFewRowsOnly = 32, kCutC = 64, kCopyB = 128, kNoSplitTiles = 256 };
+static_assert(kNoSplitTiles == 1 << (rf::kStageBits - 1), "the last flag");
 
 // The flags of a shape and its pointers (0: aligned).
 int stage_flags(int m, int n, uintptr_t a, uintptr_t b, uintptr_t c) {

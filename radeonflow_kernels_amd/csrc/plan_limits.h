@@ -35,8 +35,11 @@ constexpr bool grouped_weights_streamed(double bytes, bool queue, int columns) {
     return bytes > (queue ? 192.0 * (1 << 20) : columns > 256 ? 256.0 * (1 << 20) : 290.0e6);
 }
 
-// Slot of a shape in the table of plans already worked out (a power of two of them, up to 2^25). All products unsigned: `stage` has
-// eight bits, and as an int its product overflowed from 4 on.
+// Bits of the flags that a plan is chosen by (the launcher's kStageA and on).
+constexpr int kStageBits = 9;
+
+// Slot of a shape in the table of plans already worked out (a power of two of them, up to 2^25). All products unsigned: as an int the
+// product of `stage`, of kStageBits, overflowed from 4 on.
 constexpr unsigned plan_slot(int m, int n, int k, int stage, unsigned entries) {
     return ((((unsigned)m * 2654435761u) ^ ((unsigned)n * 2246822519u) ^ ((unsigned)k * 3266489917u) ^ ((unsigned)stage * 668265263u)) >> 7) % entries;
 }

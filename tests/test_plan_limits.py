@@ -62,9 +62,9 @@ def test_weights_the_infinity_cache_can_hold_are_read_without_the_hint(limits):
 
 def test_plan_table_slot_is_defined_for_every_set_of_staging_flags(tmp_path):
     """Evaluated by the compiler, which refuses a constant expression that overflows a signed product (flags of 4 and more did):
-    all 256 sets of flags, the largest sizes."""
+    every set of flags there is, the largest sizes."""
     src = tmp_path / "slot.cpp"
     src.write_text('#include "%s"\ntemplate <int S> constexpr bool below() {\n    constexpr unsigned a = rf::plan_slot(2147483647, 2147483647, 2147483520, S, 1024), '
                    'b = rf::plan_slot(1, 1, 128, S, 1024);\n    static_assert(a < 1024 && b < 1024, "");\n    if constexpr (S > 0) return below<S - 1>();\n'
-                   '    return true;\n}\nstatic_assert(below<255>(), "");\n' % os.path.join(ROOT, "radeonflow_kernels_amd", "csrc", "plan_limits.h"))
+                   '    return true;\n}\nstatic_assert(below<(1 << rf::kStageBits) - 1>(), "");\n' % os.path.join(ROOT, "radeonflow_kernels_amd", "csrc", "plan_limits.h"))
     subprocess.run(["g++", "-std=c++17", "-fsyntax-only", str(src)], check=True)
