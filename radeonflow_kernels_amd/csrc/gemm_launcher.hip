@@ -644,10 +644,11 @@ double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn;
 // A plan of one workgroup per tile and K part in estimated microseconds, where K is long and the chip is not full of the largest tile:
 //   3.28 + rounds * (f + K blocks of a part * (c + g * share of the units at work)) + 0.693 per million outputs
 //   + 0.057 per million bytes of A and B + 2.47 + 1.18 per million sums when K is split
-// (the more units are at work the longer each waits for L2 and the longer a K block). Fitted to the plans within 1.5 times the fastest of
-// 310 shapes (48 to 2464 rows, N = 256 to 8192, K = 1024 to 8192, 40 % of them the benchmark's pairs of N and K), every variant below with 1
-// to 8 parts on operand sets in rotation. 7.8 % off (root mean square, 43 % at worst) over all 6797 plans of these shapes, 6.6 % over those
-// fitted; 7.8 % and 42 % over 3583 plans of 158 other shapes. The model in select_config_uncached, which ranks plans first, counts a K
+// (the more units are at work the longer each waits for L2 and the longer a K block). Fitted (tuner/long_k_model.py: --measure takes the
+// times, --fit fits; estimate and choice stand there too) to the plans within 1.5 times the fastest of 290 shapes (48 to 2464 rows, N = 256
+// to 8192, K = 1024 to 8192, 40 % of them the benchmark's pairs of N and K), every variant below with 1 to 8 parts on operand sets in
+// rotation. 7.8 % off (root mean square, 43 % at worst) over all 6371 plans of these shapes, 6.7 % over those fitted; 7.9 % and 42 % over
+// 3462 plans of 151 other shapes. The model in select_config_uncached, which ranks plans first, counts a K
 // split's sums at twice what they cost against a K block, and a K block the same on half the chip as on all of it. `*out` is replaced where
 // another plan comes out 6 % lower, but for the exceptions in split_tile_plan: 8 % of the shapes in the range. Of 846 such shapes, drawn
 // for the purpose and timed in turn, the new plans are 16 % faster (geometric mean, up to 42 %), three 2 to 6 % slower (448 x 1600 x 3328 14.6 ->

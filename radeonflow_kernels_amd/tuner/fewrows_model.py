@@ -17,6 +17,8 @@ import tempfile
 
 import numpy as np
 
+from . import long_k_model as long_k
+
 BK = 128
 MAX_TILE_COUNTERS = 16384
 SPLITS = (1, 2, 3, 4, 5, 6, 8, 12, 14)
@@ -93,22 +95,8 @@ def tile_estimate(m, n, k, split, num_cu=256):
     return 3.1 + 0.67 * (t + (6.03 + 1.27e-6 * parts * m * n if parts > 1 else 0.0))
 
 
-def long_k_tile_us(m, n, k, split, num_cu=256):
-    """split_tile_us of csrc/gemm_launcher.hip for variant 28, or None where the planner does not weigh it."""
-    qk = k // BK
-    if not (num_cu == 256 and 48 <= m <= 512 and 256 <= n <= 8192 and 1024 <= k <= 8192 and n * k <= 6.0e7 and
-            _ceil(m, 256) * _ceil(n, 256) <= num_cu):
-        return None
-    kb = _ceil(qk, split)
-    parts = _ceil(qk, kb)
-    wgs, mn = _ceil(m, 128) * _ceil(n, 128) * parts, m * n * 1e-6
-    rounds = _ceil(wgs, num_cu)
-    return (3.281 + rounds * (0.229 + kb * (0.434 + 0.246 * wgs / num_cu / rounds)) + 0.693 * mn + 0.057e-6 * k * (m + n)
-            + (2.471 + 1.182 * mn * parts if parts > 1 else 0.0))
-
-
 def long_k_share(m, n, k):
-    """What part of that figure the few-rows estimate has to stay below (0: it is not weighed)."""
+    """What part of the long-K estimate of a tiled plan of one K part the few-rows estimate has to stay below (0: it is not weighed)."""
     if m > 128:
         return 0.0 if k < 14 * BK else 0.82 if n % 128 == 0 else 0.92
     return 0.90 if k < 14 * BK else 0.92
@@ -130,8 +118,7 @@ def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
             if s <= k // BK and tile_estimate(m, n, k, s, num_cu) < best[0]:
                 best = (tile_estimate(m, n, k, s, num_cu), 28, s)
         if best[1:] == (28, 1):
-            us = long_k_tile_us(m, n, k, best[2], num_cu)
-            if us is not None and few[0] < long_k_share(m, n, k) * us:
+            if m <= 512 and long_k.in_range(m, n, k, num_cu) and few[0] < long_k_share(m, n, k) * long_k.estimate(28, m, n, k, 1):
                 best = few
     return best[1:]
 

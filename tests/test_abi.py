@@ -475,3 +475,28 @@ def test_long_k_estimate_is_not_used_beyond_the_sizes_it_was_measured_on(shape, 
     import radeonflow_kernels_amd as rfk
     got = rfk.plan_for(*shape, 256)
     assert (got.variant, got.split_k, got.stream_k) == (*plan, 0)
+
+
+def test_long_k_model_states_the_choice_of_the_launcher():
+    """tuner/long_k_model.py, where the estimate is measured and fitted: the plans that it puts in place of those of the first model, and
+    every plan of its range that is not tabled is one that it would not replace."""
+    import radeonflow_kernels_amd as rfk
+    from radeonflow_kernels_amd.tuner import long_k_model as lk
+    for first, shape in (((28, 1), (1360, 1536, 7168)), ((28, 1), (544, 4096, 7168)), ((28, 1), (304, 1632, 2176)), ((12, 1), (80, 6352, 2816)),
+                         ((28, 1), (176, 7872, 5376)), ((28, 2), (160, 7968, 6656)), ((12, 1), (640, 1536, 3584)), ((12, 1), (1024, 1024, 4096)),
+                         ((28, 8), (48, 4064, 7168))):
+        got = rfk.plan_for(*shape, 256)
+        assert (got.variant, got.split_k) == lk.replaced(first, *shape), shape
+    assert lk.replaced((28, 1), 1232, 1616, 7552) == (11, 4) and lk.replaced((28, 1), 1232, 1616, 7552, 23959552) == (10, 3)
+    with open(os.path.join(ROOT, "radeonflow_kernels_amd", "csrc", "tuned_plans.inc")) as f:
+        tabled = {tuple(int(x) for x in re.findall(r"\d+", l)[:3]) for l in f if l.lstrip().startswith("{")}
+    seen = 0
+    for shape in lk.shapes(7, 1500):
+        plan = rfk.plan_for(*shape, 256)
+        if shape not in tabled and plan.variant in lk.TILES and plan.stream_k == 0:
+            parts = -(-(shape[2] // 128) // -(-(shape[2] // 128) // plan.split_k))
+            to = lk.replaced((plan.variant, parts), *shape)
+            # (a plan that took the place of variant 12 may itself give way to variant 9, which 12 does not)
+            assert to == (plan.variant, parts) or (to[0] == 9 and shape[0] > 512), (shape, plan, to)
+            seen += 1
+    assert seen > 400
