@@ -650,9 +650,9 @@ double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn;
 // rotation. 7.8 % off (root mean square, 43 % at worst) over all 6371 plans of these shapes, 6.7 % over those fitted; 7.9 % and 42 % over
 // 3462 plans of 151 other shapes. The model in select_config_uncached, which ranks plans first, counts a K
 // split's sums at twice what they cost against a K block, and a K block the same on half the chip as on all of it. `*out` is replaced where
-// another plan comes out 6 % lower, but for the exceptions in split_tile_plan: 8 % of the shapes in the range. Of 846 such shapes, drawn
-// for the purpose and timed in turn, the new plans are 16 % faster (geometric mean, up to 42 %), three 2 to 6 % slower (448 x 1600 x 3328 14.6 ->
-// 15.4). us: 1360 x 1536 x 7168 41.4 (28, one part) -> 32.4 (10, three), 543 x 4096 x 7168 with its staging 46.0 -> 37.3. Left out: the 64 x 128
+// another plan comes out 6 % lower, but for the exceptions in split_tile_plan; that is 6 % of the shapes in the range. 900 that this and the
+// few-rows comparison after it change, odd rows among them, as calls timed in turn: 15 % faster (geometric mean, up to 41 %), five 3 to 10 %
+// slower (224 x 2432 x 2560 11.1 -> 12.1, 448 x 1952 x 3328 15.2 -> 16.3). us: 1360 x 1536 x 7168 41.4 (28, one part) -> 32.4 (10, three), 543 x 4096 x 7168 with its staging 46.0 -> 37.3. Left out: the 64 x 128
 // tile in one part, which takes plans from variant 12 that are up to 9 % faster. In 64 bits' terms the results are as exact as before
 // (relative error 1.660e-3 to 1.664e-3 on either side, the bf16 of C).
 struct SplitTileFit { int variant; double f, c, g; };
@@ -871,8 +871,8 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
         // 7344 x 4608 18.1 (28, four parts), 22.0. Where 8 % are not enough, of 654 shapes that changed plan (timed in turn; ratio to the plan
         // before, geometric mean and worst): more than 128 rows and K below 1792, where the estimate of the tiles is up to 20 % high, 169
         // shapes 0.97 and 1.13 (144 x 6208 x 1408 9.1 -> 9.8), none; more than 128 rows and whole lines of B, 10 to 18 % lower, 29 shapes 0.95
-        // and 1.05; up to 128 rows and K below 1792, 8 to 10 % lower, 22 shapes 0.93 and 1.04. Of 182 other shapes that still change, drawn
-        // for the purpose, all are 12 % faster (geometric mean), none more than 2 % slower.
+        // and 1.05; up to 128 rows and K below 1792, 8 to 10 % lower, 22 shapes 0.93 and 1.04. 182 other shapes that still change are 12 % faster
+        // (geometric mean), none of them more than 2 % slower.
         // (Variant 28's best plan, which tuner/fewrows_model.py knows, has to be behind as well.)
         const double tiled = split_tile_plan(m, n, k, num_cu, out);
         const double share = m > 128 ? (qk < 14 ? 0.0 : n % 128 == 0 ? 0.82 : 0.92) : qk < 14 ? 0.90 : 0.92;
