@@ -25,7 +25,7 @@
  * stream are ordered by the stream. Calls are serialised by one lock only while they enqueue. A buffer that has to grow
  * is replaced and the old one freed by rf_gemm_destroy, so no call waits for the device; one that cannot grow stays in use. A
  * stream gets a buffer set only when a launch on it needs temporary memory: one for staging copies or for a K split's sums,
- * M * N * 4 bytes a part (with K from 1024 to 8192 and 48 to 2600 rows two plans in five split K, for up to 62 MB of sums;
+ * M * N * 4 bytes a part (with K from 1024 to 8192 and 48 to 2600 rows two plans in five split K, for up to 37 MB of sums;
  * rf_gemm_workspace_bytes tells), which it keeps until rf_gemm_destroy. Up to 32 streams per device have a set of their
  * own, and when one more asks, the least recently used set changes hands: the new stream waits on the device for the
  * old stream's work enqueued so far (an event, no host wait). A stream that is being captured into a HIP graph cannot

@@ -642,64 +642,74 @@ double skinny_staged_us(int qk, double mn, int stage) {
 double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn; }
 
 // A plan of one workgroup per tile and K part in estimated microseconds, where K is long and the chip is not full of the largest tile:
-//   3.28 + rounds * (f + K blocks of a part * (c + g * share of the units at work)) + 0.693 per million outputs
-//   + 0.057 per million bytes of A and B + 2.47 + 1.18 per million sums when K is split
-// (the more units are at work the longer each waits for L2 and the longer a K block). Fitted (tuner/long_k_model.py: --measure takes the
-// times, --fit fits; estimate and choice stand there too) to the plans within 1.5 times the fastest of 290 shapes (48 to 2464 rows, N = 256
-// to 8192, K = 1024 to 8192, 40 % of them the benchmark's pairs of N and K), every variant below with 1 to 8 parts on operand sets in
-// rotation. 7.8 % off (root mean square, 43 % at worst) over all 6371 plans of these shapes, 6.7 % over those fitted; 7.9 % and 42 % over
-// 3462 plans of 151 other shapes. The model in select_config_uncached, which ranks plans first, counts a K
-// split's sums at twice what they cost against a K block, and a K block the same on half the chip as on all of it. `*out` is replaced where
-// another plan comes out 6 % lower, but for the exceptions in split_tile_plan; that is 6 % of the shapes in the range. 900 that this and the
-// few-rows comparison after it change, odd rows among them, as calls timed in turn: 15 % faster (geometric mean, up to 41 %), five 3 to 10 %
-// slower (224 x 2432 x 2560 11.1 -> 12.1, 448 x 1952 x 3328 15.2 -> 16.3). us: 1360 x 1536 x 7168 41.4 (28, one part) -> 32.4 (10, three), 543 x 4096 x 7168 with its staging 46.0 -> 37.3. Left out: the 64 x 128
-// tile in one part, which takes plans from variant 12 that are up to 9 % faster. In 64 bits' terms the results are as exact as before
-// (relative error 1.660e-3 to 1.664e-3 on either side, the bf16 of C).
-struct SplitTileFit { int variant; double f, c, g; };
-constexpr SplitTileFit kSplitTileFits[] = {{9, 0.232, 0.462, 0.027}, {12, 0.0, 0.767, 0.401}, {28, 0.229, 0.434, 0.246}, {8, 0.716, 0.623, 0.255},
-                                           {10, 1.02, 0.77, 0.097}, {11, 0.981, 0.892, 0.085}, {0, 0.885, 1.313, 0.0}};
-static_assert(kSplitTileFits[2].variant == 28, "named below");
-double split_tile_us(const SplitTileFit &f, int m, int n, int k, int splits, int num_cu) {
-    const Variant &v = kVariants[f.variant];
+//   start + rounds * (f + K blocks of a part * (c + g * share of the units at work + b * cut B + a * cut A)) + out per million outputs
+//   + in per million bytes of A and B + split + sum per million sums when K is split
+// (the more units are at work the longer each waits for L2 and the longer a K block; cut: the share of that operand's rows that start
+// inside a cache line, of which a tile then reads one more). Two sets of constants: operands that come from the Infinity Cache (calls that
+// repeat, a layer or two) and from memory (the layers of a model in turn), where a K block of many units takes up to 1.5 times as
+// long. Fitted (tuner/long_k_model.py: --measure takes the times, --fit fits; estimates and choice stand there too) to the plans
+// within 1.5 times the fastest of 441 shapes (48 to 2464 rows, N = 256 to 8192, K = 1024 to 8192, 40 % of them the benchmark's pairs of N
+// and K), every variant below with 1 to 8 parts on operand sets in rotation. Cached 6.9 % off (root mean square, 35 % at worst) over all
+// 9922 plans of these shapes and from memory 7.0 % (41 %); fitted to two thirds of the shapes, 6.9 and 7.1 % on the others. The model in
+// select_config_uncached, which ranks plans first, counts a K split's sums at twice what they cost against a K block, and a K block the
+// same on half the chip as on all of it. `*out` is replaced where another plan comes out 7 % lower cached and 6 % lower from memory. With
+// the second estimate alone a fifth of the plans that changed were over 2 % slower cached, up to 1.45 times (272 x 8192 x 7168 29.4 us,
+// 42.4 with four parts). 295 shapes that change now, none of them fitted, plan after against plan before: cached 11 % faster (geometric mean, 5.5 % slower at
+// worst, five by more than 2 %), from memory 17 % (2.4 % at worst). 103 calls with odd rows: 7 and 17 % faster, 4.8 % slower at worst.
+// us, cached and from memory: 1232 x 1616 x 7552 38.1 -> 31.0, 53.0 -> 33.2 (28 in one part, 11 in four); 304 x 1632 x 2176 12.8 -> 11.3, 12.8 ->
+// 11.4. What the margins cost: 1360 x 1536 x 7168 stays at 29.7 and 41.7 (10 in three parts: 28.0, 31.5; estimated 2.8 % lower cached).
+// Left out: the 64 x 128 tile in one part, which takes plans from variant 12 that are up to 9 % faster. In 64 bits' terms the results are
+// as exact as before (relative error 1.660e-3 to 1.664e-3 on either side, the bf16 of C).
+struct SplitTileFit { int variant; double f, c, g, b, a; };
+struct SplitTileCosts { SplitTileFit of[7]; double start, out, in, split, sum; };
+constexpr SplitTileCosts kSplitTileCached = {
+    {{9, 0.0, 0.366, 0.0, 0.07, 0.028}, {12, 0.185, 0.592, 0.147, 0.19, 0.059}, {28, 0.194, 0.333, 0.132, 0.069, 0.039}, {8, 0.765, 0.496, 0.077, 0.033, 0.039},
+     {10, 0.759, 0.59, 0.077, 0.073, 0.058}, {11, 0.875, 0.738, 0.021, 0.036, 0.018}, {0, 1.138, 1.033, 0.023, 0.049, 0.104}},
+    4.531, 0.403, 0.0, 2.274, 1.177};
+constexpr SplitTileCosts kSplitTileMemory = {
+    {{9, 0.169, 0.397, 0.041, 0.047, 0.028}, {12, 0.0, 0.63, 0.444, 0.172, 0.066}, {28, 0.073, 0.375, 0.23, 0.072, 0.056}, {8, 0.497, 0.574, 0.217, 0.025, 0.072},
+     {10, 0.712, 0.692, 0.076, 0.086, 0.088}, {11, 0.76, 0.847, 0.056, 0.038, 0.042}, {0, 1.004, 1.207, 0.0, 0.095, 0.087}},
+    3.922, 0.531, 0.054, 2.283, 1.173};
+// Share of the rows of `bytes` bytes, one after the other, that do not start at a multiple of 128.
+double cut_rows(int bytes) { return 1.0 - std::min(bytes & -bytes, 128) / 128.0; }
+// 0 for a variant that is not estimated.
+double split_tile_us(const SplitTileCosts &costs, int variant, int m, int n, int k, int splits, int num_cu) {
+    const Variant &v = kVariants[variant];
     const int qk = k / rf::BK;
     const double wgs = (double)ceil_div(m, v.bm) * ceil_div(n, v.bn) * splits, mn = (double)m * n * 1e-6;
     const double rounds = std::ceil(wgs / num_cu), blocks = v.k_groups > 1 ? qk / v.k_groups : ceil_div(qk, splits);
-    return 3.281 + rounds * (f.f + blocks * (f.c + f.g * wgs / num_cu / rounds)) + 0.693 * mn + 0.057e-6 * k * ((double)m + n) +
-           (splits > 1 ? 2.471 + 1.182 * mn * splits : 0.0);
+    for (const SplitTileFit &f : costs.of)
+        if (f.variant == variant)
+            return costs.start + rounds * (f.f + blocks * (f.c + f.g * wgs / num_cu / rounds + f.b * cut_rows(n) + f.a * cut_rows(m))) + costs.out * mn + costs.in * 1e-6 * k * ((double)m + n) +
+                   (splits > 1 ? costs.split + costs.sum * mn * splits : 0.0);
+    return 0.0;
 }
 // The sizes it was fitted to and checked on; plans beyond them stay as the first model has them.
 bool long_k_range(int m, int n, int k) {
     return m >= 48 && m <= 2608 && n >= 256 && n <= 8192 && k >= 1024 && k <= 8192 && (double)n * k <= 6.0e7;
 }
-// Returns the figure of the plan that it leaves in *out, 0 for one that is not estimated here. K splits whose sums take more than
+// Returns the cached figure of the plan that it leaves in *out, 0 for one that is not estimated here. K splits whose sums take more than
 // `most` bytes are not tried.
 double split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out, size_t most = SIZE_MAX) {
-    const int qk = k / rf::BK;
-    const rf_gemm_config first = *out;
-    const bool many = m > kFewRowsMaxM;
-    double before = 0.0;                                    // stays 0 for a plan that is not estimated here, which stays too
-    for (const SplitTileFit &f : kSplitTileFits)
-        if (f.variant == first.variant) before = split_tile_us(f, m, n, k, ceil_div(qk, ceil_div(qk, first.split_k)), num_cu);
-    // Where 6 % are not enough, or nothing is, of 1739 shapes whose plan it changed (timed in turn; ratio to the plan before, geometric
-    // mean and worst): a K split already and 129 to 192 rows, 95 shapes 0.98 and 1.25 (160 x 7968 x 6656 28.6 us in two parts of variant
-    // 28, 35.9 in four of 10); variant 12 replaced beyond 512 rows by 9 at all, 35 shapes 0.93 and 1.16 (640 x 1536 x 3584 14.6, 16.9), or
-    // for 6 to 10 %, 25 shapes 0.86 and 1.13 (1024 x 704 x 3072 12.9, 14.7); 28 replaced beyond 512 rows by 9 for 6 to 10 %, 21 shapes 0.93
-    // and 1.06. Mostly N is a multiple of 128 there: the plan before then reads whole lines of B and is up to 15 % below its estimate.
-    if (first.split_k > 1 && m > 128 && m <= 192) return before;
-    double kept = before, best = (many && first.variant == 12 ? 0.90 : 0.94) * before;
-    for (const SplitTileFit &f : kSplitTileFits) {
+    const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, out->split_k));
+    const double cached = split_tile_us(kSplitTileCached, out->variant, m, n, k, parts, num_cu);
+    double kept = cached, best = 0.94 * split_tile_us(kSplitTileMemory, out->variant, m, n, k, parts, num_cu);
+    for (const SplitTileFit &f : kSplitTileMemory.of) {
         const Variant &v = kVariants[f.variant];
         // (up to 512 rows variant 28 in more parts is not tried: the few-rows kernels were weighed against its plan of the first model)
-        if ((f.variant == 28 && !many) || (f.variant == 9 && many && first.variant == 12)) continue;
+        if (f.variant == 28 && m <= kFewRowsMaxM) continue;
         const double tiles = (double)ceil_div(m, v.bm) * ceil_div(n, v.bn);
         for (int sp : {1, 2, 3, 4, 5, 6, 8}) {
             if (sp > qk || ceil_div(qk, ceil_div(qk, sp)) != sp || (v.k_groups > 1 && (sp > 1 || qk % v.k_groups != 0))) continue;
             if (sp == 1 && f.variant == 9) continue;
             if (sp > 1 && (tiles * sp > 600 || (double)m * n * sp > 45.0e6)) continue;      // no more than was measured
             if (sp > 1 && (size_t)m * n * sizeof(float) * sp > most) continue;
-            const double t = split_tile_us(f, m, n, k, sp, num_cu);
-            if (t < best && (f.variant != 9 || !many || t < 0.90 * before)) {
-                best = kept = t;
+            const double us = split_tile_us(kSplitTileCached, f.variant, m, n, k, sp, num_cu);
+            if (us >= 0.93 * cached) continue;
+            const double t = split_tile_us(kSplitTileMemory, f.variant, m, n, k, sp, num_cu);
+            if (t < best) {
+                best = t;
+                kept = us;
                 *out = {f.variant, sp, 8, RF_SCHEDULE_TILES};
             }
         }
@@ -866,20 +876,16 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < t) *out = other;
     if (!hit && num_cu == kTunedOnCUs && !(stage & (kStageB | kNoSplitTiles)) && out->stream_k == RF_SCHEDULE_TILES &&
         !kVariants[out->variant].takes_any_shape() && long_k_range(m, n, k) && ceil_div(m, 256) * ceil_div(n, 256) <= num_cu) {
-        // The few-rows kernels again, 8 % below that figure of a plan of one K part (a tiled plan of long K has too low a `t` above), us:
-        // 256 x 3824 x 2560 17.3 -> 13.3, 384 x 2048 x 2048 10.3 -> 9.5, 64 x 8000 x 2304 14.0 -> 9.6. Not against plans with a K split: 128 x
-        // 7344 x 4608 18.1 (28, four parts), 22.0. Where 8 % are not enough, of 654 shapes that changed plan (timed in turn; ratio to the plan
-        // before, geometric mean and worst): more than 128 rows and K below 1792, where the estimate of the tiles is up to 20 % high, 169
-        // shapes 0.97 and 1.13 (144 x 6208 x 1408 9.1 -> 9.8), none; more than 128 rows and whole lines of B, 10 to 18 % lower, 29 shapes 0.95
-        // and 1.05; up to 128 rows and K below 1792, 8 to 10 % lower, 22 shapes 0.93 and 1.04. 182 other shapes that still change are 12 % faster
-        // (geometric mean), none of them more than 2 % slower.
+        // The few-rows kernels again, 15 % below that figure of a plan of one K part (a tiled plan of long K has too low a `t` above). 121 shapes that change
+        // plan here, before against after: cached 6 % faster (geometric mean, 0.5 % slower at worst), from memory 9 % (0.1 %). us: 256 x 3824 x 2560
+        // 14.2 -> 12.6, 17.5 -> 13.1. At 8 % the slowest of 88 is 5.8 % slower (256 x 3616 x 2688). Not against plans with a K split: 128 x
+        // 7344 x 4608 18.1 (28, four parts), 22.0.
         // (Variant 28's best plan, which tuner/fewrows_model.py knows, has to be behind as well.)
         const double tiled = split_tile_plan(m, n, k, num_cu, out);
-        const double share = m > 128 ? (qk < 14 ? 0.0 : n % 128 == 0 ? 0.82 : 0.92) : qk < 14 ? 0.90 : 0.92;
         if (m <= kFewRowsMaxM && out->split_k == 1 && !(stage & kTiledOnly) && fewrows_ok(m, n)) {
             const double few = fewrows_plan(m, n, k, num_cu, false, &other);
-            const bool below_28 = split_28 == 1 ? few < share * split_tile_us(kSplitTileFits[2], m, n, k, 1, num_cu) : few < 3.1 + 0.67 * cost_28;
-            if (few < share * tiled && below_28) *out = other;
+            const bool below_28 = split_28 == 1 ? few < 0.85 * split_tile_us(kSplitTileCached, 28, m, n, k, 1, num_cu) : few < 3.1 + 0.67 * cost_28;
+            if (few < 0.85 * tiled && below_28) *out = other;
         }
     }
 }
@@ -918,9 +924,9 @@ bool fewrows_split_fits(Mem &mem, const Variant &v, int m, int n, int k, int spl
 
 // The same of a tiled plan's K split: without memory for its sums the plan is the one that split_tile_plan found. mp: the rows that are
 // planned, m: those of c, stage: the plan's flags. In the static array, beside `staged` bytes of copies, that plan in the parts that fit
-// is weighed once more against the others that fit: 1228 x 1616 x 7552, A staged, 58.4 us (28, one part) -> 41.2 (10, three instead of four of
-// 11), 400 x 5664 x 7936 48.0 -> 42.9. Of 300 shapes whose plan does not fit 25 are 10 to 31 % faster than on that plan, none slower by more
-// than the 1 % that runs differ by.
+// is weighed once more against the others that fit: 942 x 1904 x 6016, A staged, 37.5 us cached and 46.0 from memory (28, one part) -> 28.5 and
+// 32.4 (8, three parts instead of four of 10). 150 shapes whose plan does not fit, against the plan that split_tile_plan found: 11 % faster
+// cached (geometric mean), 16 % from memory, none slower by more than the 1 % that runs differ by.
 void fit_tile_split(State &s, Mem &mem, int m, int mp, int n, int k, int stage, size_t staged, rf_gemm_config *cfg) {
     if (cfg->variant < 0 || cfg->split_k == 1 || cfg->stream_k != RF_SCHEDULE_TILES || kVariants[cfg->variant].takes_any_shape()) return;
     const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, cfg->split_k));

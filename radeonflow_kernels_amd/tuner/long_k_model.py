@@ -1,11 +1,12 @@
-"""The time estimate that weighs tile plans and their K splits against each other where K is long and the chip is not full of the
-largest tile (split_tile_us and split_tile_plan in csrc/gemm_launcher.hip): the measurements behind it and its fit.
+"""The time estimates that weigh tile plans and their K splits against each other where K is long and the chip is not full of the
+largest tile (split_tile_us and split_tile_plan in csrc/gemm_launcher.hip): the measurements behind them and their fit.
 
   python -m radeonflow_kernels_amd.tuner.long_k_model --measure FILE    the tiles of TILES with 1 to 8 K parts over shapes drawn at
-                                                                        random, on operand sets in rotation
-  python -m radeonflow_kernels_amd.tuner.long_k_model --fit FILE        how far the estimate is from the times, and its constants
-                                                                        fitted to the file
-FILE has one line per plan: M N K variant split_k us. --measure needs the GPU; the estimate and the fit do not.
+                                                                        random, on operand sets in rotation that the Infinity
+                                                                        Cache holds and on sets beyond it
+  python -m radeonflow_kernels_amd.tuner.long_k_model --fit FILE        how far the estimates are from the times, and their
+                                                                        constants fitted to the file
+FILE has one line per plan: M N K variant split_k and the us of both rotations. --measure needs the GPU; the estimates and the fit do not.
 """
 import argparse
 import math
@@ -16,11 +17,20 @@ import numpy as np
 BK = 128
 # variant: tile rows, columns
 TILES = {9: (64, 128), 12: (64, 128), 28: (128, 128), 8: (128, 192), 10: (128, 256), 11: (192, 192), 0: (256, 256)}
-# a round of tiles; a K block of it; more of it with the share of the compute units at work
-FIT = {9: (0.232, 0.462, 0.027), 12: (0.0, 0.767, 0.401), 28: (0.229, 0.434, 0.246), 8: (0.716, 0.623, 0.255), 10: (1.02, 0.77, 0.097),
-       11: (0.981, 0.892, 0.085), 0: (0.885, 1.313, 0.0)}
-# launch; per million outputs; per million bytes of A and B; K split, and per million sums
-COMMON = (3.281, 0.693, 0.057, 2.471, 1.182)
+# operands from the Infinity Cache; from memory:
+#   a round of tiles; a K block of it; more of it with the share of the compute units at work, with the share of the rows of B and of A
+#   that start inside a cache line
+FITS = ({9: (0.0, 0.366, 0.0, 0.07, 0.028), 12: (0.185, 0.592, 0.147, 0.19, 0.059), 28: (0.194, 0.333, 0.132, 0.069, 0.039),
+         8: (0.765, 0.496, 0.077, 0.033, 0.039), 10: (0.759, 0.59, 0.077, 0.073, 0.058), 11: (0.875, 0.738, 0.021, 0.036, 0.018),
+         0: (1.138, 1.033, 0.023, 0.049, 0.104)},
+        {9: (0.169, 0.397, 0.041, 0.047, 0.028), 12: (0.0, 0.63, 0.444, 0.172, 0.066), 28: (0.073, 0.375, 0.23, 0.072, 0.056),
+         8: (0.497, 0.574, 0.217, 0.025, 0.072), 10: (0.712, 0.692, 0.076, 0.086, 0.088), 11: (0.76, 0.847, 0.056, 0.038, 0.042),
+         0: (1.004, 1.207, 0.0, 0.095, 0.087)})
+#   launch; per million outputs; per million bytes of A and B; K split, and per million sums
+COMMONS = ((4.531, 0.403, 0.0, 2.274, 1.177), (3.922, 0.531, 0.054, 2.283, 1.173))
+CACHED, MEMORY = 0, 1
+# what part of the estimate of the plan before another's has to stay below
+SHARES = (0.93, 0.94)
 SPLITS = (1, 2, 3, 4, 5, 6, 8)
 
 
@@ -38,43 +48,47 @@ def _parts(k, split):
     return _ceil(k // BK, _ceil(k // BK, split))
 
 
+def _cut(length):
+    return 1 - min(length & -length, 128) / 128
+
+
 def _terms(variant, m, n, k, split, num_cu=256):
     """What a variant's constants and COMMON multiply."""
     bm, bn = TILES[variant]
     blocks = k // BK // 2 if variant == 12 else _ceil(k // BK, split)      # (12 splits K inside the workgroup)
     workgroups, mn = _ceil(m, bm) * _ceil(n, bn) * split, m * n * 1e-6
     rounds = _ceil(workgroups, num_cu)
-    return ((rounds, rounds * blocks, blocks * workgroups / num_cu),
+    return ((rounds, rounds * blocks, blocks * workgroups / num_cu, rounds * blocks * _cut(n), rounds * blocks * _cut(m)),
             (1.0, mn, k * (m + n) * 1e-6, float(split > 1), mn * split if split > 1 else 0.0))
 
 
-def estimate(variant, m, n, k, split, num_cu=256, fit=None, common=COMMON):
-    """Microseconds of a plan; split: K parts that there are."""
+def estimate(variant, m, n, k, split, where, num_cu=256):
+    """Microseconds of a plan; split: K parts that there are; where: CACHED or MEMORY."""
     own, shared = _terms(variant, m, n, k, split, num_cu)
-    return sum(x * c for x, c in zip(own + shared, tuple((fit or FIT)[variant]) + tuple(common)))
+    return sum(x * c for x, c in zip(own + shared, FITS[where][variant] + COMMONS[where]))
 
 
 def replaced(first, m, n, k, most=float("inf")):
     """(variant, parts) that the planner takes in place of `first`, the plan of its first model, with sums of at most `most` bytes."""
-    if first[0] not in FIT or (first[1] > 1 and 128 < m <= 192):
+    if first[0] not in TILES:
         return first
-    many, before = m > 512, estimate(first[0], m, n, k, _parts(k, first[1]))
-    best, out = (0.90 if many and first[0] == 12 else 0.94) * before, first
+    limits = [share * estimate(first[0], m, n, k, _parts(k, first[1]), w) for w, share in enumerate(SHARES)]
+    out = first
     for v, (bm, bn) in TILES.items():
-        if (v == 28 and not many) or (v == 9 and many and first[0] == 12):
+        if v == 28 and m <= 512:
             continue
         for s in SPLITS:
             if s > k // BK or _parts(k, s) != s or (v == 12 and (s > 1 or k // BK % 2)) or (v == 9 and s == 1):
                 continue
             if s > 1 and (_ceil(m, bm) * _ceil(n, bn) * s > 600 or m * n * s > 45e6 or 4 * m * n * s > most):
                 continue
-            t = estimate(v, m, n, k, s)
-            if t < best and (v != 9 or not many or t < 0.90 * before):
-                best, out = t, (v, s)
+            us = estimate(v, m, n, k, s, MEMORY)
+            if estimate(v, m, n, k, s, CACHED) < limits[CACHED] and us < limits[MEMORY]:
+                limits[MEMORY], out = us, (v, s)
     return out
 
 
-def shapes(seed=1, count=330):
+def shapes(seed=1, count=500):
     """(M, N, K): 40 % of them the benchmark's pairs of N and K, 30 % powers of two, 30 % any multiples of 16 and 128."""
     r = random.Random(seed)
     pairs = ((1536, 7168), (4608, 7168), (7168, 2048), (576, 7168), (3072, 1536), (7168, 2304), (512, 7168), (4096, 7168))
@@ -95,7 +109,7 @@ def measure(path):
     t.settle(rfk)
     with open(path, "w") as f:
         for i, (m, n, k) in enumerate(shapes()):
-            sets = t.operand_sets(m, n, k)
+            held, beyond = t.operand_sets(m, n, k), t.operand_sets(m, n, k, 600 << 20, 24)
             for v, (bm, bn) in TILES.items():
                 for s in (1,) if v == 12 else SPLITS:
                     workgroups = _ceil(m, bm) * _ceil(n, bn) * s
@@ -103,33 +117,34 @@ def measure(path):
                         continue
                     if (v == 0 and s == 1 and workgroups > 256) or (s > 1 and m * n * s > 45e6):
                         continue
-                    f.write("%d %d %d %d %d %.2f\n" % (m, n, k, v, s, t.rotated_us(rfk, sets, rfk.GemmConfig(v, s, 8, 0), 32, 2)))
+                    us = [min(t.rotated_us(rfk, sets, rfk.GemmConfig(v, s, 8, 0), 32, 2) for _ in range(2)) for sets in (held, beyond)]
+                    f.write("%d %d %d %d %d %.2f %.2f\n" % (m, n, k, v, s, *us))
             f.flush()
             if i % 10 == 9:
                 print(i + 1, flush=True)
 
 
-def read(path):
+def read(path, where):
     """{shape: {(variant, parts): us}}"""
     out = {}
     with open(path) as f:
         for l in f:
             w = [int(x) for x in l.split()[:5]]
-            out.setdefault(tuple(w[:3]), {})[tuple(w[3:])] = float(l.split()[5])
+            out.setdefault(tuple(w[:3]), {})[tuple(w[3:])] = float(l.split()[5 + where])
     return out
 
 
 def refit(data):
-    """Constants of least relative error over the plans within 1.5 of their shape's fastest, none negative. (FIT, COMMON)."""
-    variants, rows = list(FIT), []
+    """Constants of least relative error over the plans within 1.5 of their shape's fastest, none negative: one of FITS, one of COMMONS."""
+    variants, rows, common = list(TILES), [], len(COMMONS[0])
     for shape, times in data.items():
         for (v, s), us in times.items():
             if us < 1.5 * min(times.values()):
                 own, shared = _terms(v, *shape, s)
-                row = np.zeros(3 * len(variants) + len(COMMON))
-                row[3 * variants.index(v):][:3], row[3 * len(variants):] = own, shared
+                row = np.zeros(5 * len(variants) + common)
+                row[5 * variants.index(v):][:5], row[5 * len(variants):] = own, shared
                 rows.append(row / us)
-    a, use = np.array(rows), np.ones(3 * len(variants) + len(COMMON), bool)
+    a, use = np.array(rows), np.ones(5 * len(variants) + common, bool)
     while True:
         x = np.zeros(len(use))
         x[use] = np.linalg.lstsq(a[:, use], np.ones(len(a)), rcond=None)[0]
@@ -137,14 +152,14 @@ def refit(data):
             break
         use[np.argmin(x)] = False
     x = [round(float(v), 3) for v in x]
-    return {v: tuple(x[3 * i:3 * i + 3]) for i, v in enumerate(variants)}, tuple(x[3 * len(variants):])
+    return {v: tuple(x[5 * i:5 * i + 5]) for i, v in enumerate(variants)}, tuple(x[5 * len(variants):])
 
 
-def report(data, fit, common, what):
+def report(data, where, what):
     err, near = [], []
     for shape, times in data.items():
         for (v, s), us in times.items():
-            e = estimate(v, *shape, s, fit=fit, common=common) / us - 1
+            e = estimate(v, *shape, s, where) / us - 1
             err.append(e)
             if us < 1.5 * min(times.values()):
                 near.append(e)
@@ -161,11 +176,10 @@ def main():
     if a.measure:
         measure(a.measure)
     if a.fit:
-        data = read(a.fit)
-        report(data, FIT, COMMON, "constants in use")
-        fit, common = refit(data)
-        report(data, fit, common, "refitted")
-        print("COMMON =", common, "\nFIT =", fit)
+        for where, what in ((CACHED, "operands from the Infinity Cache"), (MEMORY, "operands from memory")):
+            data = read(a.fit, where)
+            report(data, where, what)
+            print("refitted:", *refit(data))
 
 
 if __name__ == "__main__":

@@ -168,21 +168,21 @@ def _static_bits_and_plans(rfk, m, n, k, plans):
 
 
 def test_static_entry_counts_the_rows_of_c_for_a_staged_k_split(rfk):
-    """Sums that fit beside the staged A as the 625 rows that are written, but not as the 640 that are computed: the plan's three
-    parts, which were cut to two."""
-    m, n, k = 625, 3792, 7040
+    """Sums that fit beside the staged A as the 659 rows that are written, but not as the 672 that are computed: the plan's four
+    parts, which were cut to three."""
+    m, n, k = 659, 2720, 6400
     cfg = rfk.select_config(m, n, k)
-    assert cfg.split_k == 3 and cfg.stream_k == 0
-    staged = k * 640 + k // 128 * 640 * 4
-    assert staged + 3 * 4 * m * n <= rfk.lib().rf_gemm_static_scratch_bytes() < staged + 3 * 4 * 640 * n
-    got, (three, two) = _static_bits_and_plans(rfk, m, n, k, [(cfg.variant, 3), (cfg.variant, 2)])
-    assert not np.array_equal(three, two)
-    assert np.array_equal(got, three)
+    assert cfg.split_k == 4 and cfg.stream_k == 0
+    staged = k * 672 + k // 128 * 672 * 4
+    assert staged + 4 * 4 * m * n <= rfk.lib().rf_gemm_static_scratch_bytes() < staged + 4 * 4 * 672 * n
+    got, (four, three) = _static_bits_and_plans(rfk, m, n, k, [(cfg.variant, 4), (cfg.variant, 3)])
+    assert not np.array_equal(four, three)
+    assert np.array_equal(got, four)
 
 
 # aligned and beyond the array by itself, A staged beside the sums; the plan before the rule for long K in one part and in two
-@pytest.mark.parametrize("m,n,k,runs", [(272, 8192, 7168, (28, 1)), (400, 5664, 7936, (10, 2)), (1361, 1536, 7168, (28, 1)),
-                                        (1195, 1136, 7808, (28, 2)), (1228, 1616, 7552, (10, 3)), (716, 1952, 8192, (10, 4))])
+@pytest.mark.parametrize("m,n,k,runs", [(1328, 1648, 7424, (10, 3)), (560, 3216, 7040, (11, 4)), (2092, 1104, 7168, (28, 1)),
+                                        (2005, 816, 5888, (28, 2)), (1125, 1952, 7936, (8, 2)), (942, 1904, 6016, (8, 3))])
 def test_static_entry_fits_a_long_k_plan_to_its_scratch_array(rfk, m, n, k, runs):
     """Plans of split_tile_plan whose sums do not fit: the one that runs is neither theirs nor theirs with fewer parts unless that
     is estimated fastest among those that fit. Data that round tell the K parts by their bits."""
