@@ -204,6 +204,7 @@ struct StreamBuffers {
     size_t pad_bytes = 0;
     float *ws = nullptr;                 // split-K partial sums / stream-K slots
     size_t ws_bytes = 0;
+    rf::RefusedGrowth ws_refused;
     uint64_t last_use = 0;
 };
 struct State {
@@ -387,6 +388,21 @@ struct Mem {
         rc = grow(sb->ws, sb->ws_bytes, bytes);
         *out = sb->ws;
         return rc;
+    }
+    // Whether there is a workspace of that size, for a plan that another can take the place of (not for the static mode).
+    bool try_workspace(size_t bytes) {
+        float *ws = nullptr;
+        int rc = bind();
+        if (rc == RF_OK) {
+            if (bytes <= sb->ws_bytes) return true;
+            if (!sb->ws_refused.ask(bytes)) return false;
+            rc = workspace(bytes, &ws);
+            sb->ws_refused.answer(bytes, rc == RF_OK);
+        }
+        if (rc == RF_OK) return true;
+        (void)hipGetLastError();
+        g_last_error.clear();
+        return false;
     }
     int counters(CounterSet **out) {
         if (fixed) {
@@ -915,11 +931,7 @@ size_t fewrows_slot_bytes(const Variant &v, int m, int n, int parts) {
 bool fewrows_split_fits(Mem &mem, const Variant &v, int m, int n, int k, int splits) {
     if (splits == 1 || mem.fixed) return true;
     const int qk = k / rf::BK;
-    float *slots = nullptr;
-    if (mem.workspace(fewrows_slot_bytes(v, m, n, ceil_div(qk, ceil_div(qk, splits))), &slots) == RF_OK) return true;
-    (void)hipGetLastError();
-    g_last_error.clear();
-    return false;
+    return mem.try_workspace(fewrows_slot_bytes(v, m, n, ceil_div(qk, ceil_div(qk, splits))));
 }
 
 // The same of a tiled plan's K split: without memory for its sums the plan is the one that split_tile_plan found. mp: the rows that are
@@ -931,14 +943,7 @@ void fit_tile_split(State &s, Mem &mem, int m, int mp, int n, int k, int stage, 
     if (cfg->variant < 0 || cfg->split_k == 1 || cfg->stream_k != RF_SCHEDULE_TILES || kVariants[cfg->variant].takes_any_shape()) return;
     const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, cfg->split_k));
     const size_t part = (size_t)m * n * sizeof(float), left = mem.fixed_left() > staged ? mem.fixed_left() - staged : 0;
-    if (mem.fixed) {
-        if (part * parts <= left) return;
-    } else {
-        float *ws = nullptr;
-        if (mem.workspace(part * parts, &ws) == RF_OK) return;
-        (void)hipGetLastError();
-        g_last_error.clear();
-    }
+    if (mem.fixed ? part * parts <= left : mem.try_workspace(part * parts)) return;
     rf_gemm_config first;
     select_config(mp, n, k, s.num_cu, stage | kNoSplitTiles, &first);
     const bool changed = first.variant != cfg->variant || first.split_k != cfg->split_k;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cstddef>
+#include <cstdint>
 
 namespace rf {
 
@@ -20,5 +21,17 @@ auto grow_buffer(T *&buf, size_t &have, size_t need, Retired &retired, Alloc all
     have = want;
     return error;
 }
+
+// A growth that failed, of a buffer that a plan can do without: the next 63 calls that want as much or more take the plan without it
+// and do not pay for another allocation that fails. One in 64 asks again, memory may have been freed since.
+struct RefusedGrowth {
+    size_t bytes = SIZE_MAX;
+    int calls = 0;
+    bool ask(size_t need) { return need < bytes || ++calls >= 64; }
+    void answer(size_t need, bool grown) {
+        bytes = grown ? SIZE_MAX : need < bytes ? need : bytes;
+        calls = 0;
+    }
+};
 
 }  // namespace rf

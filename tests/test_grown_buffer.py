@@ -37,6 +37,22 @@ int main() {
     CHECK(rf::grow_buffer(buf, have, 401, retired, alloc) == 0 && asked == 600 && have == 600);
     CHECK(buf != first && retired.size() == 1 && retired[0] == first);
     CHECK(rf::grow_buffer(buf, have, 5000, retired, alloc) == 0 && asked == 5000 && have == 5000 && retired.size() == 2);
+    // a plan that can do without: a size that was refused is asked for once in 64 calls, a smaller one at once
+    rf::RefusedGrowth r;
+    CHECK(r.ask(9000));
+    r.answer(9000, false);
+    for (int round = 0; round < 3; round++) {
+        for (int i = 0; i < 63; i++) CHECK(!r.ask(round == 1 ? 20000 : 9000));
+        CHECK(r.ask(9000));
+        r.answer(9000, false);
+    }
+    CHECK(r.ask(8999));
+    r.answer(8999, false);
+    CHECK(!r.ask(9000) && r.ask(8998));
+    for (int i = 0; i < 62; i++) CHECK(!r.ask(9000));
+    CHECK(r.ask(9000));
+    r.answer(9000, true);
+    CHECK(r.ask(9000) && r.ask(1u << 30));
     return 0;
 }
 """
