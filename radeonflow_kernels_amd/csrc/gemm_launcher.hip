@@ -668,12 +668,12 @@ double one_round_us(int qk, double mn) { return 3.458 + 0.526 * qk + 0.434 * mn;
 // and K), every variant below with 1 to 8 parts on operand sets in rotation. Cached 6.9 % off (root mean square, 35 % at worst) over all
 // 9922 plans of these shapes and from memory 7.0 % (41 %); fitted to two thirds of the shapes, 6.9 and 7.1 % on the others. The model in
 // select_config_uncached, which ranks plans first, counts a K split's sums at twice what they cost against a K block, and a K block the
-// same on half the chip as on all of it. `*out` is replaced where another plan comes out 7 % lower cached and 6 % lower from memory. With
-// the second estimate alone a fifth of the plans that changed were over 2 % slower cached, up to 1.45 times (272 x 8192 x 7168 29.4 us,
-// 42.4 with four parts). 295 shapes that change now, none of them fitted, plan after against plan before: cached 11 % faster (geometric mean, 5.5 % slower at
-// worst, five by more than 2 %), from memory 17 % (2.4 % at worst). 103 calls with odd rows: 7 and 17 % faster, 4.8 % slower at worst.
+// same on half the chip as on all of it. `*out` is replaced (split_tile_plan) where another plan is below both estimates: with the second
+// alone a fifth of the plans that changed were over 2 % slower cached, up to 1.45 times (272 x 8192 x 7168 29.4 us, 42.4 with four parts).
+// That is 7 % of the shapes in the range. 291 of them, none fitted, plan after against plan before: cached 10 % faster (geometric mean; nine by over
+// 2 % slower, 7.3 % at worst), from memory 18 % (one, 7.3 %). 160 calls with odd rows: 7 and 17 % faster (three, 5.8 %).
 // us, cached and from memory: 1232 x 1616 x 7552 38.1 -> 31.0, 53.0 -> 33.2 (28 in one part, 11 in four); 304 x 1632 x 2176 12.8 -> 11.3, 12.8 ->
-// 11.4. What the margins cost: 1360 x 1536 x 7168 stays at 29.7 and 41.7 (10 in three parts: 28.0, 31.5; estimated 2.8 % lower cached).
+// 11.4; 544 x 4096 x 7168 28.6 -> 29.1, 41.8 -> 31.8 (28 in one part, 10 in three).
 // Left out: the 64 x 128 tile in one part, which takes plans from variant 12 that are up to 9 % faster. In 64 bits' terms the results are
 // as exact as before (relative error 1.660e-3 to 1.664e-3 on either side, the bf16 of C).
 struct SplitTileFit { int variant; double f, c, g, b, a; };
@@ -705,23 +705,30 @@ bool long_k_range(int m, int n, int k) {
     return m >= 48 && m <= 2608 && n >= 256 && n <= 8192 && k >= 1024 && k <= 8192 && (double)n * k <= 6.0e7;
 }
 // Returns the cached figure of the plan that it leaves in *out, 0 for one that is not estimated here. K splits whose sums take more than
-// `most` bytes are not tried.
+// `most` bytes are not tried. What part of the plan before's figure another's has to stay below: from memory 0.94; cached, by what the estimates of
+// 763 such pairs are off by (time over estimate, new plan against plan before): up to 512 rows K splits come out too low, 1.03 to 1.09,
+// beyond them not (variant 28 0.91, 10 0.97, 11 1.0), 9 in place of 12 too low at any size, 1.04 to 1.08. Up to 512 rows 103 of 348 pairs
+// change at 0.93 and five are over 2 % slower (54 of 198 at 0.97), beyond 512 rows 247 of 415 and 13 at 1.0 (72 and one at 0.93). Of 62 pairs
+// with 9 in place of 12 eleven were slower at 0.93 and 1.0, up to 9.7 %, none of 21 at 0.88; of 56 with 28 in place of 12 three at 1.0 (1600 x
+// 384 x 3072 12.4 -> 13.6 us), one of 39 at 0.96.
 double split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out, size_t most = SIZE_MAX) {
     const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, out->split_k));
     const double cached = split_tile_us(kSplitTileCached, out->variant, m, n, k, parts, num_cu);
+    const int first = out->variant;
     double kept = cached, best = 0.94 * split_tile_us(kSplitTileMemory, out->variant, m, n, k, parts, num_cu);
     for (const SplitTileFit &f : kSplitTileMemory.of) {
         const Variant &v = kVariants[f.variant];
         // (up to 512 rows variant 28 in more parts is not tried: the few-rows kernels were weighed against its plan of the first model)
         if (f.variant == 28 && m <= kFewRowsMaxM) continue;
         const double tiles = (double)ceil_div(m, v.bm) * ceil_div(n, v.bn);
+        const double limit = (f.variant == 9 ? (first == 12 ? 0.88 : 0.93) : m <= kFewRowsMaxM ? 0.93 : first == 12 ? 0.96 : 1.0) * cached;
         for (int sp : {1, 2, 3, 4, 5, 6, 8}) {
             if (sp > qk || ceil_div(qk, ceil_div(qk, sp)) != sp || (v.k_groups > 1 && (sp > 1 || qk % v.k_groups != 0))) continue;
             if (sp == 1 && f.variant == 9) continue;
             if (sp > 1 && (tiles * sp > 600 || (double)m * n * sp > 45.0e6)) continue;      // no more than was measured
             if (sp > 1 && (size_t)m * n * sizeof(float) * sp > most) continue;
             const double us = split_tile_us(kSplitTileCached, f.variant, m, n, k, sp, num_cu);
-            if (us >= 0.93 * cached) continue;
+            if (us >= limit) continue;
             const double t = split_tile_us(kSplitTileMemory, f.variant, m, n, k, sp, num_cu);
             if (t < best) {
                 best = t;
@@ -892,16 +899,19 @@ void select_config_uncached(int m, int n, int k, int num_cu, int stage, const st
     if ((stage & (kStageA | kStageB)) && num_cu == kTunedOnCUs && fewrows_ok(m, n) && any_tile_plan(m, n, k, num_cu, stage, &other) < t) *out = other;
     if (!hit && num_cu == kTunedOnCUs && !(stage & (kStageB | kNoSplitTiles)) && out->stream_k == RF_SCHEDULE_TILES &&
         !kVariants[out->variant].takes_any_shape() && long_k_range(m, n, k) && ceil_div(m, 256) * ceil_div(n, 256) <= num_cu) {
-        // The few-rows kernels again, 15 % below that figure of a plan of one K part (a tiled plan of long K has too low a `t` above). 121 shapes that change
-        // plan here, before against after: cached 6 % faster (geometric mean, 0.5 % slower at worst), from memory 9 % (0.1 %). us: 256 x 3824 x 2560
-        // 14.2 -> 12.6, 17.5 -> 13.1. At 8 % the slowest of 88 is 5.8 % slower (256 x 3616 x 2688). Not against plans with a K split: 128 x
-        // 7344 x 4608 18.1 (28, four parts), 22.0.
+        // The few-rows kernels again, against the cached figure of a plan of one K part (a tiled plan of long K has too low a `t` above). How far
+        // below it they have to be, by pairs of times: 28 at 0.85 25 pairs change, one is over 2 % slower (at 0.92 five of 37); 12 at 0.88 52 and
+        // one, at 0.93 89 and four; where rows of B are a multiple of 1024 bytes apart 12 takes up to 20 % longer than its figure: 46 and none,
+        // 7 % faster. 169 shapes that change plan here, before against after: cached 5 % faster (geometric mean; two by over 2 % slower, 4.3 % at
+        // worst), from memory 9 % (one, 2.6 %). us: 256 x 3824 x 2560 14.2 -> 12.6, 17.5 -> 13.1; 112 x 8192 x 2048 12.1 -> 10.2, 15.5 -> 12.6. Not
+        // against plans with a K split: 128 x 7344 x 4608 18.1 (28, four parts), 22.0.
         // (Variant 28's best plan, which tuner/fewrows_model.py knows, has to be behind as well.)
         const double tiled = split_tile_plan(m, n, k, num_cu, out);
         if (m <= kFewRowsMaxM && out->split_k == 1 && !(stage & kTiledOnly) && fewrows_ok(m, n)) {
             const double few = fewrows_plan(m, n, k, num_cu, false, &other);
-            const bool below_28 = split_28 == 1 ? few < 0.85 * split_tile_us(kSplitTileCached, 28, m, n, k, 1, num_cu) : few < 3.1 + 0.67 * cost_28;
-            if (few < 0.85 * tiled && below_28) *out = other;
+            const double share = out->variant == 28 ? 0.85 : out->variant == 12 && n % 1024 == 0 ? 1.0 : 0.88, share_28 = n % 1024 == 0 ? 1.0 : 0.85;
+            const bool below_28 = split_28 == 1 ? few < share_28 * split_tile_us(kSplitTileCached, 28, m, n, k, 1, num_cu) : few < 3.1 + 0.67 * cost_28;
+            if (few < share * tiled && below_28) *out = other;
         }
     }
 }
@@ -937,8 +947,8 @@ bool fewrows_split_fits(Mem &mem, const Variant &v, int m, int n, int k, int spl
 // The same of a tiled plan's K split: without memory for its sums the plan is the one that split_tile_plan found. mp: the rows that are
 // planned, m: those of c, stage: the plan's flags. In the static array, beside `staged` bytes of copies, that plan in the parts that fit
 // is weighed once more against the others that fit: 942 x 1904 x 6016, A staged, 37.5 us cached and 46.0 from memory (28, one part) -> 28.5 and
-// 32.4 (8, three parts instead of four of 10). 150 shapes whose plan does not fit, against the plan that split_tile_plan found: 11 % faster
-// cached (geometric mean), 16 % from memory, none slower by more than the 1 % that runs differ by.
+// 32.4 (8, three parts instead of four of 10). 150 shapes whose plan does not fit, against the plan that split_tile_plan found: 9 % faster
+// cached (geometric mean), 12 % from memory, one 2.7 % slower cached and the others within the 1 % that runs differ by.
 void fit_tile_split(State &s, Mem &mem, int m, int mp, int n, int k, int stage, size_t staged, rf_gemm_config *cfg) {
     if (cfg->variant < 0 || cfg->split_k == 1 || cfg->stream_k != RF_SCHEDULE_TILES || kVariants[cfg->variant].takes_any_shape()) return;
     const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, cfg->split_k));

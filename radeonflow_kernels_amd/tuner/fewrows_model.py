@@ -95,8 +95,9 @@ def tile_estimate(m, n, k, split, num_cu=256):
     return 3.1 + 0.67 * (t + (6.03 + 1.27e-6 * parts * m * n if parts > 1 else 0.0))
 
 
-# what part of the long-K estimate of a tiled plan of one K part the few-rows estimate has to stay below
-LONG_K_SHARE = 0.85
+def long_k_share(n):
+    """What part of the long-K estimate of variant 28's plan of one K part the few-rows estimate has to stay below."""
+    return 1.0 if n % 1024 == 0 else 0.85
 
 
 def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
@@ -115,7 +116,7 @@ def choice(m, n, k, num_cu=256, fit=None, common=COMMON, tiles=True):
             if s <= k // BK and tile_estimate(m, n, k, s, num_cu) < best[0]:
                 best = (tile_estimate(m, n, k, s, num_cu), 28, s)
         if best[1:] == (28, 1):
-            if m <= 512 and long_k.in_range(m, n, k, num_cu) and few[0] < LONG_K_SHARE * long_k.estimate(28, m, n, k, 1, long_k.CACHED):
+            if m <= 512 and long_k.in_range(m, n, k, num_cu) and few[0] < long_k_share(n) * long_k.estimate(28, m, n, k, 1, long_k.CACHED):
                 best = few
     return best[1:]
 

@@ -29,8 +29,6 @@ FITS = ({9: (0.0, 0.366, 0.0, 0.07, 0.028), 12: (0.185, 0.592, 0.147, 0.19, 0.05
 #   launch; per million outputs; per million bytes of A and B; K split, and per million sums
 COMMONS = ((4.531, 0.403, 0.0, 2.274, 1.177), (3.922, 0.531, 0.054, 2.283, 1.173))
 CACHED, MEMORY = 0, 1
-# what part of the estimate of the plan before another's has to stay below
-SHARES = (0.93, 0.94)
 SPLITS = (1, 2, 3, 4, 5, 6, 8)
 
 
@@ -68,12 +66,19 @@ def estimate(variant, m, n, k, split, where, num_cu=256):
     return sum(x * c for x, c in zip(own + shared, FITS[where][variant] + COMMONS[where]))
 
 
+def shares(first, variant, m):
+    """What part of the estimates of the plan before another's have to stay below."""
+    if variant == 9:
+        return (0.88 if first == 12 else 0.93), 0.94
+    return (0.93 if m <= 512 else 0.96 if first == 12 else 1.0), 0.94
+
+
 def replaced(first, m, n, k, most=float("inf")):
     """(variant, parts) that the planner takes in place of `first`, the plan of its first model, with sums of at most `most` bytes."""
     if first[0] not in TILES:
         return first
-    limits = [share * estimate(first[0], m, n, k, _parts(k, first[1]), w) for w, share in enumerate(SHARES)]
-    out = first
+    before = [estimate(first[0], m, n, k, _parts(k, first[1]), w) for w in (CACHED, MEMORY)]
+    best, out = float("inf"), first
     for v, (bm, bn) in TILES.items():
         if v == 28 and m <= 512:
             continue
@@ -82,9 +87,9 @@ def replaced(first, m, n, k, most=float("inf")):
                 continue
             if s > 1 and (_ceil(m, bm) * _ceil(n, bn) * s > 600 or m * n * s > 45e6 or 4 * m * n * s > most):
                 continue
-            us = estimate(v, m, n, k, s, MEMORY)
-            if estimate(v, m, n, k, s, CACHED) < limits[CACHED] and us < limits[MEMORY]:
-                limits[MEMORY], out = us, (v, s)
+            us = [estimate(v, m, n, k, s, w) for w in (CACHED, MEMORY)]
+            if us[MEMORY] < best and all(u < share * b for u, share, b in zip(us, shares(first[0], v, m), before)):
+                best, out = us[MEMORY], (v, s)
     return out
 
 

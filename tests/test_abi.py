@@ -438,11 +438,11 @@ def test_long_k_on_a_part_of_the_chip_is_split():
     import radeonflow_kernels_amd as rfk
     plan = lambda *a: (lambda c: (c.variant, c.split_k, c.stream_k))(rfk.plan_for(*a))
     assert plan(1232, 1616, 7552, 256) == plan(1228, 1616, 7552, 256) == (11, 4, 0)
-    assert plan(528, 4000, 8064, 256) == plan(527, 4000, 8064, 256) == (11, 4, 0) and plan(304, 1632, 2176, 256) == (9, 3, 0)
+    assert plan(544, 4096, 7168, 256) == plan(543, 4096, 7168, 256) == (10, 3, 0) and plan(304, 1632, 2176, 256) == (9, 3, 0)
     assert plan(1024, 1536, 7168, 256) == (28, 2, 0) and plan(1232, 1616, 7552, 304) == (28, 2, 0)
     assert plan(1232, 1608, 7552, 256) != (11, 4, 0) and plan(1232, 1616, 896, 256)[1] == 1 and plan(8192, 8192, 7168, 256)[1] == 1
     # the few-rows kernels where they are well below the tiled plan of one part, not against a K split
-    assert plan(256, 3824, 2560, 256) == (21, 1, 0) and plan(128, 7344, 4608, 256) == (28, 4, 0)
+    assert plan(256, 3824, 2560, 256) == plan(384, 2048, 2048, 256) == (21, 1, 0) and plan(128, 7344, 4608, 256) == (28, 4, 0)
 
 
 @pytest.mark.parametrize("shape,plan", [
@@ -494,7 +494,7 @@ def test_long_k_model_states_the_choice_of_the_launcher():
     every plan of its range that is not tabled is one that it would not replace."""
     import radeonflow_kernels_amd as rfk
     from radeonflow_kernels_amd.tuner import long_k_model as lk
-    for first, shape in (((28, 1), (1360, 1536, 7168)), ((28, 1), (528, 4000, 8064)), ((28, 1), (304, 1632, 2176)), ((12, 1), (80, 6352, 2816)),
+    for first, shape in (((28, 1), (1360, 1536, 7168)), ((28, 1), (544, 4096, 7168)), ((28, 1), (304, 1632, 2176)), ((12, 1), (848, 512, 3328)),
                          ((28, 1), (176, 7872, 5376)), ((28, 2), (160, 7968, 6656)), ((12, 1), (640, 1536, 3584)), ((12, 1), (1024, 1024, 4096)),
                          ((28, 8), (48, 4064, 7168))):
         got = rfk.plan_for(*shape, 256)

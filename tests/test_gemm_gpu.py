@@ -783,7 +783,7 @@ def test_k_split_inside_the_workgroup_on_random_shapes_equals_the_two_launch_for
 # K parts that divide the K blocks unevenly (17 in three), a single m-tile, odd rows (A staged); sums of 33.4 and 34.6 MiB beyond the 32 MiB
 # static array; sums that fit it alone but not beside a staged A (942 rows); the large ones against one K part. The sums are exact in any order: this
 # is a test of the bits, not of the plan that runs (test_static_entry_fits_a_long_k_plan_to_its_scratch_array tells which one does)
-@pytest.mark.parametrize("m,n,k,oracle", [(304, 1632, 2176, True), (45, 5504, 7296, True), (48, 7856, 2304, True), (1328, 1648, 7424, False),
+@pytest.mark.parametrize("m,n,k,oracle", [(304, 1632, 2176, True), (45, 5504, 7296, True), (48, 6912, 8064, True), (1328, 1648, 7424, False),
                                           (560, 3216, 7040, False), (942, 1904, 6016, False)])
 def test_split_tile_plans_in_both_entries(rfk, m, n, k, oracle):
     """Shapes that split_tile_plan moves to a K split: the bits of the oracle from the entry that allocates and from the one that cannot."""
