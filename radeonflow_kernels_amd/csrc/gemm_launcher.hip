@@ -710,7 +710,8 @@ bool long_k_range(int m, int n, int k) {
 // beyond them not (variant 28 0.91, 10 0.97, 11 1.0), 9 in place of 12 too low at any size, 1.04 to 1.08. Up to 512 rows 103 of 348 pairs
 // change at 0.93 and five are over 2 % slower (54 of 198 at 0.97), beyond 512 rows 247 of 415 and 13 at 1.0 (72 and one at 0.93). Of 62 pairs
 // with 9 in place of 12 eleven were slower at 0.93 and 1.0, up to 9.7 %, none of 21 at 0.88; of 56 with 28 in place of 12 three at 1.0 (1600 x
-// 384 x 3072 12.4 -> 13.6 us), one of 39 at 0.96.
+// 384 x 3072 12.4 -> 13.6 us), one of 39 at 0.96. Where rows of B are a multiple of 1024 bytes apart 12 takes up to 20 % longer than its figure:
+// 32 shapes that change there are 8 % faster, 1.7 % slower at worst (551 x 2048 x 4096 20.6 -> 18.8 us).
 double split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out, size_t most = SIZE_MAX) {
     const int qk = k / rf::BK, parts = ceil_div(qk, ceil_div(qk, out->split_k));
     const double cached = split_tile_us(kSplitTileCached, out->variant, m, n, k, parts, num_cu);
@@ -721,7 +722,7 @@ double split_tile_plan(int m, int n, int k, int num_cu, rf_gemm_config *out, siz
         // (up to 512 rows variant 28 in more parts is not tried: the few-rows kernels were weighed against its plan of the first model)
         if (f.variant == 28 && m <= kFewRowsMaxM) continue;
         const double tiles = (double)ceil_div(m, v.bm) * ceil_div(n, v.bn);
-        const double limit = (f.variant == 9 ? (first == 12 ? 0.88 : 0.93) : m <= kFewRowsMaxM ? 0.93 : first == 12 ? 0.96 : 1.0) * cached;
+        const double limit = (f.variant == 9 ? (first == 12 ? 0.88 : 0.93) : m <= kFewRowsMaxM ? 0.93 : first != 12 ? 1.0 : n % 1024 == 0 ? 1.06 : 0.96) * cached;
         for (int sp : {1, 2, 3, 4, 5, 6, 8}) {
             if (sp > qk || ceil_div(qk, ceil_div(qk, sp)) != sp || (v.k_groups > 1 && (sp > 1 || qk % v.k_groups != 0))) continue;
             if (sp == 1 && f.variant == 9) continue;

@@ -66,11 +66,11 @@ def estimate(variant, m, n, k, split, where, num_cu=256):
     return sum(x * c for x, c in zip(own + shared, FITS[where][variant] + COMMONS[where]))
 
 
-def shares(first, variant, m):
+def shares(first, variant, m, n):
     """What part of the estimates of the plan before another's have to stay below."""
     if variant == 9:
         return (0.88 if first == 12 else 0.93), 0.94
-    return (0.93 if m <= 512 else 0.96 if first == 12 else 1.0), 0.94
+    return (0.93 if m <= 512 else 1.0 if first != 12 else 1.06 if n % 1024 == 0 else 0.96), 0.94
 
 
 def replaced(first, m, n, k, most=float("inf")):
@@ -88,7 +88,7 @@ def replaced(first, m, n, k, most=float("inf")):
             if s > 1 and (_ceil(m, bm) * _ceil(n, bn) * s > 600 or m * n * s > 45e6 or 4 * m * n * s > most):
                 continue
             us = [estimate(v, m, n, k, s, w) for w in (CACHED, MEMORY)]
-            if us[MEMORY] < best and all(u < share * b for u, share, b in zip(us, shares(first[0], v, m), before)):
+            if us[MEMORY] < best and all(u < share * b for u, share, b in zip(us, shares(first[0], v, m, n), before)):
                 best, out = us[MEMORY], (v, s)
     return out
 
